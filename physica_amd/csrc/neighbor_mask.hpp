@@ -530,6 +530,56 @@ __device__ __forceinline__ bool masks_apply(const MaskView& m, uint32_t slot, ui
     return !crowded && __all(may) != 0;
 }
 
+// Tests the members of the 27 cells around (cx, cy, cz): test(s) says whether
+// the candidate with sorted index s is marked, emit(k, bits) takes stencil
+// slot k's mask (every slot, in order). Returns false if a cell holds more
+// than kMaskBits particles (its members beyond them are not tested). The
+// ranges of three cells and then four members are fetched together: with few
+// waves in flight the scan is a chain of loads.
+template <class Test, class Emit>
+__device__ __forceinline__ bool scan_stencil(const SortedGrid& g, int cx, int cy, int cz, Test&& test, Emit&& emit) {
+    constexpr uint32_t kTogether = 4;
+    bool complete = true;
+    uint32_t k = 0u;
+#pragma unroll 1
+    for (int ox = -1; ox <= 1; ++ox) {
+#pragma unroll 1
+        for (int oy = -1; oy <= 1; ++oy, k += 3u) {
+            const int X = cx + ox, Y = cy + oy;
+            const bool row = X >= 0 && X < static_cast<int>(g.cx) && Y >= 0 && Y < static_cast<int>(g.cy);
+            uint32_t first[3] = {0u, 0u, 0u}, last[3] = {0u, 0u, 0u};
+            if (row) {
+#pragma unroll
+                for (int z = 0; z < 3; ++z) {
+                    const int Z = cz + z - 1;
+                    const bool inside = Z >= 0 && Z < static_cast<int>(g.cz);
+                    const uint32_t c = cell_of(g, X, Y, inside ? Z : cz);
+                    first[z] = g.offsets[c];
+                    last[z] = inside ? g.offsets[c + 1u] : first[z];
+                }
+            }
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+                uint32_t end = last[z];
+                if (end - first[z] > kMaskBits) {
+                    complete = false;
+                    end = first[z] + kMaskBits;
+                }
+                uint32_t bits = 0u;
+                for (uint32_t s = first[z]; s < end; s += kTogether) {
+#pragma unroll
+                    for (uint32_t u = 0; u < kTogether; ++u) {
+                        const bool marked = test(min(s + u, end - 1u)) && s + u < end;
+                        bits |= marked ? 1u << (s + u - first[z]) : 0u;
+                    }
+                }
+                emit(k + static_cast<uint32_t>(z), bits);
+            }
+        }
+    }
+    return complete;
+}
+
 // Visits the candidates of particle i in the reference order: the marked
 // ones of its masks (copied to its LDS column) or every particle of the 27
 // cells around (cx, cy, cz).
@@ -664,19 +714,45 @@ __device__ __forceinline__ void visit_records(const SortedGrid& g, const MaskVie
 // the kept candidates of each stencil slot k are written as the mask
 // out[k * n + i] (every slot is written) like visit_and_mask. Crowded lanes
 // of a wave-shared cell write no masks (a crowded particle's masks are never
-// read). Returns false if a kept candidate lies beyond the first kMaskBits
-// particles of its cell.
-template <int kDepth, class Load, class Keep>
+// read). near(s) is keep()'s answer from the position alone (true also where the
+// distance is NaN): a lane that
+// has neither masks nor a crowded cell marks its candidates with it and
+// evaluates only the marked ones. Returns false if a kept candidate lies
+// beyond the first kMaskBits particles of its cell.
+template <int kDepth, class Near, class Load, class Keep>
 __device__ __forceinline__ bool visit_records_and_mask(const SortedGrid& g, const MaskView& m, bool masked,
                                                        uint32_t i, int cx, int cy, int cz, const int* delta,
                                                        uint16_t* column, uint32_t stride,
-                                                       uint16_t* __restrict__ out, uint32_t n, Load&& load,
-                                                       Keep&& keep) {
+                                                       uint16_t* __restrict__ out, uint32_t n, Near&& near,
+                                                       Load&& load, Keep&& keep) {
     uint32_t leader = 0u;
     const bool crowded = is_crowded(m, i);
     const bool shared = shared_crowded_cell(crowded, cell_of(g, cx, cy, cz), leader);
     bool complete = true;
-    if (!shared || !crowded) {
+    if (!masked && !crowded && m.crowded != nullptr) {
+        // mark first, then walk the marked candidates: of the 27 cells' 216
+        // candidates about 33 are kept, but in nearly every trip some lane of
+        // the wave keeps its own, so a walk that evaluates as it goes pays
+        // for the pair terms 216 times (12 uneven scenes stepped together,
+        // 0.9 M particles: lambda passes 318 -> 247 us, vorticity 368 -> 297)
+        uint32_t nonzero = 0u;
+        complete = scan_stencil(g, cx, cy, cz, near, [&](uint32_t k, uint32_t bits) {
+            out[static_cast<size_t>(k) * n + i] = static_cast<uint16_t>(bits);
+            column[k * stride] = static_cast<uint16_t>(bits);
+            nonzero |= bits != 0u ? 1u << k : 0u;
+        });
+        const uint32_t center = cell_of(g, cx, cy, cz);
+        if constexpr (kDepth == 0) {
+            walk_masked(g.offsets, center, delta, column, stride, nonzero,
+                        [&](uint32_t s) { (void)keep(load(s), s); });
+        } else {
+            using Record = decltype(load(0u));
+            walk_masked_prefetch<kDepth>(
+                g.offsets, center, delta, column, stride, nonzero, i,
+                [&](uint32_t s) { return Tagged<Record>{load(s), s}; },
+                [&](const Tagged<Record>& t) { (void)keep(t.r, t.s); });
+        }
+    } else if (!shared || !crowded) {
         if constexpr (kDepth == 0) {
             complete = visit_and_mask(g, m, masked, i, cx, cy, cz, delta, column, stride, out, n,
                                       [&](uint32_t s) { return keep(load(s), s); });

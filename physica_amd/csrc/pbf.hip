@@ -180,6 +180,10 @@ __global__ void __launch_bounds__(kBlock) pbf_lambda_kernel(LambdaArgs a, BatchV
         }
         return dot(d, d) < a.t_exact;
     };
+    auto near = [&](uint32_t s) {
+        const Float3 d = sub(p, load(a.pos, s));
+        return !(dot(d, d) >= a.t_exact);
+    };
     auto visit = [&](uint32_t s) { return pair(load(a.pos, s), a.m[s], s); };
     if (a.boundary.offsets != nullptr) {
         for_each_candidate(
@@ -192,7 +196,7 @@ __global__ void __launch_bounds__(kBlock) pbf_lambda_kernel(LambdaArgs a, BatchV
             });
     } else {
         const bool complete = visit_records_and_mask<kPbfWalkDepth<kBatch>>(
-            grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n,
+            grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n, near,
             [&](uint32_t s) { return PointMass{load(a.pos, s), a.m[s]}; },
             [&](const PointMass& c, uint32_t s) { return pair(c.x, c.m, s); });
         flag_incomplete(complete, mv, i, &a.exact_flags[kFlagOverflow]);
@@ -365,8 +369,12 @@ __global__ void __launch_bounds__(kBlock) pbf_vorticity_kernel(PostArgs a, Batch
         if (s != i) w = add(w, cross(sub(vq, v), spiky_gradient(d, a.h, a.spiky)));
         return dot(d, d) < a.t_exact;
     };
+    auto near = [&](uint32_t s) {
+        const Float3 d = sub(p, load(a.pos, s));
+        return !(dot(d, d) >= a.t_exact);
+    };
     const bool complete = visit_records_and_mask<kPbfWalkDepth<kBatch>>(
-        grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n,
+        grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n, near,
         [&](uint32_t s) { return PointVector{load(a.pos, s), load(a.vel, s)}; },
         [&](const PointVector& c, uint32_t s) { return pair(c.x, c.v, s); });
     flag_incomplete(complete, mv, i, &a.exact_flags[kFlagOverflow]);
