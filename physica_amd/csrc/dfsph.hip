@@ -134,6 +134,10 @@ DfsphSolver::DfsphSolver(const phx_domain_configuration* domain, const phx_dfsph
     const uint32_t predictions = tolerance > 0.0F ? 2u * config_.max_iterations + 1u
                                                   : config_.divergence_iterations + config_.density_iterations + 1u;
     masks_.allocate(n, predictions, domain_.config.support_radius);
+    if (boundary_.count() > 0u) {
+        exact_samples_.resize(static_cast<size_t>(kStencil) * n);
+        skin_samples_.resize(static_cast<size_t>(kStencil) * n);
+    }
     if (mode == PHX_MODE_FORWARD) {
         for (DeviceBuffer<float>* b : {&moved_, &moved_sorted_}) b->resize(n);
         cell_bound_.resize(domain_.cells);
@@ -141,7 +145,7 @@ DfsphSolver::DfsphSolver(const phx_domain_configuration* domain, const phx_dfsph
         fill_u32(stream_, taint_.data(), domain_.cells, 0u);
     }
     if (tolerance > 0.0F) {
-        tol_partials_.resize(static_cast<size_t>(pass_blocks(n)) * kWaves);  // one per projection wave
+        tol_partials_.resize(static_cast<size_t>(pass_blocks(n, pass_group(n, boundary_.count() > 0u))) * kWaves);  // one per projection wave
         tol_done_.resize(2u);
         PHX_HIP(hipHostMalloc(reinterpret_cast<void**>(&tol_host_), 4u * sizeof(uint32_t), hipHostMallocDefault));
         PHX_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&tol_host_device_), tol_host_, 0u));
@@ -219,7 +223,7 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
         gather.add(state.method.warm_density_pressure, p_den0);
     }
     // per-cell skins need the previous step's displacements
-    const bool cell_skins = !rec && have_moved_ && boundary_.count() == 0u;
+    const bool cell_skins = !rec && have_moved_;
     if (cell_skins) gather.add(moved_.data(), moved_sorted_.data());
     // stamps of this step's predicting passes: stamp_base_ + slot
     const uint32_t predictions = config_.density_error_tolerance > 0.0F ? 2u * config_.max_iterations + 1u
@@ -236,8 +240,7 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
             fill_f32(stream_, p_div0, n, 0.0F);
             fill_f32(stream_, p_den0, n, 0.0F);
         }
-        // boundary samples: every pass walks the full stencil
-        masks_.begin_step(stream_, boundary_.count() > 0u);
+        masks_.begin_step(stream_);
         // the mask pass marks unequal masses with this step's stamp
         if (++mass_stamp_ == 0u) {
             fill_u32(stream_, mass_state_.data(), 1u, 0u);
@@ -257,7 +260,9 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     }
     const SortedGrid grid = cache.neighborhood.grid();
     const BoundaryGrid boundary = cache.neighborhood.boundary();
-    const uint32_t blocks = pass_blocks(n);
+    const bool with_boundary = boundary_.count() > 0u;
+    const int group = pass_group(n, with_boundary);
+    const uint32_t blocks = pass_blocks(n, group);
 
     MaskDensityArgs ma{n,
                        constants_,
@@ -275,12 +280,15 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
                        masks_.flags(),
                        rho0};
     ma.crowded = crowded;
+    ma.cell = masks_.cells();
     if (cell_skins) ma.cell_bound = cell_bound_.data();
     ma.xt_div = xt_div_.data();
     ma.xt_den = xt_den_.data();
     ma.mass_state = mass_state_.data();
     ma.mass_stamp = mass_stamp_;
-    launch_mask_density<false>(profiler_, stream_, blocks, ma, kDfsphDensity);
+    ma.exact_samples = exact_samples_.data();
+    ma.skin_samples = skin_samples_.data();
+    launch_mask_density<false>(profiler_, stream_, ma, kDfsphDensity);
 
     ForceArgs fa{};
     fa.n = n;
@@ -307,6 +315,7 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     fa.boundary = boundary;
     fa.rest_density = rho0;
     fa.crowded = crowded;
+    fa.cell = masks_.cells();
     if (cell_skins) {
         fa.cell_bound = cell_bound_.data();
         fa.taint = taint_.data();
@@ -314,6 +323,7 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     if (!rec) fa.moved_out = moved_.data();
     fa.mass_state = mass_state_.data();
     fa.mass_stamp = mass_stamp_;
+    fa.exact_samples = exact_samples_.data();
     // prediction `slot` writes x* (recorded per slot) and, recorded, its collision bits
     auto set_slot = [&](uint32_t slot) {
         fa.slot = slot;
@@ -337,6 +347,8 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     pa.boundary = boundary;
     pa.rest_density = rho0;
     pa.crowded = crowded;
+    pa.cell = masks_.cells();
+    pa.skin_samples = skin_samples_.data();
     if (cell_skins) pa.taint = taint_.data();
     // update `it` of phase `phase` reads the x* of prediction `slot`
     auto set_update = [&](uint32_t phase, uint32_t it, uint32_t slot) {
@@ -370,7 +382,7 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
         fa.t2 = t_den_.data();
         fa.final_step = 0u;
         set_slot(slot);
-        launch_force<true, kDivPredict>(profiler_, stream_, blocks, fa, kDfsphForceInit);
+        launch_force<true, kDivPredict>(profiler_, stream_, group, fa, kDfsphForceInit);
         uint32_t executed[2] = {0u, 0u};
         for (uint32_t phase = 0; phase < 2u; ++phase) {
             uint32_t* done = tol_done_.data() + phase;
@@ -394,9 +406,9 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
                 set_update(phase, it, first_slot + it - 1u);
                 pa.cv = Convergence{tol_partials_.data(), done, rho0};
                 if (phase == 0u) {
-                    launch_projection(profiler_, stream_, blocks, pa, kDfsphProjectionDivergence, kProjectDivergence);
+                    launch_projection(profiler_, stream_, group, pa, kDfsphProjectionDivergence, kProjectDivergence);
                 } else {
-                    launch_projection(profiler_, stream_, blocks, pa, kDfsphProjectionDensity, kProjectDensity);
+                    launch_projection(profiler_, stream_, group, pa, kDfsphProjectionDensity, kProjectDensity);
                 }
                 converge_kernel<<<1, kConvergeBlock, 0, stream_>>>(tol_partials_.data(), blocks * kWaves, n,
                                                                    tolerance, it, max_it, done,
@@ -408,9 +420,9 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
                 fa.iteration = it;
                 fa.final_step = 0u;
                 if (phase == 0u) {
-                    launch_force<false, kDivAuto>(profiler_, stream_, blocks, fa, kDfsphForceDivergence);
+                    launch_force<false, kDivAuto>(profiler_, stream_, group, fa, kDfsphForceDivergence);
                 } else {
-                    launch_force<false, kDenPredict>(profiler_, stream_, blocks, fa, kDfsphForceDensity);
+                    launch_force<false, kDenPredict>(profiler_, stream_, group, fa, kDfsphForceDensity);
                 }
             };
             launch_iteration(1u);
@@ -445,23 +457,23 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     set_slot(slot);
     if (nd == 0u) {
         fa.final_step = ne == 0u ? 1u : 0u;
-        launch_force<true, kDivEnd>(profiler_, stream_, blocks, fa, kDfsphForceInit);
+        launch_force<true, kDivEnd>(profiler_, stream_, group, fa, kDfsphForceInit);
     } else {
         fa.final_step = 0u;
-        launch_force<true, kDivPredict>(profiler_, stream_, blocks, fa, kDfsphForceInit);
+        launch_force<true, kDivPredict>(profiler_, stream_, group, fa, kDfsphForceInit);
         pa.target = cache.densities.data();
         pa.relaxation = relax_div;
         pa.t = t_div_.data();
         pa.xt_out = xt_div_.data();
         for (uint32_t it = 1; it <= nd; ++it) {  // sph.cpp:580-587
             set_update(0u, it, slot);
-            launch_projection(profiler_, stream_, blocks, pa, kDfsphProjectionDivergence, kProjectDivergence);
+            launch_projection(profiler_, stream_, group, pa, kDfsphProjectionDivergence, kProjectDivergence);
             set_slot(++slot);
             if (it < nd) {
-                launch_force<false, kDivPredict>(profiler_, stream_, blocks, fa, kDfsphForceDivergence);
+                launch_force<false, kDivPredict>(profiler_, stream_, group, fa, kDfsphForceDivergence);
             } else {
                 fa.final_step = ne == 0u ? 1u : 0u;
-                launch_force<false, kDivEnd>(profiler_, stream_, blocks, fa, kDfsphForceDivergenceEnd);
+                launch_force<false, kDivEnd>(profiler_, stream_, group, fa, kDfsphForceDivergenceEnd);
             }
         }
     }
@@ -476,14 +488,16 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
     fa.warm_div_out = nullptr;
     for (uint32_t it = 1; it <= ne; ++it) {
         set_update(1u, it, slot);
-        launch_projection(profiler_, stream_, blocks, pa, kDfsphProjectionDensity, kProjectDensity);
+        launch_projection(profiler_, stream_, group, pa, kDfsphProjectionDensity, kProjectDensity);
         set_slot(++slot);
         fa.final_step = it == ne ? 1u : 0u;
-        launch_force<false, kDenPredict>(profiler_, stream_, blocks, fa, kDfsphForceDensity);
+        launch_force<false, kDenPredict>(profiler_, stream_, group, fa, kDfsphForceDensity);
     }
     if (rec) {
         PHX_HIP(hipMemcpyAsync(cache.mask_flags.data(), masks_.flags(), sizeof(uint32_t) * masks_.flag_count(),
                                hipMemcpyDeviceToDevice, stream_));
+        // the derivative passes walk the full stencil with samples
+        if (with_boundary) fill_u32(stream_, cache.mask_flags.data() + kFlagOverflow, 1u, 1u);
         cache.mask_limit2 = masks_.limit2();
         cache.step_index = step;
         cache.warm_start = warm;

@@ -143,7 +143,9 @@ class DfsphSolver {
     VecBuffer u_;
     DeviceBuffer<float> rho0_, relax_div_, relax_den_, p_div_, p_den_, t_div_, t_den_;
     MaskSet masks_;
-    // Per-cell skins (forward mode, no boundary samples): each particle's
+    // masks of the cells' boundary samples (a domain with samples)
+    DeviceBuffer<uint16_t> exact_samples_, skin_samples_;
+    // Per-cell skins (forward mode): each particle's
     // displacement in the last forward step (original order), its sorted
     // copy, the step's per-cell bounds, and the cells' taint stamps (one
     // stamp per predicting pass, never reused until the counter wraps).

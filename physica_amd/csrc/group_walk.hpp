@@ -1,0 +1,226 @@
+// Neighbour sums with a group of G lanes per particle.
+//
+// One lane per particle leaves most of the GPU idle below about 100,000
+// particles (1,024 SIMDs of 64 lanes), and a pass then lasts as long as one
+// lane's chain of some 40 candidates. Here G lanes (4 or 16) share a
+// particle: each evaluates the pair terms of every G-th candidate, and the
+// terms are then added one after the other, in the candidates' order, by
+// every lane of the group through DPP broadcasts. The additions are the same
+// as one lane's, in the same order, so the sums are equal bit for bit.
+//
+// A workgroup of kGroupBlock threads serves kGroupBlock / G particles in two
+// mappings:
+//   expand  thread t turns ceil(27 / G) stencil slots of particle t % P into
+//           sorted candidate indices in the particle's LDS list (P particles
+//           per workgroup); the slots of the G threads follow each other, so
+//           the list is in the reference order
+//   walk    lane t % G of particle t / G takes every G-th entry of that list
+#pragma once
+
+#include "neighbor_mask.hpp"
+
+namespace phx {
+
+constexpr uint32_t kGroupBlock = 256;
+// candidates listed at a time; a particle with more is served in rounds
+constexpr uint32_t kGroupList = 64;
+// list entries with this bit are boundary samples (the launch has fewer
+// particles and samples than that)
+constexpr uint32_t kSampleEntry = 0x80000000u;
+
+template <int G>
+constexpr uint32_t kGroupParticles = kGroupBlock / G;
+
+template <int G>
+struct GroupLds {
+    // the row stride puts the entries that a wave reads together in distinct banks
+    static constexpr uint32_t kStride = kGroupList + G;
+    uint32_t list[kGroupParticles<G> * kStride];
+    uint32_t counts[kGroupBlock];
+    uint32_t totals[kGroupParticles<G>];
+};
+
+// The value lane k of the caller's group holds.
+template <int G, int k>
+__device__ __forceinline__ float group_broadcast(float v) {
+    static_assert(G == 4 || G == 16, "groups are DPP quads or rows");
+    constexpr int control = G == 4 ? k * 0x55 : 0x150 + k;  // quad_perm:[k,k,k,k], row_newbcast:k
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), control, 0xf, 0xf, true));
+}
+
+// sum[f] + terms[f] of lane 0, then of lane 1, ... of the group.
+template <int G, int F, int k = 0>
+__device__ __forceinline__ void group_add(float (&sum)[F], const float (&terms)[F]) {
+#pragma unroll
+    for (int f = 0; f < F; ++f) sum[f] = sum[f] + group_broadcast<G, k>(terms[f]);
+    if constexpr (k + 1 < G) group_add<G, F, k + 1>(sum, terms);
+}
+
+// Walks entries 0 .. count - 1 of a group's list. load(entry) fetches an
+// entry's record (it must accept `fallback`), pair(record, entry, terms)
+// writes its terms, and fold(terms) adds every lane's to the sums (group_add);
+// -0, which adds nothing to any value, stands in where the last trip has no
+// entry. Records are fetched one trip ahead. The whole group calls this
+// together.
+template <int G, int F, class Load, class Pair, class Fold>
+__device__ __forceinline__ void group_walk_list(const uint32_t* row, uint32_t count, uint32_t fallback, Load&& load,
+                                                Pair&& pair, Fold&& fold) {
+    const uint32_t lane = threadIdx.x % G;
+    uint32_t entry = lane < count ? row[lane] : fallback;
+    auto record = load(entry);
+    for (uint32_t k = lane; k < count + lane; k += G) {
+        const uint32_t ahead = k + G < count ? row[k + G] : fallback;
+        const auto fetched = load(ahead);
+        asm volatile("" ::: "memory");
+        float terms[F];
+#pragma unroll
+        for (int f = 0; f < F; ++f) terms[f] = -0.0F;
+        if (k < count) pair(record, entry, terms);
+        fold(terms);
+        entry = ahead;
+        record = fetched;
+    }
+}
+
+// group_walk_list over every particle of the 27 cells around (cx, cy, cz),
+// and with sample_offsets each cell's boundary samples after its particles:
+// the walk of a particle whose candidates are not listed. Entry `skip` is
+// left out.
+template <int G, int F, class Load, class Pair, class Fold>
+__device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const uint32_t* sample_offsets, int cx, int cy,
+                                                   int cz, uint32_t skip, Load&& load, Pair&& pair, Fold&& fold) {
+    const uint32_t lane = threadIdx.x % G;
+    auto run = [&](uint32_t first, uint32_t last, uint32_t flag) {
+        for (uint32_t base = first; base < last; base += G) {
+            const uint32_t s = base + lane;
+            const uint32_t entry = (s < last ? s : base) | flag;
+            const auto record = load(entry);
+            float terms[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) terms[f] = -0.0F;
+            if (s < last && entry != skip) pair(record, entry, terms);
+            fold(terms);
+        }
+    };
+    for_each_cell(g, cx, cy, cz, [&](uint32_t c) {
+        run(g.offsets[c], g.offsets[c + 1u], 0u);
+        if (sample_offsets != nullptr) run(sample_offsets[c], sample_offsets[c + 1u], kSampleEntry);
+    });
+}
+
+// Lists the candidates of a workgroup's particles and walks them. slot(j, k,
+// first) returns the mask of the expanding thread's particle in stencil slot
+// k, the thread's j-th, and sets `first` to the sorted index of that cell's
+// first particle (an empty mask for a particle that is not listed); with
+// kSamples, sample_slot(j, k, first) does the same for the cell's boundary
+// samples.
+// run(row, count) walks a list; it is called once for each round of
+// kGroupList candidates. Every thread of the workgroup calls this together.
+template <int G, bool kSamples, class Slot, class SampleSlot, class Run>
+__device__ __forceinline__ void group_expand(GroupLds<G>& lds, Slot&& slot, SampleSlot&& sample_slot, Run&& run) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    const uint32_t particle = threadIdx.x % kParticles;
+    const uint32_t part = threadIdx.x / kParticles;
+    uint32_t bits[kSlots], first[kSlots];
+    [[maybe_unused]] uint32_t sample_bits[kSlots], sample_first[kSlots];
+    uint32_t mine = 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) {
+        const uint32_t k = part * kSlots + j;
+        bits[j] = 0u;
+        first[j] = 0u;
+        if (k < static_cast<uint32_t>(kStencil)) bits[j] = slot(j, k, first[j]);
+        mine += static_cast<uint32_t>(__popc(bits[j]));
+        if constexpr (kSamples) {
+            sample_bits[j] = 0u;
+            sample_first[j] = 0u;
+            if (k < static_cast<uint32_t>(kStencil)) sample_bits[j] = sample_slot(j, k, sample_first[j]);
+            mine += static_cast<uint32_t>(__popc(sample_bits[j]));
+        }
+    }
+    lds.counts[threadIdx.x] = mine;
+    __syncthreads();
+    uint32_t start = 0u, total = 0u;
+#pragma unroll
+    for (uint32_t v = 0; v < static_cast<uint32_t>(G); ++v) {
+        const uint32_t c = lds.counts[v * kParticles + particle];
+        start += v < part ? c : 0u;
+        total += c;
+    }
+    uint32_t* list = lds.list + particle * GroupLds<G>::kStride;
+    const uint32_t walked = threadIdx.x / G;
+    const uint32_t* row = lds.list + walked * GroupLds<G>::kStride;
+    for (uint32_t low = 0u;; low += kGroupList) {
+        uint32_t place = start - low;  // wraps below the round's first entry
+#pragma unroll
+        for (uint32_t j = 0; j < kSlots; ++j) {
+            for (uint32_t m = bits[j]; m != 0u; m &= m - 1u, ++place)
+                if (place < kGroupList) list[place] = first[j] + static_cast<uint32_t>(__builtin_ctz(m));
+            if constexpr (kSamples) {
+                for (uint32_t m = sample_bits[j]; m != 0u; m &= m - 1u, ++place)
+                    if (place < kGroupList)
+                        list[place] = (sample_first[j] + static_cast<uint32_t>(__builtin_ctz(m))) | kSampleEntry;
+            }
+        }
+        if (part == 0u) lds.totals[particle] = total;
+        __syncthreads();
+        const uint32_t all = lds.totals[walked];
+        run(row, min(all > low ? all - low : 0u, kGroupList));
+        if (__syncthreads_or(total > low + kGroupList ? 1 : 0) == 0) break;
+    }
+}
+
+// Cell-index offset of stencil slot k (fill_slot_deltas).
+__device__ __forceinline__ uint32_t slot_delta(const SortedGrid& g, uint32_t k) {
+    const int ox = static_cast<int>(k / 9u) - 1;
+    const int oy = static_cast<int>((k / 3u) % 3u) - 1;
+    const int oz = static_cast<int>(k % 3u) - 1;
+    return static_cast<uint32_t>(ox + (oz * static_cast<int>(g.cy) + oy) * static_cast<int>(g.cx));
+}
+
+// Slot k of particle i's stored masks, for group_expand: with drop_self the
+// particle's own bit is cleared.
+template <bool kDropSelf>
+__device__ __forceinline__ uint32_t stored_slot(const uint16_t* __restrict__ masks,
+                                                const uint32_t* __restrict__ offsets, uint32_t n, uint32_t i,
+                                                uint32_t cell, uint32_t k, uint32_t& first) {
+    uint32_t m = masks[static_cast<size_t>(k) * n + i];
+    if (m == 0u) return 0u;
+    first = offsets[cell];
+    if constexpr (kDropSelf) {
+        if (k == 13u) {
+            const uint32_t own = i - first;
+            m &= ~(own < kMaskBits ? 1u << own : 0u);
+        }
+    }
+    return m;
+}
+
+// The mask of the particles of cell `cell` with near(s), for a slot of a
+// particle that is not crowded and whose stored masks do not apply; `first`
+// is set as by stored_slot. Four members are tested together.
+template <class Near>
+__device__ __forceinline__ uint32_t scanned_slot(const SortedGrid& g, int x, int y, int z, uint32_t k, uint32_t& first,
+                                                 Near&& near) {
+    const int X = x + static_cast<int>(k / 9u) - 1;
+    const int Y = y + static_cast<int>((k / 3u) % 3u) - 1;
+    const int Z = z + static_cast<int>(k % 3u) - 1;
+    if (X < 0 || X >= static_cast<int>(g.cx) || Y < 0 || Y >= static_cast<int>(g.cy) || Z < 0 ||
+        Z >= static_cast<int>(g.cz))
+        return 0u;
+    const uint32_t c = cell_of(g, X, Y, Z);
+    first = g.offsets[c];
+    const uint32_t last = min(g.offsets[c + 1u], first + kMaskBits);
+    uint32_t bits = 0u;
+    for (uint32_t s = first; s < last; s += 4u) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const bool marked = near(min(s + u, last - 1u)) && s + u < last;
+            bits |= marked ? 1u << (s + u - first) : 0u;
+        }
+    }
+    return bits;
+}
+
+}  // namespace phx

@@ -34,6 +34,7 @@ void MaskSet::allocate(uint32_t n, uint32_t predicting_passes, float support_rad
     exact_.resize(static_cast<size_t>(kStencil) * n);
     skin_mask_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
+    cells_.resize(n);
     flag_count_ = kFlagDisplacement + predicting_passes;
     flags_.resize(flag_count_);
     flags_host_.resize(sizeof(uint32_t) * flag_count_ * kReadbacks);
@@ -45,7 +46,7 @@ void MaskSet::allocate(uint32_t n, uint32_t predicting_passes, float support_rad
 // whose read-back completed: twice the displacement (both particles of a
 // pair move) with a 30 % margin, in [0.02, 0.6] h. Older read-backs are
 // dropped.
-void MaskSet::begin_step(hipStream_t stream, bool full_stencil) {
+void MaskSet::begin_step(hipStream_t stream) {
     for (uint32_t back = 1; back <= kReadbacks; ++back) {
         const uint32_t k = (readback_next_ + kReadbacks - back) % kReadbacks;
         if (!readback_pending_[k] || hipEventQuery(readback_[k]) != hipSuccess) continue;
@@ -64,7 +65,6 @@ void MaskSet::begin_step(hipStream_t stream, bool full_stencil) {
         break;
     }
     fill_u32(stream, flags_.data(), flag_count_, 0u);
-    if (full_stencil) fill_u32(stream, flags_.data() + kFlagOverflow, 1u, 1u);
 }
 
 void MaskSet::end_step(hipStream_t stream) {

@@ -54,10 +54,8 @@ class MaskSet {
     // Masks of n particles and flags for `predicting_passes` displacement
     // slots (one per pass that writes predicted positions).
     void allocate(uint32_t n, uint32_t predicting_passes, float support_radius);
-    // Adopts the skin of the newest completed read-back, if any, and clears the flags;
-    // with full_stencil the step's masks are marked unusable (overflow), so
-    // every pass walks the whole 27-cell stencil.
-    void begin_step(hipStream_t stream, bool full_stencil = false);
+    // Adopts the skin of the newest completed read-back, if any, and clears the flags.
+    void begin_step(hipStream_t stream);
     // Enqueues the read-back of this step's displacement flags.
     void end_step(hipStream_t stream);
 
@@ -73,6 +71,9 @@ class MaskSet {
     uint32_t* flags() { return flags_.data(); }
     // per particle: walks the full stencil (written by the mask pass)
     uint8_t* crowded() { return crowded_.data(); }
+    // the grid cell of each particle (sorted order, written by the mask
+    // pass): later passes read 4 bytes instead of dividing by the cell size
+    uint32_t* cells() { return cells_.data(); }
 
   private:
     float h_ = 0.0F;
@@ -80,7 +81,7 @@ class MaskSet {
     uint32_t flag_count_ = 0;
     DeviceBuffer<uint16_t> exact_, skin_mask_;
     DeviceBuffer<uint8_t> crowded_;
-    DeviceBuffer<uint32_t> flags_;
+    DeviceBuffer<uint32_t> flags_, cells_;
     // A ring of read-backs: a step's copy may still be queued behind its
     // last pass when the next step starts (always so when the host waits
     // inside a step), so begin_step adopts the newest one that completed.

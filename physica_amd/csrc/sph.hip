@@ -48,93 +48,15 @@ struct WcsphForceArgs {
     const float* rest_density;      // rho0, for the boundary terms
     const float* boundary_tension;  // WCSPH boundary_surface_tension, for the boundary cohesion
     const uint8_t* crowded;         // per particle: walks the full stencil
+    const uint32_t* cell;           // MaskDensityArgs::cell
+    const uint16_t* exact_samples;  // MaskDensityArgs::exact_samples
 };
 
-// pressure_forward_kernel (common.cu:165-194), viscosity_forward_kernel
-// (wcsph.cu:136-174), surface_forward_kernel (wcsph.cu:306-339) as three
-// accumulators over one neighbour walk, then the sums of WCSPH::forward
-// (sph.cpp:219-222), external_forward_kernel (wcsph.cu:86-90) and
-// integrate_forward_kernel (common.cu:302-320). A boundary sample b, after
-// each cell's particles, adds the pressure term grad W (-rho0_i V_b p_i /
-// rho_i^2), on approach the artificial viscosity with
-// nu = mu_i h c_i / rho_i and mass rho0_i V_b, and within h the cohesion
-// -sigma_b,i rho0_i V_b W / m_i d (wcsph.cu:160-170, 326-335).
-__global__ void __launch_bounds__(kBlock) wcsph_force_kernel(WcsphForceArgs a) {
-    __shared__ uint16_t smask[kStencil * kBlock];
-    __shared__ int delta[kStencil];
-    fill_slot_deltas(a.grid, delta);
-    __syncthreads();
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.n) return;
-    const float h = a.kc.h;
-    const float4 self = a.xm[i];
-    const Float3 p = xyz(self);
-    const float4 vm = a.vmu[i];
-    const Float3 vel = xyz(vm);
-    const float4 own = a.aux[i];
-    const float rho_i = own.x;
-    const float t_i = own.y;
-    const float c_i = own.z;
-    const float sigma_i = own.w;
-    const float softening = 0.01F * h * h;
-    const float contact_weight = cubic_value(pair_distance(Float3{a.diameter, 0.0F, 0.0F}), a.kc);
-    Float3 ap{0.0F, 0.0F, 0.0F};
-    Float3 av{0.0F, 0.0F, 0.0F};
-    Float3 as{0.0F, 0.0F, 0.0F};
-    auto visit = [&](uint32_t s) {
-        if (s == i) return;
-        const float4 q = a.xm[s];
-        const float ms = q.w;
-        const Float3 d = sub(p, xyz(q));
-        const float dist = pair_distance(d);
-        const Float3 gradient = scale(d, cubic_gradient_factor(dist, a.kc));
-        const float4 other = a.aux[s];
-        ap = add(ap, scale(gradient, -ms * (t_i + other.y)));
-        const float4 vq = a.vmu[s];
-        const float compression = dot(sub(vel, xyz(vq)), d);
-        if (!(compression >= 0.0F)) {
-            const float alpha = 0.5F * (vm.w + vq.w);
-            const float speed = 0.5F * (c_i + other.z);
-            const float nu = 2.0F * alpha * h * speed / (rho_i + other.x);
-            const float pi_value = -nu * compression / (dot(d, d) + softening);
-            av = add(av, scale(gradient, -ms * pi_value));
-        }
-        if (!(dist >= h)) {
-            const float weight = dist > a.diameter ? cubic_value(dist, a.kc) : contact_weight;
-            const float factor = -sigma_i * ms * weight / self.w;
-            as = add(as, scale(d, factor));
-        }
-    };
-    int cx, cy, cz;
-    particle_cell(a.grid, p, cx, cy, cz);
-    if (a.boundary.offsets != nullptr) {
-        const float rest = a.rest_density[i];
-        const float tension = a.boundary_tension[i];
-        for_each_candidate(a.grid, a.boundary, cx, cy, cz, visit, [&](uint32_t s) {
-            const float4 b = a.boundary.x[s];
-            const Float3 d = sub(p, xyz(b));
-            const float dist = pair_distance(d);
-            const Float3 gradient = scale(d, cubic_gradient_factor(dist, a.kc));
-            ap = add(ap, scale(gradient, -rest * b.w * t_i));
-            const float compression = dot(sub(vel, xyz(a.boundary.v[s])), d);
-            if (!(compression >= 0.0F)) {
-                const float nu = vm.w * h * c_i / rho_i;
-                const float pi_value = -nu * compression / (dot(d, d) + softening);
-                av = add(av, scale(gradient, -rest * b.w * pi_value));
-            }
-            if (!(dist >= h)) {
-                const float weight = dist > a.diameter ? cubic_value(dist, a.kc) : contact_weight;
-                const float factor = -tension * rest * b.w * weight / self.w;
-                as = add(as, scale(d, factor));
-            }
-        });
-    } else if (a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u) {
-        uint16_t* column = smask + threadIdx.x;
-        const uint32_t nonzero = load_lane_column(a.exact, a.n, i, column, kBlock);
-        walk_masked(a.grid.offsets, cell_of(a.grid, cx, cy, cz), delta, column, kBlock, nonzero, visit);
-    } else {
-        for_each_candidate(a.grid, cx, cy, cz, visit);
-    }
+// The sums of WCSPH::forward (sph.cpp:219-222), external_forward_kernel
+// (wcsph.cu:86-90) and integrate_forward_kernel (common.cu:302-320) from
+// particle i's pressure, viscosity and surface accelerations.
+__device__ __forceinline__ void finish_wcsph(const WcsphForceArgs& a, uint32_t i, Float3 p, Float3 vel, Float3 ap,
+                                             Float3 av, Float3 as) {
     Float3 total = add(ap, av);
     total = add(total, as);
     total = add(total, add(a.gravity, load(a.u, i)));
@@ -144,6 +66,107 @@ __global__ void __launch_bounds__(kBlock) wcsph_force_kernel(WcsphForceArgs a) {
     const uint32_t j = a.perm[i];
     store(a.next_x, j, nx);
     store(a.next_v, j, nv);
+}
+
+// pressure_forward_kernel (common.cu:165-194), viscosity_forward_kernel
+// (wcsph.cu:136-174), surface_forward_kernel (wcsph.cu:306-339) as three
+// accumulators over one neighbour walk, then finish_wcsph. Always in groups:
+// the pair terms are long enough that four lanes beat one at any size
+// (16,000 particles 113 -> 63 us a step, 1,048,576: 614 -> 482 us, this pass
+// 325 -> 213 us).
+// With kSamples a boundary sample b, after each cell's particles, adds the pressure term
+// grad W (-rho0_i V_b p_i / rho_i^2), on approach the artificial viscosity
+// with nu = mu_i h c_i / rho_i and mass rho0_i V_b, and within h the cohesion
+// -sigma_b,i rho0_i V_b W / m_i d (wcsph.cu:160-170, 326-335).
+template <int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) wcsph_force_kernel(WcsphForceArgs a) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    constexpr int kSums = 9;
+    __shared__ GroupLds<G> lds;
+    const uint32_t base = xcd_block() * kParticles;
+    const uint32_t i = base + threadIdx.x % kParticles;
+    const bool usable = a.flags[kFlagOverflow] == 0u;
+    uint32_t center = 0u;
+    bool listed = false;
+    if (i < a.n) {
+        center = a.cell[i];
+        listed = usable && a.crowded[i] == 0u;
+    }
+    const uint32_t w = base + threadIdx.x / G;
+    const bool active = w < a.n;
+    const uint32_t own_index = active ? w : 0u;
+    const float h = a.kc.h;
+    const float4 self = a.xm[own_index];
+    const Float3 p = xyz(self);
+    const float4 vm = a.vmu[own_index];
+    const Float3 vel = xyz(vm);
+    const float4 own = a.aux[own_index];
+    const float rest = kSamples ? a.rest_density[own_index] : 0.0F;
+    const float tension = kSamples ? a.boundary_tension[own_index] : 0.0F;
+    const float softening = 0.01F * h * h;
+    const float contact_weight = cubic_value(pair_distance(Float3{a.diameter, 0.0F, 0.0F}), a.kc);
+    float sum[kSums] = {0.0F, 0.0F, 0.0F, 0.0F, 0.0F, 0.0F, 0.0F, 0.0F, 0.0F};
+    struct Record {
+        float4 q, v, aux;
+    };
+    auto fetch = [&](uint32_t entry) {
+        if constexpr (kSamples) {
+            if ((entry & kSampleEntry) != 0u) {
+                const uint32_t b = entry & ~kSampleEntry;
+                return Record{a.boundary.x[b], a.boundary.v[b], float4{}};
+            }
+        }
+        return Record{a.xm[entry], a.vmu[entry], a.aux[entry]};
+    };
+    auto put = [](float* terms, Float3 v) {
+        terms[0] = v.x;
+        terms[1] = v.y;
+        terms[2] = v.z;
+    };
+    auto pair = [&](const Record& r, uint32_t entry, float (&terms)[kSums]) {
+        const bool sample = kSamples && (entry & kSampleEntry) != 0u;
+        const Float3 d = sub(p, xyz(r.q));
+        const float dist = pair_distance(d);
+        const Float3 gradient = scale(d, cubic_gradient_factor(dist, a.kc));
+        put(terms, scale(gradient, sample ? -rest * r.q.w * own.y : -r.q.w * (own.y + r.aux.y)));
+        const float compression = dot(sub(vel, xyz(r.v)), d);
+        if (!(compression >= 0.0F)) {
+            const float alpha = 0.5F * (vm.w + r.v.w);
+            const float speed = 0.5F * (own.z + r.aux.z);
+            const float nu = sample ? vm.w * h * own.z / own.x : 2.0F * alpha * h * speed / (own.x + r.aux.x);
+            const float pi_value = -nu * compression / (dot(d, d) + softening);
+            put(terms + 3, scale(gradient, sample ? -rest * r.q.w * pi_value : -r.q.w * pi_value));
+        }
+        if (!(dist >= h)) {
+            const float weight = dist > a.diameter ? cubic_value(dist, a.kc) : contact_weight;
+            const float factor = sample ? -tension * rest * r.q.w * weight / self.w : -own.w * r.q.w * weight / self.w;
+            put(terms + 6, scale(d, factor));
+        }
+    };
+    auto fold = [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); };
+    group_expand<G, kSamples>(
+        lds,
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            return listed ? stored_slot<true>(a.exact, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first)
+                          : 0u;
+        },
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            return listed ? stored_slot<false>(a.exact_samples, a.boundary.offsets, a.n, i,
+                                               center + slot_delta(a.grid, k), k, first)
+                          : 0u;
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (active) group_walk_list<G, kSums>(row, count, w, fetch, pair, fold);
+        });
+    if (!active) return;
+    if (!usable || a.crowded[w] != 0u) {
+        int cx, cy, cz;
+        cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
+        group_walk_stencil<G, kSums>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, fetch, pair, fold);
+    }
+    if (threadIdx.x % G == 0u)
+        finish_wcsph(a, w, p, vel, Float3{sum[0], sum[1], sum[2]}, Float3{sum[3], sum[4], sum[5]},
+                     Float3{sum[6], sum[7], sum[8]});
 }
 
 }  // namespace
@@ -219,6 +242,10 @@ SphSolver::SphSolver(const phx_domain_configuration* domain, const phx_sph_confi
     // one displacement slot per predicting pass
     const uint32_t predictions = (tolerance > 0.0F ? config_.max_iterations : config_.pressure_iterations) + 1u;
     masks_.allocate(n, predictions, domain_.config.support_radius);
+    if (boundary_.count() > 0u) {
+        exact_samples_.resize(static_cast<size_t>(kStencil) * n);
+        skin_samples_.resize(static_cast<size_t>(kStencil) * n);
+    }
     if (mode == PHX_MODE_FORWARD && config_.method != PHX_SPH_WCSPH) {
         xt_.resize(n);
         mass_state_.resize(2u);
@@ -229,7 +256,7 @@ SphSolver::SphSolver(const phx_domain_configuration* domain, const phx_sph_confi
         fill_u32(stream_, taint_.data(), domain_.cells, 0u);
     }
     if (tolerance > 0.0F) {
-        tol_partials_.resize(static_cast<size_t>(pass_blocks(n)) * kWaves);  // one per projection wave
+        tol_partials_.resize(static_cast<size_t>(pass_blocks(n, pass_group(n, boundary_.count() > 0u))) * kWaves);  // one per projection wave
         tol_done_.resize(1u);
         tol_host_.resize(2u * sizeof(uint32_t));
         for (hipEvent_t& e : tol_events_) PHX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -389,11 +416,10 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
         PassScope scope(profiler_, stream_, kSphGrid);
         cache.neighborhood.build(stream_, domain_, step, cvec(state.particles.positions), nullptr, gather.get(),
                                  &boundary_);
-        masks_.begin_step(stream_, with_boundary);
+        masks_.begin_step(stream_);
     }
     const SortedGrid grid = cache.neighborhood.grid();
     const BoundaryGrid boundary = cache.neighborhood.boundary();
-    const uint32_t blocks = pass_blocks(n);
 
     MaskDensityArgs ma{};
     ma.n = n;
@@ -411,7 +437,10 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
     ma.pressures = cache.pressures.data();
     ma.aux = aux;
     ma.crowded = crowded;
-    launch_mask_density<true>(profiler_, stream_, blocks, ma, kSphDensity);
+    ma.cell = masks_.cells();
+    ma.exact_samples = exact_samples_.data();
+    ma.skin_samples = skin_samples_.data();
+    launch_mask_density<true>(profiler_, stream_, ma, kSphDensity);
 
     WcsphForceArgs wa{};
     wa.n = n;
@@ -435,14 +464,21 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
     wa.rest_density = rho0;
     wa.boundary_tension = btension;
     wa.crowded = crowded;
+    wa.cell = masks_.cells();
+    wa.exact_samples = exact_samples_.data();
     {
         PassScope scope(profiler_, stream_, kSphForces);
-        wcsph_force_kernel<<<blocks, kBlock, 0, stream_>>>(wa);
+        const int group = wide_group(n);
+        with_group(group, with_boundary, [&](auto g, auto samples) {
+            wcsph_force_kernel<g(), samples()><<<pass_blocks(n, group), kGroupBlock, 0, stream_>>>(wa);
+        });
         PHX_LAUNCH_CHECK();
     }
     if (rec) {
         PHX_HIP(hipMemcpyAsync(r->flags.data(), masks_.flags(), sizeof(uint32_t) * masks_.flag_count(),
                                hipMemcpyDeviceToDevice, stream_));
+        // the derivative passes walk the full stencil with samples
+        if (with_boundary) fill_u32(stream_, r->flags.data() + kFlagOverflow, 1u, 1u);
         r->step_index = step;
         r->recorded = true;
     }
@@ -469,7 +505,7 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     gather.add(relaxation, relax_.data());
     const bool with_boundary = boundary_.count() > 0u;
     // per-cell skins (DfsphSolver::forward_step) from the previous step's displacements
-    const bool cell_skins = have_moved_ && !with_boundary;
+    const bool cell_skins = have_moved_;
     if (cell_skins) gather.add(moved_.data(), moved_sorted_.data());
     const uint32_t predictions =
         (config_.density_error_tolerance > 0.0F ? config_.max_iterations : config_.pressure_iterations) + 1u;
@@ -481,7 +517,7 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
         PassScope scope(profiler_, stream_, kSphGrid);
         cache.neighborhood.build(stream_, domain_, step, cvec(state.particles.positions), nullptr, gather.get(),
                                  &boundary_);
-        masks_.begin_step(stream_, with_boundary);
+        masks_.begin_step(stream_);
         fill_f32(stream_, cache.pressures.data(), n, 0.0F);  // clear_iteration (sph.cpp:298)
         // the mask pass marks unequal masses with this step's stamp
         if (++mass_stamp_ == 0u) {
@@ -498,7 +534,8 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     }
     const SortedGrid grid = cache.neighborhood.grid();
     const BoundaryGrid boundary = cache.neighborhood.boundary();
-    const uint32_t blocks = pass_blocks(n);
+    const int group = pass_group(n, with_boundary);
+    const uint32_t blocks = pass_blocks(n, group);
 
     MaskDensityArgs ma{};
     ma.n = n;
@@ -513,10 +550,13 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     ma.rho = cache.densities.data();
     ma.flags = masks_.flags();
     ma.crowded = masks_.crowded();
+    ma.cell = masks_.cells();
+    ma.exact_samples = exact_samples_.data();
+    ma.skin_samples = skin_samples_.data();
     if (cell_skins) ma.cell_bound = cell_bound_.data();
     ma.mass_state = mass_state_.data();
     ma.mass_stamp = mass_stamp_;
-    launch_mask_density<false>(profiler_, stream_, blocks, ma, kSphDensity);
+    launch_mask_density<false>(profiler_, stream_, ma, kSphDensity);
 
     ForceArgs fa{};
     fa.n = n;
@@ -540,10 +580,12 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     fa.boundary = boundary;
     fa.rest_density = rho0_.data();
     fa.crowded = masks_.crowded();
+    fa.cell = masks_.cells();
     fa.moved_out = moved_.data();
     fa.xt1 = xt_.data();
     fa.mass_state = mass_state_.data();
     fa.mass_stamp = mass_stamp_;
+    fa.exact_samples = exact_samples_.data();
     if (cell_skins) {
         fa.cell_bound = cell_bound_.data();
         fa.taint = taint_.data();
@@ -570,6 +612,8 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     pa.boundary = boundary;
     pa.rest_density = rho0_.data();
     pa.crowded = masks_.crowded();
+    pa.cell = masks_.cells();
+    pa.skin_samples = skin_samples_.data();
     pa.xt_out = xt_.data();
     if (cell_skins) pa.taint = taint_.data();
     // the stamps of this step's predictions: stamp_base_ + slot
@@ -601,11 +645,11 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
         fill_u32(stream_, done, 1u, 0u);
         set_force_slot(0u);
         fa.final_step = 0u;
-        launch_force<true, kInitPredict>(profiler_, stream_, blocks, fa, kSphForceInit);
+        launch_force<true, kInitPredict>(profiler_, stream_, group, fa, kSphForceInit);
         auto launch_iteration = [&](uint32_t it) {
             set_projection_slot(it - 1u);  // the prediction of the previous pass
             pa.cv = Convergence{tol_partials_.data(), done, rho0_.data()};
-            launch_projection(profiler_, stream_, blocks, pa, kSphProjection, kProjectDensity);
+            launch_projection(profiler_, stream_, group, pa, kSphProjection, kProjectDensity);
             converge_kernel<<<1, kConvergeBlock, 0, stream_>>>(tol_partials_.data(), blocks * kWaves, n, tolerance,
                                                                it, max_it, done, host_device + (it & 1u));
             PHX_HIP(hipGetLastError());
@@ -614,7 +658,7 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
             fa.done = done;
             fa.iteration = it;
             fa.final_step = 0u;
-            launch_force<false, kDivPredict>(profiler_, stream_, blocks, fa, kSphForce);
+            launch_force<false, kDivPredict>(profiler_, stream_, group, fa, kSphForce);
         };
         launch_iteration(1u);
         uint32_t it = 1u;
@@ -636,13 +680,13 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     uint32_t slot = 0;  // displacement slot written by the latest predicting pass
     set_force_slot(slot);
     fa.final_step = iterations == 0u ? 1u : 0u;
-    launch_force<true, kInitPredict>(profiler_, stream_, blocks, fa, kSphForceInit);
+    launch_force<true, kInitPredict>(profiler_, stream_, group, fa, kSphForceInit);
     for (uint32_t it = 1; it <= iterations; ++it) {  // sph.cpp:300-307 / 413-420
         set_projection_slot(slot);
-        launch_projection(profiler_, stream_, blocks, pa, kSphProjection, kProjectDensity);
+        launch_projection(profiler_, stream_, group, pa, kSphProjection, kProjectDensity);
         set_force_slot(++slot);
         fa.final_step = it == iterations ? 1u : 0u;
-        launch_force<false, kDivPredict>(profiler_, stream_, blocks, fa, kSphForce);
+        launch_force<false, kDivPredict>(profiler_, stream_, group, fa, kSphForce);
     }
     end_step();
 }

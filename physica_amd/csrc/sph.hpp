@@ -130,6 +130,8 @@ class SphSolver {
     KernelConstants constants_{};
     PassProfiler profiler_;
     MaskSet masks_;
+    // masks of the cells' boundary samples (a domain with samples)
+    DeviceBuffer<uint16_t> exact_samples_, skin_samples_;
     // per-cell skins of the forward PCISPH/IISPH step (as DfsphSolver's):
     // last displacements (original order), their sorted copy, the per-cell
     // bounds and the cells' taint stamps

@@ -10,8 +10,11 @@
 #pragma once
 
 #include "engine.hpp"
+#include "group_walk.hpp"
 #include "neighbor_mask.hpp"
 #include "profiler.hpp"
+
+#include <type_traits>
 
 namespace phx {
 namespace {
@@ -22,6 +25,15 @@ constexpr uint32_t kBlock = 256;
 constexpr uint32_t kWaves = kBlock / 64;  // waves of a pass workgroup
 // candidates a masked walk fetches ahead of the one it processes
 constexpr int kWalkDepth = 2;
+// Particle counts up to which 16 and 4 lanes share a particle. More lanes
+// shorten a pass that does not fill the GPU and add work (listing the
+// candidates, idle lanes in a particle's last trip) to one that does. DFSPH
+// steps of 4 + 6 iterations, us, with 1 / 4 / 16 lanes: 2,000 particles
+// 419 / 278 / 194, 16,000 476 / 303 / 270, 32,000 432 / 297 / 346, 64,000
+// 458 / 379 / 501, 130,000 529 / 613 / 829, 1,048,576 3,071 / 3,309 / 5,780;
+// IISPH and PCISPH cross at the same counts.
+constexpr uint32_t kGroup16Particles = 20000;
+constexpr uint32_t kGroup4Particles = 90000;
 
 // Marks the 27 cells around (cx, cy, cz) with `stamp` (plain stores: every
 // writer writes the same value).
@@ -72,6 +84,7 @@ struct MaskDensityArgs {
     // per particle: set where a stencil cell holds more than kMaskBits
     // particles (that particle walks the full stencil in every pass)
     uint8_t* crowded;
+    uint32_t* cell;  // out: the grid cell of each particle
     // per cell: a bound on how far its particles move this step; non-null:
     // the skin mask keeps a pair while d2 < (h + B_ci + B_cj)^2 (plus a
     // rounding margin) instead of d2 < t_skin
@@ -85,65 +98,15 @@ struct MaskDensityArgs {
     // particle whose mass has other bits
     uint32_t* mass_state = nullptr;
     uint32_t mass_stamp = 0u;
+    // masks of the cells' boundary samples, as exact and skin (a launch with
+    // samples)
+    uint16_t* exact_samples = nullptr;
+    uint16_t* skin_samples = nullptr;
 };
 
-// Mask build, then density_forward_kernel (density.cu:18-40, cubic kernel,
-// topology = positions) over the exact mask and the first_term p/rho^2 of
-// pressure_forward_kernel (common.cu:171) for the given pressures, or with
-// kEos the Tait pressure of eos_forward_kernel (wcsph.cu:92-100) and its
-// first_term. With boundary samples no masks are built (the host marks the
-// step's masks unusable) and the density walks the full stencil, each cell's
-// samples b after its particles adding rho0_i V_b W (density.cu:34-37). A
-// particle with a stencil cell of more than kMaskBits particles is marked
-// crowded and walks the full stencil here and in every later pass.
+// What the mask pass writes for particle i at p with density `result`.
 template <bool kEos>
-__global__ void __launch_bounds__(kBlock) mask_density_kernel(MaskDensityArgs a) {
-    __shared__ uint16_t smask[kStencil * kBlock];
-    __shared__ int delta[kStencil];
-    fill_slot_deltas(a.grid, delta);
-    __syncthreads();
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.n) return;
-    uint16_t* column = smask + threadIdx.x;
-    const float4 self = a.xm[i];
-    const Float3 p = xyz(self);
-    if (a.mass_state != nullptr) {
-        const uint32_t bits = __float_as_uint(self.w);
-        if (i == 0u) a.mass_state[1] = bits;
-        if (bits != __float_as_uint(a.xm[0].w)) a.mass_state[0] = a.mass_stamp;  // one value for every writer
-    }
-    int cx, cy, cz;
-    particle_cell(a.grid, p, cx, cy, cz);
-    uint32_t nonzero = 0u;
-    float result = 0.0F;
-    if (a.boundary.offsets != nullptr) {
-        a.crowded[i] = 1u;  // no masks are built with boundary samples
-        const float rest = a.rest_density[i];
-        for_each_candidate(
-            a.grid, a.boundary, cx, cy, cz,
-            [&](uint32_t s) {
-                const float4 q = a.xm[s];
-                result += q.w * cubic_value(pair_distance(sub(p, xyz(q))), a.kc);
-            },
-            [&](uint32_t s) {
-                const float4 b = a.boundary.x[s];
-                result += rest * b.w * cubic_value(pair_distance(sub(p, xyz(b))), a.kc);
-            });
-    } else if (build_masks(a.grid, a.xm, a.n, i, p, cx, cy, cz, a.kc.sqrt_support, a.t_skin, a.exact, a.skin, column,
-                           kBlock, &nonzero, a.cell_bound, a.kc.h)) {
-        a.crowded[i] = 0u;
-        walk_masked(a.grid.offsets, cell_of(a.grid, cx, cy, cz), delta, column, kBlock, nonzero, [&](uint32_t s) {
-            const float4 q = a.xm[s];
-            const float dist = pair_distance(sub(p, xyz(q)));
-            result += q.w * cubic_value(dist, a.kc);
-        });
-    } else {
-        a.crowded[i] = 1u;
-        for_each_candidate(a.grid, cx, cy, cz, [&](uint32_t s) {
-            const float4 q = a.xm[s];
-            result += q.w * cubic_value(pair_distance(sub(p, xyz(q))), a.kc);
-        });
-    }
+__device__ __forceinline__ void write_density(const MaskDensityArgs& a, uint32_t i, Float3 p, float result) {
     a.rho[i] = result;
     if constexpr (kEos) {
         const float4 aux = a.aux[i];
@@ -166,6 +129,166 @@ __global__ void __launch_bounds__(kBlock) mask_density_kernel(MaskDensityArgs a)
             if (a.xt_den != nullptr) a.xt_den[i] = make_float4(p.x, p.y, p.z, t);
         }
     }
+}
+
+// Notes particle i's mass in the step's mass state (MaskDensityArgs::mass_state).
+__device__ __forceinline__ void note_mass(const MaskDensityArgs& a, uint32_t i, float mass) {
+    if (a.mass_state == nullptr) return;
+    const uint32_t bits = __float_as_uint(mass);
+    if (i == 0u) a.mass_state[1] = bits;
+    if (bits != __float_as_uint(a.xm[0].w)) a.mass_state[0] = a.mass_stamp;  // one value for every writer
+}
+
+// Mask build, then density_forward_kernel (density.cu:18-40, cubic kernel,
+// topology = positions) over the exact mask and the first_term p/rho^2 of
+// pressure_forward_kernel (common.cu:171) for the given pressures, or with
+// kEos the Tait pressure of eos_forward_kernel (wcsph.cu:92-100) and its
+// first_term. A particle with a stencil cell of more than kMaskBits
+// particles is marked crowded and walks the full stencil here and in every
+// later pass. The expanding threads build the masks, each for its own stencil
+// slots, so a particle's 27 cells are scanned by G threads at once: one lane
+// per particle scanned them in turn, a chain of loads that took 50 us however
+// few the particles (3,315 particles: 49 -> 8 us with 16 lanes; 64,000:
+// 50 -> 19 us with four; 1,048,576: 206 -> 181 us). With kSamples the cells'
+// boundary samples get masks of their own (a sample moves with the step, not
+// within it, so its skin covers the particle's displacement alone), and each
+// cell's samples b add rho0_i V_b W after its particles (density.cu:34-37).
+template <bool kEos, int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityArgs a) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    __shared__ GroupLds<G> lds;
+    __shared__ uint32_t crowd[kParticles];
+    const uint32_t base = xcd_block() * kParticles;
+    const uint32_t expanded = threadIdx.x % kParticles;
+    const uint32_t part = threadIdx.x / kParticles;
+    const uint32_t i = base + expanded;
+    const bool valid = i < a.n;
+    if (threadIdx.x < kParticles) crowd[threadIdx.x] = 0u;
+    __syncthreads();
+    Float3 p{0.0F, 0.0F, 0.0F};
+    uint32_t first[kSlots], last[kSlots];
+    [[maybe_unused]] uint32_t sample_first[kSlots], sample_last[kSlots];
+    [[maybe_unused]] float bound_i = 0.0F;
+    float bound[kSlots];
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) {
+        first[j] = last[j] = 0u;
+        bound[j] = 0.0F;
+        if constexpr (kSamples) sample_first[j] = sample_last[j] = 0u;
+    }
+    if (valid) {
+        const float4 self = a.xm[i];
+        p = xyz(self);
+        if (part == 0u) note_mass(a, i, self.w);
+        int cx, cy, cz;
+        particle_cell(a.grid, p, cx, cy, cz);
+        const uint32_t center = cell_of(a.grid, cx, cy, cz);
+        if (part == 0u) a.cell[i] = center;
+        if (a.cell_bound != nullptr) bound_i = a.cell_bound[center];
+        bool crowded = false;
+#pragma unroll
+        for (uint32_t j = 0; j < kSlots; ++j) {
+            const uint32_t k = part * kSlots + j;
+            const int X = cx + static_cast<int>(k / 9u) - 1;
+            const int Y = cy + static_cast<int>((k / 3u) % 3u) - 1;
+            const int Z = cz + static_cast<int>(k % 3u) - 1;
+            if (k >= static_cast<uint32_t>(kStencil) || X < 0 || X >= static_cast<int>(a.grid.cx) || Y < 0 ||
+                Y >= static_cast<int>(a.grid.cy) || Z < 0 || Z >= static_cast<int>(a.grid.cz))
+                continue;
+            const uint32_t c = cell_of(a.grid, X, Y, Z);
+            first[j] = a.grid.offsets[c];
+            last[j] = a.grid.offsets[c + 1u];
+            if (a.cell_bound != nullptr) bound[j] = a.cell_bound[c];
+            if constexpr (kSamples) {
+                sample_first[j] = a.boundary.offsets[c];
+                sample_last[j] = a.boundary.offsets[c + 1u];
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kSlots; ++j) {
+            crowded = crowded || last[j] - first[j] > kMaskBits;
+            if constexpr (kSamples) crowded = crowded || sample_last[j] - sample_first[j] > kMaskBits;
+        }
+        if (crowded) crowd[expanded] = 1u;
+    }
+    // the exact mask of members from .. to - 1 at positions x[s], their skin
+    // mask in `skin`; four members are fetched together
+    auto mark = [&](const float4* x, uint32_t from, uint32_t to, float t_skin, uint32_t& skin) {
+        uint32_t exact = 0u;
+        skin = 0u;
+        const uint32_t end = min(to, from + kMaskBits);
+        for (uint32_t s = from; s < end; s += 4u) {
+            float4 q[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) q[u] = x[min(s + u, end - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const Float3 d = sub(p, xyz(q[u]));
+                const float d2 = dot(d, d);
+                const uint32_t bit = s + u < end ? 1u << (s + u - from) : 0u;
+                exact |= d2 < a.kc.sqrt_support ? bit : 0u;
+                skin |= d2 < t_skin ? bit : 0u;
+            }
+        }
+        return exact;
+    };
+    // the threshold of pairs within h after moving up to `reach` together
+    // (the relative margin covers rounding), or the step's global one
+    auto threshold = [&](float reach) {
+        if (a.cell_bound == nullptr) return a.t_skin;
+        const float radius = a.kc.h + reach;
+        return radius * radius * (1.0F + 2e-5F);
+    };
+    auto slot = [&](uint32_t j, uint32_t k, uint32_t& start) {
+        if (!valid) return 0u;
+        start = first[j];
+        uint32_t skin;
+        const uint32_t exact = mark(a.xm, first[j], last[j], threshold(bound_i + bound[j]), skin);
+        a.exact[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(exact);
+        a.skin[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
+        return exact;
+    };
+    auto sample_slot = [&](uint32_t j, uint32_t k, uint32_t& start) {
+        if constexpr (kSamples) {
+            if (!valid) return 0u;
+            start = sample_first[j];
+            uint32_t skin;
+            const uint32_t exact = mark(a.boundary.x, sample_first[j], sample_last[j], threshold(bound_i), skin);
+            a.exact_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(exact);
+            a.skin_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
+            return exact;
+        }
+        return 0u;
+    };
+    const uint32_t walked = threadIdx.x / G;
+    const uint32_t w = base + walked;
+    const bool active = w < a.n;
+    const float4 own = a.xm[active ? w : 0u];
+    const float rest = kSamples && active ? a.rest_density[w] : 0.0F;
+    float sum[1] = {0.0F};
+    auto fetch = [&](uint32_t entry) {
+        if constexpr (kSamples) {
+            if ((entry & kSampleEntry) != 0u) return a.boundary.x[entry & ~kSampleEntry];
+        }
+        return a.xm[entry];
+    };
+    auto pair = [&](float4 q, uint32_t entry, float (&terms)[1]) {
+        const float weight = cubic_value(pair_distance(sub(xyz(own), xyz(q))), a.kc);
+        terms[0] = kSamples && (entry & kSampleEntry) != 0u ? rest * q.w * weight : q.w * weight;
+    };
+    auto fold = [&](const float (&terms)[1]) { group_add<G, 1>(sum, terms); };
+    group_expand<G, kSamples>(lds, slot, sample_slot, [&](const uint32_t* row, uint32_t count) {
+        if (active && crowd[walked] == 0u) group_walk_list<G, 1>(row, count, w, fetch, pair, fold);
+    });
+    if (valid && part == 0u) a.crowded[i] = static_cast<uint8_t>(crowd[expanded]);
+    if (!active) return;
+    if (crowd[walked] != 0u) {
+        int cx, cy, cz;
+        particle_cell(a.grid, xyz(own), cx, cy, cz);
+        group_walk_stencil<G, 1>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, fetch, pair, fold);
+    }
+    if (threadIdx.x % G == 0u) write_density<kEos>(a, w, xyz(own), sum[0]);
 }
 
 // Tolerance mode: the convergence state of a pressure phase. The projection
@@ -261,6 +384,7 @@ struct ProjectionArgs {
     BoundaryGrid boundary;     // offsets null: no boundary samples
     const float* rest_density;  // rho0, for the boundary terms
     const uint8_t* crowded;     // per particle: walks the full stencil
+    const uint32_t* cell;       // MaskDensityArgs::cell
     // per-cell skins: the skin mask applies to particle i unless its cell
     // holds `stamp` (a particle of a neighbouring cell moved past its cell's
     // bound in the prediction this pass reads); null: the global rule
@@ -268,7 +392,48 @@ struct ProjectionArgs {
     const uint32_t* taint = nullptr;
     uint32_t stamp = 0u;
     float4* xt_out = nullptr;  // optional: (x, y, z, t) per particle, the force pass's candidate record
+    const uint16_t* skin_samples = nullptr;  // MaskDensityArgs::skin_samples
 };
+
+// Whether the skin masks apply to particle i of cell `cell` in this pass.
+__device__ __forceinline__ bool projection_masked(const ProjectionArgs& a, uint32_t i, uint32_t cell) {
+    const bool moved_within = a.taint != nullptr
+                                  ? a.taint[cell] != a.stamp
+                                  : __uint_as_float(a.flags[kFlagDisplacement + a.slot]) <= a.limit2;
+    return a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u && moved_within;
+}
+
+// Whether a predicted position q can be within the support of p (a distance
+// that is NaN can, as its term is NaN).
+__device__ __forceinline__ bool projection_near(const ProjectionArgs& a, Float3 p, Float3 q) {
+    const Float3 d = sub(p, q);
+    return !(dot(d, d) >= a.kc.sqrt_support);
+}
+
+// The pressure update of particle i from its predicted density rs; returns
+// its compression error in tolerance mode.
+__device__ __forceinline__ double update_pressure(const ProjectionArgs& a, uint32_t i, float4 topology, float mass,
+                                                  float rs) {
+    const float rho = a.rho[i];
+    const float target = a.target[i];
+    const float volume = mass / a.volume_density[i];
+    const float delta_p = 1.0F / (2.0F * a.dt * a.dt * volume * volume * a.gradient_norm);
+    const float pressure = fmaxf(0.0F, a.p_prev[i] + a.relaxation[i] * delta_p * (rs - target));
+    a.p[i] = pressure;
+    const float t = pressure / (rho * rho);
+    a.t[i] = t;
+    if (a.xt_out != nullptr) a.xt_out[i] = make_float4(topology.x, topology.y, topology.z, t);
+    if (a.rs_out != nullptr) a.rs_out[i] = rs;
+    if (a.cv.partials == nullptr) return 0.0;
+    return fmax(0.0, static_cast<double>(rs) - static_cast<double>(target)) / static_cast<double>(a.cv.rest[i]);
+}
+
+// Adds the wave's errors and stores the sum; every lane of the wave calls it.
+__device__ __forceinline__ void store_wave_error(const ProjectionArgs& a, double error) {
+    double wave_error = error;
+    for (int offset = 32; offset > 0; offset >>= 1) wave_error += __shfl_xor(wave_error, offset, 64);
+    if ((threadIdx.x & 63u) == 0u) a.cv.partials[blockIdx.x * kWaves + (threadIdx.x >> 6)] = wave_error;
+}
 
 // The pressure phase a projection serves. The kernel is the same for both;
 // the two instantiations only give profiles one kernel name per phase.
@@ -292,57 +457,117 @@ __global__ void __launch_bounds__(kBlock) projection_kernel(ProjectionArgs a) {
     double error = 0.0;
     if (i < a.n) {
         const float4 topology = a.xm[i];
-        int cx, cy, cz;
-        particle_cell(a.grid, xyz(topology), cx, cy, cz);
-        const bool moved_within = a.taint != nullptr
-                                      ? a.taint[cell_of(a.grid, cx, cy, cz)] != a.stamp
-                                      : __uint_as_float(a.flags[kFlagDisplacement + a.slot]) <= a.limit2;
-        const bool masked =
-            a.flags[kFlagOverflow] == 0u && a.boundary.offsets == nullptr && a.crowded[i] == 0u && moved_within;
+        const uint32_t center = a.cell[i];
+        const bool crowded = a.flags[kFlagOverflow] != 0u || a.crowded[i] != 0u;
+        const bool masked = projection_masked(a, i, center);
         const float4 self = a.xs[i];
         const Float3 ps = xyz(self);
         float rs = 0.0F;
-        auto visit = [&](uint32_t s) {
-            const float4 q = a.xs[s];
-            rs += q.w * cubic_value(pair_distance(sub(ps, xyz(q))), a.kc);
-        };
-        if (masked) {
+        if (!crowded) {
             uint16_t* column = smask + threadIdx.x;
-            const uint32_t nonzero = load_lane_column(a.skin, a.n, i, column, kBlock);
+            uint32_t nonzero = 0u;
+            if (masked) {
+                nonzero = load_lane_column(a.skin, a.n, i, column, kBlock);
+            } else {
+                // moved past the skin: mark the candidates at the predicted
+                // positions, then walk those (scan_stencil)
+                int cx, cy, cz;
+                cell_coordinates(a.grid, center, cx, cy, cz);
+                scan_stencil(
+                    a.grid, cx, cy, cz, [&](uint32_t s) { return projection_near(a, ps, xyz(a.xs[s])); },
+                    [&](uint32_t k, uint32_t bits) {
+                        column[k * kBlock] = static_cast<uint16_t>(bits);
+                        nonzero |= bits != 0u ? 1u << k : 0u;
+                    });
+            }
             walk_masked_prefetch<kWalkDepth>(
-                a.grid.offsets, cell_of(a.grid, cx, cy, cz), delta, column, kBlock, nonzero, i,
+                a.grid.offsets, center, delta, column, kBlock, nonzero, i,
                 [&](uint32_t s) { return a.xs[s]; },
                 [&](float4 q) { rs += q.w * cubic_value(pair_distance(sub(ps, xyz(q))), a.kc); });
-        } else if (a.boundary.offsets != nullptr) {
-            // the predicted density's boundary terms rho0_i V_b W(x*_i - x_b)
-            const float rest = a.rest_density[i];
-            for_each_candidate(a.grid, a.boundary, cx, cy, cz, visit, [&](uint32_t s) {
-                const float4 b = a.boundary.x[s];
-                rs += rest * b.w * cubic_value(pair_distance(sub(ps, xyz(b))), a.kc);
-            });
         } else {
-            for_each_candidate(a.grid, cx, cy, cz, visit);
+            int cx, cy, cz;
+            cell_coordinates(a.grid, center, cx, cy, cz);
+            for_each_candidate(a.grid, cx, cy, cz, [&](uint32_t s) {
+                const float4 q = a.xs[s];
+                rs += q.w * cubic_value(pair_distance(sub(ps, xyz(q))), a.kc);
+            });
         }
-        const float rho = a.rho[i];
-        const float target = a.target[i];
-        const float volume = self.w / a.volume_density[i];
-        const float delta_p = 1.0F / (2.0F * a.dt * a.dt * volume * volume * a.gradient_norm);
-        const float pressure = fmaxf(0.0F, a.p_prev[i] + a.relaxation[i] * delta_p * (rs - target));
-        a.p[i] = pressure;
-        const float t = pressure / (rho * rho);
-        a.t[i] = t;
-        if (a.xt_out != nullptr) a.xt_out[i] = make_float4(topology.x, topology.y, topology.z, t);
-        if (a.rs_out != nullptr) a.rs_out[i] = rs;
-        if (tolerance)
-            error = fmax(0.0, static_cast<double>(rs) - static_cast<double>(target)) /
-                    static_cast<double>(a.cv.rest[i]);
+        error = update_pressure(a, i, topology, self.w, rs);
     }
-    if (tolerance) {
-        // every lane of the wave is here (no early return above)
-        double wave_error = error;
-        for (int offset = 32; offset > 0; offset >>= 1) wave_error += __shfl_xor(wave_error, offset, 64);
-        if ((threadIdx.x & 63u) == 0u) a.cv.partials[blockIdx.x * kWaves + (threadIdx.x >> 6)] = wave_error;
+    if (tolerance) store_wave_error(a, error);  // every lane of the wave is here (no early return above)
+}
+
+// projection_kernel with a group of G lanes per particle; with kSamples each
+// cell's boundary samples add rho0_i V_b W(x*_i - x_b) after its particles.
+template <int kPhase, int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(ProjectionArgs a) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    __shared__ GroupLds<G> lds;
+    const bool tolerance = a.cv.partials != nullptr;
+    if (tolerance && *a.cv.done != 0u) return;  // the phase ended at an earlier iteration
+    const uint32_t base = xcd_block() * kParticles;
+    const uint32_t i = base + threadIdx.x % kParticles;
+    const bool usable = a.flags[kFlagOverflow] == 0u;
+    uint32_t center = 0u;
+    bool listed = false, masked = false;
+    Float3 expanded{0.0F, 0.0F, 0.0F};
+    int cx = 0, cy = 0, cz = 0;
+    if (i < a.n) {
+        center = a.cell[i];
+        listed = usable && a.crowded[i] == 0u;
+        masked = projection_masked(a, i, center);
+        if (listed && !masked) {  // moved past the skin: marked at the predicted positions below
+            expanded = xyz(a.xs[i]);
+            cell_coordinates(a.grid, center, cx, cy, cz);
+        }
     }
+    const uint32_t w = base + threadIdx.x / G;
+    const bool active = w < a.n;
+    const float4 self = a.xs[active ? w : 0u];
+    const float rest = kSamples && active ? a.rest_density[w] : 0.0F;
+    float sum[1] = {0.0F};
+    auto fetch = [&](uint32_t entry) {
+        if constexpr (kSamples) {
+            if ((entry & kSampleEntry) != 0u) return a.boundary.x[entry & ~kSampleEntry];
+        }
+        return a.xs[entry];
+    };
+    auto pair = [&](float4 q, uint32_t entry, float (&terms)[1]) {
+        const float weight = cubic_value(pair_distance(sub(xyz(self), xyz(q))), a.kc);
+        terms[0] = kSamples && (entry & kSampleEntry) != 0u ? rest * q.w * weight : q.w * weight;
+    };
+    auto fold = [&](const float (&terms)[1]) { group_add<G, 1>(sum, terms); };
+    group_expand<G, kSamples>(
+        lds,
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            if (masked) return stored_slot<false>(a.skin, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first);
+            if (!listed) return 0u;
+            return scanned_slot(a.grid, cx, cy, cz, k, first,
+                                [&](uint32_t s) { return projection_near(a, expanded, xyz(a.xs[s])); });
+        },
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            if (masked)
+                return stored_slot<false>(a.skin_samples, a.boundary.offsets, a.n, i, center + slot_delta(a.grid, k), k,
+                                          first);
+            if (!listed) return 0u;
+            SortedGrid samples = a.grid;
+            samples.offsets = a.boundary.offsets;
+            return scanned_slot(samples, cx, cy, cz, k, first,
+                                [&](uint32_t s) { return projection_near(a, expanded, xyz(a.boundary.x[s])); });
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (active) group_walk_list<G, 1>(row, count, w, fetch, pair, fold);
+        });
+    double error = 0.0;
+    if (active) {
+        if (!usable || a.crowded[w] != 0u) {
+            cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
+            group_walk_stencil<G, 1>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, fetch, pair,
+                                     fold);
+        }
+        if (threadIdx.x % G == 0u) error = update_pressure(a, w, a.xm[w], self.w, sum[0]);
+    }
+    if (tolerance) store_wave_error(a, error);
 }
 
 enum Epilogue : int {
@@ -387,6 +612,7 @@ struct ForceArgs {
     BoundaryGrid boundary;      // offsets null: no boundary samples
     const float* rest_density;  // rho0, for the boundary pressure terms
     const uint8_t* crowded;     // per particle: walks the full stencil
+    const uint32_t* cell;       // MaskDensityArgs::cell
     // per-cell skins: a predicting pass marks the 27 cells around every
     // particle that moved farther than its cell's bound with `stamp`
     const float* cell_bound = nullptr;
@@ -401,16 +627,67 @@ struct ForceArgs {
     const float4* xt1 = nullptr;
     const uint32_t* mass_state = nullptr;
     uint32_t mass_stamp = 0u;
+    const uint16_t* exact_samples = nullptr;  // MaskDensityArgs::exact_samples
 };
+
+// What a force pass does with particle i's non-pressure acceleration `acc`
+// and pressure accelerations ap1, ap2 (the latter with `two`): the prediction
+// or next state. Returns the squared displacement of a prediction.
+template <bool kNonPressure, int kEpilogue>
+__device__ __forceinline__ float finish_force(const ForceArgs& a, uint32_t i, float4 self, Float3 vel, bool two,
+                                              uint32_t final_step, uint32_t cell, Float3 acc, Float3 ap1, Float3 ap2) {
+    const Float3 p = xyz(self);
+    if constexpr (kNonPressure) {
+        a.anp[i] = make_float4(acc.x, acc.y, acc.z, 0.0F);
+    } else {
+        acc = xyz(a.anp[i]);
+    }
+    Float3 total;
+    if constexpr (kEpilogue == kInitPredict) {
+        total = Float3{0.0F, 0.0F, 0.0F};
+    } else if constexpr (kEpilogue == kDenPredict) {
+        total = add(xyz(a.adiv[i]), ap1);
+    } else if (two) {
+        a.adiv[i] = make_float4(ap1.x, ap1.y, ap1.z, 0.0F);
+        total = add(ap1, ap2);
+    } else {
+        total = ap1;
+    }
+    Float3 nx, nv;
+    const Float3 a_total = add(acc, total);
+    predict_clamped(a.box, a.dt, p, vel, a_total, nx, nv);
+    if (a.collisions != nullptr)
+        a.collisions[i] = static_cast<uint8_t>(predict_collisions(a.box, a.dt, p, vel, a_total));
+    if (two && a.warm_div_out != nullptr) a.warm_div_out[a.perm[i]] = a.p_div[i];
+    const Float3 moved = sub(nx, p);
+    if (final_step != 0u) {
+        const uint32_t j = a.perm[i];
+        store(a.next_x, j, nx);
+        store(a.next_v, j, nv);
+        if (a.warm_den_out != nullptr) a.warm_den_out[j] = a.p_den[i];
+        if (a.moved_out != nullptr) a.moved_out[j] = sqrtf(dot(moved, moved));
+        return 0.0F;
+    }
+    a.xs[i] = make_float4(nx.x, nx.y, nx.z, self.w);
+    const float moved2 = dot(moved, moved);
+    if (a.taint != nullptr) {
+        const float bound = a.cell_bound[cell];
+        if (moved2 > bound * bound) {
+            int cx, cy, cz;
+            cell_coordinates(a.grid, cell, cx, cy, cz);
+            taint_neighbour_cells(a.grid, cx, cy, cz, a.taint, a.stamp);
+        }
+    }
+    return moved2;
+}
 
 // Pressure acceleration (pressure_forward_kernel, common.cu:165-194),
 // optionally fused with the non-pressure acceleration
 // (non_pressure_forward_kernel, common.cu:14-47), then the predict of the
 // next iteration (dfsph.cu:26-44) or, on the last pass, the next state.
 // cubic_gradient(d, h) is evaluated as f * d with f its radial factor, the
-// same operations as the reference's expression. Boundary samples add, after
-// each cell's particles, mu_i V_b lap W (v_b - v_i) (common.cu:38-43) and
-// grad W (-rho0_i V_b p_i / rho_i^2) (common.cu:185-190).
+// same operations as the reference's expression. Launches with boundary
+// samples go to the group kernel.
 template <bool kNonPressure, int kEpilogue>
 __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
     constexpr bool kAuto = kEpilogue == kDivAuto;
@@ -432,7 +709,7 @@ __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
     const bool active = i < a.n;
     float moved2 = 0.0F;
     if (active) {
-        const bool masked = a.flags[kFlagOverflow] == 0u && a.boundary.offsets == nullptr && a.crowded[i] == 0u;
+        const bool masked = a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u;
         const float4 self = a.xm[i];
         const Float3 p = xyz(self);
         const float4 vm = a.vmu[i];
@@ -444,8 +721,7 @@ __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
         if (kTwo) t2_i = a.t2[i];
         Float3 ap1{0.0F, 0.0F, 0.0F};
         Float3 ap2{0.0F, 0.0F, 0.0F};
-        int cx, cy, cz;
-        particle_cell(a.grid, p, cx, cy, cz);
+        const uint32_t center = a.cell[i];
         // candidates as (x, y, z, t1) records with one mass (uniform over the launch)
         const bool packed = kPressure && a.xt1 != nullptr && a.mass_state[0] != a.mass_stamp;
         const float mass = packed ? __uint_as_float(a.mass_state[1]) : 0.0F;
@@ -465,7 +741,6 @@ __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
         };
         if (masked) {
             uint16_t* column = smask + threadIdx.x;
-            const uint32_t center = cell_of(a.grid, cx, cy, cz);
             uint32_t nonzero = load_lane_column(a.exact, a.n, i, column, kBlock);
             nonzero = drop_self(i, a.grid.offsets[center], column, kBlock, nonzero);
             if (packed) {
@@ -522,94 +797,238 @@ __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
                 const Float3 d = sub(p, xyz(q));
                 pair(s, q, t1_s, t2_s, d, kPressure ? cubic_gradient_factor(pair_distance(d), a.kc) : 0.0F);
             };
-            if (a.boundary.offsets != nullptr) {
-                const float rest = a.rest_density[i];
-                for_each_candidate(a.grid, a.boundary, cx, cy, cz, visit, [&](uint32_t s) {
-                    const float4 b = a.boundary.x[s];
-                    const Float3 d = sub(p, xyz(b));
-                    if constexpr (kNonPressure) {
-                        const float weight = vm.w * b.w * viscosity_laplacian_c(d, a.kc);
-                        acc = add(acc, scale(sub(xyz(a.boundary.v[s]), vel), weight));
-                    }
-                    if constexpr (kPressure) {
-                        const Float3 gradient = scale(d, cubic_gradient_factor(pair_distance(d), a.kc));
-                        ap1 = add(ap1, scale(gradient, -rest * b.w * t1_i));
-                        if (kTwo) ap2 = add(ap2, scale(gradient, -rest * b.w * t2_i));
-                    }
-                });
-            } else {
-                for_each_candidate(a.grid, cx, cy, cz, visit);
-            }
+            int cx, cy, cz;
+            cell_coordinates(a.grid, center, cx, cy, cz);
+            for_each_candidate(a.grid, cx, cy, cz, visit);
         }
-        if constexpr (kNonPressure) {
-            a.anp[i] = make_float4(acc.x, acc.y, acc.z, 0.0F);
-        } else {
-            acc = xyz(a.anp[i]);
-        }
-        Float3 total;
-        if constexpr (kEpilogue == kInitPredict) {
-            total = Float3{0.0F, 0.0F, 0.0F};
-        } else if constexpr (kEpilogue == kDenPredict) {
-            total = add(xyz(a.adiv[i]), ap1);
-        } else if (kTwo) {
-            a.adiv[i] = make_float4(ap1.x, ap1.y, ap1.z, 0.0F);
-            total = add(ap1, ap2);
-        } else {
-            total = ap1;
-        }
-        Float3 nx, nv;
-        const Float3 a_total = add(acc, total);
-        predict_clamped(a.box, a.dt, p, vel, a_total, nx, nv);
-        if (a.collisions != nullptr)
-            a.collisions[i] = static_cast<uint8_t>(predict_collisions(a.box, a.dt, p, vel, a_total));
-        if (kTwo && a.warm_div_out != nullptr) a.warm_div_out[a.perm[i]] = a.p_div[i];
-        const Float3 moved = sub(nx, p);
-        if (final_step != 0u) {
-            const uint32_t j = a.perm[i];
-            store(a.next_x, j, nx);
-            store(a.next_v, j, nv);
-            if (a.warm_den_out != nullptr) a.warm_den_out[j] = a.p_den[i];
-            if (a.moved_out != nullptr) a.moved_out[j] = sqrtf(dot(moved, moved));
-        } else {
-            a.xs[i] = make_float4(nx.x, nx.y, nx.z, self.w);
-            moved2 = dot(moved, moved);
-            if (a.taint != nullptr) {
-                const float bound = a.cell_bound[cell_of(a.grid, cx, cy, cz)];
-                if (moved2 > bound * bound) taint_neighbour_cells(a.grid, cx, cy, cz, a.taint, a.stamp);
-            }
-        }
+        moved2 = finish_force<kNonPressure, kEpilogue>(a, i, self, vel, kTwo, final_step, center, acc, ap1, ap2);
     }
     if (final_step == 0u) block_max_to<kBlock>(moved2, &a.flags[kFlagDisplacement + a.slot]);
 }
 
+// force_kernel with a group of G lanes per particle. With kSamples the
+// boundary samples add, after each cell's particles, mu_i V_b lap W
+// (v_b - v_i) (common.cu:38-43) and grad W (-rho0_i V_b p_i / rho_i^2)
+// (common.cu:185-190).
+template <bool kNonPressure, int kEpilogue, int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) force_group_kernel(ForceArgs a) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    constexpr bool kAuto = kEpilogue == kDivAuto;
+    constexpr bool kPressure = kEpilogue != kInitPredict;
+    constexpr bool kMayTwo = kEpilogue == kDivEnd || kAuto;
+    // the sums: non-pressure, first pressure and second pressure acceleration
+    constexpr int kFirst = kNonPressure ? 3 : 0;
+    constexpr int kSecond = kFirst + (kPressure ? 3 : 0);
+    constexpr int kSums = kSecond + (kMayTwo ? 3 : 0);
+    __shared__ GroupLds<G> lds;
+    // the iteration that ends its phase (tolerance mode), uniform over the grid
+    const uint32_t ended = a.done != nullptr ? *a.done : 0u;
+    if (ended != 0u && ended < a.iteration) return;
+    const bool ends = ended != 0u && ended == a.iteration;
+    const bool two = kEpilogue == kDivEnd || (kAuto && ends);
+    const uint32_t final_step =
+        a.final_step != 0u || ((kEpilogue == kDenPredict || kEpilogue == kDivPredict) && ends) ? 1u : 0u;
+    const uint32_t base = xcd_block() * kParticles;
+    const uint32_t i = base + threadIdx.x % kParticles;
+    uint32_t center = 0u;
+    const bool usable = a.flags[kFlagOverflow] == 0u;
+    bool listed = false;
+    if (i < a.n) {
+        center = a.cell[i];
+        listed = usable && a.crowded[i] == 0u;
+    }
+    const uint32_t w = base + threadIdx.x / G;
+    const bool active = w < a.n;
+    const uint32_t own = active ? w : 0u;
+    const float4 self = a.xm[own];
+    const Float3 p = xyz(self);
+    const float4 vm = a.vmu[own];
+    const Float3 vel = xyz(vm);
+    const float t1_i = kPressure ? a.t1[own] : 0.0F;
+    const float t2_i = kMayTwo && two ? a.t2[own] : 0.0F;
+    const float rest = kSamples ? a.rest_density[own] : 0.0F;
+    // candidates as (x, y, z, t1) records with one mass (uniform over the launch)
+    const bool packed = kPressure && a.xt1 != nullptr && a.mass_state[0] != a.mass_stamp;
+    const float mass = packed ? __uint_as_float(a.mass_state[1]) : 0.0F;
+    float sum[kSums];
+#pragma unroll
+    for (int f = 0; f < kSums; ++f) sum[f] = 0.0F;
+    if constexpr (kNonPressure) {
+        const Float3 start = add(a.gravity, load(a.u, own));
+        sum[0] = start.x;
+        sum[1] = start.y;
+        sum[2] = start.z;
+    }
+    struct Record {
+        float4 q;  // position and mass, or a sample's volume
+        float t1, t2;
+        float4 v;  // velocity and viscosity
+        float rho;
+    };
+    auto fetch = [&](uint32_t entry) {
+        Record r{};
+        if constexpr (kSamples) {
+            if ((entry & kSampleEntry) != 0u) {
+                const uint32_t b = entry & ~kSampleEntry;
+                r.q = a.boundary.x[b];
+                if constexpr (kNonPressure) r.v = a.boundary.v[b];
+                return r;
+            }
+        }
+        if (packed) {
+            const float4 x = a.xt1[entry];
+            r.q = make_float4(x.x, x.y, x.z, mass);
+            r.t1 = x.w;
+        } else {
+            r.q = a.xm[entry];
+            if constexpr (kPressure) r.t1 = a.t1[entry];
+        }
+        if constexpr (kMayTwo) {
+            if (two) r.t2 = a.t2[entry];
+        }
+        if constexpr (kNonPressure) {
+            r.v = a.vmu[entry];
+            r.rho = a.rho[entry];
+        }
+        return r;
+    };
+    auto put = [](float* terms, Float3 v) {
+        terms[0] = v.x;
+        terms[1] = v.y;
+        terms[2] = v.z;
+    };
+    auto pair = [&](const Record& r, uint32_t entry, float (&terms)[kSums]) {
+        const Float3 d = sub(p, xyz(r.q));
+        const bool sample = kSamples && (entry & kSampleEntry) != 0u;
+        if constexpr (kNonPressure) {
+            const float laplacian = viscosity_laplacian_c(d, a.kc);
+            const float weight = sample ? vm.w * r.q.w * laplacian
+                                        : 0.5F * (vm.w + r.v.w) * r.q.w * laplacian / r.rho;
+            put(terms, scale(sub(xyz(r.v), vel), weight));
+        }
+        if constexpr (kPressure) {
+            const Float3 gradient = scale(d, cubic_gradient_factor(pair_distance(d), a.kc));
+            put(terms + kFirst, scale(gradient, sample ? -rest * r.q.w * t1_i : -r.q.w * (t1_i + r.t1)));
+            if constexpr (kMayTwo) {
+                if (two) put(terms + kSecond, scale(gradient, sample ? -rest * r.q.w * t2_i : -r.q.w * (t2_i + r.t2)));
+            }
+        }
+    };
+    auto fold = [&](const float (&terms)[kSums]) {
+        group_add<G, kSums>(sum, terms);
+    };
+    group_expand<G, kSamples>(
+        lds,
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            return listed ? stored_slot<true>(a.exact, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first)
+                          : 0u;
+        },
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            return listed ? stored_slot<false>(a.exact_samples, a.boundary.offsets, a.n, i,
+                                               center + slot_delta(a.grid, k), k, first)
+                          : 0u;
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (active) group_walk_list<G, kSums>(row, count, w, fetch, pair, fold);
+        });
+    float moved2 = 0.0F;
+    if (active) {
+        const uint32_t cell = a.cell[w];
+        if (!usable || a.crowded[w] != 0u) {
+            int cx, cy, cz;
+            cell_coordinates(a.grid, cell, cx, cy, cz);
+            group_walk_stencil<G, kSums>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, fetch, pair,
+                                         fold);
+        }
+        if (threadIdx.x % G == 0u) {
+            Float3 acc{0.0F, 0.0F, 0.0F}, ap1{0.0F, 0.0F, 0.0F}, ap2{0.0F, 0.0F, 0.0F};
+            if constexpr (kNonPressure) acc = Float3{sum[0], sum[1], sum[2]};
+            if constexpr (kPressure) ap1 = Float3{sum[kFirst], sum[kFirst + 1], sum[kFirst + 2]};
+            if constexpr (kMayTwo) ap2 = Float3{sum[kSecond], sum[kSecond + 1], sum[kSecond + 2]};
+            moved2 = finish_force<kNonPressure, kEpilogue>(a, w, self, vel, two, final_step, cell, acc, ap1, ap2);
+        }
+    }
+    if (final_step == 0u) block_max_to<kGroupBlock>(moved2, &a.flags[kFlagDisplacement + a.slot]);
+}
+
+// Lanes per particle of a pass that always runs in groups.
+inline int wide_group(uint32_t n) { return n <= kGroup16Particles ? 16 : 4; }
+
+// Lanes per particle of a projection or force pass (1: the kernels without
+// groups, which do not take boundary samples).
+inline int pass_group(uint32_t n, bool samples) { return samples || n <= kGroup4Particles ? wide_group(n) : 1; }
+
+// Whole workgroups of a launch with groups of `group` lanes, padded to a
+// multiple of the XCD count.
+inline uint32_t pass_blocks(uint32_t n, int group) {
+    return (blocks_for(n, kBlock / static_cast<uint32_t>(group)) + 7u) / 8u * 8u;
+}
+
+// Calls launch(std::integral_constant<int, G>, std::bool_constant<samples>)
+// for a launch with groups.
+template <class Launch>
+void with_group(int group, bool samples, Launch&& launch) {
+    if (group == 16) {
+        if (samples) {
+            launch(std::integral_constant<int, 16>{}, std::true_type{});
+        } else {
+            launch(std::integral_constant<int, 16>{}, std::false_type{});
+        }
+    } else {
+        if (samples) {
+            launch(std::integral_constant<int, 4>{}, std::true_type{});
+        } else {
+            launch(std::integral_constant<int, 4>{}, std::false_type{});
+        }
+    }
+}
+
 template <bool kNonPressure, int kEpilogue>
-void launch_force(PassProfiler& profiler, hipStream_t stream, uint32_t blocks, const ForceArgs& args, int pass) {
+void launch_force(PassProfiler& profiler, hipStream_t stream, int group, const ForceArgs& args, int pass) {
     PassScope scope(profiler, stream, pass);
-    force_kernel<kNonPressure, kEpilogue><<<blocks, kBlock, 0, stream>>>(args);
+    const uint32_t blocks = pass_blocks(args.n, group);
+    if (group == 1) {
+        force_kernel<kNonPressure, kEpilogue><<<blocks, kBlock, 0, stream>>>(args);
+    } else {
+        with_group(group, args.boundary.offsets != nullptr, [&](auto g, auto samples) {
+            force_group_kernel<kNonPressure, kEpilogue, g(), samples()><<<blocks, kGroupBlock, 0, stream>>>(args);
+        });
+    }
     PHX_LAUNCH_CHECK();
 }
 
-void launch_projection(PassProfiler& profiler, hipStream_t stream, uint32_t blocks, const ProjectionArgs& args,
-                       int pass, ProjectionPhase phase) {
+template <int kPhase>
+void launch_projection_phase(hipStream_t stream, int group, const ProjectionArgs& args) {
+    const uint32_t blocks = pass_blocks(args.n, group);
+    if (group == 1) {
+        projection_kernel<kPhase><<<blocks, kBlock, 0, stream>>>(args);
+    } else {
+        with_group(group, args.boundary.offsets != nullptr, [&](auto g, auto samples) {
+            projection_group_kernel<kPhase, g(), samples()><<<blocks, kGroupBlock, 0, stream>>>(args);
+        });
+    }
+}
+
+void launch_projection(PassProfiler& profiler, hipStream_t stream, int group, const ProjectionArgs& args, int pass,
+                       ProjectionPhase phase) {
     PassScope scope(profiler, stream, pass);
     if (phase == kProjectDivergence) {
-        projection_kernel<kProjectDivergence><<<blocks, kBlock, 0, stream>>>(args);
+        launch_projection_phase<kProjectDivergence>(stream, group, args);
     } else {
-        projection_kernel<kProjectDensity><<<blocks, kBlock, 0, stream>>>(args);
+        launch_projection_phase<kProjectDensity>(stream, group, args);
     }
     PHX_LAUNCH_CHECK();
 }
 
 template <bool kEos>
-void launch_mask_density(PassProfiler& profiler, hipStream_t stream, uint32_t blocks, const MaskDensityArgs& args,
-                         int pass) {
+void launch_mask_density(PassProfiler& profiler, hipStream_t stream, const MaskDensityArgs& args, int pass) {
     PassScope scope(profiler, stream, pass);
-    mask_density_kernel<kEos><<<blocks, kBlock, 0, stream>>>(args);
+    const int group = wide_group(args.n);
+    with_group(group, args.boundary.offsets != nullptr, [&](auto g, auto samples) {
+        mask_density_kernel<kEos, g(), samples()><<<pass_blocks(args.n, group), kGroupBlock, 0, stream>>>(args);
+    });
     PHX_LAUNCH_CHECK();
 }
-
-// Whole blocks of kBlock particles, padded to a multiple of the XCD count.
-inline uint32_t pass_blocks(uint32_t n) { return (blocks_for(n, kBlock) + 7u) / 8u * 8u; }
 
 }  // namespace
 }  // namespace phx
