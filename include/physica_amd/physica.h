@@ -694,7 +694,7 @@ phx_status phx_write_vectors(phx_stream stream, uint32_t count, phx_const_vector
 typedef struct phx_pbf_batch phx_pbf_batch;
 
 typedef struct phx_pbf_batch_configuration {
-    float mask_skin;    /* neighbour-mask skin in units of h (0: 0.3); results do not depend on it */
+    float mask_skin;    /* 0, or 0.01 to 1; unused: the passes keep no skin masks (results never depended on it) */
     uint32_t use_graph; /* replay a captured substep (only when every box is static) */
 } phx_pbf_batch_configuration;
 

@@ -28,7 +28,8 @@ TUNING = Path(__file__).resolve().parent / "tuning" / "pbf_batch.json"
 
 def tuned_settings() -> dict:
     """The autotuner's choice for this GPU (physica_amd/tuning/pbf_batch.json),
-    or the defaults (mask skin 0.3 h, graph replay)."""
+    or the defaults (graph replay; the mask skin is accepted by the engine but
+    sizes nothing, since its passes keep no skin masks)."""
     settings = {"mask_skin": 0.3, "use_graph": True}
     if TUNING.exists():
         try:

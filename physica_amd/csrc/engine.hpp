@@ -192,7 +192,7 @@ struct BatchBlock {
     uint32_t scene;
     uint32_t first;  // first particle of the workgroup (batch index)
     uint32_t count;  // particles of the workgroup (0: padding)
-    uint32_t pad;
+    uint32_t group_block;  // the first workgroup of the passes among its particles
 };
 struct BatchScene {
     uint32_t cell_base;  // first cell of the scene's grid in the batch's offsets

@@ -40,6 +40,12 @@ struct GroupLds {
     uint32_t totals[kGroupParticles<G>];
 };
 
+// The list of the particle the caller walks.
+template <int G>
+__device__ __forceinline__ uint32_t* group_row(GroupLds<G>& lds) {
+    return lds.list + threadIdx.x / G * GroupLds<G>::kStride;
+}
+
 // The value lane k of the caller's group holds.
 template <int G, int k>
 __device__ __forceinline__ float group_broadcast(float v) {
@@ -82,30 +88,45 @@ __device__ __forceinline__ void group_walk_list(const uint32_t* row, uint32_t co
     }
 }
 
-// group_walk_list over every particle of the 27 cells around (cx, cy, cz),
-// and with sample_offsets each cell's boundary samples after its particles:
-// the walk of a particle whose candidates are not listed. Entry `skip` is
-// left out.
-template <int G, int F, class Load, class Pair, class Fold>
+// group_walk_list over the particles of the 27 cells around (cx, cy, cz), and
+// with sample_offsets each cell's boundary samples after its particles: the
+// walk of a particle with a crowded cell, whose candidates have no masks.
+// The group tests G candidates at a time with near(entry), which is false
+// only where the terms are exact zeros, and collects the others in its list
+// `row`; a full list is walked on the way. Of the candidates of a crowded
+// neighbourhood a sixth to a half are kept, and the ordered additions make
+// each one dear. Entry `skip` is left out.
+template <int G, int F, class Near, class Load, class Pair, class Fold>
 __device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const uint32_t* sample_offsets, int cx, int cy,
-                                                   int cz, uint32_t skip, Load&& load, Pair&& pair, Fold&& fold) {
+                                                   int cz, uint32_t skip, uint32_t fallback, uint32_t* row,
+                                                   Near&& near, Load&& load, Pair&& pair, Fold&& fold) {
     const uint32_t lane = threadIdx.x % G;
+    const uint32_t group_shift = __lane_id() - lane;
+    uint32_t count = 0u;
+    auto empty = [&] {
+        // the list is written and read by this group alone, within its wave
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        group_walk_list<G, F>(row, count, fallback, load, pair, fold);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        count = 0u;
+    };
     auto run = [&](uint32_t first, uint32_t last, uint32_t flag) {
         for (uint32_t base = first; base < last; base += G) {
             const uint32_t s = base + lane;
             const uint32_t entry = (s < last ? s : base) | flag;
-            const auto record = load(entry);
-            float terms[F];
-#pragma unroll
-            for (int f = 0; f < F; ++f) terms[f] = -0.0F;
-            if (s < last && entry != skip) pair(record, entry, terms);
-            fold(terms);
+            const bool kept = near(entry) && s < last && entry != skip;
+            const uint32_t members =
+                static_cast<uint32_t>(__ballot(kept) >> group_shift) & ((1u << static_cast<uint32_t>(G)) - 1u);
+            if (kept) row[count + static_cast<uint32_t>(__popc(members & ((1u << lane) - 1u)))] = entry;
+            count += static_cast<uint32_t>(__popc(members));
+            if (count > kGroupList - G) empty();
         }
     };
     for_each_cell(g, cx, cy, cz, [&](uint32_t c) {
         run(g.offsets[c], g.offsets[c + 1u], 0u);
         if (sample_offsets != nullptr) run(sample_offsets[c], sample_offsets[c + 1u], kSampleEntry);
     });
+    empty();
 }
 
 // Lists the candidates of a workgroup's particles and walks them. slot(j, k,
@@ -197,12 +218,57 @@ __device__ __forceinline__ uint32_t stored_slot(const uint16_t* __restrict__ mas
     return m;
 }
 
-// The mask of the particles of cell `cell` with near(s), for a slot of a
-// particle that is not crowded and whose stored masks do not apply; `first`
-// is set as by stored_slot. Four members are tested together.
+// The ranges [first, last) of the expanding thread's stencil slots of the cell
+// (x, y, z), empty outside the grid; returns whether one holds more than
+// kMaskBits. Fetched together, ahead of the members.
+template <int G>
+__device__ __forceinline__ bool group_ranges(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
+                                             uint32_t (&first)[(kStencil + G - 1) / G],
+                                             uint32_t (&last)[(kStencil + G - 1) / G]) {
+    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    const uint32_t part = threadIdx.x / kGroupParticles<G>;
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) {
+        first[j] = last[j] = 0u;
+        const uint32_t k = part * kSlots + j;
+        const int X = x + static_cast<int>(k / 9u) - 1;
+        const int Y = y + static_cast<int>((k / 3u) % 3u) - 1;
+        const int Z = z + static_cast<int>(k % 3u) - 1;
+        if (k >= static_cast<uint32_t>(kStencil) || X < 0 || X >= static_cast<int>(g.cx) || Y < 0 ||
+            Y >= static_cast<int>(g.cy) || Z < 0 || Z >= static_cast<int>(g.cz))
+            continue;
+        const uint32_t c = cell_of(g, X, Y, Z);
+        first[j] = offsets[c];
+        last[j] = offsets[c + 1u];
+    }
+    bool many = false;
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) many = many || last[j] - first[j] > kMaskBits;
+    return many;
+}
+
+// The mask of members from .. to - 1 (the first kMaskBits of them) with
+// near(s). Four are tested together, so that their loads overlap.
 template <class Near>
-__device__ __forceinline__ uint32_t scanned_slot(const SortedGrid& g, int x, int y, int z, uint32_t k, uint32_t& first,
-                                                 Near&& near) {
+__device__ __forceinline__ uint32_t mark_members(uint32_t from, uint32_t to, Near&& near) {
+    const uint32_t end = min(to, from + kMaskBits);
+    uint32_t bits = 0u;
+    for (uint32_t s = from; s < end; s += 4u) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const bool marked = near(min(s + u, end - 1u)) && s + u < end;
+            bits |= marked ? 1u << (s + u - from) : 0u;
+        }
+    }
+    return bits;
+}
+
+// Slot k of a particle of cell (x, y, z) that is not crowded and whose stored
+// masks do not apply: the members with near(s); `first` is set as by
+// stored_slot.
+template <class Near>
+__device__ __forceinline__ uint32_t scanned_slot(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
+                                                 uint32_t k, uint32_t& first, Near&& near) {
     const int X = x + static_cast<int>(k / 9u) - 1;
     const int Y = y + static_cast<int>((k / 3u) % 3u) - 1;
     const int Z = z + static_cast<int>(k % 3u) - 1;
@@ -210,17 +276,8 @@ __device__ __forceinline__ uint32_t scanned_slot(const SortedGrid& g, int x, int
         Z >= static_cast<int>(g.cz))
         return 0u;
     const uint32_t c = cell_of(g, X, Y, Z);
-    first = g.offsets[c];
-    const uint32_t last = min(g.offsets[c + 1u], first + kMaskBits);
-    uint32_t bits = 0u;
-    for (uint32_t s = first; s < last; s += 4u) {
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
-            const bool marked = near(min(s + u, last - 1u)) && s + u < last;
-            bits |= marked ? 1u << (s + u - first) : 0u;
-        }
-    }
-    return bits;
+    first = offsets[c];
+    return mark_members(first, offsets[c + 1u], near);
 }
 
 }  // namespace phx

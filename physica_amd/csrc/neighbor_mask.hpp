@@ -146,58 +146,6 @@ __device__ __forceinline__ void walk_slots_prefetch(SlotBase&& slot_base, const 
     }
 }
 
-// walk_slots_prefetch that hands each candidate's place to process: its
-// sorted index s, stencil slot k and bit b within that cell's mask, as
-// process(value, s, k, b).
-template <int kDepth, class SlotBase, class Load, class Process>
-__device__ __forceinline__ void walk_slots_prefetch_tagged(SlotBase&& slot_base, const uint16_t* column,
-                                                           uint32_t stride, uint32_t nonzero, uint32_t fallback,
-                                                           Load&& load, Process&& process) {
-    auto fetch = [&](uint32_t& mask, uint32_t& base, uint32_t& slot) {
-        mask = 0u;
-        if (nonzero != 0u) {
-            slot = static_cast<uint32_t>(__builtin_ctz(nonzero));
-            nonzero &= nonzero - 1u;
-            mask = column[slot * stride];
-            base = slot_base(slot);
-        }
-    };
-    uint32_t m = 0u, base = 0u, slot = 0u, m_next = 0u, base_next = 0u, slot_next = 0u;
-    fetch(m, base, slot);
-    fetch(m_next, base_next, slot_next);
-    auto next = [&](bool& have, uint32_t& s, uint32_t& k, uint32_t& b) -> uint32_t {
-        if (m == 0u) {
-            m = m_next;
-            base = base_next;
-            slot = slot_next;
-            fetch(m_next, base_next, slot_next);
-        }
-        have = m != 0u;
-        b = static_cast<uint32_t>(__builtin_ctz(m));
-        s = base + b;
-        k = slot;
-        m &= m - 1u;
-        return have ? s : fallback;
-    };
-    using Data = decltype(load(0u));
-    Data data[kDepth];
-    bool have[kDepth];
-    uint32_t ss[kDepth], ks[kDepth], bs[kDepth];
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d) data[d] = load(next(have[d], ss[d], ks[d], bs[d]));
-    for (;;) {
-#pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            if (!have[d]) return;
-            const Data current = data[d];
-            const uint32_t s = ss[d], k = ks[d], b = bs[d];
-            data[d] = load(next(have[d], ss[d], ks[d], bs[d]));
-            asm volatile("" ::: "memory");
-            process(current, s, k, b);
-        }
-    }
-}
-
 // Every candidate of the 27 cells around (cx, cy, cz) in the reference order
 // (for_each_candidate) with the memory latency taken off the critical path as
 // in walk_slots_prefetch: the range of the next in-grid stencil cell is
@@ -375,38 +323,7 @@ struct MaskView {
     // per particle (sorted order): non-zero where a stencil cell holds more
     // than kMaskBits particles; null: no particle is crowded
     const uint8_t* crowded = nullptr;
-    // per cell: the largest displacement (float bits, rounded up) of its
-    // particles from the positions the masks were built at, over the position
-    // sets written so far in the step; null: only the step-wide limit applies.
-    // Where that limit fails, a particle whose own displacement plus the
-    // largest of its stencil cells' stays within pair_limit keeps its masks.
-    const uint32_t* cell_moved = nullptr;
-    float pair_limit = -1.0F;
 };
-
-// The displacement |moved| rounded up for the per-cell bounds: the relative
-// margin covers the rounding of the difference, the dot product and the
-// square root.
-__device__ __forceinline__ float displacement_bound(Float3 moved) {
-    return sqrtf(dot(moved, moved)) * (1.0F + 4e-6F);
-}
-
-// Raises cell_moved[cell] to at least `moved` for each lane's cell. The lanes
-// of one cell are consecutive in sorted order, so a segmented maximum over the
-// wave leaves one atomic per run of equal cells. Every lane of the wave calls
-// this; a lane without a particle passes cell = ~0u.
-__device__ __forceinline__ void raise_cell_bound(uint32_t* cell_moved, uint32_t cell, float moved) {
-    const int lane = static_cast<int>(__lane_id());
-    float v = moved;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-        const float up = __shfl_up(v, offset);
-        const uint32_t up_cell = __shfl_up(cell, offset);
-        if (lane >= offset && up_cell == cell) v = fmaxf(v, up);
-    }
-    const uint32_t next_cell = __shfl_down(cell, 1);
-    if (cell != ~0u && (lane == 63 || next_cell != cell)) atomicMax(cell_moved + cell, __float_as_uint(v));
-}
 
 // Whether particle i is crowded in the step of these masks (it then walks the
 // full stencil in every pass).
@@ -434,44 +351,6 @@ __device__ __forceinline__ bool masks_apply(const MaskView& m, uint32_t slot, ui
     if (m.masks == nullptr || m.flags[kFlagOverflow] != 0u) return false;
     if (m.crowded != nullptr && m.crowded[i] != 0u) return false;
     return m.exact != 0u || __uint_as_float(m.flags[kFlagDisplacement + slot]) <= m.limit2;
-}
-
-// masks_apply, and where the step-wide displacement limit fails, the
-// per-cell rule: particle i may keep its masks if own() (its displacement
-// bound) plus the largest cell_moved of its stencil stays within pair_limit.
-// A pair within h at the current positions was then within h + pair_limit at
-// the positions the masks were built at. A wave whose lanes decided both ways
-// would run the masked and the full walk one after the other, so a wave walks
-// its masks only if every lane that is not crowded may. Every lane of the
-// wave with a particle calls this.
-template <class Own>
-__device__ __forceinline__ bool masks_apply(const MaskView& m, uint32_t slot, uint32_t i, const SortedGrid& g, int cx,
-                                            int cy, int cz, Own&& own) {
-    if (m.masks == nullptr || m.flags[kFlagOverflow] != 0u) return false;
-    const bool crowded = m.crowded != nullptr && m.crowded[i] != 0u;
-    if (m.exact != 0u || __uint_as_float(m.flags[kFlagDisplacement + slot]) <= m.limit2) return !crowded;
-    if (m.cell_moved == nullptr) return false;
-    bool may = crowded;  // crowded lanes walk the full stencil, whatever the wave does
-    if (!crowded) {
-        float largest = 0.0F;
-#pragma unroll 1
-        for (int oz = -1; oz <= 1; ++oz) {
-            const int Z = cz + oz;
-            if (Z < 0 || Z >= static_cast<int>(g.cz)) continue;
-#pragma unroll 1
-            for (int oy = -1; oy <= 1; ++oy) {
-                const int Y = cy + oy;
-                if (Y < 0 || Y >= static_cast<int>(g.cy)) continue;
-                for (int ox = -1; ox <= 1; ++ox) {
-                    const int X = cx + ox;
-                    if (X < 0 || X >= static_cast<int>(g.cx)) continue;
-                    largest = fmaxf(largest, __uint_as_float(m.cell_moved[cell_of(g, X, Y, Z)]));
-                }
-            }
-        }
-        may = own() + largest <= m.pair_limit;
-    }
-    return !crowded && __all(may) != 0;
 }
 
 // Tests the members of the 27 cells around (cx, cy, cz): test(s) says whether
@@ -539,81 +418,6 @@ __device__ __forceinline__ void visit_candidates(const SortedGrid& g, const Mask
     }
 }
 
-// Visits the candidates of particle i like visit_candidates, where visit(s)
-// returns whether candidate s is kept, and writes the kept candidates of each
-// stencil slot k as the mask out[k * n + i] (every slot is written). Returns
-// false if a kept candidate lies beyond the first kMaskBits particles of its
-// cell: the masks are then incomplete and must not be used.
-template <class Visit>
-__device__ __forceinline__ bool visit_and_mask(const SortedGrid& g, const MaskView& m, bool masked, uint32_t i,
-                                               int cx, int cy, int cz, const int* delta, uint16_t* column,
-                                               uint32_t stride, uint16_t* __restrict__ out, uint32_t n,
-                                               Visit&& visit) {
-    uint32_t written = 0u;
-    auto emit = [&](uint32_t k, uint32_t bits) {
-        for (; written < k; ++written) out[static_cast<size_t>(written) * n + i] = 0u;
-        out[static_cast<size_t>(k) * n + i] = static_cast<uint16_t>(bits);
-        written = k + 1u;
-    };
-    bool complete = true;
-    if (masked) {
-        // one candidate per loop trip, as in walk_masked (a loop per slot
-        // would run, slot after slot, as many trips as the wave's fullest
-        // lane in that slot); a lane writes a slot's mask as it moves on
-        uint32_t nonzero = load_lane_column(m.masks, m.n, i, column, stride);
-        const uint32_t center = cell_of(g, cx, cy, cz);
-        constexpr uint32_t kNone = static_cast<uint32_t>(kStencil);
-        uint32_t candidates = 0u, base = 0u, bits = 0u, k = kNone;
-        while ((candidates | nonzero) != 0u) {
-            if (candidates == 0u) {
-                if (k != kNone) emit(k, bits);
-                k = static_cast<uint32_t>(__builtin_ctz(nonzero));
-                nonzero &= nonzero - 1u;
-                candidates = column[k * stride];
-                base = g.offsets[center + static_cast<uint32_t>(delta[k])];
-                bits = 0u;
-            }
-            const uint32_t b = static_cast<uint32_t>(__builtin_ctz(candidates));
-            candidates &= candidates - 1u;
-            if (visit(base + b)) bits |= 1u << b;
-        }
-        if (k != kNone) emit(k, bits);
-    } else {
-        uint32_t k = 0u;
-#pragma unroll 1
-        for (int ox = -1; ox <= 1; ++ox) {
-            const int X = cx + ox;
-#pragma unroll 1
-            for (int oy = -1; oy <= 1; ++oy) {
-                const int Y = cy + oy;
-#pragma unroll 1
-                for (int oz = -1; oz <= 1; ++oz, ++k) {
-                    const int Z = cz + oz;
-                    if (X < 0 || X >= static_cast<int>(g.cx) || Y < 0 || Y >= static_cast<int>(g.cy) || Z < 0 ||
-                        Z >= static_cast<int>(g.cz))
-                        continue;
-                    const uint32_t c = cell_of(g, X, Y, Z);
-                    const uint32_t first = g.offsets[c];
-                    const uint32_t last = g.offsets[c + 1u];
-                    uint32_t bits = 0u;
-                    for (uint32_t s = first; s < last; ++s) {
-                        if (visit(s)) {
-                            if (s - first < kMaskBits) {
-                                bits |= 1u << (s - first);
-                            } else {
-                                complete = false;
-                            }
-                        }
-                    }
-                    emit(k, bits);
-                }
-            }
-        }
-    }
-    for (; written < static_cast<uint32_t>(kStencil); ++written) out[static_cast<size_t>(written) * n + i] = 0u;
-    return complete;
-}
-
 // A candidate's record and sorted index.
 template <class Record>
 struct Tagged {
@@ -652,135 +456,6 @@ __device__ __forceinline__ void visit_records(const SortedGrid& g, const MaskVie
         }
     }
     if (shared) walk_stencil_shared(g, leader, cx, cy, cz, crowded, load, pair);
-}
-
-// visit_records where keep(record, s) says whether candidate s is kept, and
-// the kept candidates of each stencil slot k are written as the mask
-// out[k * n + i] (every slot is written) like visit_and_mask. Crowded lanes
-// of a wave-shared cell write no masks (a crowded particle's masks are never
-// read). near(s) is keep()'s answer from the position alone (true also where the
-// distance is NaN): a lane that
-// has neither masks nor a crowded cell marks its candidates with it and
-// evaluates only the marked ones. Returns false if a kept candidate lies
-// beyond the first kMaskBits particles of its cell.
-template <int kDepth, class Near, class Load, class Keep>
-__device__ __forceinline__ bool visit_records_and_mask(const SortedGrid& g, const MaskView& m, bool masked,
-                                                       uint32_t i, int cx, int cy, int cz, const int* delta,
-                                                       uint16_t* column, uint32_t stride,
-                                                       uint16_t* __restrict__ out, uint32_t n, Near&& near,
-                                                       Load&& load, Keep&& keep) {
-    uint32_t leader = 0u;
-    const bool crowded = is_crowded(m, i);
-    const bool shared = shared_crowded_cell(crowded, cell_of(g, cx, cy, cz), leader);
-    bool complete = true;
-    if (!masked && !crowded && m.crowded != nullptr) {
-        // mark first, then walk the marked candidates: of the 27 cells' 216
-        // candidates about 33 are kept, but in nearly every trip some lane of
-        // the wave keeps its own, so a walk that evaluates as it goes pays
-        // for the pair terms 216 times (12 uneven scenes stepped together,
-        // 0.9 M particles: lambda passes 318 -> 247 us, vorticity 368 -> 297)
-        uint32_t nonzero = 0u;
-        complete = scan_stencil(g, cx, cy, cz, near, [&](uint32_t k, uint32_t bits) {
-            out[static_cast<size_t>(k) * n + i] = static_cast<uint16_t>(bits);
-            column[k * stride] = static_cast<uint16_t>(bits);
-            nonzero |= bits != 0u ? 1u << k : 0u;
-        });
-        const uint32_t center = cell_of(g, cx, cy, cz);
-        if constexpr (kDepth == 0) {
-            walk_masked(g.offsets, center, delta, column, stride, nonzero,
-                        [&](uint32_t s) { (void)keep(load(s), s); });
-        } else {
-            using Record = decltype(load(0u));
-            walk_masked_prefetch<kDepth>(
-                g.offsets, center, delta, column, stride, nonzero, i,
-                [&](uint32_t s) { return Tagged<Record>{load(s), s}; },
-                [&](const Tagged<Record>& t) { (void)keep(t.r, t.s); });
-        }
-    } else if (!shared || !crowded) {
-        if constexpr (kDepth == 0) {
-            complete = visit_and_mask(g, m, masked, i, cx, cy, cz, delta, column, stride, out, n,
-                                      [&](uint32_t s) { return keep(load(s), s); });
-        } else {
-            constexpr uint32_t kNone = static_cast<uint32_t>(kStencil);
-            uint32_t written = 0u, open = kNone, bits = 0u;
-            // closes the open slot (zero masks before it) and opens slot k
-            auto open_slot = [&](uint32_t k) {
-                if (open != kNone) {
-                    for (; written < open; ++written) out[static_cast<size_t>(written) * n + i] = 0u;
-                    out[static_cast<size_t>(open) * n + i] = static_cast<uint16_t>(bits);
-                    written = open + 1u;
-                }
-                open = k;
-                bits = 0u;
-            };
-            auto take = [&](const auto& r, uint32_t s, uint32_t k, uint32_t b) {
-                if (k != open) open_slot(k);
-                if (keep(r, s)) {
-                    if (b < kMaskBits) {
-                        bits |= 1u << b;
-                    } else {
-                        complete = false;
-                    }
-                }
-            };
-            if (masked) {
-                const uint32_t nonzero = load_lane_column(m.masks, m.n, i, column, stride);
-                const uint32_t center = cell_of(g, cx, cy, cz);
-                walk_slots_prefetch_tagged<kDepth>(
-                    [&](uint32_t k) { return g.offsets[center + static_cast<uint32_t>(delta[k])]; }, column, stride,
-                    nonzero, i, load, take);
-            } else {
-                walk_stencil_prefetch<kDepth>(
-                    g, cx, cy, cz, i, load,
-                    [&](const auto& r, uint32_t s, uint32_t k, uint32_t first) { take(r, s, k, s - first); });
-            }
-            open_slot(kNone);
-            for (; written < static_cast<uint32_t>(kStencil); ++written)
-                out[static_cast<size_t>(written) * n + i] = 0u;
-        }
-    }
-    if (shared) walk_stencil_shared(g, leader, cx, cy, cz, crowded, load, [&](const auto& r, uint32_t s) {
-        (void)keep(r, s);
-    });
-    return complete;
-}
-
-// Skin mask of particle i at p from SoA positions: bit b of slot k marks the
-// b-th particle of that stencil cell with squared distance below t. Returns
-// false if a stencil cell holds more than kMaskBits particles.
-__device__ __forceinline__ bool build_skin_mask(const SortedGrid& g, CVec pos, uint32_t n, uint32_t i, Float3 p,
-                                                int cx, int cy, int cz, float t, uint16_t* __restrict__ masks) {
-    bool complete = true;
-    int k = 0;
-#pragma unroll 1
-    for (int ox = -1; ox <= 1; ++ox) {
-        const int X = cx + ox;
-#pragma unroll 1
-        for (int oy = -1; oy <= 1; ++oy) {
-            const int Y = cy + oy;
-#pragma unroll 1
-            for (int oz = -1; oz <= 1; ++oz, ++k) {
-                const int Z = cz + oz;
-                uint32_t bits = 0u;
-                if (X >= 0 && X < static_cast<int>(g.cx) && Y >= 0 && Y < static_cast<int>(g.cy) && Z >= 0 &&
-                    Z < static_cast<int>(g.cz)) {
-                    const uint32_t c = cell_of(g, X, Y, Z);
-                    const uint32_t first = g.offsets[c];
-                    uint32_t last = g.offsets[c + 1u];
-                    if (last - first > kMaskBits) {
-                        complete = false;
-                        last = first + kMaskBits;
-                    }
-                    for (uint32_t s = first; s < last; ++s) {
-                        const Float3 d = sub(p, load(pos, s));
-                        bits |= dot(d, d) < t ? 1u << (s - first) : 0u;
-                    }
-                }
-                masks[static_cast<size_t>(k) * n + i] = static_cast<uint16_t>(bits);
-            }
-        }
-    }
-    return complete;
 }
 
 // Block-wide maximum of a non-negative float, folded into *target

@@ -2,10 +2,6 @@
 //
 // Reference: PBF::forward_step (pbf/pbf.cpp:167-191) and pbf/pbf.cu. Fusion:
 //   grid       predict x* fused into the cell-key pass (pbf.cu:73-78)
-//   mask       skin masks at x* (radius h (1 + skin)); every later pass walks
-//              them while no particle moved more than half the skin from x*
-//              (checked on the device from the correction passes' largest
-//              displacement), and the full 27-cell stencil otherwise
 //   per iter   A: density + lambda in one neighbour loop (density.cu:18-40,
 //                 pbf.cu:95-127; the two sums keep their own order)
 //              B: correction + project (pbf.cu:254-288, 417-431), written to
@@ -14,28 +10,59 @@
 //   post       vorticity + magnitude (pbf.cu:476-497, 565-569)
 //              normal + confinement (pbf.cu:571-593, 674-678)
 //              XSPH + scatter of the next state (pbf.cu:700-721)
+// A pass gives each particle a group of 4 or 16 lanes (group_walk.hpp). The
+// first pass at a set of positions (lambda, vorticity) scans the 27 cells and
+// writes the exact neighbour masks that the others at those positions walk.
 // Per-particle sums run in the reference order, so each value is the IEEE
 // result of the reference expression.
 #include "pbf.hpp"
 
+#include "group_walk.hpp"
 #include "neighbor_mask.hpp"
+
+#include <type_traits>
 
 namespace phx {
 namespace {
 
 constexpr uint32_t kBlock = 256;
-// Records a neighbour walk fetches ahead: two in a single scene's launch
-// (too few waves to hide the loads of long crowded walks), none in a batch
-// launch, which fills the GPU.
-template <bool kBatch>
-constexpr int kPbfWalkDepth = kBatch ? 0 : 2;
+// Particle counts up to which 16 lanes share a particle; above, 4. One lane
+// per particle, over skin masks built once a step, is slower at every size.
+// Steps, us, with 1 / 4 / 16 lanes: 1,300 particles 532 / 169 / 106, 16,000
+// 514 / 174 / 136, 32,000 524 / 179 / 181 (30 clumps 1,799 / 613 / 524),
+// 64,000 517 / 239 / 289, 260,000 809 / 663 / 903, 1,048,576 4,080 / 2,313 /
+// 3,424.
+constexpr uint32_t kGroup16Particles = 32768;
 
-// LDS of a masked neighbour pass: the lanes' mask columns and the slot table.
-#define PHX_MASK_LDS(grid)                          \
-    __shared__ uint16_t smask[kStencil * kBlock];   \
-    __shared__ int delta[kStencil];                 \
-    fill_slot_deltas(grid, delta);                  \
-    __syncthreads()
+// Workgroups with crowded particles that a pass starts before all others.
+constexpr uint32_t kEarlyBlocks = 512;
+// Particle count from which a single scene orders its workgroups so (a batch
+// always does): below, a pass's workgroups all start at once anyway.
+constexpr uint32_t kEarlyParticles = 100000;
+
+// The order of a pass's workgroups. A workgroup with crowded particles can
+// last many times as long as the others; started last, it runs on alone.
+// pbf_cell_kernel lists such workgroups, and the first kEarlyBlocks blocks of
+// a launch serve the listed ones; a listed workgroup's own block returns at
+// once. 262,144 particles with 60
+// clumps: 1,317 -> 1,057 us a step.
+struct Schedule {
+    uint32_t* count;   // workgroups listed (may exceed kEarlyBlocks: the rest are not served early)
+    uint32_t* listed;  // [kEarlyBlocks] their ids
+    uint32_t* place;   // per workgroup: its place in `listed` + 1; 0: not listed
+    uint32_t* seen;    // per workgroup: non-zero once a crowded particle was found
+    uint32_t early;    // kEarlyBlocks, or 0: workgroups in order
+};
+
+// The workgroup id a block serves; ~0u for none.
+__device__ __forceinline__ uint32_t scheduled_block(const Schedule& s) {
+    if (s.early == 0u) return xcd_block();
+    if (blockIdx.x < s.early) return blockIdx.x < *s.count ? s.listed[blockIdx.x] : ~0u;
+    const uint32_t per_xcd = (gridDim.x - s.early) / 8u;
+    const uint32_t b = blockIdx.x - s.early;
+    const uint32_t id = b % 8u * per_xcd + b / 8u;
+    return s.place[id] - 1u < s.early ? ~0u : id;
+}
 
 // The particle, grid and collision box of a lane: one scene (kBatch false),
 // or in a batch the scene of the workgroup's block, whose grid starts at
@@ -48,10 +75,11 @@ struct Lane {
 };
 
 template <bool kBatch>
-__device__ __forceinline__ Lane lane_of(uint32_t n, const SortedGrid& grid, const Box& box, const BatchView& batch) {
+__device__ __forceinline__ Lane lane_of(uint32_t id, uint32_t n, const SortedGrid& grid, const Box& box,
+                                        const BatchView& batch) {
     Lane l;
     if constexpr (kBatch) {
-        const BatchBlock blk = batch.blocks[xcd_block()];
+        const BatchBlock blk = batch.blocks[id];
         const BatchScene& sc = batch.scenes[blk.scene];
         l.i = blk.first + threadIdx.x;
         l.valid = threadIdx.x < blk.count;
@@ -74,7 +102,7 @@ __device__ __forceinline__ Lane lane_of(uint32_t n, const SortedGrid& grid, cons
         }
         l.box.no_slip = sc.no_slip;
     } else {
-        l.i = xcd_block() * kBlock + threadIdx.x;
+        l.i = id * kBlock + threadIdx.x;
         l.valid = l.i < n;
         l.grid = grid;
         l.box = box;
@@ -82,42 +110,51 @@ __device__ __forceinline__ Lane lane_of(uint32_t n, const SortedGrid& grid, cons
     return l;
 }
 
-// The lane's mask view: in a batch the per-cell displacement bounds of the
-// lane's scene start at its cell base, like its grid's offsets.
-__device__ __forceinline__ MaskView lane_masks(const MaskView& mv, const SortedGrid& launch, const SortedGrid& lane) {
-    MaskView v = mv;
-    if (v.cell_moved != nullptr) v.cell_moved += lane.offsets - launch.offsets;
-    return v;
-}
-
-struct MaskArgs {
-    uint32_t n;
+// The particles of workgroup `id` of a launch with groups of G lanes: base ..
+// base + count - 1, of one scene.
+struct GroupScene {
+    uint32_t base, count;
     SortedGrid grid;
-    CVec xs;
-    float t_skin;
-    uint16_t* masks;
-    uint8_t* crowded;
+    Box box;
 };
 
-// Skin masks at x*; a particle with a stencil cell of more than kMaskBits
-// particles is marked crowded and walks the full stencil in every pass of
-// the step (the others keep their masks).
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_mask_kernel(MaskArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, Box{}, batch);
-    const uint32_t i = lane.i;
-    if (!lane.valid) return;
-    const SortedGrid& grid = lane.grid;
-    const Float3 p = load(a.xs, i);
-    int cx, cy, cz;
-    particle_cell(grid, p, cx, cy, cz);
-    a.crowded[i] = build_skin_mask(grid, a.xs, a.n, i, p, cx, cy, cz, a.t_skin, a.masks) ? 0u : 1u;
+template <bool kBatch, int G>
+__device__ __forceinline__ GroupScene group_scene(uint32_t id, uint32_t n, const SortedGrid& grid, const Box& box,
+                                                  const BatchView& batch) {
+    if constexpr (kBatch) {
+        const BatchBlock blk = batch.blocks[id];
+        const Lane l = lane_of<true>(id, n, grid, box, batch);
+        return GroupScene{blk.first, blk.count, l.grid, l.box};
+    } else {
+        const uint32_t base = id * kGroupParticles<G>;
+        return GroupScene{base, base < n ? min(n - base, kGroupParticles<G>) : 0u, grid, box};
+    }
 }
 
-// A particle that is not crowded always gets complete exact masks; the set's
-// overflow word is raised only if that ever fails.
-__device__ __forceinline__ void flag_incomplete(bool complete, const MaskView& mv, uint32_t i, uint32_t* set_flag) {
-    if (!complete && (mv.crowded == nullptr || mv.crowded[i] == 0u)) atomicOr(set_flag, 1u);
+// The cell and crowded byte of each particle, and the workgroups (of
+// `particles` particles each) that hold crowded ones.
+template <bool kBatch>
+__global__ void __launch_bounds__(kBlock) pbf_cell_kernel(uint32_t n, SortedGrid launch_grid, CVec xs, uint32_t* cell,
+                                                          uint8_t* crowded, uint32_t particles, Schedule schedule,
+                                                          BatchView batch) {
+    const uint32_t id = xcd_block();
+    const Lane lane = lane_of<kBatch>(id, n, launch_grid, Box{}, batch);
+    if (!lane.valid) return;
+    const SortedGrid& grid = lane.grid;
+    int cx, cy, cz;
+    particle_cell(grid, load(xs, lane.i), cx, cy, cz);
+    cell[lane.i] = cell_of(grid, cx, cy, cz);
+    bool many = false;
+    for_each_cell(grid, cx, cy, cz,
+                  [&](uint32_t c) { many = many || grid.offsets[c + 1u] - grid.offsets[c] > kMaskBits; });
+    crowded[lane.i] = many ? 1u : 0u;
+    if (!many) return;
+    const uint32_t first = kBatch ? batch.blocks[id].group_block : id * (kBlock / particles);
+    const uint32_t group_block = first + threadIdx.x / particles;
+    if (atomicExch(schedule.seen + group_block, 1u) != 0u) return;
+    const uint32_t place = atomicAdd(schedule.count, 1u);
+    if (place < kEarlyBlocks) schedule.listed[place] = group_block;
+    schedule.place[group_block] = place + 1u;
 }
 
 struct LambdaArgs {
@@ -134,73 +171,34 @@ struct LambdaArgs {
     float* lambda;
     float* den;  // optional (recorded step)
     Vec gsum;    // optional (recorded step)
-    MaskView mv;
-    uint32_t slot;  // displacement slot of the positions read
     // exact masks of the positions read (pairs inside exact_mask_threshold),
     // for the correction pass and the derivatives (crowded particles walk the
     // full stencil instead)
     float t_exact;
     uint16_t* exact_out;
-    uint32_t* exact_flags;
     BoundaryGrid boundary;  // offsets null: no boundary samples
+    // the cell and crowded byte of each particle, written by the step's first
+    // pass (first_pass != 0) and read by the others
+    uint32_t* cell;
+    uint8_t* crowded;
+    uint32_t first_pass;
 };
 
-// density_forward_kernel (density.cu:18-40, poly6) and lambda_forward_kernel
-// (pbf.cu:95-127); the walk also writes the exact masks of the positions.
-// With boundary samples the walk is the full stencil, each cell's samples b
-// after its particles adding rho0_i V_b W to the density and V_b grad W to
-// the gradient sum (pbf.cu:118-121); no exact masks are written (the host
-// marks those sets unusable).
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_lambda_kernel(LambdaArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, Box{}, batch);
-    PHX_MASK_LDS(lane.grid);
-    const uint32_t i = lane.i;
-    if (!lane.valid) return;
-    const SortedGrid& grid = lane.grid;
-    const MaskView mv = lane_masks(a.mv, a.grid, grid);
-    const Float3 p = load(a.pos, i);
-    const float rest = a.rho0[i];
-    const Float3 x_star = load(a.topo, i);
-    int cx, cy, cz;
-    particle_cell(grid, x_star, cx, cy, cz);
-    const bool masked =
-        masks_apply(mv, a.slot, i, grid, cx, cy, cz, [&] { return displacement_bound(sub(p, x_star)); });
-    float density = 0.0F;
-    Float3 gradient_sum{0.0F, 0.0F, 0.0F};
-    float denominator = a.eps[i];
-    auto pair = [&](Float3 q, float ms, uint32_t s) {
-        const Float3 d = sub(p, q);
-        density += ms * poly6(d, a.h);
-        if (s != i) {
-            const Float3 g = spiky_gradient(d, a.h, a.spiky);
-            const float coefficient = ms / rest;
-            gradient_sum = add(gradient_sum, scale(g, coefficient));
-            denominator += coefficient * coefficient * dot(g, g);
-        }
-        return dot(d, d) < a.t_exact;
-    };
-    auto near = [&](uint32_t s) {
-        const Float3 d = sub(p, load(a.pos, s));
-        return !(dot(d, d) >= a.t_exact);
-    };
-    auto visit = [&](uint32_t s) { return pair(load(a.pos, s), a.m[s], s); };
-    if (a.boundary.offsets != nullptr) {
-        for_each_candidate(
-            grid, a.boundary, cx, cy, cz, [&](uint32_t s) { (void)visit(s); },
-            [&](uint32_t s) {
-                const float4 b = a.boundary.x[s];
-                const Float3 d = sub(p, Float3{b.x, b.y, b.z});
-                density += rest * b.w * poly6(d, a.h);
-                gradient_sum = add(gradient_sum, scale(spiky_gradient(d, a.h, a.spiky), b.w));
-            });
-    } else {
-        const bool complete = visit_records_and_mask<kPbfWalkDepth<kBatch>>(
-            grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n, near,
-            [&](uint32_t s) { return PointMass{load(a.pos, s), a.m[s]}; },
-            [&](const PointMass& c, uint32_t s) { return pair(c.x, c.m, s); });
-        flag_incomplete(complete, mv, i, &a.exact_flags[kFlagOverflow]);
-    }
+// The terms of one candidate in the density and lambda sums: the density,
+// the gradient sum and the denominator.
+struct LambdaTerms {
+    float density;
+    Float3 gradient;
+    float square;
+};
+__device__ __forceinline__ LambdaTerms lambda_terms(const LambdaArgs& a, Float3 d, float ms, float rest) {
+    const Float3 g = spiky_gradient(d, a.h, a.spiky);
+    const float coefficient = ms / rest;
+    return LambdaTerms{ms * poly6(d, a.h), scale(g, coefficient), coefficient * coefficient * dot(g, g)};
+}
+
+__device__ __forceinline__ void finish_lambda(const LambdaArgs& a, uint32_t i, float rest, float density,
+                                              Float3 gradient_sum, float denominator) {
     denominator += dot(gradient_sum, gradient_sum);
     a.rho[i] = density;
     a.lambda[i] = -(density / rest - 1.0F) / denominator;
@@ -208,6 +206,204 @@ __global__ void __launch_bounds__(kBlock) pbf_lambda_kernel(LambdaArgs a, BatchV
         a.den[i] = denominator;
         store(a.gsum, i, gradient_sum);
     }
+}
+
+// The position of a list entry.
+template <bool kSamples>
+__device__ __forceinline__ Float3 entry_position(CVec pos, const BoundaryGrid& samples, uint32_t entry) {
+    if constexpr (kSamples) {
+        if ((entry & kSampleEntry) != 0u) {
+            const float4 b = samples.x[entry & ~kSampleEntry];
+            return Float3{b.x, b.y, b.z};
+        }
+    }
+    return load(pos, entry);
+}
+
+// What the first walk of a set of positions (lambda, vorticity) does: each
+// expanding thread scans its stencil slots at the positions `pos` and writes
+// their exact masks. A scan shared by G lanes takes little longer than
+// reading masks would, so a step keeps no skin masks. `samples`, with kSamples, lists the boundary samples
+// near the particle. pair and fold are group_walk_list's; sum is kept by the
+// caller. Returns the walked particle, or ~0u for a lane without one.
+template <int G, bool kSamples, int F, class Args, class Load, class Pair, class Fold>
+__device__ __forceinline__ uint32_t group_first_walk(const Args& a, const GroupScene& scene, GroupLds<G>& lds,
+                                                     uint32_t* crowd, const BoundaryGrid& samples, uint32_t skip,
+                                                     Load&& load_record, Pair&& pair, Fold&& fold) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    const uint32_t expanded = threadIdx.x % kParticles;
+    const uint32_t part = threadIdx.x / kParticles;
+    const uint32_t i = scene.base + expanded;
+    const bool valid = expanded < scene.count;
+    if (threadIdx.x < kParticles) crowd[threadIdx.x] = 0u;
+    __syncthreads();
+    Float3 p{0.0F, 0.0F, 0.0F};
+    uint32_t first[kSlots] = {}, last[kSlots] = {};
+    [[maybe_unused]] uint32_t sample_first[kSlots] = {}, sample_last[kSlots] = {};
+    if (valid) {
+        p = load(a.pos, i);
+        int cx, cy, cz;
+        if (a.first_pass != 0u) {
+            particle_cell(scene.grid, load(a.topo, i), cx, cy, cz);
+            if (part == 0u) a.cell[i] = cell_of(scene.grid, cx, cy, cz);
+        } else {
+            cell_coordinates(scene.grid, a.cell[i], cx, cy, cz);
+        }
+        bool crowded = group_ranges<G>(scene.grid, scene.grid.offsets, cx, cy, cz, first, last);
+        if constexpr (kSamples)
+            crowded = group_ranges<G>(scene.grid, samples.offsets, cx, cy, cz, sample_first, sample_last) || crowded;
+        if (crowded) crowd[expanded] = 1u;
+    }
+    auto near = [&](Float3 from, Float3 to) {
+        const Float3 d = sub(from, to);
+        return !(dot(d, d) >= a.t_exact);
+    };
+    const uint32_t walked = threadIdx.x / G;
+    const uint32_t w = scene.base + walked;
+    const bool active = walked < scene.count;
+    group_expand<G, kSamples>(
+        lds,
+        [&](uint32_t j, uint32_t k, uint32_t& start) {
+            if (!valid) return 0u;
+            start = first[j];
+            const uint32_t bits = mark_members(first[j], last[j], [&](uint32_t s) { return near(p, load(a.pos, s)); });
+            a.exact_out[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits);
+            return bits;
+        },
+        [&](uint32_t j, uint32_t, uint32_t& start) {
+            start = sample_first[j];
+            return mark_members(sample_first[j], sample_last[j], [&](uint32_t b) {
+                const float4 q = samples.x[b];
+                return near(p, Float3{q.x, q.y, q.z});
+            });
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (active && crowd[walked] == 0u) group_walk_list<G, F>(row, count, w, load_record, pair, fold);
+        });
+    if (a.first_pass != 0u && valid && part == 0u) a.crowded[i] = static_cast<uint8_t>(crowd[expanded]);
+    if (!active) return ~0u;
+    if (crowd[walked] != 0u) {
+        int cx, cy, cz;
+        particle_cell(scene.grid, load(a.topo, w), cx, cy, cz);
+        const Float3 own = load(a.pos, w);
+        group_walk_stencil<G, F>(
+            scene.grid, kSamples ? samples.offsets : nullptr, cx, cy, cz, skip, w, group_row(lds),
+            [&](uint32_t entry) { return near(own, entry_position<kSamples>(a.pos, samples, entry)); }, load_record,
+            pair, fold);
+    }
+    return w;
+}
+
+// A later walk at the same positions, over the exact masks of the first one;
+// the samples near the particle are scanned again. The particle itself is
+// left out.
+template <int G, bool kSamples, int F, class Args, class Load, class Pair, class Fold>
+__device__ __forceinline__ uint32_t group_exact_walk(const Args& a, const GroupScene& scene, GroupLds<G>& lds,
+                                                     const BoundaryGrid& samples, float t_exact, Load&& load_record,
+                                                     Pair&& pair, Fold&& fold) {
+    constexpr uint32_t kParticles = kGroupParticles<G>;
+    const uint32_t expanded = threadIdx.x % kParticles;
+    const uint32_t i = scene.base + expanded;
+    bool listed = false;
+    uint32_t center = 0u;
+    [[maybe_unused]] Float3 p{0.0F, 0.0F, 0.0F};
+    [[maybe_unused]] int x = 0, y = 0, z = 0;
+    if (expanded < scene.count) {
+        center = a.cell[i];
+        listed = a.crowded[i] == 0u;
+        if constexpr (kSamples) {
+            p = load(a.pos, i);
+            cell_coordinates(scene.grid, center, x, y, z);
+        }
+    }
+    const uint32_t walked = threadIdx.x / G;
+    const uint32_t w = scene.base + walked;
+    const bool active = walked < scene.count;
+    group_expand<G, kSamples>(
+        lds,
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            return listed ? stored_slot<true>(a.exact, scene.grid.offsets, a.n, i,
+                                              center + slot_delta(scene.grid, k), k, first)
+                          : 0u;
+        },
+        [&](uint32_t, uint32_t k, uint32_t& first) {
+            if (!listed) return 0u;
+            return scanned_slot(scene.grid, samples.offsets, x, y, z, k, first, [&](uint32_t b) {
+                const float4 q = samples.x[b];
+                const Float3 d = sub(p, Float3{q.x, q.y, q.z});
+                return !(dot(d, d) >= t_exact);
+            });
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (active) group_walk_list<G, F>(row, count, w, load_record, pair, fold);
+        });
+    if (!active) return ~0u;
+    if (a.crowded[w] != 0u) {
+        int cx, cy, cz;
+        cell_coordinates(scene.grid, a.cell[w], cx, cy, cz);
+        const Float3 own = load(a.pos, w);
+        group_walk_stencil<G, F>(
+            scene.grid, kSamples ? samples.offsets : nullptr, cx, cy, cz, w, w, group_row(lds),
+            [&](uint32_t entry) {
+                const Float3 d = sub(own, entry_position<kSamples>(a.pos, samples, entry));
+                return !(dot(d, d) >= t_exact);
+            },
+            load_record, pair, fold);
+    }
+    return w;
+}
+
+__device__ __forceinline__ void put(float* terms, Float3 v) {
+    terms[0] = v.x;
+    terms[1] = v.y;
+    terms[2] = v.z;
+}
+
+// density_forward_kernel (density.cu:18-40, poly6) and lambda_forward_kernel
+// (pbf.cu:95-127). With kSamples each cell's boundary samples b add, after
+// its particles, rho0_i V_b W to the density and V_b grad W to the gradient
+// sum (pbf.cu:118-121).
+template <bool kBatch, int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) pbf_lambda_kernel(LambdaArgs a, Schedule schedule, BatchView batch) {
+    constexpr int kSums = 5;
+    __shared__ GroupLds<G> lds;
+    __shared__ uint32_t crowd[kGroupParticles<G>];
+    const uint32_t id = scheduled_block(schedule);
+    if (id == ~0u) return;
+    const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
+    const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
+    const Float3 p = load(a.pos, own);
+    const float rest = a.rho0[own];
+    float sum[kSums] = {0.0F, 0.0F, 0.0F, 0.0F, a.eps[own]};
+    const uint32_t w = group_first_walk<G, kSamples, kSums>(
+        a, scene, lds, crowd, a.boundary, ~0u,
+        [&](uint32_t entry) {
+            if constexpr (kSamples) {
+                if ((entry & kSampleEntry) != 0u) {
+                    const float4 b = a.boundary.x[entry & ~kSampleEntry];
+                    return PointMass{Float3{b.x, b.y, b.z}, b.w};
+                }
+            }
+            return PointMass{load(a.pos, entry), a.m[entry]};
+        },
+        [&](const PointMass& c, uint32_t entry, float (&terms)[kSums]) {
+            const Float3 d = sub(p, c.x);
+            if (kSamples && (entry & kSampleEntry) != 0u) {
+                terms[0] = rest * c.m * poly6(d, a.h);
+                put(terms + 1, scale(spiky_gradient(d, a.h, a.spiky), c.m));
+                return;
+            }
+            const LambdaTerms t = lambda_terms(a, d, c.m, rest);
+            terms[0] = t.density;
+            if (entry != own) {
+                put(terms + 1, t.gradient);
+                terms[4] = t.square;
+            }
+        },
+        [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
+    if (w != ~0u && threadIdx.x % G == 0u)
+        finish_lambda(a, w, rest, sum[0], Float3{sum[1], sum[2], sum[3]}, sum[4]);
 }
 
 struct CorrectionArgs {
@@ -230,89 +426,85 @@ struct CorrectionArgs {
     CVec x0;
     float inv_dt;
     Vec vel;
-    MaskView mv;
-    uint32_t slot;           // displacement slot of the positions read
-    uint32_t* moved_to;      // largest squared displacement of the output from x*
-    uint32_t* cell_moved;    // optional: per-cell displacement bounds of the output (MaskView::cell_moved)
-    BoundaryGrid boundary;   // offsets null: no boundary samples
+    const uint16_t* exact;  // exact masks of the positions read
+    BoundaryGrid boundary;  // offsets null: no boundary samples
+    const uint32_t* cell;   // LambdaArgs::cell and crowded
+    const uint8_t* crowded;
+    float t_exact;
 };
 
-// correction_forward_kernel (pbf.cu:254-288) and project_forward_kernel
-// (pbf.cu:417-431), plus the largest displacement of the projected positions
-// from x* for the mask checks of later passes. A boundary sample b adds
-// V_b (lambda_i + s_corr(d)) grad W after each cell's particles
-// (pbf.cu:278-284).
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_correction_kernel(CorrectionArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, a.box, batch);
-    PHX_MASK_LDS(lane.grid);
-    const uint32_t i = lane.i;
-    const SortedGrid& grid = lane.grid;
-    const Box& box = lane.box;
-    float moved2 = 0.0F;
-    uint32_t moved_cell = ~0u;
-    float moved_bound = 0.0F;
-    if (lane.valid) {
-        const bool masked = masks_apply(a.mv, a.slot, i);
-        const Float3 p = load(a.pos, i);
-        const float rest = a.rho0[i];
-        const float lambda_i = a.lambda[i];
-        const float strength = a.strength[i];
-        const float exponent = a.exponent[i];
-        const float reference = poly6(Float3{a.radius[i], 0.0F, 0.0F}, a.h);
-        // with k = +-0 the term is -k wherever W(d) > 0 (no powf per pair)
-        const bool vanishes = artificial_vanishes(a.h, strength, exponent, reference);
-        int cx, cy, cz;
-        particle_cell(grid, load(a.topo, i), cx, cy, cz);
-        Float3 correction{0.0F, 0.0F, 0.0F};
-        auto artificial_at = [&](Float3 d) {
-            return vanishes ? (poly6(d, a.h) == 0.0F ? 0.0F : -strength)
-                            : artificial_value(d, a.h, strength, exponent, reference);
-        };
-        auto pair = [&](Float3 q, float ms, float lambda_s, uint32_t s) {
-            if (s == i) return;
-            const Float3 d = sub(p, q);
-            const float artificial = artificial_at(d);
-            const float coefficient = ms / rest;
-            correction = add(correction, scale(spiky_gradient(d, a.h, a.spiky),
-                                               coefficient * (lambda_i + lambda_s + artificial)));
-        };
-        auto visit = [&](uint32_t s) { pair(load(a.pos, s), a.m[s], a.lambda[s], s); };
-        if (a.boundary.offsets != nullptr) {
-            for_each_candidate(grid, a.boundary, cx, cy, cz, visit, [&](uint32_t s) {
-                const float4 b = a.boundary.x[s];
-                const Float3 d = sub(p, Float3{b.x, b.y, b.z});
-                const float artificial = artificial_at(d);
-                correction = add(correction, scale(spiky_gradient(d, a.h, a.spiky), b.w * (lambda_i + artificial)));
-            });
-        } else {
-            visit_records<kPbfWalkDepth<kBatch>>(
-                grid, a.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock,
-                [&](uint32_t s) { return PointMassLambda{load(a.pos, s), a.m[s], a.lambda[s]}; },
-                [&](const PointMassLambda& c, uint32_t s) { pair(c.x, c.m, c.lambda, s); });
-        }
-        const Float3 candidate = add(p, correction);
-        if (a.mask != nullptr) {
-            uint32_t bits = 0u;
-            if (candidate.x < box.lo[0] || candidate.x > box.hi[0]) bits |= 1u;
-            if (candidate.y < box.lo[1] || candidate.y > box.hi[1]) bits |= 2u;
-            if (candidate.z < box.lo[2] || candidate.z > box.hi[2]) bits |= 4u;
-            a.mask[i] = static_cast<uint8_t>(bits);
-        }
-        const Float3 projected{fminf(box.hi[0], fmaxf(box.lo[0], candidate.x)),
-                               fminf(box.hi[1], fmaxf(box.lo[1], candidate.y)),
-                               fminf(box.hi[2], fmaxf(box.lo[2], candidate.z))};
-        store(a.out, i, projected);
-        if (a.reconstruct != 0u) store(a.vel, i, scale(sub(projected, load(a.x0, i)), a.inv_dt));
-        const Float3 moved = sub(projected, load(a.topo, i));
-        moved2 = dot(moved, moved);
-        if (a.cell_moved != nullptr) {
-            moved_cell = static_cast<uint32_t>(grid.offsets - a.grid.offsets) + cell_of(grid, cx, cy, cz);
-            moved_bound = displacement_bound(moved);
-        }
+// The artificial pressure of a particle, as its correction pass evaluates it.
+struct ArtificialPressure {
+    float strength, exponent, reference;
+    bool vanishes;  // with k = +-0 the term is -k wherever W(d) > 0 (no powf per pair)
+};
+__device__ __forceinline__ ArtificialPressure artificial_of(const CorrectionArgs& a, uint32_t i) {
+    ArtificialPressure s{a.strength[i], a.exponent[i], poly6(Float3{a.radius[i], 0.0F, 0.0F}, a.h), false};
+    s.vanishes = artificial_vanishes(a.h, s.strength, s.exponent, s.reference);
+    return s;
+}
+__device__ __forceinline__ float artificial_at(const CorrectionArgs& a, const ArtificialPressure& s, Float3 d) {
+    return s.vanishes ? (poly6(d, a.h) == 0.0F ? 0.0F : -s.strength)
+                      : artificial_value(d, a.h, s.strength, s.exponent, s.reference);
+}
+
+// project_forward_kernel (pbf.cu:417-431) of particle i at p with its
+// correction.
+__device__ __forceinline__ void finish_correction(const CorrectionArgs& a, const Box& box, uint32_t i, Float3 p,
+                                                    Float3 correction) {
+    const Float3 candidate = add(p, correction);
+    if (a.mask != nullptr) {
+        uint32_t bits = 0u;
+        if (candidate.x < box.lo[0] || candidate.x > box.hi[0]) bits |= 1u;
+        if (candidate.y < box.lo[1] || candidate.y > box.hi[1]) bits |= 2u;
+        if (candidate.z < box.lo[2] || candidate.z > box.hi[2]) bits |= 4u;
+        a.mask[i] = static_cast<uint8_t>(bits);
     }
-    if (a.cell_moved != nullptr) raise_cell_bound(a.cell_moved, moved_cell, moved_bound);
-    block_max_to<kBlock>(moved2, a.moved_to);
+    const Float3 projected{fminf(box.hi[0], fmaxf(box.lo[0], candidate.x)),
+                           fminf(box.hi[1], fmaxf(box.lo[1], candidate.y)),
+                           fminf(box.hi[2], fmaxf(box.lo[2], candidate.z))};
+    store(a.out, i, projected);
+    if (a.reconstruct != 0u) store(a.vel, i, scale(sub(projected, load(a.x0, i)), a.inv_dt));
+}
+
+// correction_forward_kernel (pbf.cu:254-288) and project_forward_kernel. With
+// kSamples a boundary sample b adds V_b (lambda_i + s_corr(d)) grad W after
+// each cell's particles (pbf.cu:278-284).
+template <bool kBatch, int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) pbf_correction_kernel(CorrectionArgs a, Schedule schedule, BatchView batch) {
+    constexpr int kSums = 3;
+    __shared__ GroupLds<G> lds;
+    const uint32_t id = scheduled_block(schedule);
+    if (id == ~0u) return;
+    const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, a.box, batch);
+    const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
+    const Float3 p = load(a.pos, own);
+    const float rest = a.rho0[own];
+    const float lambda_i = a.lambda[own];
+    const ArtificialPressure pressure = artificial_of(a, own);
+    float sum[kSums] = {0.0F, 0.0F, 0.0F};
+    const uint32_t w = group_exact_walk<G, kSamples, kSums>(
+        a, scene, lds, a.boundary, a.t_exact,
+        [&](uint32_t entry) {
+            if constexpr (kSamples) {
+                if ((entry & kSampleEntry) != 0u) {
+                    const float4 b = a.boundary.x[entry & ~kSampleEntry];
+                    return PointMassLambda{Float3{b.x, b.y, b.z}, b.w, 0.0F};
+                }
+            }
+            return PointMassLambda{load(a.pos, entry), a.m[entry], a.lambda[entry]};
+        },
+        [&](const PointMassLambda& c, uint32_t entry, float (&terms)[kSums]) {
+            const Float3 d = sub(p, c.x);
+            const float artificial = artificial_at(a, pressure, d);
+            const float factor = kSamples && (entry & kSampleEntry) != 0u
+                                     ? c.m * (lambda_i + artificial)
+                                     : c.m / rest * (lambda_i + c.lambda + artificial);
+            put(terms, scale(spiky_gradient(d, a.h, a.spiky), factor));
+        },
+        [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
+    if (w != ~0u && threadIdx.x % G == 0u)
+        finish_correction(a, scene.box, w, p, Float3{sum[0], sum[1], sum[2]});
 }
 
 __global__ void __launch_bounds__(kBlock) pbf_reconstruct_kernel(uint32_t n, CVec pos, CVec x0, float inv_dt, Vec vel) {
@@ -339,70 +531,23 @@ struct PostArgs {
     const float* xsph;
     const uint32_t* perm;
     Vec next_x, next_v;
-    MaskView mv;
-    uint32_t slot;  // displacement slot of the final positions
     // exact masks of the final positions: written by the vorticity pass and
-    // walked by the normal and XSPH passes (through mv, slot 0)
+    // walked by the normal and XSPH passes
     float t_exact;
     uint16_t* exact_out;
-    uint32_t* exact_flags;
+    const uint16_t* exact;
+    // LambdaArgs::cell, crowded and first_pass
+    uint32_t* cell;
+    uint8_t* crowded;
+    uint32_t first_pass;
 };
 
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_vorticity_kernel(PostArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, Box{}, batch);
-    PHX_MASK_LDS(lane.grid);
-    const uint32_t i = lane.i;
-    if (!lane.valid) return;
-    const SortedGrid& grid = lane.grid;
-    const MaskView mv = lane_masks(a.mv, a.grid, grid);
-    const Float3 p = load(a.pos, i);
-    const Float3 v = load(a.vel, i);
-    const Float3 x_star = load(a.topo, i);
-    int cx, cy, cz;
-    particle_cell(grid, x_star, cx, cy, cz);
-    const bool masked =
-        masks_apply(mv, a.slot, i, grid, cx, cy, cz, [&] { return displacement_bound(sub(p, x_star)); });
-    Float3 w{0.0F, 0.0F, 0.0F};
-    auto pair = [&](Float3 q, Float3 vq, uint32_t s) {
-        const Float3 d = sub(p, q);
-        if (s != i) w = add(w, cross(sub(vq, v), spiky_gradient(d, a.h, a.spiky)));
-        return dot(d, d) < a.t_exact;
-    };
-    auto near = [&](uint32_t s) {
-        const Float3 d = sub(p, load(a.pos, s));
-        return !(dot(d, d) >= a.t_exact);
-    };
-    const bool complete = visit_records_and_mask<kPbfWalkDepth<kBatch>>(
-        grid, mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, a.exact_out, a.n, near,
-        [&](uint32_t s) { return PointVector{load(a.pos, s), load(a.vel, s)}; },
-        [&](const PointVector& c, uint32_t s) { return pair(c.x, c.v, s); });
-    flag_incomplete(complete, mv, i, &a.exact_flags[kFlagOverflow]);
+__device__ __forceinline__ void finish_vorticity(const PostArgs& a, uint32_t i, Float3 w) {
     store(a.vort, i, w);
     a.magnitude[i] = length(w);
 }
 
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_normal_kernel(PostArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, Box{}, batch);
-    PHX_MASK_LDS(lane.grid);
-    const uint32_t i = lane.i;
-    if (!lane.valid) return;
-    const SortedGrid& grid = lane.grid;
-    const bool masked = masks_apply(a.mv, a.slot, i);
-    const Float3 p = load(a.pos, i);
-    const float mag_i = a.magnitude[i];
-    int cx, cy, cz;
-    particle_cell(grid, load(a.topo, i), cx, cy, cz);
-    Float3 g{0.0F, 0.0F, 0.0F};
-    auto pair = [&](Float3 q, float mag_s, uint32_t s) {
-        if (s == i) return;
-        g = add(g, scale(spiky_gradient(sub(p, q), a.h, a.spiky), mag_s - mag_i));
-    };
-    visit_records<kPbfWalkDepth<kBatch>>(
-        grid, a.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock,
-        [&](uint32_t s) { return PointMass{load(a.pos, s), a.magnitude[s]}; },
-        [&](const PointMass& c, uint32_t s) { pair(c.x, c.m, s); });
+__device__ __forceinline__ void finish_normal(const PostArgs& a, uint32_t i, Float3 g) {
     const float normalizer = length(g);
     const Float3 normal = normalizer > 0.0F ? scale(g, 1.0F / normalizer) : Float3{0.0F, 0.0F, 0.0F};
     if (a.normalizers != nullptr) {
@@ -413,32 +558,137 @@ __global__ void __launch_bounds__(kBlock) pbf_normal_kernel(PostArgs a, BatchVie
     store(a.vc, i, add(load(a.vel, i), scale(cross(normal, w), a.dt * a.confinement[i])));
 }
 
-template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_xsph_kernel(PostArgs a, BatchView batch) {
-    const Lane lane = lane_of<kBatch>(a.n, a.grid, Box{}, batch);
-    PHX_MASK_LDS(lane.grid);
-    const uint32_t i = lane.i;
-    if (!lane.valid) return;
-    const SortedGrid& grid = lane.grid;
-    const bool masked = masks_apply(a.mv, a.slot, i);
-    const CVec vc{a.vc.x, a.vc.y, a.vc.z};
-    const Float3 p = load(a.pos, i);
-    const Float3 v = load(vc, i);
-    int cx, cy, cz;
-    particle_cell(grid, load(a.topo, i), cx, cy, cz);
-    Float3 smoothing{0.0F, 0.0F, 0.0F};
-    auto pair = [&](Float3 q, Float3 vq, uint32_t s) {
-        if (s == i) return;
-        smoothing = add(smoothing, scale(sub(vq, v), poly6(sub(p, q), a.h)));
-    };
-    visit_records<kPbfWalkDepth<kBatch>>(
-        grid, a.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock,
-        [&](uint32_t s) { return PointVector{load(a.pos, s), load(vc, s)}; },
-        [&](const PointVector& c, uint32_t s) { pair(c.x, c.v, s); });
+__device__ __forceinline__ void finish_xsph(const PostArgs& a, uint32_t i, Float3 p, Float3 v, Float3 smoothing) {
     const uint32_t j = a.perm[i];
     store(a.next_v, j, add(v, scale(smoothing, a.xsph[i])));
     store(a.next_x, j, p);
 }
+
+template <bool kBatch, int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vorticity_kernel(PostArgs a, Schedule schedule, BatchView batch) {
+    constexpr int kSums = 3;
+    __shared__ GroupLds<G> lds;
+    __shared__ uint32_t crowd[kGroupParticles<G>];
+    const uint32_t id = scheduled_block(schedule);
+    if (id == ~0u) return;
+    const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
+    const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
+    const Float3 p = load(a.pos, own);
+    const Float3 v = load(a.vel, own);
+    float sum[kSums] = {0.0F, 0.0F, 0.0F};
+    const uint32_t w = group_first_walk<G, false, kSums>(
+        a, scene, lds, crowd, BoundaryGrid{}, own,
+        [&](uint32_t s) { return PointVector{load(a.pos, s), load(a.vel, s)}; },
+        [&](const PointVector& c, uint32_t s, float (&terms)[kSums]) {
+            if (s != own) put(terms, cross(sub(c.v, v), spiky_gradient(sub(p, c.x), a.h, a.spiky)));
+        },
+        [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
+    if (w != ~0u && threadIdx.x % G == 0u) finish_vorticity(a, w, Float3{sum[0], sum[1], sum[2]});
+}
+
+template <bool kBatch, int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_normal_kernel(PostArgs a, Schedule schedule, BatchView batch) {
+    constexpr int kSums = 3;
+    __shared__ GroupLds<G> lds;
+    const uint32_t id = scheduled_block(schedule);
+    if (id == ~0u) return;
+    const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
+    const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
+    const Float3 p = load(a.pos, own);
+    const float mag_i = a.magnitude[own];
+    float sum[kSums] = {0.0F, 0.0F, 0.0F};
+    const uint32_t w = group_exact_walk<G, false, kSums>(
+        a, scene, lds, BoundaryGrid{}, a.t_exact,
+        [&](uint32_t s) { return PointMass{load(a.pos, s), a.magnitude[s]}; },
+        [&](const PointMass& c, uint32_t, float (&terms)[kSums]) {
+            put(terms, scale(spiky_gradient(sub(p, c.x), a.h, a.spiky), c.m - mag_i));
+        },
+        [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
+    if (w != ~0u && threadIdx.x % G == 0u) finish_normal(a, w, Float3{sum[0], sum[1], sum[2]});
+}
+
+template <bool kBatch, int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_xsph_kernel(PostArgs a, Schedule schedule, BatchView batch) {
+    constexpr int kSums = 3;
+    __shared__ GroupLds<G> lds;
+    const uint32_t id = scheduled_block(schedule);
+    if (id == ~0u) return;
+    const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
+    const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
+    const CVec vc{a.vc.x, a.vc.y, a.vc.z};
+    const Float3 p = load(a.pos, own);
+    const Float3 v = load(vc, own);
+    float sum[kSums] = {0.0F, 0.0F, 0.0F};
+    const uint32_t w = group_exact_walk<G, false, kSums>(
+        a, scene, lds, BoundaryGrid{}, a.t_exact,
+        [&](uint32_t s) { return PointVector{load(a.pos, s), load(vc, s)}; },
+        [&](const PointVector& c, uint32_t, float (&terms)[kSums]) {
+            put(terms, scale(sub(c.v, v), poly6(sub(p, c.x), a.h)));
+        },
+        [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
+    if (w != ~0u && threadIdx.x % G == 0u) finish_xsph(a, w, p, v, Float3{sum[0], sum[1], sum[2]});
+}
+
+// Lanes per particle of a step's passes.
+inline int pbf_group(uint32_t n) { return n <= kGroup16Particles ? 16 : 4; }
+
+// Workgroups of a pass over n particles, padded to a multiple of the XCD count.
+inline uint32_t pbf_blocks(uint32_t n, int group) {
+    return (blocks_for(n, kBlock / static_cast<uint32_t>(group)) + 7u) / 8u * 8u;
+}
+
+// The launches of a step's passes with `group` lanes per particle over
+// `blocks` blocks (the schedule's early ones included).
+template <bool kBatch>
+struct PassLauncher {
+    int group;
+    uint32_t blocks;
+    hipStream_t stream;
+    Schedule schedule;
+    BatchView batch;
+
+    // launch(std::integral_constant<int, G>) with G the launch's group
+    template <class Launch>
+    void with_group(Launch&& launch) const {
+        if (group == 16) {
+            launch(std::integral_constant<int, 16>{});
+        } else {
+            launch(std::integral_constant<int, 4>{});
+        }
+        PHX_LAUNCH_CHECK();
+    }
+    void lambda(const LambdaArgs& a) const {
+        with_group([&](auto g) {
+            if constexpr (!kBatch) {
+                if (a.boundary.offsets != nullptr) {
+                    pbf_lambda_kernel<false, g(), true><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch);
+                    return;
+                }
+            }
+            pbf_lambda_kernel<kBatch, g(), false><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch);
+        });
+    }
+    void correction(const CorrectionArgs& a) const {
+        with_group([&](auto g) {
+            if constexpr (!kBatch) {
+                if (a.boundary.offsets != nullptr) {
+                    pbf_correction_kernel<false, g(), true><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch);
+                    return;
+                }
+            }
+            pbf_correction_kernel<kBatch, g(), false><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch);
+        });
+    }
+    void vorticity(const PostArgs& a) const {
+        with_group([&](auto g) { pbf_vorticity_kernel<kBatch, g()><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch); });
+    }
+    void normal(const PostArgs& a) const {
+        with_group([&](auto g) { pbf_normal_kernel<kBatch, g()><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch); });
+    }
+    void xsph(const PostArgs& a) const {
+        with_group([&](auto g) { pbf_xsph_kernel<kBatch, g()><<<blocks, kGroupBlock, 0, stream>>>(a, schedule, batch); });
+    }
+};
 
 }  // namespace
 
@@ -490,9 +740,7 @@ void PbfCache::allocate(uint32_t n, uint32_t cells, uint32_t pressure_iterations
     den.resize(per);
     masks.resize(per);
     normalizers.resize(n);
-    masks_skin.resize(static_cast<size_t>(kStencil) * n);
     crowded.resize(n);
-    mask_flags.resize(kFlagDisplacement + pressure_iterations + 1u);
     exact_masks.resize(static_cast<size_t>(pressure_iterations + 1u) * kStencil * n);
     exact_flags.resize(pressure_iterations + 1u);
 }
@@ -515,9 +763,7 @@ PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_confi
         b->resize(n);
     exact_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
-    exact_flags_.resize(config_.pressure_iterations + 1u);
-    // displacement slots: one per iterate (the first, x* itself, stays zero)
-    masks_.allocate(n, config_.pressure_iterations + 1u, domain_.config.support_radius);
+    cells_.resize(n);
 }
 
 void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& control,
@@ -573,52 +819,52 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
         PassScope scope(profiler_, stream_, kPbfGrid);
         cache.neighborhood.build(stream_, domain_, step + 1u, cvec(state.particles.positions), &predict,
                                  gather.get(), &boundary_);
-        masks_.begin_step(stream_);
     }
 
     const SortedGrid grid = cache.neighborhood.grid();
     const BoundaryGrid boundary = cache.neighborhood.boundary();
-    const bool with_boundary = boundary.offsets != nullptr;
-    // whole blocks of kBlock particles, padded to a multiple of the XCD count
-    const uint32_t blocks = (blocks_for(n, kBlock) + 7u) / 8u * 8u;
+    const int group = pbf_group(n);
+    // a large scene serves workgroups with crowded particles first; its cells
+    // are then found by a launch of their own
+    const bool ordered = n >= kEarlyParticles;
+    const uint32_t group_blocks = pbf_blocks(n, group);
+    Schedule schedule{};
+    if (ordered) {
+        schedule_.resize(1u + kEarlyBlocks + 2u * static_cast<size_t>(group_blocks));
+        schedule = Schedule{schedule_.data(), schedule_.data() + 1u, schedule_.data() + 1u + kEarlyBlocks,
+                            schedule_.data() + 1u + kEarlyBlocks + group_blocks, kEarlyBlocks};
+    }
+    const PassLauncher<false> launch{group, group_blocks + schedule.early, stream_, schedule, BatchView{}};
     const float h = c.support_radius;
     const float inv_dt = 1.0F / c.time_step;
-    // a recorded step keeps its masks and flags for its derivative passes
-    uint16_t* skin = rec ? cache.masks_skin.data() : masks_.skin_mask();
+    // a recorded step keeps its exact masks for its derivative passes
     uint8_t* crowded = rec ? cache.crowded.data() : crowded_.data();
-    {
+    if (ordered) {
         PassScope scope(profiler_, stream_, kPbfMask);
-        MaskArgs ma{n, grid, xs.cview(), masks_.t_skin(), skin, crowded};
-        pbf_mask_kernel<false><<<blocks, kBlock, 0, stream_>>>(ma, BatchView{});
+        fill_u32(stream_, schedule_.data(), schedule_.size(), 0u);
+        pbf_cell_kernel<false><<<pbf_blocks(n, 1), kBlock, 0, stream_>>>(n, grid, xs.cview(), cells_.data(), crowded,
+                                                                         kBlock / static_cast<uint32_t>(group), schedule,
+                                                                         BatchView{});
         PHX_LAUNCH_CHECK();
     }
-    // the skin adapts to the largest displacement of the previous step, so
-    // the step-wide limit holds nearly always: no per-cell bounds (the
-    // batch's fixed skin uses them)
-    MaskView mv{skin, masks_.flags(), n, masks_.limit2()};
-    mv.crowded = crowded;
     // exact masks of position set k (iterate k, the final positions last):
     // written by the pass that first walks those positions, walked by the
-    // later passes at them; a recorded step keeps every set. Each set has one
-    // overflow word.
+    // later passes at them; a recorded step keeps every set. Each recorded set
+    // has one overflow word.
     const float t_exact = exact_mask_threshold(h);
     const uint32_t sets = config_.pressure_iterations + 1u;
-    uint32_t* exact_flags = rec ? cache.exact_flags.data() : exact_flags_.data();
-    fill_u32(stream_, exact_flags, sets, 0u);
-    // with boundary samples the iterations' passes walk the full stencil and
-    // write no exact masks; the final positions' set (vorticity, normal,
-    // XSPH: no boundary terms) is built as usual
-    if (with_boundary && sets > 1u) fill_u32(stream_, exact_flags, sets - 1u, 1u);
+    if (rec) fill_u32(stream_, cache.exact_flags.data(), sets, 0u);
     auto exact_set = [&](uint32_t k) {
         require(k < sets, PHX_ERROR_INVALID_ARGUMENT, "exact mask set out of range");
         return rec ? cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n : exact_.data();
     };
-    auto exact_view = [&](uint32_t k) { return MaskView{exact_set(k), exact_flags + k, n, 0.0F, 1u, crowded}; };
 
     LambdaArgs la{n,           h,        spiky_,     grid, xs.cview(), xs.cview(), m_.data(), rho0_.data(),
-                  eps_.data(), cache.densities.data(), cache.lambdas.data(), nullptr, Vec{}, mv, 0u};
+                  eps_.data(), cache.densities.data(), cache.lambdas.data(), nullptr, Vec{}};
     la.t_exact = t_exact;
     la.boundary = boundary;
+    la.cell = cells_.data();
+    la.crowded = crowded;
     CorrectionArgs ca{};
     ca.n = n;
     ca.h = h;
@@ -635,8 +881,10 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     ca.x0 = x0.cview();
     ca.inv_dt = inv_dt;
     ca.vel = vel.view();
-    ca.mv = mv;
     ca.boundary = boundary;
+    ca.cell = cells_.data();
+    ca.crowded = crowded;
+    ca.t_exact = t_exact;
 
     // positions start at x* (pbf.cpp:171) and ping-pong between two buffers
     // (a recorded step keeps every iterate)
@@ -645,12 +893,9 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     const uint32_t iterations = config_.pressure_iterations;
     for (uint32_t it = 0; it < iterations; ++it) {
         la.pos = current;
-        la.slot = it;
+        la.first_pass = it == 0u && !ordered ? 1u : 0u;
         la.exact_out = exact_set(it);
-        la.exact_flags = exact_flags + it;
-        ca.mv = exact_view(it);
-        ca.slot = 0u;
-        ca.moved_to = masks_.flags() + kFlagDisplacement + it + 1u;
+        ca.exact = exact_set(it);
         if (rec) {
             const size_t off = static_cast<size_t>(it) * n;
             la.rho = cache.rho.data() + off;
@@ -662,8 +907,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
         }
         {
             PassScope scope(profiler_, stream_, kPbfLambda);
-            pbf_lambda_kernel<false><<<blocks, kBlock, 0, stream_>>>(la, BatchView{});
-            PHX_LAUNCH_CHECK();
+            launch.lambda(la);
         }
         const Vec target = rec ? cache.positions.view(it) : targets[it & 1u]->view();
         ca.pos = current;
@@ -671,8 +915,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
         ca.reconstruct = it + 1u == iterations ? 1u : 0u;
         {
             PassScope scope(profiler_, stream_, kPbfCorrection);
-            pbf_correction_kernel<false><<<blocks, kBlock, 0, stream_>>>(ca, BatchView{});
-            PHX_LAUNCH_CHECK();
+            launch.correction(ca);
         }
         current = CVec{target.x, target.y, target.z};
     }
@@ -685,7 +928,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
                                hipMemcpyDeviceToDevice, stream_));
     }
     if (iterations == 0u) {
-        pbf_reconstruct_kernel<<<blocks, kBlock, 0, stream_>>>(n, current, x0.cview(), inv_dt, vel.view());
+        pbf_reconstruct_kernel<<<pbf_blocks(n, 1), kBlock, 0, stream_>>>(n, current, x0.cview(), inv_dt, vel.view());
         PHX_LAUNCH_CHECK();
     }
 
@@ -708,41 +951,31 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     }
     post.xsph = xsph_.data();
     post.perm = cache.neighborhood.perm.data();
-    post.mv = mv;
-    post.slot = iterations;
     post.t_exact = t_exact;
     post.exact_out = exact_set(iterations);
-    post.exact_flags = exact_flags + iterations;
+    post.exact = exact_set(iterations);
+    post.cell = cells_.data();
+    post.crowded = crowded;
+    post.first_pass = iterations == 0u && !ordered ? 1u : 0u;
     post.next_x = vec(next.particles.positions);
     post.next_v = vec(next.particles.velocities);
-    // the normal and XSPH passes: every field of `post`, with the exact masks
-    PostArgs post_exact = post;
-    post_exact.mv = exact_view(iterations);
-    post_exact.slot = 0u;
     {
         PassScope scope(profiler_, stream_, kPbfVorticity);
-        pbf_vorticity_kernel<false><<<blocks, kBlock, 0, stream_>>>(post, BatchView{});
-        PHX_LAUNCH_CHECK();
+        launch.vorticity(post);
     }
     {
         PassScope scope(profiler_, stream_, kPbfNormal);
-        pbf_normal_kernel<false><<<blocks, kBlock, 0, stream_>>>(post_exact, BatchView{});
-        PHX_LAUNCH_CHECK();
+        launch.normal(post);
     }
     {
         PassScope scope(profiler_, stream_, kPbfXsph);
-        pbf_xsph_kernel<false><<<blocks, kBlock, 0, stream_>>>(post_exact, BatchView{});
-        PHX_LAUNCH_CHECK();
+        launch.xsph(post);
     }
     if (rec) {
-        PHX_HIP(hipMemcpyAsync(cache.mask_flags.data(), masks_.flags(), sizeof(uint32_t) * masks_.flag_count(),
-                               hipMemcpyDeviceToDevice, stream_));
-        cache.mask_limit2 = masks_.limit2();
         cache.recorded = true;
         cache.iterations = iterations;
         cache.step_index = step;
     }
-    masks_.end_step(stream_);
     next.particles.step_index = step + 1u;
 }
 
@@ -760,10 +993,10 @@ PbfBatch::PbfBatch(const phx_domain_configuration* domains, uint32_t scene_count
     config_ = *configuration;
     require(config_.pressure_iterations < 1024u, PHX_ERROR_INVALID_ARGUMENT, "too many pressure iterations");
     if (batch_configuration != nullptr) {
+        // accepted as before; the passes keep no skin masks that it would size
         const float skin = batch_configuration->mask_skin;
         require(skin == 0.0F || (skin >= 0.01F && skin <= 1.0F), PHX_ERROR_INVALID_ARGUMENT,
                 "mask_skin must be 0 (default) or in [0.01, 1]");
-        if (skin > 0.0F) skin_ = skin;
         use_graph_ = batch_configuration->use_graph != 0u;
     }
     uint64_t particles = 0, cells = 0;
@@ -808,38 +1041,47 @@ PbfBatch::PbfBatch(const phx_domain_configuration* domains, uint32_t scene_count
     use_graph_ = use_graph_ && static_boxes_;
     spiky_ = spiky_coefficient(h_);
 
-    // workgroup table: each scene's particles in blocks of kBlock, padded to
-    // a multiple of the XCD count
-    std::vector<BatchBlock> table;
-    for (uint32_t k = 0; k < scene_count; ++k) {
-        for (uint64_t first = offsets_[k]; first < offsets_[k + 1]; first += kBlock) {
-            const uint64_t count = std::min<uint64_t>(kBlock, offsets_[k + 1] - first);
-            table.push_back(BatchBlock{k, static_cast<uint32_t>(first), static_cast<uint32_t>(count), 0u});
+    // workgroup tables: each scene's particles in blocks of kBlock (the grid
+    // build) and of the passes' workgroups, padded to a multiple of the XCD count
+    group_ = pbf_group(n_);
+    const uint32_t group_particles = kBlock / static_cast<uint32_t>(group_);
+    auto build_table = [&](uint32_t size, DeviceBuffer<BatchBlock>& device) {
+        std::vector<BatchBlock> table;
+        uint32_t scene_block = 0u;  // the scene's first workgroup of the passes
+        for (uint32_t k = 0; k < scene_count; ++k) {
+            for (uint64_t first = offsets_[k]; first < offsets_[k + 1]; first += size) {
+                const uint64_t count = std::min<uint64_t>(size, offsets_[k + 1] - first);
+                const auto within = static_cast<uint32_t>((first - offsets_[k]) / group_particles);
+                table.push_back(
+                    BatchBlock{k, static_cast<uint32_t>(first), static_cast<uint32_t>(count), scene_block + within});
+            }
+            scene_block += blocks_for(offsets_[k + 1] - offsets_[k], group_particles);
         }
-    }
-    while (table.empty() || table.size() % 8u != 0u) table.push_back(BatchBlock{0u, 0u, 0u, 0u});
-    blocks_ = static_cast<uint32_t>(table.size());
-    block_table_.resize(table.size());
+        while (table.empty() || table.size() % 8u != 0u) table.push_back(BatchBlock{0u, 0u, 0u, 0u});
+        device.resize(table.size());
+        PHX_HIP(hipMemcpy(device.data(), table.data(), sizeof(BatchBlock) * table.size(), hipMemcpyHostToDevice));
+        return static_cast<uint32_t>(table.size());
+    };
+    blocks_ = build_table(kBlock, block_table_);
+    pass_blocks_ = build_table(group_particles, pass_table_);
+    schedule_.resize(1u + kEarlyBlocks);
+    for (DeviceBuffer<uint32_t>* b : {&schedule_place_, &schedule_seen_}) b->resize(pass_blocks_);
     scene_table_.resize(scenes_.size());
-    PHX_HIP(hipMemcpy(block_table_.data(), table.data(), sizeof(BatchBlock) * table.size(), hipMemcpyHostToDevice));
     PHX_HIP(hipMemcpy(scene_table_.data(), scenes_.data(), sizeof(BatchScene) * scenes_.size(),
                       hipMemcpyHostToDevice));
 
     const uint32_t n = n_;
     grid_.allocate(n, cells_);
-    cell_moved_.resize(cells_);
     for (VecBuffer* b : {&positions_[0], &positions_[1], &velocities_[0], &velocities_[1], &predicted_, &xs_, &x0_,
                          &pa_, &pb_, &vel_, &vort_, &vc_})
         b->resize(n);
     for (DeviceBuffer<float>* b :
          {&m_, &rho0_, &eps_, &strength_, &exponent_, &radius_, &xsph_, &confinement_, &rho_, &lambda_, &magnitude_})
         b->resize(n);
-    skin_masks_.resize(static_cast<size_t>(kStencil) * n);
     exact_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
-    flags_.resize(kFlagDisplacement + config_.pressure_iterations + 1u);
-    exact_flags_.resize(config_.pressure_iterations + 1u);
-    // grid build 9, flag and cell-bound fills 3, masks 1, two per iteration, three post passes
+    cell_index_.resize(n);
+    // grid build 9, schedule fills 3, cells 1, two per iteration, three post passes
     const uint32_t it = config_.pressure_iterations;
     kernels_per_step_ = 9u + 3u + 1u + 2u * it + (it == 0u ? 1u : 0u) + 3u;
     PHX_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
@@ -897,33 +1139,28 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     build_batch_grid(s, n, cells_, blocks_, bv, x.cview(), predict, gather.get(), grid_.scratch, grid_.perm.data(),
                      grid_.offsets.data());
     kernels_per_step_ += 9u;  // counts fill, key, three scan kernels, scatter, rank, big-cell sort, gather
-    const uint32_t sets = config_.pressure_iterations + 1u;
-    fill_u32(s, flags_.data(), kFlagDisplacement + sets, 0u);
-    fill_u32(s, exact_flags_.data(), sets, 0u);
-    fill_u32(s, cell_moved_.data(), cells_, 0u);
+    const Schedule schedule{schedule_.data(), schedule_.data() + 1u, schedule_place_.data(), schedule_seen_.data(),
+                            kEarlyBlocks};
+    const PassLauncher<true> launch{group_, pass_blocks_ + kEarlyBlocks, s, schedule,
+                                    BatchView{pass_table_.data(), scene_table_.data(), bv.time, h_}};
+    fill_u32(s, schedule_.data(), schedule_.size(), 0u);
+    fill_u32(s, schedule_place_.data(), pass_blocks_, 0u);
+    fill_u32(s, schedule_seen_.data(), pass_blocks_, 0u);
     kernels_per_step_ += 3u;
-
     // the batch's offsets; each lane's grid starts at its scene's cell base
     const SortedGrid grid{grid_.offsets.data(), 0u, 0u, 0u, 0.0F, 0.0F, 0.0F, h_};
-    const float radius = h_ * (1.0F + skin_);
-    const float t_skin = radius * radius * (1.0F + 1e-5F);
-    const float limit = 0.5F * (radius - h_ * (1.0F + 2e-5F));
-    const float limit2 = limit > 0.0F ? limit * limit : -1.0F;
-    MaskArgs ma{n, grid, xs_.cview(), t_skin, skin_masks_.data(), crowded_.data()};
-    pbf_mask_kernel<true><<<blocks_, kBlock, 0, s>>>(ma, bv);
+    pbf_cell_kernel<true><<<blocks_, kBlock, 0, s>>>(n, grid, xs_.cview(), cell_index_.data(), crowded_.data(),
+                                                     kBlock / static_cast<uint32_t>(group_), schedule, bv);
     PHX_LAUNCH_CHECK();
     ++kernels_per_step_;
-    MaskView mv{skin_masks_.data(), flags_.data(), n, limit2};
-    mv.crowded = crowded_.data();
-    mv.cell_moved = cell_moved_.data();
-    mv.pair_limit = 2.0F * limit;
-    const MaskView exact_view{exact_.data(), exact_flags_.data(), n, 0.0F, 1u, crowded_.data()};
     const float t_exact = exact_mask_threshold(h_);
 
     LambdaArgs la{n,           h_,         spiky_,        grid, xs_.cview(), xs_.cview(), m_.data(), rho0_.data(),
-                  eps_.data(), rho_.data(), lambda_.data(), nullptr, Vec{},       mv,          0u};
+                  eps_.data(), rho_.data(), lambda_.data(), nullptr, Vec{}};
     la.t_exact = t_exact;
     la.exact_out = exact_.data();
+    la.cell = cell_index_.data();
+    la.crowded = crowded_.data();
     CorrectionArgs ca{};
     ca.n = n;
     ca.h = h_;
@@ -939,9 +1176,10 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     ca.x0 = x0_.cview();
     ca.inv_dt = 1.0F / dt_;
     ca.vel = vel_.view();
-    ca.mv = exact_view;
-    ca.slot = 0u;
-    ca.cell_moved = cell_moved_.data();
+    ca.exact = exact_.data();
+    ca.cell = cell_index_.data();
+    ca.crowded = crowded_.data();
+    ca.t_exact = t_exact;
     // the exact masks of each set of positions are rebuilt by the pass that
     // first walks them, so one buffer serves every set in forward mode
     CVec current = xs_.cview();
@@ -949,18 +1187,12 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     const uint32_t iterations = config_.pressure_iterations;
     for (uint32_t it = 0; it < iterations; ++it) {
         la.pos = current;
-        la.slot = it;
-        la.exact_flags = exact_flags_.data() + it;
-        ca.mv.flags = exact_flags_.data() + it;
-        ca.moved_to = flags_.data() + kFlagDisplacement + it + 1u;
-        pbf_lambda_kernel<true><<<blocks_, kBlock, 0, s>>>(la, bv);
-        PHX_LAUNCH_CHECK();
+        launch.lambda(la);
         const Vec target = targets[it & 1u]->view();
         ca.pos = current;
         ca.out = target;
         ca.reconstruct = it + 1u == iterations ? 1u : 0u;
-        pbf_correction_kernel<true><<<blocks_, kBlock, 0, s>>>(ca, bv);
-        PHX_LAUNCH_CHECK();
+        launch.correction(ca);
         kernels_per_step_ += 2u;
         current = CVec{target.x, target.y, target.z};
     }
@@ -985,23 +1217,16 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     post.vc = vc_.view();
     post.xsph = xsph_.data();
     post.perm = grid_.perm.data();
-    post.mv = mv;
-    post.slot = iterations;
     post.t_exact = t_exact;
     post.exact_out = exact_.data();
-    post.exact_flags = exact_flags_.data() + iterations;
+    post.exact = exact_.data();
+    post.cell = cell_index_.data();
+    post.crowded = crowded_.data();
     post.next_x = next_x.view();
     post.next_v = next_v.view();
-    PostArgs post_exact = post;
-    post_exact.mv = exact_view;
-    post_exact.mv.flags = exact_flags_.data() + iterations;
-    post_exact.slot = 0u;
-    pbf_vorticity_kernel<true><<<blocks_, kBlock, 0, s>>>(post, bv);
-    PHX_LAUNCH_CHECK();
-    pbf_normal_kernel<true><<<blocks_, kBlock, 0, s>>>(post_exact, bv);
-    PHX_LAUNCH_CHECK();
-    pbf_xsph_kernel<true><<<blocks_, kBlock, 0, s>>>(post_exact, bv);
-    PHX_LAUNCH_CHECK();
+    launch.vorticity(post);
+    launch.normal(post);
+    launch.xsph(post);
     kernels_per_step_ += 3u;
 }
 }  // namespace phx

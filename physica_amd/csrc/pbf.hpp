@@ -51,12 +51,7 @@ struct PbfCache {
     VecBuffer velocities, vorticities, normals, confined;
     DeviceBuffer<float> magnitudes;  // vorticity magnitudes (cell order), every mode
     DeviceBuffer<float> normalizers;
-    // the step's neighbour masks and mask flags, so the derivative passes
-    // walk the same candidates as the forward passes
-    DeviceBuffer<uint16_t> masks_skin;
     DeviceBuffer<uint8_t> crowded;  // per particle: walks the full stencil (a stencil cell overflows the masks)
-    DeviceBuffer<uint32_t> mask_flags;
-    float mask_limit2 = -1.0F;
     // exact masks of every set of positions (iterates 0 .. I - 1, then the
     // final positions), [set][kStencil][n], and one overflow word per set
     DeviceBuffer<uint16_t> exact_masks;
@@ -126,14 +121,14 @@ class PbfSolver {
     hipStream_t stream_;
     float spiky_ = 0.0F;
     PassProfiler profiler_;
-    MaskSet masks_;
     BoundarySamples boundary_;  // the domain's boundary samples on the device
     // sorted-order workspace
     VecBuffer xs_, x0_, pa_, pb_, vel_, vort_, vc_;
     DeviceBuffer<float> m_, rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
     DeviceBuffer<uint16_t> exact_;  // exact masks of the current set of positions (forward mode)
     DeviceBuffer<uint8_t> crowded_;  // per particle: walks the full stencil (forward mode)
-    DeviceBuffer<uint32_t> exact_flags_;
+    DeviceBuffer<uint32_t> cells_;   // per particle: its grid cell
+    DeviceBuffer<uint32_t> schedule_;  // the order of the passes' workgroups (a large scene)
     PbfDerivativeWorkspace dw_;
 };
 
@@ -172,21 +167,22 @@ class PbfBatch {
     hipEvent_t ready_ = nullptr, done_ = nullptr;
     std::vector<BatchScene> scenes_;
     std::vector<uint64_t> offsets_;
-    uint32_t n_ = 0, cells_ = 0, blocks_ = 0;
-    float h_ = 0.0F, dt_ = 0.0F, spiky_ = 0.0F, skin_ = 0.3F;
+    uint32_t n_ = 0, cells_ = 0, blocks_ = 0, pass_blocks_ = 0;
+    int group_ = 1;  // lanes per particle of the passes
+    float h_ = 0.0F, dt_ = 0.0F, spiky_ = 0.0F;
     bool static_boxes_ = true, use_graph_ = false;
     uint32_t kernels_per_step_ = 0;
-    DeviceBuffer<BatchBlock> block_table_;
+    DeviceBuffer<BatchBlock> block_table_, pass_table_;
     DeviceBuffer<BatchScene> scene_table_;
     Neighborhood grid_;
     VecBuffer positions_[2], velocities_[2];  // the state in original order, ping-pong
     VecBuffer predicted_, xs_, x0_, pa_, pb_, vel_, vort_, vc_;
     DeviceBuffer<float> m_, rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
     DeviceBuffer<float> rho_, lambda_, magnitude_;
-    DeviceBuffer<uint16_t> skin_masks_, exact_;
+    DeviceBuffer<uint16_t> exact_;
     DeviceBuffer<uint8_t> crowded_;
-    DeviceBuffer<uint32_t> flags_, exact_flags_;
-    DeviceBuffer<uint32_t> cell_moved_;  // per cell: displacement bound of the substep (MaskView::cell_moved)
+    DeviceBuffer<uint32_t> schedule_, schedule_place_, schedule_seen_;  // the order of the passes' workgroups
+    DeviceBuffer<uint32_t> cell_index_;  // per particle: its cell in its scene's grid
     // captured substeps 0 -> 1 and 1 -> 0, and the control and parameter
     // arrays they read
     hipGraphExec_t graph_[2] = {nullptr, nullptr};

@@ -921,12 +921,6 @@ MaskView exact_view(const PbfCache& cache, uint32_t k, uint32_t n) {
     return MaskView{cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n, cache.exact_flags.data() + k, n,
                     0.0F, 1u, cache.crowded.data()};
 }
-
-// The recorded skin masks of the step and their displacement flags.
-MaskView skin_view(const PbfCache& cache, uint32_t n) {
-    return MaskView{cache.masks_skin.data(), cache.mask_flags.data(), n, cache.mask_limit2, 0u,
-                    cache.crowded.data()};
-}
 }  // namespace
 
 void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& cache,
@@ -979,7 +973,7 @@ void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.radius.data(),
            dw_.xsph.data(),
            dw_.confinement.data(),
-           skin_view(cache, n),
+           exact_view(cache, iterations, n),
            nullptr,
            cache.neighborhood.boundary()};
     const TangentParams tp{dw_.m_t.data(),        dw_.rho0_t.data(),   dw_.eps_t.data(),  dw_.strength_t.data(),
@@ -1077,7 +1071,7 @@ void PbfSolver::vjp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.radius.data(),
            dw_.xsph.data(),
            dw_.confinement.data(),
-           skin_view(cache, n),
+           exact_view(cache, iterations, n),
            dw_.inv_rho0.data(),
            cache.neighborhood.boundary()};
     // sorted parameter adjoints start at zero (+0.0 is the all-zero bit pattern)

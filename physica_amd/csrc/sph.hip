@@ -162,7 +162,13 @@ __global__ void __launch_bounds__(kGroupBlock) wcsph_force_kernel(WcsphForceArgs
     if (!usable || a.crowded[w] != 0u) {
         int cx, cy, cz;
         cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
-        group_walk_stencil<G, kSums>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, fetch, pair, fold);
+        group_walk_stencil<G, kSums>(
+            a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, w, group_row(lds),
+            [&](uint32_t entry) {
+                const bool sample = kSamples && (entry & kSampleEntry) != 0u;
+                return within_support(a.kc, p, xyz(sample ? a.boundary.x[entry & ~kSampleEntry] : a.xm[entry]));
+            },
+            fetch, pair, fold);
     }
     if (threadIdx.x % G == 0u)
         finish_wcsph(a, w, p, vel, Float3{sum[0], sum[1], sum[2]}, Float3{sum[3], sum[4], sum[5]},

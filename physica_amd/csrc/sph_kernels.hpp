@@ -21,6 +21,13 @@ namespace {
 
 __device__ __forceinline__ Float3 xyz(float4 q) { return Float3{q.x, q.y, q.z}; }
 
+// Whether q can be within the support of p (a distance that is NaN can, as
+// its terms are NaN); the kernels' values are exact zeros where it is not.
+__device__ __forceinline__ bool within_support(const KernelConstants& k, Float3 p, Float3 q) {
+    const Float3 d = sub(p, q);
+    return !(dot(d, d) >= k.sqrt_support);
+}
+
 constexpr uint32_t kBlock = 256;
 constexpr uint32_t kWaves = kBlock / 64;  // waves of a pass workgroup
 // candidates a masked walk fetches ahead of the one it processes
@@ -167,16 +174,10 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
     if (threadIdx.x < kParticles) crowd[threadIdx.x] = 0u;
     __syncthreads();
     Float3 p{0.0F, 0.0F, 0.0F};
-    uint32_t first[kSlots], last[kSlots];
-    [[maybe_unused]] uint32_t sample_first[kSlots], sample_last[kSlots];
-    [[maybe_unused]] float bound_i = 0.0F;
-    float bound[kSlots];
-#pragma unroll
-    for (uint32_t j = 0; j < kSlots; ++j) {
-        first[j] = last[j] = 0u;
-        bound[j] = 0.0F;
-        if constexpr (kSamples) sample_first[j] = sample_last[j] = 0u;
-    }
+    uint32_t first[kSlots] = {}, last[kSlots] = {};
+    [[maybe_unused]] uint32_t sample_first[kSlots] = {}, sample_last[kSlots] = {};
+    float bound_i = 0.0F;
+    float bound[kSlots] = {};
     if (valid) {
         const float4 self = a.xm[i];
         p = xyz(self);
@@ -185,30 +186,14 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
         particle_cell(a.grid, p, cx, cy, cz);
         const uint32_t center = cell_of(a.grid, cx, cy, cz);
         if (part == 0u) a.cell[i] = center;
-        if (a.cell_bound != nullptr) bound_i = a.cell_bound[center];
-        bool crowded = false;
+        bool crowded = group_ranges<G>(a.grid, a.grid.offsets, cx, cy, cz, first, last);
+        if constexpr (kSamples)
+            crowded = group_ranges<G>(a.grid, a.boundary.offsets, cx, cy, cz, sample_first, sample_last) || crowded;
+        if (a.cell_bound != nullptr) {
+            bound_i = a.cell_bound[center];
 #pragma unroll
-        for (uint32_t j = 0; j < kSlots; ++j) {
-            const uint32_t k = part * kSlots + j;
-            const int X = cx + static_cast<int>(k / 9u) - 1;
-            const int Y = cy + static_cast<int>((k / 3u) % 3u) - 1;
-            const int Z = cz + static_cast<int>(k % 3u) - 1;
-            if (k >= static_cast<uint32_t>(kStencil) || X < 0 || X >= static_cast<int>(a.grid.cx) || Y < 0 ||
-                Y >= static_cast<int>(a.grid.cy) || Z < 0 || Z >= static_cast<int>(a.grid.cz))
-                continue;
-            const uint32_t c = cell_of(a.grid, X, Y, Z);
-            first[j] = a.grid.offsets[c];
-            last[j] = a.grid.offsets[c + 1u];
-            if (a.cell_bound != nullptr) bound[j] = a.cell_bound[c];
-            if constexpr (kSamples) {
-                sample_first[j] = a.boundary.offsets[c];
-                sample_last[j] = a.boundary.offsets[c + 1u];
-            }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kSlots; ++j) {
-            crowded = crowded || last[j] - first[j] > kMaskBits;
-            if constexpr (kSamples) crowded = crowded || sample_last[j] - sample_first[j] > kMaskBits;
+            for (uint32_t j = 0; j < kSlots; ++j)
+                if (last[j] != first[j]) bound[j] = a.cell_bound[center + slot_delta(a.grid, part * kSlots + j)];
         }
         if (crowded) crowd[expanded] = 1u;
     }
@@ -286,7 +271,9 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
     if (crowd[walked] != 0u) {
         int cx, cy, cz;
         particle_cell(a.grid, xyz(own), cx, cy, cz);
-        group_walk_stencil<G, 1>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, fetch, pair, fold);
+        group_walk_stencil<G, 1>(
+            a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, w, group_row(lds),
+            [&](uint32_t entry) { return within_support(a.kc, xyz(own), xyz(fetch(entry))); }, fetch, pair, fold);
     }
     if (threadIdx.x % G == 0u) write_density<kEos>(a, w, xyz(own), sum[0]);
 }
@@ -403,13 +390,6 @@ __device__ __forceinline__ bool projection_masked(const ProjectionArgs& a, uint3
     return a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u && moved_within;
 }
 
-// Whether a predicted position q can be within the support of p (a distance
-// that is NaN can, as its term is NaN).
-__device__ __forceinline__ bool projection_near(const ProjectionArgs& a, Float3 p, Float3 q) {
-    const Float3 d = sub(p, q);
-    return !(dot(d, d) >= a.kc.sqrt_support);
-}
-
 // The pressure update of particle i from its predicted density rs; returns
 // its compression error in tolerance mode.
 __device__ __forceinline__ double update_pressure(const ProjectionArgs& a, uint32_t i, float4 topology, float mass,
@@ -474,7 +454,7 @@ __global__ void __launch_bounds__(kBlock) projection_kernel(ProjectionArgs a) {
                 int cx, cy, cz;
                 cell_coordinates(a.grid, center, cx, cy, cz);
                 scan_stencil(
-                    a.grid, cx, cy, cz, [&](uint32_t s) { return projection_near(a, ps, xyz(a.xs[s])); },
+                    a.grid, cx, cy, cz, [&](uint32_t s) { return within_support(a.kc, ps, xyz(a.xs[s])); },
                     [&](uint32_t k, uint32_t bits) {
                         column[k * kBlock] = static_cast<uint16_t>(bits);
                         nonzero |= bits != 0u ? 1u << k : 0u;
@@ -542,18 +522,16 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
         [&](uint32_t, uint32_t k, uint32_t& first) {
             if (masked) return stored_slot<false>(a.skin, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first);
             if (!listed) return 0u;
-            return scanned_slot(a.grid, cx, cy, cz, k, first,
-                                [&](uint32_t s) { return projection_near(a, expanded, xyz(a.xs[s])); });
+            return scanned_slot(a.grid, a.grid.offsets, cx, cy, cz, k, first,
+                                [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.xs[s])); });
         },
         [&](uint32_t, uint32_t k, uint32_t& first) {
             if (masked)
                 return stored_slot<false>(a.skin_samples, a.boundary.offsets, a.n, i, center + slot_delta(a.grid, k), k,
                                           first);
             if (!listed) return 0u;
-            SortedGrid samples = a.grid;
-            samples.offsets = a.boundary.offsets;
-            return scanned_slot(samples, cx, cy, cz, k, first,
-                                [&](uint32_t s) { return projection_near(a, expanded, xyz(a.boundary.x[s])); });
+            return scanned_slot(a.grid, a.boundary.offsets, cx, cy, cz, k, first,
+                                [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.boundary.x[s])); });
         },
         [&](const uint32_t* row, uint32_t count) {
             if (active) group_walk_list<G, 1>(row, count, w, fetch, pair, fold);
@@ -562,8 +540,9 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
     if (active) {
         if (!usable || a.crowded[w] != 0u) {
             cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
-            group_walk_stencil<G, 1>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, fetch, pair,
-                                     fold);
+            group_walk_stencil<G, 1>(
+                a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, w, group_row(lds),
+                [&](uint32_t entry) { return within_support(a.kc, xyz(self), xyz(fetch(entry))); }, fetch, pair, fold);
         }
         if (threadIdx.x % G == 0u) error = update_pressure(a, w, a.xm[w], self.w, sum[0]);
     }
@@ -937,8 +916,13 @@ __global__ void __launch_bounds__(kGroupBlock) force_group_kernel(ForceArgs a) {
         if (!usable || a.crowded[w] != 0u) {
             int cx, cy, cz;
             cell_coordinates(a.grid, cell, cx, cy, cz);
-            group_walk_stencil<G, kSums>(a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, fetch, pair,
-                                         fold);
+            group_walk_stencil<G, kSums>(
+                a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, w, w, group_row(lds),
+                [&](uint32_t entry) {
+                    const bool sample = kSamples && (entry & kSampleEntry) != 0u;
+                    return within_support(a.kc, p, xyz(sample ? a.boundary.x[entry & ~kSampleEntry] : a.xm[entry]));
+                },
+                fetch, pair, fold);
         }
         if (threadIdx.x % G == 0u) {
             Float3 acc{0.0F, 0.0F, 0.0F}, ap1{0.0F, 0.0F, 0.0F}, ap2{0.0F, 0.0F, 0.0F};
