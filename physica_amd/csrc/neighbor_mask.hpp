@@ -331,21 +331,6 @@ __device__ __forceinline__ bool is_crowded(const MaskView& m, uint32_t i) {
     return m.crowded != nullptr && m.crowded[i] != 0u;
 }
 
-// Candidate records of the wave-shared walks (whole dwords).
-struct PointMass {
-    Float3 x;
-    float m;
-};
-struct PointMassLambda {
-    Float3 x;
-    float m;
-    float lambda;
-};
-struct PointVector {
-    Float3 x;
-    Float3 v;
-};
-
 // Whether particle i walks its masks in a pass reading displacement slot `slot`.
 __device__ __forceinline__ bool masks_apply(const MaskView& m, uint32_t slot, uint32_t i) {
     if (m.masks == nullptr || m.flags[kFlagOverflow] != 0u) return false;

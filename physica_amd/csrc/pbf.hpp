@@ -123,8 +123,9 @@ class PbfSolver {
     PassProfiler profiler_;
     BoundarySamples boundary_;  // the domain's boundary samples on the device
     // sorted-order workspace
-    VecBuffer xs_, x0_, pa_, pb_, vel_, vort_, vc_;
-    DeviceBuffer<float> m_, rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
+    VecBuffer x0_, vort_;
+    DeviceBuffer<float4> xs_, pa_, pb_, vel_, vc_, pos_magnitude_;  // candidate records: 16 bytes in one load
+    DeviceBuffer<float> rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
     DeviceBuffer<uint16_t> exact_;  // exact masks of the current set of positions (forward mode)
     DeviceBuffer<uint8_t> crowded_;  // per particle: walks the full stencil (forward mode)
     DeviceBuffer<uint32_t> cells_;   // per particle: its grid cell
@@ -176,8 +177,9 @@ class PbfBatch {
     DeviceBuffer<BatchScene> scene_table_;
     Neighborhood grid_;
     VecBuffer positions_[2], velocities_[2];  // the state in original order, ping-pong
-    VecBuffer predicted_, xs_, x0_, pa_, pb_, vel_, vort_, vc_;
-    DeviceBuffer<float> m_, rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
+    VecBuffer predicted_, x0_, vort_;
+    DeviceBuffer<float4> xs_, pa_, pb_, vel_, vc_, pos_magnitude_;  // candidate records
+    DeviceBuffer<float> rho0_, eps_, strength_, exponent_, radius_, xsph_, confinement_;
     DeviceBuffer<float> rho_, lambda_, magnitude_;
     DeviceBuffer<uint16_t> exact_;
     DeviceBuffer<uint8_t> crowded_;
