@@ -30,6 +30,9 @@ constexpr uint32_t kSampleEntry = 0x80000000u;
 
 template <int G>
 constexpr uint32_t kGroupParticles = kGroupBlock / G;
+// stencil slots an expanding thread serves
+template <int G>
+constexpr uint32_t kGroupSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
 
 template <int G>
 struct GroupLds {
@@ -129,36 +132,29 @@ __device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const ui
     empty();
 }
 
-// Lists the candidates of a workgroup's particles and walks them. slot(j, k,
-// first) returns the mask of the expanding thread's particle in stencil slot
-// k, the thread's j-th, and sets `first` to the sorted index of that cell's
-// first particle (an empty mask for a particle that is not listed); with
-// kSamples, sample_slot(j, k, first) does the same for the cell's boundary
-// samples.
+// Lists the candidates of a workgroup's particles and walks them.
+// slots(bits, first) sets, for each stencil slot k = part * kGroupSlots<G> + j
+// of the expanding thread, bits[j] to the mask of its particle in that slot
+// (empty for a particle that is not listed) and first[j] to the sorted index
+// of that cell's first particle; with kSamples, sample_slots does the same
+// for the cells' boundary samples.
 // run(row, count) walks a list; it is called once for each round of
 // kGroupList candidates. Every thread of the workgroup calls this together.
-template <int G, bool kSamples, class Slot, class SampleSlot, class Run>
-__device__ __forceinline__ void group_expand(GroupLds<G>& lds, Slot&& slot, SampleSlot&& sample_slot, Run&& run) {
+template <int G, bool kSamples, class Slots, class SampleSlots, class Run>
+__device__ __forceinline__ void group_expand(GroupLds<G>& lds, Slots&& slots, SampleSlots&& sample_slots, Run&& run) {
     constexpr uint32_t kParticles = kGroupParticles<G>;
-    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    constexpr uint32_t kSlots = kGroupSlots<G>;
     const uint32_t particle = threadIdx.x % kParticles;
     const uint32_t part = threadIdx.x / kParticles;
-    uint32_t bits[kSlots], first[kSlots];
-    [[maybe_unused]] uint32_t sample_bits[kSlots], sample_first[kSlots];
+    uint32_t bits[kSlots] = {}, first[kSlots] = {};
+    [[maybe_unused]] uint32_t sample_bits[kSlots] = {}, sample_first[kSlots] = {};
+    slots(bits, first);
+    if constexpr (kSamples) sample_slots(sample_bits, sample_first);
     uint32_t mine = 0u;
 #pragma unroll
     for (uint32_t j = 0; j < kSlots; ++j) {
-        const uint32_t k = part * kSlots + j;
-        bits[j] = 0u;
-        first[j] = 0u;
-        if (k < static_cast<uint32_t>(kStencil)) bits[j] = slot(j, k, first[j]);
         mine += static_cast<uint32_t>(__popc(bits[j]));
-        if constexpr (kSamples) {
-            sample_bits[j] = 0u;
-            sample_first[j] = 0u;
-            if (k < static_cast<uint32_t>(kStencil)) sample_bits[j] = sample_slot(j, k, sample_first[j]);
-            mine += static_cast<uint32_t>(__popc(sample_bits[j]));
-        }
+        if constexpr (kSamples) mine += static_cast<uint32_t>(__popc(sample_bits[j]));
     }
     lds.counts[threadIdx.x] = mine;
     __syncthreads();
@@ -200,22 +196,36 @@ __device__ __forceinline__ uint32_t slot_delta(const SortedGrid& g, uint32_t k) 
     return static_cast<uint32_t>(ox + (oz * static_cast<int>(g.cy) + oy) * static_cast<int>(g.cx));
 }
 
-// Slot k of particle i's stored masks, for group_expand: with drop_self the
-// particle's own bit is cleared.
-template <bool kDropSelf>
-__device__ __forceinline__ uint32_t stored_slot(const uint16_t* __restrict__ masks,
-                                                const uint32_t* __restrict__ offsets, uint32_t n, uint32_t i,
-                                                uint32_t cell, uint32_t k, uint32_t& first) {
-    uint32_t m = masks[static_cast<size_t>(k) * n + i];
-    if (m == 0u) return 0u;
-    first = offsets[cell];
-    if constexpr (kDropSelf) {
-        if (k == 13u) {
-            const uint32_t own = i - first;
-            m &= ~(own < kMaskBits ? 1u << own : 0u);
+// The expanding thread's slots from particle i's stored masks, for
+// group_expand: with kDropSelf the particle's own bit is cleared. Every mask
+// and every cell start is fetched at once, whether or not the mask turns out
+// empty (a cell outside the grid has an empty mask; its start is read from
+// the nearest cell index): a thread that waits for each mask before it
+// fetches the cell start runs through G / 2 dependent pairs of loads.
+template <int G, bool kDropSelf>
+__device__ __forceinline__ void stored_slots(const uint16_t* __restrict__ masks, const SortedGrid& g,
+                                             const uint32_t* __restrict__ offsets, uint32_t n, uint32_t i,
+                                             uint32_t center, uint32_t (&bits)[kGroupSlots<G>],
+                                             uint32_t (&first)[kGroupSlots<G>]) {
+    constexpr uint32_t kSlots = kGroupSlots<G>;
+    const uint32_t part = threadIdx.x / kGroupParticles<G>;
+    const int last_cell = static_cast<int>(g.cx * g.cy * g.cz) - 1;
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) {
+        const uint32_t k = min(part * kSlots + j, static_cast<uint32_t>(kStencil) - 1u);
+        bits[j] = masks[static_cast<size_t>(k) * n + i];
+        const int c = static_cast<int>(center + slot_delta(g, k));
+        first[j] = offsets[min(max(c, 0), last_cell)];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kSlots; ++j) {
+        const uint32_t k = part * kSlots + j;
+        if (k >= static_cast<uint32_t>(kStencil)) bits[j] = 0u;
+        if (kDropSelf && k == 13u) {
+            const uint32_t own = i - first[j];
+            bits[j] &= ~(own < kMaskBits ? 1u << own : 0u);
         }
     }
-    return m;
 }
 
 // The ranges [first, last) of the expanding thread's stencil slots of the cell
@@ -223,9 +233,9 @@ __device__ __forceinline__ uint32_t stored_slot(const uint16_t* __restrict__ mas
 // kMaskBits. Fetched together, ahead of the members.
 template <int G>
 __device__ __forceinline__ bool group_ranges(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
-                                             uint32_t (&first)[(kStencil + G - 1) / G],
-                                             uint32_t (&last)[(kStencil + G - 1) / G]) {
-    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+                                             uint32_t (&first)[kGroupSlots<G>],
+                                             uint32_t (&last)[kGroupSlots<G>]) {
+    constexpr uint32_t kSlots = kGroupSlots<G>;
     const uint32_t part = threadIdx.x / kGroupParticles<G>;
 #pragma unroll
     for (uint32_t j = 0; j < kSlots; ++j) {
@@ -263,21 +273,16 @@ __device__ __forceinline__ uint32_t mark_members(uint32_t from, uint32_t to, Nea
     return bits;
 }
 
-// Slot k of a particle of cell (x, y, z) that is not crowded and whose stored
-// masks do not apply: the members with near(s); `first` is set as by
-// stored_slot.
-template <class Near>
-__device__ __forceinline__ uint32_t scanned_slot(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
-                                                 uint32_t k, uint32_t& first, Near&& near) {
-    const int X = x + static_cast<int>(k / 9u) - 1;
-    const int Y = y + static_cast<int>((k / 3u) % 3u) - 1;
-    const int Z = z + static_cast<int>(k % 3u) - 1;
-    if (X < 0 || X >= static_cast<int>(g.cx) || Y < 0 || Y >= static_cast<int>(g.cy) || Z < 0 ||
-        Z >= static_cast<int>(g.cz))
-        return 0u;
-    const uint32_t c = cell_of(g, X, Y, Z);
-    first = offsets[c];
-    return mark_members(first, offsets[c + 1u], near);
+// The expanding thread's slots of a particle of cell (x, y, z) that is not
+// crowded and whose stored masks do not apply: the members with near(s).
+template <int G, class Near>
+__device__ __forceinline__ void scanned_slots(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
+                                              uint32_t (&bits)[kGroupSlots<G>], uint32_t (&first)[kGroupSlots<G>],
+                                              Near&& near) {
+    uint32_t last[kGroupSlots<G>];
+    (void)group_ranges<G>(g, offsets, x, y, z, first, last);
+#pragma unroll
+    for (uint32_t j = 0; j < kGroupSlots<G>; ++j) bits[j] = mark_members(first[j], last[j], near);
 }
 
 }  // namespace phx

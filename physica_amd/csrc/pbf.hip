@@ -233,7 +233,7 @@ __device__ __forceinline__ uint32_t group_first_walk(const Args& a, const GroupS
                                                      uint32_t* crowd, const BoundaryGrid& samples, uint32_t skip,
                                                      Load&& load_record, Pair&& pair, Fold&& fold) {
     constexpr uint32_t kParticles = kGroupParticles<G>;
-    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    constexpr uint32_t kSlots = kGroupSlots<G>;
     const uint32_t expanded = threadIdx.x % kParticles;
     const uint32_t part = threadIdx.x / kParticles;
     const uint32_t i = scene.base + expanded;
@@ -266,19 +266,23 @@ __device__ __forceinline__ uint32_t group_first_walk(const Args& a, const GroupS
     const bool active = walked < scene.count;
     group_expand<G, kSamples>(
         lds,
-        [&](uint32_t j, uint32_t k, uint32_t& start) {
-            if (!valid) return 0u;
-            start = first[j];
-            const uint32_t bits = mark_members(first[j], last[j], [&](uint32_t s) { return near(p, xyz(a.pos[s])); });
-            a.exact_out[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits);
-            return bits;
+        [&](uint32_t (&bits)[kSlots], uint32_t (&start)[kSlots]) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSlots; ++j) {
+                const uint32_t k = part * kSlots + j;
+                start[j] = first[j];
+                if (!valid || k >= static_cast<uint32_t>(kStencil)) continue;
+                bits[j] = mark_members(first[j], last[j], [&](uint32_t s) { return near(p, xyz(a.pos[s])); });
+                a.exact_out[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits[j]);
+            }
         },
-        [&](uint32_t j, uint32_t, uint32_t& start) {
-            start = sample_first[j];
-            return mark_members(sample_first[j], sample_last[j], [&](uint32_t b) {
-                const float4 q = samples.x[b];
-                return near(p, Float3{q.x, q.y, q.z});
-            });
+        [&](uint32_t (&bits)[kSlots], uint32_t (&start)[kSlots]) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSlots; ++j) {
+                start[j] = sample_first[j];
+                bits[j] = mark_members(sample_first[j], sample_last[j],
+                                       [&](uint32_t b) { return near(p, xyz(samples.x[b])); });
+            }
         },
         [&](const uint32_t* row, uint32_t count) {
             if (active && crowd[walked] == 0u) group_walk_list<G, F>(row, count, w, load_record, pair, fold);
@@ -328,16 +332,13 @@ __device__ __forceinline__ uint32_t group_exact_walk(const Args& a, const GroupS
     const bool active = walked < scene.count;
     group_expand<G, kSamples>(
         lds,
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            return listed ? stored_slot<true>(a.exact, scene.grid.offsets, a.n, i,
-                                              center + slot_delta(scene.grid, k), k, first)
-                          : 0u;
+        [&](auto& bits, auto& first) {
+            if (listed) stored_slots<G, true>(a.exact, scene.grid, scene.grid.offsets, a.n, i, center, bits, first);
         },
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            if (!listed) return 0u;
-            return scanned_slot(scene.grid, samples.offsets, x, y, z, k, first, [&](uint32_t b) {
-                const float4 q = samples.x[b];
-                const Float3 d = sub(p, Float3{q.x, q.y, q.z});
+        [&](auto& bits, auto& first) {
+            if (!listed) return;
+            scanned_slots<G>(scene.grid, samples.offsets, x, y, z, bits, first, [&](uint32_t b) {
+                const Float3 d = sub(p, xyz(samples.x[b]));
                 return !(dot(d, d) >= t_exact);
             });
         },

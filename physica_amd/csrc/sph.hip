@@ -146,14 +146,11 @@ __global__ void __launch_bounds__(kGroupBlock) wcsph_force_kernel(WcsphForceArgs
     auto fold = [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); };
     group_expand<G, kSamples>(
         lds,
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            return listed ? stored_slot<true>(a.exact, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first)
-                          : 0u;
+        [&](auto& bits, auto& first) {
+            if (listed) stored_slots<G, true>(a.exact, a.grid, a.grid.offsets, a.n, i, center, bits, first);
         },
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            return listed ? stored_slot<false>(a.exact_samples, a.boundary.offsets, a.n, i,
-                                               center + slot_delta(a.grid, k), k, first)
-                          : 0u;
+        [&](auto& bits, auto& first) {
+            if (listed) stored_slots<G, false>(a.exact_samples, a.grid, a.boundary.offsets, a.n, i, center, bits, first);
         },
         [&](const uint32_t* row, uint32_t count) {
             if (active) group_walk_list<G, kSums>(row, count, w, fetch, pair, fold);

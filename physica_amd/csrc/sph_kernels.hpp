@@ -163,7 +163,7 @@ __device__ __forceinline__ void note_mass(const MaskDensityArgs& a, uint32_t i, 
 template <bool kEos, int G, bool kSamples>
 __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityArgs a) {
     constexpr uint32_t kParticles = kGroupParticles<G>;
-    constexpr uint32_t kSlots = (static_cast<uint32_t>(kStencil) + G - 1u) / G;
+    constexpr uint32_t kSlots = kGroupSlots<G>;
     __shared__ GroupLds<G> lds;
     __shared__ uint32_t crowd[kParticles];
     const uint32_t base = xcd_block() * kParticles;
@@ -225,26 +225,31 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
         const float radius = a.kc.h + reach;
         return radius * radius * (1.0F + 2e-5F);
     };
-    auto slot = [&](uint32_t j, uint32_t k, uint32_t& start) {
-        if (!valid) return 0u;
-        start = first[j];
-        uint32_t skin;
-        const uint32_t exact = mark(a.xm, first[j], last[j], threshold(bound_i + bound[j]), skin);
-        a.exact[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(exact);
-        a.skin[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
-        return exact;
-    };
-    auto sample_slot = [&](uint32_t j, uint32_t k, uint32_t& start) {
-        if constexpr (kSamples) {
-            if (!valid) return 0u;
-            start = sample_first[j];
+    auto slots = [&](uint32_t (&bits)[kSlots], uint32_t (&start)[kSlots]) {
+#pragma unroll
+        for (uint32_t j = 0; j < kSlots; ++j) {
+            const uint32_t k = part * kSlots + j;
+            start[j] = first[j];
+            if (!valid || k >= static_cast<uint32_t>(kStencil)) continue;
             uint32_t skin;
-            const uint32_t exact = mark(a.boundary.x, sample_first[j], sample_last[j], threshold(bound_i), skin);
-            a.exact_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(exact);
-            a.skin_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
-            return exact;
+            bits[j] = mark(a.xm, first[j], last[j], threshold(bound_i + bound[j]), skin);
+            a.exact[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits[j]);
+            a.skin[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
         }
-        return 0u;
+    };
+    auto sample_slots = [&](uint32_t (&bits)[kSlots], uint32_t (&start)[kSlots]) {
+        if constexpr (kSamples) {
+#pragma unroll
+            for (uint32_t j = 0; j < kSlots; ++j) {
+                const uint32_t k = part * kSlots + j;
+                start[j] = sample_first[j];
+                if (!valid || k >= static_cast<uint32_t>(kStencil)) continue;
+                uint32_t skin;
+                bits[j] = mark(a.boundary.x, sample_first[j], sample_last[j], threshold(bound_i), skin);
+                a.exact_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits[j]);
+                a.skin_samples[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(skin);
+            }
+        }
     };
     const uint32_t walked = threadIdx.x / G;
     const uint32_t w = base + walked;
@@ -263,7 +268,7 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
         terms[0] = kSamples && (entry & kSampleEntry) != 0u ? rest * q.w * weight : q.w * weight;
     };
     auto fold = [&](const float (&terms)[1]) { group_add<G, 1>(sum, terms); };
-    group_expand<G, kSamples>(lds, slot, sample_slot, [&](const uint32_t* row, uint32_t count) {
+    group_expand<G, kSamples>(lds, slots, sample_slots, [&](const uint32_t* row, uint32_t count) {
         if (active && crowd[walked] == 0u) group_walk_list<G, 1>(row, count, w, fetch, pair, fold);
     });
     if (valid && part == 0u) a.crowded[i] = static_cast<uint8_t>(crowd[expanded]);
@@ -519,19 +524,21 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
     auto fold = [&](const float (&terms)[1]) { group_add<G, 1>(sum, terms); };
     group_expand<G, kSamples>(
         lds,
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            if (masked) return stored_slot<false>(a.skin, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first);
-            if (!listed) return 0u;
-            return scanned_slot(a.grid, a.grid.offsets, cx, cy, cz, k, first,
-                                [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.xs[s])); });
+        [&](auto& bits, auto& first) {
+            if (masked) {
+                stored_slots<G, false>(a.skin, a.grid, a.grid.offsets, a.n, i, center, bits, first);
+            } else if (listed) {
+                scanned_slots<G>(a.grid, a.grid.offsets, cx, cy, cz, bits, first,
+                                 [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.xs[s])); });
+            }
         },
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            if (masked)
-                return stored_slot<false>(a.skin_samples, a.boundary.offsets, a.n, i, center + slot_delta(a.grid, k), k,
-                                          first);
-            if (!listed) return 0u;
-            return scanned_slot(a.grid, a.boundary.offsets, cx, cy, cz, k, first,
-                                [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.boundary.x[s])); });
+        [&](auto& bits, auto& first) {
+            if (masked) {
+                stored_slots<G, false>(a.skin_samples, a.grid, a.boundary.offsets, a.n, i, center, bits, first);
+            } else if (listed) {
+                scanned_slots<G>(a.grid, a.boundary.offsets, cx, cy, cz, bits, first,
+                                 [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.boundary.x[s])); });
+            }
         },
         [&](const uint32_t* row, uint32_t count) {
             if (active) group_walk_list<G, 1>(row, count, w, fetch, pair, fold);
@@ -898,14 +905,11 @@ __global__ void __launch_bounds__(kGroupBlock) force_group_kernel(ForceArgs a) {
     };
     group_expand<G, kSamples>(
         lds,
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            return listed ? stored_slot<true>(a.exact, a.grid.offsets, a.n, i, center + slot_delta(a.grid, k), k, first)
-                          : 0u;
+        [&](auto& bits, auto& first) {
+            if (listed) stored_slots<G, true>(a.exact, a.grid, a.grid.offsets, a.n, i, center, bits, first);
         },
-        [&](uint32_t, uint32_t k, uint32_t& first) {
-            return listed ? stored_slot<false>(a.exact_samples, a.boundary.offsets, a.n, i,
-                                               center + slot_delta(a.grid, k), k, first)
-                          : 0u;
+        [&](auto& bits, auto& first) {
+            if (listed) stored_slots<G, false>(a.exact_samples, a.grid, a.boundary.offsets, a.n, i, center, bits, first);
         },
         [&](const uint32_t* row, uint32_t count) {
             if (active) group_walk_list<G, kSums>(row, count, w, fetch, pair, fold);
