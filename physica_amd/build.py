@@ -99,17 +99,23 @@ def build_cpp_tests(verbose: bool = False) -> list:
 
 
 MATH_CHECK = ROOT / "tests" / "native" / "libphx_math_check.so"
+PAIR_MATH_CHECK = ROOT / "tests" / "native" / "libphx_pair_math_check.so"
 
 
 def build_math_check(verbose: bool = False) -> Path:
-    """Compile the rounding-helper checks (tests/native/math_check.hip)."""
-    src = ROOT / "tests" / "native" / "math_check.hip"
-    tmp = MATH_CHECK.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-shared", "-I", str(CSRC), str(src), "-o", str(tmp)]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
-    os.replace(tmp, MATH_CHECK)
+    """Compile the checks of the device arithmetic (tests/native/*.hip); the
+    pair checks take their constants from the library."""
+    for library, source, links in ((MATH_CHECK, "math_check.hip", []),
+                                   (PAIR_MATH_CHECK, "pair_math_check.hip",
+                                    ["-L", str(PACKAGE), "-lphysica_amd",
+                                     "-Wl,-rpath,$ORIGIN/../../physica_amd"])):
+        tmp = library.with_suffix(".so.tmp")
+        cmd = [hipcc(), *HIPCC_FLAGS, "-shared", "-I", str(CSRC), str(ROOT / "tests" / "native" / source), *links,
+               "-o", str(tmp)]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
+        os.replace(tmp, library)
     return MATH_CHECK
 
 

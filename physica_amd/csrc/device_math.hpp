@@ -99,6 +99,7 @@ struct KernelConstants {
     float sqrt_support; // smallest float t with sqrtf(t) >= h
     float inv_h;        // RN(1 / h)
     float inv_viscosity; // RN(1 / viscosity)
+    uint32_t plain;      // h lies outside [2^-20, 2^20], where div_in_range is not used
 };
 
 // Correctly rounded x / b from inv_b = RN(1 / b), for b > 0: the estimate
@@ -119,25 +120,39 @@ __host__ __device__ inline float div_rn(float x, float b, float inv_b) {
     return fmaf(r1, inv_b, q1);
 }
 
-// Correctly rounded square root of 0 <= x < 2^64: the hardware estimate s of
-// sqrt(y), y = x 2^64 (a normal number or zero for every such x), moved to
-// the float neighbour that the signs of y - s' s select (the correction of
-// the AMDGPU backend's sqrtf), then scaled back by 2^-32, which is exact
-// since every nonzero result is at least 2^-74.5. It equals sqrtf(x) on that
-// range (checked on the GPU for every float below 2^64) without the tests
-// sqrtf makes for denormal and special arguments; from 2^64 on it returns
-// +inf, which the pair kernels only compare with the support radius.
-__device__ __forceinline__ float sqrt_rn(float x) {
-    const float y = x * 0x1p64F;
-    const float s = __builtin_amdgcn_sqrtf(y);
-    const float down = __uint_as_float(__float_as_uint(s) - 1u);
-    const float up = __uint_as_float(__float_as_uint(s) + 1u);
-    const float below = fmaf(-down, s, y);
-    const float above = fmaf(-up, s, y);
-    float r = below <= 0.0F ? down : s;
-    r = above > 0.0F ? up : r;
-    return r * 0x1p-32F;
+// a / b for operands whose quotient, remainders and reciprocal stay normal:
+// the compiler's own sequence of reciprocal estimate, one Newton step and two
+// quotient refinements, hence its correctly rounded result, without the
+// scaling and special cases around it (8 instructions for 11). With
+// positive_sqrt it took PBF steps of 1,048,576 particles from 1,738 to
+// 1,625 us and WCSPH steps from 466 to 456; DFSPH's passes, held by their
+// gathers, did not move.
+__device__ __forceinline__ float div_in_range(float a, float b) {
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0F), r, r);
+    float q = a * r;
+    q = fmaf(fmaf(-b, q, a), r, q);
+    return fmaf(fmaf(-b, q, a), r, q);
 }
+
+// sqrt(x) for x > 0, correctly rounded, from the reciprocal square root s of
+// y = x 2^64 (a normal number for every such x below 2^64): g = y s is within
+// an ulp of sqrt(y), its residual y - g^2 is exact, and g + (y - g^2) s / 2
+// rounds correctly (checked on the GPU for every float below 2^64); the scale
+// is undone exactly. Two operations fewer than correcting the hardware's
+// square root by the signs of its neighbours' residuals, which also needs two
+// comparisons. x = 0 gives a root below 2^-77, which no kernel value tells
+// from 0; from 2^64 on the result is +inf; NaN stays NaN.
+__device__ __forceinline__ float positive_sqrt(float x) {
+    const float y = x * 0x1p64F;
+    const float in_range = __builtin_amdgcn_fmed3f(y, 0x1p-90F, 0x1.fffffep127F);
+    const float s = __builtin_amdgcn_rsqf(in_range);
+    const float g = in_range * s;
+    return fmaf(fmaf(-g, g, y), 0.5F * s, g) * 0x1p-32F;
+}
+
+// Correctly rounded square root of 0 <= x < 2^64 (positive_sqrt, and 0 at 0).
+__device__ __forceinline__ float sqrt_rn(float x) { return x == 0.0F ? 0.0F : positive_sqrt(x); }
 
 // length(d) of a neighbour pair (the same value; any |d| >= 2^32 gives +inf,
 // which lies outside every support).
@@ -164,7 +179,9 @@ __device__ __forceinline__ float cubic_gradient_factor(float dist, const KernelC
     const float diff = 1.0F - q;
     const float far = -6.0F * diff * diff;
     const float deriv = q <= 0.5F ? near : far;
-    const float f = k.cubic * deriv / (k.h * dist);
+    const float top = k.cubic * deriv;
+    const float bottom = k.h * dist;
+    const float f = k.plain != 0u ? top / bottom : div_in_range(top, bottom);
     return dist == 0.0F || dist >= k.h ? 0.0F : f;
 }
 
@@ -190,16 +207,6 @@ __device__ __forceinline__ Float3 spiky_gradient(Float3 d, float h, float coeffi
     return scale(d, coefficient * diff * diff / dist);
 }
 
-// artificial pressure value, pbf.cu:56-71 (value only). `reference` is
-// poly6((radius,0,0), h) of the particle.
-__device__ __forceinline__ float artificial_value(Float3 d, float h, float strength, float exponent, float reference) {
-    const float kernel = poly6(d, h);
-    if (kernel == 0.0F) return 0.0F;
-    const float ratio = kernel / reference;
-    const float power = powf(ratio, exponent);
-    return -strength * power;
-}
-
 // True when the artificial pressure -k (W(d) / W(dq))^n of a particle is the
 // signed zero -k for every pair with W(d) > 0: k is +-0 and the power stays
 // finite for every ratio up to W(0) / W(dq) (powf is non-decreasing in the
@@ -208,6 +215,54 @@ __device__ __forceinline__ bool artificial_vanishes(float h, float strength, flo
     if (strength != 0.0F || !(reference > 0.0F) || !(exponent >= 0.0F)) return false;
     const float largest = poly6(Float3{0.0F, 0.0F, 0.0F}, h) / reference;
     return powf(largest, exponent) < 1.0e37F;
+}
+
+// The PBF kernels' constants for one support radius, evaluated with the
+// reference's FP32 expressions on the host: the poly6 denominator
+// 64 pi h^9 scaled by a power of two into [1, 2) (poly6_value scales its
+// numerator alike, so no remainder underflows), and the spiky coefficient.
+struct PbfKernel {
+    float h;
+    float hr;           // h h
+    float spiky;        // spiky_coefficient(h)
+    float poly6;        // 64 pi hr hr hr h h h
+    float poly6_scaled; // poly6 scale
+    float inv_poly6;    // RN(1 / poly6_scaled)
+    float scale;
+    uint32_t plain;     // h lies outside [2^-11, 2^8], where the quotients below are taken by the compiler's division
+};
+
+// poly6(d, h) from d2 = dot(d, d).
+__device__ __forceinline__ float poly6_value(float d2, const PbfKernel& k) {
+    const float diff = k.hr - d2;
+    const float top = 315.0F * diff * diff * diff;
+    const float w = k.plain != 0u ? top / k.poly6 : div_rn(top * k.scale, k.poly6_scaled, k.inv_poly6);
+    return d2 >= k.hr ? 0.0F : w;
+}
+
+// Whether poly6(d, h) is zero.
+__device__ __forceinline__ bool poly6_vanishes(float d2, const PbfKernel& k) {
+    return k.plain != 0u ? poly6_value(d2, k) == 0.0F : d2 >= k.hr;
+}
+
+// The factor f of spiky_gradient(d, h) = f d from d2 = dot(d, d); both sides
+// of its condition are evaluated and selected, so that a wave does not
+// diverge.
+__device__ __forceinline__ float spiky_factor(float d2, const PbfKernel& k) {
+    const float dist = sqrt_rn(d2);
+    const float diff = k.h - dist;
+    const float top = k.spiky * diff * diff;
+    const float f = k.plain != 0u ? top / dist : div_in_range(top, dist);
+    return dist == 0.0F || dist >= k.h ? 0.0F : f;
+}
+
+// artificial pressure value, pbf.cu:56-71 (value only), from d2 = dot(d, d).
+// `reference` is poly6((radius,0,0), h) of the particle.
+__device__ __forceinline__ float artificial_value(float d2, const PbfKernel& k, float strength, float exponent,
+                                                  float reference) {
+    const float kernel = poly6_value(d2, k);
+    if (kernel == 0.0F) return 0.0F;
+    return -strength * powf(kernel / reference, exponent);
 }
 
 // min(C-1, max(0, floor(v))) with NaN and negatives mapped to 0, as the

@@ -25,6 +25,7 @@
 #include "group_walk.hpp"
 #include "neighbor_mask.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace phx {
@@ -166,8 +167,7 @@ __global__ void __launch_bounds__(kBlock) pbf_cell_kernel(uint32_t n, SortedGrid
 
 struct LambdaArgs {
     uint32_t n;
-    float h;
-    float spiky;
+    PbfKernel k;
     SortedGrid grid;
     const float4* pos;  // positions and masses
     const float* rho0;
@@ -189,6 +189,20 @@ struct LambdaArgs {
     uint32_t first_pass;
 };
 
+// A particle's rest density as the divisor of its candidates' masses: the
+// reciprocal is taken once (div_rn), or, outside [2^-60, 2^60], the quotient
+// of each pair by the compiler's division.
+struct RestDensity {
+    float value, inverse;
+    bool plain;
+};
+__device__ __forceinline__ RestDensity rest_density_of(float rest) {
+    return RestDensity{rest, 1.0F / rest, !(rest >= 0x1p-60F && rest <= 0x1p60F)};
+}
+__device__ __forceinline__ float over_rest(float mass, const RestDensity& rest) {
+    return rest.plain ? mass / rest.value : div_rn(mass, rest.value, rest.inverse);
+}
+
 // The terms of one candidate in the density and lambda sums: the density,
 // the gradient sum and the denominator.
 struct LambdaTerms {
@@ -196,10 +210,11 @@ struct LambdaTerms {
     Float3 gradient;
     float square;
 };
-__device__ __forceinline__ LambdaTerms lambda_terms(const LambdaArgs& a, Float3 d, float ms, float rest) {
-    const Float3 g = spiky_gradient(d, a.h, a.spiky);
-    const float coefficient = ms / rest;
-    return LambdaTerms{ms * poly6(d, a.h), scale(g, coefficient), coefficient * coefficient * dot(g, g)};
+__device__ __forceinline__ LambdaTerms lambda_terms(const LambdaArgs& a, Float3 d, float ms, const RestDensity& rest) {
+    const float d2 = dot(d, d);
+    const Float3 g = scale(d, spiky_factor(d2, a.k));
+    const float coefficient = over_rest(ms, rest);
+    return LambdaTerms{ms * poly6_value(d2, a.k), scale(g, coefficient), coefficient * coefficient * dot(g, g)};
 }
 
 __device__ __forceinline__ void finish_lambda(const LambdaArgs& a, uint32_t i, float rest, float density,
@@ -381,7 +396,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_lambda_kernel(LambdaArgs a, S
     const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
     const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
     const Float3 p = xyz(a.pos[own]);
-    const float rest = a.rho0[own];
+    const RestDensity rest = rest_density_of(a.rho0[own]);
     float sum[kSums] = {0.0F, 0.0F, 0.0F, 0.0F, a.eps[own]};
     const uint32_t w = group_first_walk<G, kSamples, kSums>(
         a, scene, lds, crowd, a.boundary, ~0u,
@@ -389,8 +404,9 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_lambda_kernel(LambdaArgs a, S
         [&](float4 c, uint32_t entry, float (&terms)[kSums]) {
             const Float3 d = sub(p, xyz(c));
             if (kSamples && (entry & kSampleEntry) != 0u) {
-                terms[0] = rest * c.w * poly6(d, a.h);
-                put(terms + 1, scale(spiky_gradient(d, a.h, a.spiky), c.w));
+                const float d2 = dot(d, d);
+                terms[0] = rest.value * c.w * poly6_value(d2, a.k);
+                put(terms + 1, scale(scale(d, spiky_factor(d2, a.k)), c.w));
                 return;
             }
             const LambdaTerms t = lambda_terms(a, d, c.w, rest);
@@ -402,7 +418,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_lambda_kernel(LambdaArgs a, S
         },
         [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
     if (w != ~0u && threadIdx.x % G == 0u)
-        finish_lambda(a, w, rest, sum[0], Float3{sum[1], sum[2], sum[3]}, sum[4]);
+        finish_lambda(a, w, rest.value, sum[0], Float3{sum[1], sum[2], sum[3]}, sum[4]);
 }
 
 // Candidate records.
@@ -422,8 +438,7 @@ __device__ __forceinline__ void store_both(float4* records, Vec recorded, uint32
 
 struct CorrectionArgs {
     uint32_t n;
-    float h;
-    float spiky;
+    PbfKernel k;
     SortedGrid grid;
     Box box;
     const float4* pos;  // positions and masses
@@ -453,13 +468,13 @@ struct ArtificialPressure {
     bool vanishes;  // with k = +-0 the term is -k wherever W(d) > 0 (no powf per pair)
 };
 __device__ __forceinline__ ArtificialPressure artificial_of(const CorrectionArgs& a, uint32_t i) {
-    ArtificialPressure s{a.strength[i], a.exponent[i], poly6(Float3{a.radius[i], 0.0F, 0.0F}, a.h), false};
-    s.vanishes = artificial_vanishes(a.h, s.strength, s.exponent, s.reference);
+    ArtificialPressure s{a.strength[i], a.exponent[i], poly6(Float3{a.radius[i], 0.0F, 0.0F}, a.k.h), false};
+    s.vanishes = artificial_vanishes(a.k.h, s.strength, s.exponent, s.reference);
     return s;
 }
-__device__ __forceinline__ float artificial_at(const CorrectionArgs& a, const ArtificialPressure& s, Float3 d) {
-    return s.vanishes ? (poly6(d, a.h) == 0.0F ? 0.0F : -s.strength)
-                      : artificial_value(d, a.h, s.strength, s.exponent, s.reference);
+__device__ __forceinline__ float artificial_at(const CorrectionArgs& a, const ArtificialPressure& s, float d2) {
+    return s.vanishes ? (poly6_vanishes(d2, a.k) ? 0.0F : -s.strength)
+                      : artificial_value(d2, a.k, s.strength, s.exponent, s.reference);
 }
 
 // project_forward_kernel (pbf.cu:417-431) of particle i at p with its
@@ -495,7 +510,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_correction_kernel(CorrectionA
     const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
     const float4 self = a.pos[own];
     const Float3 p = xyz(self);
-    const float rest = a.rho0[own];
+    const RestDensity rest = rest_density_of(a.rho0[own]);
     const float lambda_i = a.lambda[own];
     const ArtificialPressure pressure = artificial_of(a, own);
     float sum[kSums] = {0.0F, 0.0F, 0.0F};
@@ -507,11 +522,12 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_correction_kernel(CorrectionA
         },
         [&](const PointLambda& c, uint32_t entry, float (&terms)[kSums]) {
             const Float3 d = sub(p, xyz(c.x));
-            const float artificial = artificial_at(a, pressure, d);
+            const float d2 = dot(d, d);
+            const float artificial = artificial_at(a, pressure, d2);
             const float factor = kSamples && (entry & kSampleEntry) != 0u
                                      ? c.x.w * (lambda_i + artificial)
-                                     : c.x.w / rest * (lambda_i + c.lambda + artificial);
-            put(terms, scale(spiky_gradient(d, a.h, a.spiky), factor));
+                                     : over_rest(c.x.w, rest) * (lambda_i + c.lambda + artificial);
+            put(terms, scale(scale(d, spiky_factor(d2, a.k)), factor));
         },
         [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
     if (w != ~0u && threadIdx.x % G == 0u)
@@ -527,8 +543,7 @@ __global__ void __launch_bounds__(kBlock) pbf_reconstruct_kernel(uint32_t n, con
 
 struct PostArgs {
     uint32_t n;
-    float h;
-    float spiky;
+    PbfKernel k;
     float dt;
     SortedGrid grid;
     const float4* pos;  // positions and masses
@@ -595,7 +610,8 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_vorticity_kernel(PostArgs a, 
         a, scene, lds, crowd, BoundaryGrid{}, own,
         [&](uint32_t s) { return PointVector{a.pos[s], a.vel[s]}; },
         [&](const PointVector& c, uint32_t s, float (&terms)[kSums]) {
-            if (s != own) put(terms, cross(sub(xyz(c.v), v), spiky_gradient(sub(p, xyz(c.x)), a.h, a.spiky)));
+            const Float3 d = sub(p, xyz(c.x));
+            if (s != own) put(terms, cross(sub(xyz(c.v), v), scale(d, spiky_factor(dot(d, d), a.k))));
         },
         [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
     if (w != ~0u && threadIdx.x % G == 0u) finish_vorticity(a, w, p, Float3{sum[0], sum[1], sum[2]});
@@ -617,7 +633,8 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_normal_kernel(PostArgs a, Sch
         a, scene, lds, BoundaryGrid{}, a.t_exact,
         [&](uint32_t s) { return a.pos_magnitude[s]; },
         [&](float4 c, uint32_t, float (&terms)[kSums]) {
-            put(terms, scale(spiky_gradient(sub(p, xyz(c)), a.h, a.spiky), c.w - mag_i));
+            const Float3 d = sub(p, xyz(c));
+            put(terms, scale(scale(d, spiky_factor(dot(d, d), a.k)), c.w - mag_i));
         },
         [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
     if (w != ~0u && threadIdx.x % G == 0u) finish_normal(a, w, Float3{sum[0], sum[1], sum[2]});
@@ -638,7 +655,8 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_xsph_kernel(PostArgs a, Sched
         a, scene, lds, BoundaryGrid{}, a.t_exact,
         [&](uint32_t s) { return PointVector{a.pos[s], a.vc[s]}; },
         [&](const PointVector& c, uint32_t, float (&terms)[kSums]) {
-            put(terms, scale(sub(xyz(c.v), v), poly6(sub(p, xyz(c.x)), a.h)));
+            const Float3 d = sub(p, xyz(c.x));
+            put(terms, scale(sub(xyz(c.v), v), poly6_value(dot(d, d), a.k)));
         },
         [&](const float (&terms)[kSums]) { group_add<G, kSums>(sum, terms); });
     if (w != ~0u && threadIdx.x % G == 0u) finish_xsph(a, w, p, v, Float3{sum[0], sum[1], sum[2]});
@@ -739,6 +757,23 @@ double pbf_pass_bytes(int pass, uint32_t particles, uint32_t cells) {
     }
 }
 
+PbfKernel pbf_kernel(float h) {
+    PbfKernel k{};
+    k.h = h;
+    k.hr = h * h;
+    k.spiky = spiky_coefficient(h);
+    k.poly6 = 64.0F * kPi * k.hr * k.hr * k.hr * h * h * h;
+    k.plain = h >= 0x1p-11F && h <= 0x1p8F ? 0u : 1u;
+    if (k.plain == 0u) {
+        int exponent = 0;
+        (void)std::frexp(k.poly6, &exponent);
+        k.scale = std::ldexp(1.0F, 1 - exponent);
+        k.poly6_scaled = k.poly6 * k.scale;
+        k.inv_poly6 = 1.0F / k.poly6_scaled;
+    }
+    return k;
+}
+
 void PbfCache::allocate(uint32_t n, uint32_t cells, uint32_t pressure_iterations) {
     neighborhood.allocate(n, cells);
     predicted.resize(n);
@@ -772,6 +807,7 @@ PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_confi
     boundary_.upload(domain_.config);
     domain_.config.boundary_particles = nullptr;  // the caller's host array is not kept
     spiky_ = spiky_coefficient(domain_.config.support_radius);
+    kernel_ = pbf_kernel(domain_.config.support_radius);
     const uint32_t n = domain_.config.particle_count;
     for (VecBuffer* b : {&x0_, &vort_}) b->resize(n);
     for (DeviceBuffer<float4>* b : {&xs_, &pa_, &pb_, &vel_, &vc_, &pos_magnitude_}) b->resize(n);
@@ -873,17 +909,16 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
         return rec ? cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n : exact_.data();
     };
 
-    LambdaArgs la{n,           h,           spiky_,
-                  grid,        xs_.data(),  rho0_.data(),
-                  eps_.data(), cache.densities.data(), cache.lambdas.data()};
+    LambdaArgs la{n,           kernel_,     grid,
+                  xs_.data(),  rho0_.data(), eps_.data(),
+                  cache.densities.data(), cache.lambdas.data()};
     la.t_exact = t_exact;
     la.boundary = boundary;
     la.cell = cells_.data();
     la.crowded = crowded;
     CorrectionArgs ca{};
     ca.n = n;
-    ca.h = h;
-    ca.spiky = spiky_;
+    ca.k = kernel_;
     ca.grid = grid;
     ca.box = collision_box(c, step + 1u);
     ca.rho0 = rho0_.data();
@@ -950,8 +985,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
 
     PostArgs post{};
     post.n = n;
-    post.h = h;
-    post.spiky = spiky_;
+    post.k = kernel_;
     post.dt = c.time_step;
     post.grid = grid;
     post.pos = current;
@@ -1056,7 +1090,7 @@ PbfBatch::PbfBatch(const phx_domain_configuration* domains, uint32_t scene_count
     cells_ = static_cast<uint32_t>(cells);
     // a captured substep bakes in the step time, which moving boxes change
     use_graph_ = use_graph_ && static_boxes_;
-    spiky_ = spiky_coefficient(h_);
+    kernel_ = pbf_kernel(h_);
 
     // workgroup tables: each scene's particles in blocks of kBlock (the grid
     // build) and of the passes' workgroups, padded to a multiple of the XCD count
@@ -1173,7 +1207,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     ++kernels_per_step_;
     const float t_exact = exact_mask_threshold(h_);
 
-    LambdaArgs la{n,           h_,         spiky_,         grid, xs_.data(), rho0_.data(),
+    LambdaArgs la{n,           kernel_,     grid, xs_.data(), rho0_.data(),
                   eps_.data(), rho_.data(), lambda_.data()};
     la.t_exact = t_exact;
     la.exact_out = exact_.data();
@@ -1181,8 +1215,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     la.crowded = crowded_.data();
     CorrectionArgs ca{};
     ca.n = n;
-    ca.h = h_;
-    ca.spiky = spiky_;
+    ca.k = kernel_;
     ca.grid = grid;
     ca.rho0 = rho0_.data();
     ca.lambda = lambda_.data();
@@ -1220,8 +1253,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     }
     PostArgs post{};
     post.n = n;
-    post.h = h_;
-    post.spiky = spiky_;
+    post.k = kernel_;
     post.dt = dt_;
     post.grid = grid;
     post.pos = current;

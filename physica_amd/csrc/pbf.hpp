@@ -92,6 +92,9 @@ struct PbfDerivativeWorkspace {
     void allocate(uint32_t n);
 };
 
+// Constants of the poly6 and spiky kernels for support radius h.
+PbfKernel pbf_kernel(float h);
+
 class PbfSolver {
   public:
     PbfSolver(const phx_domain_configuration* domain, const phx_pbf_configuration* configuration,
@@ -120,6 +123,7 @@ class PbfSolver {
     phx_execution_mode mode_;
     hipStream_t stream_;
     float spiky_ = 0.0F;
+    PbfKernel kernel_{};
     PassProfiler profiler_;
     BoundarySamples boundary_;  // the domain's boundary samples on the device
     // sorted-order workspace
@@ -170,7 +174,8 @@ class PbfBatch {
     std::vector<uint64_t> offsets_;
     uint32_t n_ = 0, cells_ = 0, blocks_ = 0, pass_blocks_ = 0;
     int group_ = 1;  // lanes per particle of the passes
-    float h_ = 0.0F, dt_ = 0.0F, spiky_ = 0.0F;
+    float h_ = 0.0F, dt_ = 0.0F;
+    PbfKernel kernel_{};
     bool static_boxes_ = true, use_graph_ = false;
     uint32_t kernels_per_step_ = 0;
     DeviceBuffer<BatchBlock> block_table_, pass_table_;

@@ -1,0 +1,29 @@
+"""The pair kernels' arithmetic (physica_amd/csrc/device_math.hpp) against the
+same expressions with the compiler's square root and division, for every float
+squared distance from 2^-90 h^2 to just past the support, and for 0. The range
+of support radii includes the ends of the ones whose quotients skip the
+compiler's scaling, and radii beyond them."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from physica_amd import build
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(x) -> int:
+    return int(np.array([x], dtype=np.float32).view(np.uint32)[0])
+
+
+@pytest.mark.parametrize("h", [0.02, 0.04, 0.1, 1.0 / 30.0, 2.0**-11, 2.0**8, 1.0e-4, 700.0])
+def test_pair_functions_equal_their_expressions(gpu_device, h):
+    lib = ctypes.CDLL(str(build.PAIR_MATH_CHECK))
+    lib.phx_test_pair_math.argtypes = [ctypes.c_float, ctypes.c_uint32, ctypes.c_uint32,
+                                       ctypes.POINTER(ctypes.c_ulonglong)]
+    h = float(np.float32(h))
+    wrong = (ctypes.c_ulonglong * 4)()
+    for first, count in ((_bits(2.0**-90 * h * h), _bits(1.01 * h * h) - _bits(2.0**-90 * h * h)), (0, 1)):
+        assert lib.phx_test_pair_math(h, first, count, wrong) == 0
+        assert list(wrong) == [0, 0, 0, 0], (h, first)
