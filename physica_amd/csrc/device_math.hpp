@@ -334,6 +334,10 @@ __device__ __forceinline__ void particle_cell(const SortedGrid& g, Float3 p, int
 // the samples in ascending original index, each stored as its position at
 // the step's time t, x0 + t v (boundary_position, neighborhood/device.cuh:
 // 16-22), with its volume, and its velocity.
+// Candidate records are read up to kScanPadding past the end of a cell
+// (mark_members), so the arrays of records that are scanned are that longer.
+constexpr uint32_t kScanPadding = 3;
+
 struct BoundaryGrid {
     const uint32_t* offsets;  // C + 1 cell starts; null when the domain has no boundary samples
     const float4* x;          // position at t (xyz), volume (w)

@@ -125,7 +125,8 @@ DfsphSolver::DfsphSolver(const phx_domain_configuration* domain, const phx_dfsph
     gradient_norm_ = reference_gradient_norm(domain_.config);
     constants_ = kernel_constants(domain_.config.support_radius);
     const uint32_t n = domain_.config.particle_count;
-    for (DeviceBuffer<float4>* b : {&xm_, &vmu_, &xs_, &adiv_, &xt_div_, &xt_den_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&vmu_, &adiv_, &xt_div_, &xt_den_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&xm_, &xs_}) b->resize(n + static_cast<size_t>(kScanPadding));
     mass_state_.resize(2u);
     fill_u32(stream_, mass_state_.data(), 2u, 0u);
     u_.resize(n);

@@ -327,7 +327,7 @@ struct Neighborhood {
         if (boundary_perm.size() != boundary_count || boundary_offsets.size() != static_cast<size_t>(cells) + 1u) {
             boundary_perm.resize(boundary_count);
             boundary_offsets.resize(static_cast<size_t>(cells) + 1u);
-            boundary_x.resize(boundary_count);
+            boundary_x.resize(boundary_count + static_cast<size_t>(kScanPadding));
             boundary_v.resize(boundary_count);
             const size_t bytes = boundary_scratch_bytes(boundary_count);
             boundary_scratch_bytes_.resize(bytes);

@@ -257,32 +257,16 @@ __device__ __forceinline__ bool group_ranges(const SortedGrid& g, const uint32_t
     return many;
 }
 
-// The mask of members from .. to - 1 (the first kMaskBits of them) with
-// near(s). Four are tested together, so that their loads overlap.
-template <class Near>
-__device__ __forceinline__ uint32_t mark_members(uint32_t from, uint32_t to, Near&& near) {
-    const uint32_t end = min(to, from + kMaskBits);
-    uint32_t bits = 0u;
-    for (uint32_t s = from; s < end; s += 4u) {
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
-            const bool marked = near(min(s + u, end - 1u)) && s + u < end;
-            bits |= marked ? 1u << (s + u - from) : 0u;
-        }
-    }
-    return bits;
-}
-
 // The expanding thread's slots of a particle of cell (x, y, z) that is not
-// crowded and whose stored masks do not apply: the members with near(s).
+// crowded and whose stored masks do not apply: the members with near(position).
 template <int G, class Near>
-__device__ __forceinline__ void scanned_slots(const SortedGrid& g, const uint32_t* offsets, int x, int y, int z,
-                                              uint32_t (&bits)[kGroupSlots<G>], uint32_t (&first)[kGroupSlots<G>],
+__device__ __forceinline__ void scanned_slots(const SortedGrid& g, const uint32_t* offsets, const float4* records,
+                                              int x, int y, int z, uint32_t (&bits)[kGroupSlots<G>], uint32_t (&first)[kGroupSlots<G>],
                                               Near&& near) {
     uint32_t last[kGroupSlots<G>];
     (void)group_ranges<G>(g, offsets, x, y, z, first, last);
 #pragma unroll
-    for (uint32_t j = 0; j < kGroupSlots<G>; ++j) bits[j] = mark_members(first[j], last[j], near);
+    for (uint32_t j = 0; j < kGroupSlots<G>; ++j) bits[j] = mark_members(records, first[j], last[j], near);
 }
 
 }  // namespace phx

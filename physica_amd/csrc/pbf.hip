@@ -287,7 +287,7 @@ __device__ __forceinline__ uint32_t group_first_walk(const Args& a, const GroupS
                 const uint32_t k = part * kSlots + j;
                 start[j] = first[j];
                 if (!valid || k >= static_cast<uint32_t>(kStencil)) continue;
-                bits[j] = mark_members(first[j], last[j], [&](uint32_t s) { return near(p, xyz(a.pos[s])); });
+                bits[j] = mark_members(a.pos, first[j], last[j], [&](Float3 q) { return near(p, q); });
                 a.exact_out[static_cast<size_t>(k) * a.n + i] = static_cast<uint16_t>(bits[j]);
             }
         },
@@ -295,8 +295,8 @@ __device__ __forceinline__ uint32_t group_first_walk(const Args& a, const GroupS
 #pragma unroll
             for (uint32_t j = 0; j < kSlots; ++j) {
                 start[j] = sample_first[j];
-                bits[j] = mark_members(sample_first[j], sample_last[j],
-                                       [&](uint32_t b) { return near(p, xyz(samples.x[b])); });
+                bits[j] = mark_members(samples.x, sample_first[j], sample_last[j],
+                                       [&](Float3 q) { return near(p, q); });
             }
         },
         [&](const uint32_t* row, uint32_t count) {
@@ -352,8 +352,8 @@ __device__ __forceinline__ uint32_t group_exact_walk(const Args& a, const GroupS
         },
         [&](auto& bits, auto& first) {
             if (!listed) return;
-            scanned_slots<G>(scene.grid, samples.offsets, x, y, z, bits, first, [&](uint32_t b) {
-                const Float3 d = sub(p, xyz(samples.x[b]));
+            scanned_slots<G>(scene.grid, samples.offsets, samples.x, x, y, z, bits, first, [&](Float3 q) {
+                const Float3 d = sub(p, q);
                 return !(dot(d, d) >= t_exact);
             });
         },
@@ -810,7 +810,8 @@ PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_confi
     kernel_ = pbf_kernel(domain_.config.support_radius);
     const uint32_t n = domain_.config.particle_count;
     for (VecBuffer* b : {&x0_, &vort_}) b->resize(n);
-    for (DeviceBuffer<float4>* b : {&xs_, &pa_, &pb_, &vel_, &vc_, &pos_magnitude_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&vel_, &vc_, &pos_magnitude_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&xs_, &pa_, &pb_}) b->resize(n + static_cast<size_t>(kScanPadding));
     for (DeviceBuffer<float>* b : {&rho0_, &eps_, &strength_, &exponent_, &radius_, &xsph_, &confinement_})
         b->resize(n);
     exact_.resize(static_cast<size_t>(kStencil) * n);
@@ -1126,7 +1127,8 @@ PbfBatch::PbfBatch(const phx_domain_configuration* domains, uint32_t scene_count
     for (VecBuffer* b :
          {&positions_[0], &positions_[1], &velocities_[0], &velocities_[1], &predicted_, &x0_, &vort_})
         b->resize(n);
-    for (DeviceBuffer<float4>* b : {&xs_, &pa_, &pb_, &vel_, &vc_, &pos_magnitude_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&vel_, &vc_, &pos_magnitude_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&xs_, &pa_, &pb_}) b->resize(n + static_cast<size_t>(kScanPadding));
     for (DeviceBuffer<float>* b :
          {&rho0_, &eps_, &strength_, &exponent_, &radius_, &xsph_, &confinement_, &rho_, &lambda_, &magnitude_})
         b->resize(n);

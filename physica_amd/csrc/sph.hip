@@ -238,7 +238,8 @@ SphSolver::SphSolver(const phx_domain_configuration* domain, const phx_sph_confi
     gradient_norm_ = reference_gradient_norm(domain_.config);
     constants_ = kernel_constants(domain_.config.support_radius);
     const uint32_t n = domain_.config.particle_count;
-    for (DeviceBuffer<float4>* b : {&xm_, &vmu_, &xs_, &aux_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&vmu_, &aux_}) b->resize(n);
+    for (DeviceBuffer<float4>* b : {&xm_, &xs_}) b->resize(n + static_cast<size_t>(kScanPadding));
     u_.resize(n);
     for (DeviceBuffer<float>* b : {&rho0_, &relax_, &tait_, &t_}) b->resize(n);
     if (boundary_.count() > 0u && config_.method == PHX_SPH_WCSPH) btension_.resize(n);

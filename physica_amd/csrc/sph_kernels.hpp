@@ -198,25 +198,17 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
         if (crowded) crowd[expanded] = 1u;
     }
     // the exact mask of members from .. to - 1 at positions x[s], their skin
-    // mask in `skin`; four members are fetched together
+    // mask in `skin`
     auto mark = [&](const float4* x, uint32_t from, uint32_t to, float t_skin, uint32_t& skin) {
-        uint32_t exact = 0u;
-        skin = 0u;
-        const uint32_t end = min(to, from + kMaskBits);
-        for (uint32_t s = from; s < end; s += 4u) {
-            float4 q[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4u; ++u) q[u] = x[min(s + u, end - 1u)];
-#pragma unroll
-            for (uint32_t u = 0; u < 4u; ++u) {
-                const Float3 d = sub(p, xyz(q[u]));
-                const float d2 = dot(d, d);
-                const uint32_t bit = s + u < end ? 1u << (s + u - from) : 0u;
-                exact |= d2 < a.kc.sqrt_support ? bit : 0u;
-                skin |= d2 < t_skin ? bit : 0u;
-            }
-        }
-        return exact;
+        uint32_t bits[2];
+        mark_members<2>(x, from, to, bits, [&](Float3 q, bool (&marked)[2]) {
+            const Float3 d = sub(p, q);
+            const float d2 = dot(d, d);
+            marked[0] = d2 < a.kc.sqrt_support;
+            marked[1] = d2 < t_skin;
+        });
+        skin = bits[1];
+        return bits[0];
     };
     // the threshold of pairs within h after moving up to `reach` together
     // (the relative margin covers rounding), or the step's global one
@@ -459,7 +451,7 @@ __global__ void __launch_bounds__(kBlock) projection_kernel(ProjectionArgs a) {
                 int cx, cy, cz;
                 cell_coordinates(a.grid, center, cx, cy, cz);
                 scan_stencil(
-                    a.grid, cx, cy, cz, [&](uint32_t s) { return within_support(a.kc, ps, xyz(a.xs[s])); },
+                    a.grid, a.xs, cx, cy, cz, [&](Float3 q) { return within_support(a.kc, ps, q); },
                     [&](uint32_t k, uint32_t bits) {
                         column[k * kBlock] = static_cast<uint16_t>(bits);
                         nonzero |= bits != 0u ? 1u << k : 0u;
@@ -528,16 +520,16 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
             if (masked) {
                 stored_slots<G, false>(a.skin, a.grid, a.grid.offsets, a.n, i, center, bits, first);
             } else if (listed) {
-                scanned_slots<G>(a.grid, a.grid.offsets, cx, cy, cz, bits, first,
-                                 [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.xs[s])); });
+                scanned_slots<G>(a.grid, a.grid.offsets, a.xs, cx, cy, cz, bits, first,
+                                 [&](Float3 q) { return within_support(a.kc, expanded, q); });
             }
         },
         [&](auto& bits, auto& first) {
             if (masked) {
                 stored_slots<G, false>(a.skin_samples, a.grid, a.boundary.offsets, a.n, i, center, bits, first);
             } else if (listed) {
-                scanned_slots<G>(a.grid, a.boundary.offsets, cx, cy, cz, bits, first,
-                                 [&](uint32_t s) { return within_support(a.kc, expanded, xyz(a.boundary.x[s])); });
+                scanned_slots<G>(a.grid, a.boundary.offsets, a.boundary.x, cx, cy, cz, bits, first,
+                                 [&](Float3 q) { return within_support(a.kc, expanded, q); });
             }
         },
         [&](const uint32_t* row, uint32_t count) {
