@@ -139,12 +139,14 @@ __device__ __forceinline__ GroupScene group_scene(uint32_t id, uint32_t n, const
     }
 }
 
-// The cell and crowded byte of each particle, and the workgroups (of
-// `particles` particles each) that hold crowded ones.
+// The cell and crowded byte of each particle (a stencil cell holds more than
+// kMaskBits particles, or boundary samples), and the workgroups (of `particles`
+// particles each) that hold crowded ones.
 template <bool kBatch>
-__global__ void __launch_bounds__(kBlock) pbf_cell_kernel(uint32_t n, SortedGrid launch_grid, const float4* xs, uint32_t* cell,
-                                                          uint8_t* crowded, uint32_t particles, Schedule schedule,
-                                                          BatchView batch) {
+__global__ void __launch_bounds__(kBlock) pbf_cell_kernel(uint32_t n, SortedGrid launch_grid,
+                                                          const uint32_t* sample_offsets, const float4* xs,
+                                                          uint32_t* cell, uint8_t* crowded, uint32_t particles,
+                                                          Schedule schedule, BatchView batch) {
     const uint32_t id = xcd_block();
     const Lane lane = lane_of<kBatch>(id, n, launch_grid, Box{}, batch);
     if (!lane.valid) return;
@@ -153,8 +155,10 @@ __global__ void __launch_bounds__(kBlock) pbf_cell_kernel(uint32_t n, SortedGrid
     particle_cell(grid, xyz(xs[lane.i]), cx, cy, cz);
     cell[lane.i] = cell_of(grid, cx, cy, cz);
     bool many = false;
-    for_each_cell(grid, cx, cy, cz,
-                  [&](uint32_t c) { many = many || grid.offsets[c + 1u] - grid.offsets[c] > kMaskBits; });
+    for_each_cell(grid, cx, cy, cz, [&](uint32_t c) {
+        many = many || grid.offsets[c + 1u] - grid.offsets[c] > kMaskBits;
+        if (sample_offsets != nullptr) many = many || sample_offsets[c + 1u] - sample_offsets[c] > kMaskBits;
+    });
     crowded[lane.i] = many ? 1u : 0u;
     if (!many) return;
     const uint32_t first = kBatch ? batch.blocks[id].group_block : id * (kBlock / particles);
@@ -893,9 +897,9 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     if (ordered) {
         PassScope scope(profiler_, stream_, kPbfMask);
         fill_u32(stream_, schedule_.data(), schedule_.size(), 0u);
-        pbf_cell_kernel<false><<<pbf_blocks(n, 1), kBlock, 0, stream_>>>(n, grid, xs_.data(), cells_.data(), crowded,
-                                                                         kBlock / static_cast<uint32_t>(group), schedule,
-                                                                         BatchView{});
+        pbf_cell_kernel<false><<<pbf_blocks(n, 1), kBlock, 0, stream_>>>(
+            n, grid, boundary.offsets, xs_.data(), cells_.data(), crowded, kBlock / static_cast<uint32_t>(group),
+            schedule, BatchView{});
         PHX_LAUNCH_CHECK();
     }
     // exact masks of position set k (iterate k, the final positions last):
@@ -1203,7 +1207,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     kernels_per_step_ += 3u;
     // the batch's offsets; each lane's grid starts at its scene's cell base
     const SortedGrid grid{grid_.offsets.data(), 0u, 0u, 0u, 0.0F, 0.0F, 0.0F, h_};
-    pbf_cell_kernel<true><<<blocks_, kBlock, 0, s>>>(n, grid, xs_.data(), cell_index_.data(), crowded_.data(),
+    pbf_cell_kernel<true><<<blocks_, kBlock, 0, s>>>(n, grid, nullptr, xs_.data(), cell_index_.data(), crowded_.data(),
                                                      kBlock / static_cast<uint32_t>(group_), schedule, bv);
     PHX_LAUNCH_CHECK();
     ++kernels_per_step_;

@@ -124,3 +124,25 @@ def test_sph_methods(gpu_device, count, spread, method):
             assert bits_equal(x, exp["positions"]), step
             assert bits_equal(v, exp["velocities"]), step
         state, nxt = nxt, state
+
+
+@pytest.mark.parametrize("shape", [(30, 20, 30), (60, 30, 60)])
+def test_pbf_cells_with_many_boundary_samples(gpu_device, shape):
+    """More than 16 boundary samples in a cell, in a scene whose passes run
+    their workgroups in order (18,000 particles) and in one that starts the
+    workgroups with crowded particles first (108,000)."""
+    sc = scenes.pbf_dam_break(shape=shape)
+    s = 2.0 * float(sc.domain.particle_radius)
+    x = np.arange(30) * s / 3.0
+    gx, gz = np.meshgrid(x + sc.positions[0].min(), x + sc.positions[2].min(), indexing="ij")
+    pos = np.stack([gx.ravel(), np.full(gx.size, -0.5 * s), gz.ravel()]).astype(np.float32)
+    vel = np.zeros_like(pos)
+    vol = np.full(pos.shape[1], s ** 3 / 9.0, np.float32)
+    sc.domain.boundary_particles = [(tuple(p), (0.0, 0.0, 0.0), float(w)) for p, w in zip(pos.T, vol)]
+    solver, state, nxt, control, params, cache = pbf_setup(sc, gpu_device, PBF.Configuration(2))
+    solver.forward_step(state, control, params, nxt, cache)
+    torch.cuda.synchronize()
+    d = oracle.make_domain(sc.domain, (pos, vel, vol))
+    exp = oracle.pbf_step(d, 0, sc.positions, sc.velocities, np.zeros_like(sc.positions), sc.parameters, 2)
+    assert bits_equal(nxt.particles.positions.numpy(), exp["positions"])
+    assert bits_equal(nxt.particles.velocities.numpy(), exp["velocities"])
