@@ -91,25 +91,71 @@ __device__ __forceinline__ void group_walk_list(const uint32_t* row, uint32_t co
     }
 }
 
-// group_walk_list over the particles of the 27 cells around (cx, cy, cz), and
-// with sample_offsets each cell's boundary samples after its particles: the
-// walk of a particle with a crowded cell, whose candidates have no masks.
-// The group tests G candidates at a time with near(entry), which is false
-// only where the terms are exact zeros, and collects the others in its list
-// `row`; a full list is walked on the way. Of the candidates of a crowded
-// neighbourhood a sixth to a half are kept, and the ordered additions make
-// each one dear. Entry `skip` is left out.
-template <int G, int F, class Near, class Load, class Pair, class Fold>
-__device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const uint32_t* sample_offsets, int cx, int cy,
-                                                   int cz, uint32_t skip, uint32_t fallback, uint32_t* row,
-                                                   Near&& near, Load&& load, Pair&& pair, Fold&& fold) {
+// Visits entries 0 .. count - 1 of a group's list for sums whose order is
+// free: each lane takes its own entries, pair(load(entry), entry), fetching one
+// ahead, and keeps partial sums (group_total).
+template <int G, class Load, class Pair>
+__device__ __forceinline__ void group_visit_list(const uint32_t* row, uint32_t count, Load&& load, Pair&& pair) {
+    uint32_t k = threadIdx.x % G;
+    if (k >= count) return;
+    uint32_t entry = row[k];
+    auto record = load(entry);
+    while (true) {
+        k += G;
+        uint32_t ahead = entry;
+        auto fetched = record;
+        if (k < count) {
+            ahead = row[k];
+            fetched = load(ahead);
+        }
+        asm volatile("" ::: "memory");
+        pair(record, entry);
+        if (k >= count) return;
+        entry = ahead;
+        record = fetched;
+    }
+}
+
+// v of the lane that DPP `control` reads for this one.
+template <int control>
+__device__ __forceinline__ double group_other(double v) {
+    const long long bits = __double_as_longlong(v);
+    const int low = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), control, 0xf, 0xf, true);
+    const int high = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), control, 0xf, 0xf, true);
+    return __longlong_as_double((static_cast<long long>(high) << 32) | static_cast<unsigned int>(low));
+}
+
+// The sum of the group's values, in every lane of the group.
+template <int G>
+__device__ __forceinline__ double group_total(double v) {
+    static_assert(G == 4 || G == 16, "groups are DPP quads or rows");
+    v += group_other<0xB1>(v);  // quad_perm:[1,0,3,2]
+    v += group_other<0x4E>(v);  // quad_perm:[2,3,0,1]
+    if constexpr (G == 16) {
+        v += group_other<0x124>(v);  // row_ror:4
+        v += group_other<0x128>(v);  // row_ror:8
+    }
+    return v;
+}
+
+// Walks the particles of the 27 cells around (cx, cy, cz), and with
+// sample_offsets each cell's boundary samples after its particles: the walk of
+// a particle with a crowded cell, whose candidates have no masks. The group
+// tests G candidates at a time with near(entry), which is false only where the
+// terms are exact zeros, and collects the others in its list `row`; a full
+// list is walked on the way with run(row, count). Of the candidates of a
+// crowded neighbourhood a sixth to a half are kept, and each one walked is
+// dear. Entry `skip` is left out.
+template <int G, class Near, class Run>
+__device__ __forceinline__ void group_near_stencil(const SortedGrid& g, const uint32_t* sample_offsets, int cx, int cy,
+                                                   int cz, uint32_t skip, uint32_t* row, Near&& near, Run&& walk) {
     const uint32_t lane = threadIdx.x % G;
     const uint32_t group_shift = __lane_id() - lane;
     uint32_t count = 0u;
     auto empty = [&] {
         // the list is written and read by this group alone, within its wave
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        group_walk_list<G, F>(row, count, fallback, load, pair, fold);
+        walk(row, count);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         count = 0u;
     };
@@ -130,6 +176,16 @@ __device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const ui
         if (sample_offsets != nullptr) run(sample_offsets[c], sample_offsets[c + 1u], kSampleEntry);
     });
     empty();
+}
+
+// group_near_stencil with the walks of group_walk_list.
+template <int G, int F, class Near, class Load, class Pair, class Fold>
+__device__ __forceinline__ void group_walk_stencil(const SortedGrid& g, const uint32_t* sample_offsets, int cx, int cy,
+                                                   int cz, uint32_t skip, uint32_t fallback, uint32_t* row,
+                                                   Near&& near, Load&& load, Pair&& pair, Fold&& fold) {
+    group_near_stencil<G>(g, sample_offsets, cx, cy, cz, skip, row, near, [&](const uint32_t* list, uint32_t count) {
+        group_walk_list<G, F>(list, count, fallback, load, pair, fold);
+    });
 }
 
 // Lists the candidates of a workgroup's particles and walks them.

@@ -83,8 +83,13 @@ struct PbfDerivativeWorkspace {
     VecBuffer x_t, v_t, u_t, p_t[2], vrec_t, w_t, vc_t;
     DeviceBuffer<float> rho_t, lambda_t, magnitude_t;
     // adjoints (FP64), sorted
-    DVecBuffer p_a[2], vrec_a, w_a, g_a, next_x_a, next_v_a, x_a, vel_a;
-    DeviceBuffer<double> lambda_a, magnitude_a;
+    DVecBuffer p_a, vrec_a, next_x_a, x_a;
+    DeviceBuffer<double> lambda_a;
+    // candidate records of the reverse passes: two of 16 bytes a particle
+    // (three doubles and one more), and of 16 bytes a particle
+    DeviceBuffer<double2> w_a, g_a, next_v_a, p_in;
+    DeviceBuffer<float4> point[2], gradient[2], confined, reconstructed, artificial;
+    DeviceBuffer<uint32_t> cell;
     DeviceBuffer<double> m_a, rho0_a, eps_a, strength_a, exponent_a, radius_a, xsph_a, confinement_a;
     DeviceBuffer<uint8_t> vanishes;  // per particle: the artificial pressure is the signed zero -k
     DeviceBuffer<double> inv_rho0;   // 1 / rho0

@@ -24,6 +24,7 @@
 // projection, vorticity (+ reconstruct), normal + confinement, XSPH.
 #include <cmath>
 
+#include "group_walk.hpp"
 #include "neighbor_mask.hpp"
 #include "pbf.hpp"
 
@@ -31,10 +32,6 @@ namespace phx {
 namespace {
 
 constexpr uint32_t kBlock = 256;
-// records a derivative pass's walks fetch ahead (two were no faster: the
-// deeper ring costs occupancy)
-constexpr int kVjpDepth = 1;
-
 // LDS of a masked neighbour pass: the lanes' mask columns and the slot table
 // (every thread reaches the barrier before any returns).
 #define PHX_MASK_LDS(grid)                          \
@@ -49,11 +46,26 @@ struct D3 {
 __device__ __forceinline__ D3 d3(Float3 a) {
     return {static_cast<double>(a.x), static_cast<double>(a.y), static_cast<double>(a.z)};
 }
-__device__ __forceinline__ D3 add(D3 a, D3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ D3 sub(D3 a, D3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ D3 scale(D3 v, double f) { return {f * v.x, f * v.y, f * v.z}; }
-__device__ __forceinline__ double dot(D3 a, D3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// The FP64 arithmetic of the reverse passes is fused where it can be (their
+// FP32 functions of the primal values, which are promoted, stay as written).
+__device__ __forceinline__ D3 add(D3 a, D3 b) {
+#pragma clang fp contract(fast)
+    return {a.x + b.x, a.y + b.y, a.z + b.z};
+}
+__device__ __forceinline__ D3 sub(D3 a, D3 b) {
+#pragma clang fp contract(fast)
+    return {a.x - b.x, a.y - b.y, a.z - b.z};
+}
+__device__ __forceinline__ D3 scale(D3 v, double f) {
+#pragma clang fp contract(fast)
+    return {f * v.x, f * v.y, f * v.z};
+}
+__device__ __forceinline__ double dot(D3 a, D3 b) {
+#pragma clang fp contract(fast)
+    return a.x * b.x + a.y * b.y + a.z * b.z;
+}
 __device__ __forceinline__ D3 cross(D3 a, D3 b) {
+#pragma clang fp contract(fast)
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 __device__ __forceinline__ D3 load(DVec f, uint32_t i) { return {f.x[i], f.y[i], f.z[i]}; }
@@ -94,17 +106,16 @@ struct Artificial {
 // can notice; only the strength derivative -(W / W(dq))^n needs a powf, and
 // only when `strength_wanted`.
 // `kernel` is poly6(d, h), which a pair's two directions share (d and -d
-// give the same value).
+// give the same value); `reference` is W(dq).
 __device__ __forceinline__ Artificial artificial_at(float kernel, Float3 d, float h, float strength, float exponent,
-                                                    float radius, bool vanishes = false, bool strength_wanted = true) {
+                                                    float radius, float reference, bool vanishes, bool strength_wanted) {
     Artificial a{0.0F, {0.0F, 0.0F, 0.0F}, 0.0F, 0.0F, 0.0F};
     if (kernel == 0.0F) return a;
     if (vanishes) {
         a.value = -strength;
-        if (strength_wanted) a.d_strength = -powf(kernel / poly6(Float3{radius, 0.0F, 0.0F}, h), exponent);
+        if (strength_wanted) a.d_strength = -powf(kernel / reference, exponent);
         return a;
     }
-    const float reference = poly6(Float3{radius, 0.0F, 0.0F}, h);
     const float ratio = kernel / reference;
     const float power = powf(ratio, exponent);
     a.value = -strength * power;
@@ -119,9 +130,9 @@ __device__ __forceinline__ Artificial artificial_at(float kernel, Float3 d, floa
     return a;
 }
 
-__device__ __forceinline__ Artificial artificial_full(Float3 d, float h, float strength, float exponent, float radius,
-                                                      bool vanishes = false, bool strength_wanted = true) {
-    return artificial_at(poly6(d, h), d, h, strength, exponent, radius, vanishes, strength_wanted);
+__device__ __forceinline__ Artificial artificial_full(Float3 d, float h, float strength, float exponent, float radius) {
+    return artificial_at(poly6(d, h), d, h, strength, exponent, radius, poly6(Float3{radius, 0.0F, 0.0F}, h), false,
+                         true);
 }
 
 // Sorted-order views of a recorded step and the sorted parameters.
@@ -132,8 +143,11 @@ struct Step {
     CVec xs, x0;
     const float *m, *rho0, *eps, *strength, *exponent, *radius, *xsph, *confinement;
     MaskView mv;  // the recorded step's masks and flags
-    const double* inv_rho0;  // 1 / rho0 (reverse passes)
     BoundaryGrid boundary;   // the step's sorted boundary samples; offsets null: none
+    // reverse passes
+    PbfKernel k;
+    float t_exact;  // exact_mask_threshold
+    const uint32_t* cell;
 };
 
 // Visits particle i's fluid candidates through its masks where they apply or,
@@ -149,20 +163,6 @@ __device__ __forceinline__ void walk_with_samples(const Step& s, bool masked, ui
         for_each_candidate(s.grid, s.boundary, cx, cy, cz, visit, visit_boundary);
     } else {
         visit_candidates(s.grid, s.mv, masked, i, cx, cy, cz, delta, column, kBlock, visit);
-    }
-}
-
-// The same with fluid candidate j visited as pair(load(j), j) (visit_records
-// without samples).
-template <class Load, class Pair, class VisitBoundary>
-__device__ __forceinline__ void walk_with_samples(const Step& s, bool masked, uint32_t i, int cx, int cy, int cz,
-                                                  const int* delta, uint16_t* column, Load&& load, Pair&& pair,
-                                                  VisitBoundary&& visit_boundary) {
-    if (s.boundary.offsets != nullptr) {
-        for_each_candidate(
-            s.grid, s.boundary, cx, cy, cz, [&](uint32_t j) { pair(load(j), j); }, visit_boundary);
-    } else {
-        visit_records<kVjpDepth>(s.grid, s.mv, masked, i, cx, cy, cz, delta, column, kBlock, load, pair);
     }
 }
 
@@ -183,165 +183,315 @@ __device__ __forceinline__ D3 unclamped(D3 b, uint8_t m) {
 }
 
 // ----------------------------------------------------------------------- VJP
+// A reverse pass serves each particle with a group of G lanes: each lane sums
+// the pair terms of every G-th candidate, and the lanes' FP64 sums are added
+// at the end (no order is prescribed for adjoints). With one lane per particle
+// a scene of 100,000 left three quarters of the wave slots empty. What a pass
+// reads of a candidate is packed into records of 16 bytes, written by the
+// passes before it: the address unit serves one wave load of 16 bytes a lane in
+// about the time of two of 4, and the fields taken one by one were 9 to 14
+// loads a candidate. 104,000 particles, us a pass before and now: correction
+// 72 / 54, lambda 48 / 41, post 47 / 29, normal 35 / 26, vorticity 42 / 30; the
+// FP64 arithmetic of the pairs bounds them now (three waves a SIMD; without the
+// candidate fetched ahead, or at four waves with spills, they are no faster).
+
+// Three doubles and one more as two records of a candidate.
+struct D4 {
+    D3 v;
+    double w;
+};
+__device__ __forceinline__ D4 load_d4(const double2* records, uint32_t i) {
+    const double2 a = records[2u * static_cast<size_t>(i)], b = records[2u * static_cast<size_t>(i) + 1u];
+    return D4{{a.x, a.y, b.x}, b.y};
+}
+__device__ __forceinline__ void store_d4(double2* records, uint32_t i, D3 v, double w) {
+    records[2u * static_cast<size_t>(i)] = make_double2(v.x, v.y);
+    records[2u * static_cast<size_t>(i) + 1u] = make_double2(v.z, w);
+}
+__device__ __forceinline__ Float3 xyz(float4 q) { return Float3{q.x, q.y, q.z}; }
+__device__ __forceinline__ float4 record(Float3 v, float w) { return make_float4(v.x, v.y, v.z, w); }
+
+template <int G>
+__device__ __forceinline__ D3 group_sum(D3 v) {
+    return D3{group_total<G>(v.x), group_total<G>(v.y), group_total<G>(v.z)};
+}
+
+// Visits the candidates of a workgroup's particles (base ..) with groups of G
+// lanes: pair(load(j), j) for the fluid particles of particle w's exact masks,
+// or of its stencil where they do not apply, and with kSamples sample(b) for
+// the boundary samples within the reach of the masks. pos holds the positions
+// of the masks.
+template <int G, bool kSamples, class Load, class Pair, class Sample>
+__device__ __forceinline__ void reverse_walk(const Step& s, const float4* pos, GroupLds<G>& lds, uint32_t base,
+                                             uint32_t w, Load&& load_record, Pair&& pair, Sample&& sample) {
+    const uint32_t i = base + threadIdx.x % kGroupParticles<G>;
+    const bool active = w < s.n;
+    bool masked = false;
+    uint32_t center = 0u;
+    if (i < s.n) {
+        center = s.cell[i];
+        masked = masks_apply(s.mv, 0u, i);
+    }
+    const bool listed = active && masks_apply(s.mv, 0u, w);
+    auto near = [&](Float3 p, Float3 q) {
+        const Float3 d = sub(p, q);
+        return !(dot(d, d) >= s.t_exact);
+    };
+    auto walk = [&](const uint32_t* row, uint32_t count) {
+        group_visit_list<G>(
+            row, count,
+            [&](uint32_t entry) { return load_record(kSamples && (entry & kSampleEntry) != 0u ? w : entry); },
+            [&](const auto& r, uint32_t entry) {
+                if constexpr (kSamples) {
+                    if ((entry & kSampleEntry) != 0u) {
+                        sample(s.boundary.x[entry & ~kSampleEntry]);
+                        return;
+                    }
+                }
+                pair(r, entry);
+            });
+    };
+    group_expand<G, kSamples>(
+        lds,
+        [&](auto& bits, auto& first) {
+            if (masked) stored_slots<G, false>(s.mv.masks, s.grid, s.grid.offsets, s.n, i, center, bits, first);
+        },
+        [&](auto& bits, auto& first) {
+            if (!masked) return;
+            const Float3 p = xyz(pos[i]);
+            int cx, cy, cz;
+            cell_coordinates(s.grid, center, cx, cy, cz);
+            scanned_slots<G>(s.grid, s.boundary.offsets, s.boundary.x, cx, cy, cz, bits, first,
+                             [&](Float3 q) { return near(p, q); });
+        },
+        [&](const uint32_t* row, uint32_t count) {
+            if (listed) walk(row, count);
+        });
+    if (!active || listed) return;
+    const Float3 p = xyz(pos[w]);
+    int cx, cy, cz;
+    cell_coordinates(s.grid, s.cell[w], cx, cy, cz);
+    group_near_stencil<G>(
+        s.grid, kSamples ? s.boundary.offsets : nullptr, cx, cy, cz, ~0u, group_row(lds),
+        [&](uint32_t entry) {
+            const bool is_sample = kSamples && (entry & kSampleEntry) != 0u;
+            return near(p, xyz(is_sample ? s.boundary.x[entry & ~kSampleEntry] : pos[entry]));
+        },
+        walk);
+}
+
+// The particle a group serves; every lane of the group has the same one.
+template <int G>
+__device__ __forceinline__ uint32_t walked_particle(uint32_t base) {
+    return base + threadIdx.x / G;
+}
+
+// The records of a constraint iteration, written before its passes by the
+// pass ahead of it (position adjoints are ready then), by one lane a particle.
+struct IterationRecords {
+    CVec pos;  // positions entering the iteration; x null: no iteration follows
+    const float* lambda;
+    CVec gsum;
+    const float* m;
+    const uint8_t* mask;  // box-collision bits of the iteration's projection
+    const double* inv_rho0;
+    float4* point;       // out: position, lambda
+    float4* gradient;    // out: gradient sum, mass
+    double2* p_in;       // out: adjoint of the positions leaving the iteration without its clamped components, 1 / rho0
+};
+__device__ __forceinline__ void write_records(const IterationRecords& r, uint32_t i, D3 adjoint) {
+    r.point[i] = record(load(r.pos, i), r.lambda[i]);
+    r.gradient[i] = record(load(r.gsum, i), r.m[i]);
+    store_d4(r.p_in, i, unclamped(adjoint, r.mask[i]), r.inv_rho0[i]);
+}
+
 struct PostVjpArgs {
     Step s;
-    uint32_t slot;  // displacement slot of the positions read
-    CVec pos, vc, w, nrm;
+    const float4* point;  // final positions (and vorticity magnitudes)
+    const float4* vc;
+    const double2* next_v_a;  // adjoint of the next velocity, and the XSPH viscosity
+    CVec w, nrm;
     const float* nz;
-    DVec next_x_a, next_v_a;  // adjoints of the next state, sorted
-    DVec p_a, vrec_a, w_a, g_a;
+    DVec next_x_a;  // adjoint of the next position, sorted
+    DVec p_a, vrec_a;
+    double2 *w_a, *g_a;
     double* xsph_a;
     double* confinement_a;
 };
 
 // xsph_vjp_kernel (pbf.cu:756-794), confinement_vjp_kernel (pbf.cu:688-698)
 // and the adjoint of the normalised gradient (pbf.cu:630-633).
-__global__ void __launch_bounds__(kBlock) pbf_vjp_post_kernel(PostVjpArgs a) {
-    PHX_MASK_LDS(a.s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vjp_post_kernel(PostVjpArgs a) {
+#pragma clang fp contract(fast)
+    __shared__ GroupLds<G> lds;
     const Step& s = a.s;
-    const Float3 pi = load(a.pos, i);
-    const D3 out = load(a.next_v_a, i);
-    const D3 vci = d3(load(a.vc, i));
-    const double ci = static_cast<double>(s.xsph[i]);
+    const uint32_t base = xcd_block() * kGroupParticles<G>;
+    const uint32_t w = walked_particle<G>(base);
+    const uint32_t own = w < s.n ? w : 0u;
+    const Float3 pi = xyz(a.point[own]);
+    const D4 self = load_d4(a.next_v_a, own);
+    const D3 out = self.v;
+    const D3 vci = d3(xyz(a.vc[own]));
+    const double ci = self.w;
     D3 pcon{0.0, 0.0, 0.0};
-    D3 vcon = out;
+    D3 vcon{0.0, 0.0, 0.0};
     double ccon = 0.0;
-    int cx, cy, cz;
-    cell_of_topology(s, i, cx, cy, cz);
     struct Record {
-        Float3 x, vc;
-        D3 vb;
-        float c;
+        float4 x, vc;
+        D4 vb;
     };
-    auto fetch = [&](uint32_t j) { return Record{load(a.pos, j), load(a.vc, j), load(a.next_v_a, j), s.xsph[j]}; };
-    visit_records<kVjpDepth>(s.grid, s.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, fetch,
-                  [&](const Record& r, uint32_t j) {
-        if (j == i) return;
-        const Float3 dd = sub(pi, r.x);
-        const double wgt = static_cast<double>(poly6(dd, s.h));
-        const D3 gw = d3(poly6_gradient(dd, s.h));
-        const D3 diff = sub(d3(r.vc), vci);
-        const D3 vb = r.vb;
-        const double cj = static_cast<double>(r.c);
-        vcon = add(vcon, scale(out, -ci * wgt));
-        vcon = add(vcon, scale(vb, cj * wgt));
-        pcon = add(pcon, scale(gw, ci * dot(out, diff) - cj * dot(vb, diff)));
-        ccon += wgt * dot(out, diff);
-    });
-    store(a.p_a, i, add(load(a.next_x_a, i), pcon));
-    a.xsph_a[i] += ccon;
+    reverse_walk<G, false>(
+        s, a.point, lds, base, w,
+        [&](uint32_t j) { return Record{a.point[j], a.vc[j], load_d4(a.next_v_a, j)}; },
+        [&](const Record& r, uint32_t j) {
+            if (j == w) return;
+            const Float3 dd = sub(pi, xyz(r.x));
+            const double wgt = static_cast<double>(poly6_value(dot(dd, dd), s.k));
+            const D3 gw = d3(poly6_gradient(dd, s.h));
+            const D3 diff = sub(d3(xyz(r.vc)), vci);
+            const D3 vb = r.vb.v;
+            const double cj = r.vb.w;
+            vcon = add(vcon, scale(out, -ci * wgt));
+            vcon = add(vcon, scale(vb, cj * wgt));
+            pcon = add(pcon, scale(gw, ci * dot(out, diff) - cj * dot(vb, diff)));
+            ccon += wgt * dot(out, diff);
+        },
+        [](float4) {});
+    pcon = group_sum<G>(pcon);
+    vcon = add(out, group_sum<G>(vcon));
+    ccon = group_total<G>(ccon);
+    if (w >= s.n || threadIdx.x % G != 0u) return;
+    store(a.p_a, w, add(load(a.next_x_a, w), pcon));
+    a.xsph_a[w] += ccon;
     // confinement: v_c = v + dt eps (n x w)
-    const D3 wv = d3(load(a.w, i));
-    const D3 nv = d3(load(a.nrm, i));
-    const double f = static_cast<double>(s.dt) * static_cast<double>(s.confinement[i]);
-    store(a.vrec_a, i, vcon);
-    store(a.w_a, i, scale(cross(vcon, nv), f));
+    const D3 wv = d3(load(a.w, w));
+    const D3 nv = d3(load(a.nrm, w));
+    const double f = static_cast<double>(s.dt) * static_cast<double>(s.confinement[w]);
+    store(a.vrec_a, w, vcon);
+    store_d4(a.w_a, w, scale(cross(vcon, nv), f), 0.0);
     const D3 n_bar = scale(cross(wv, vcon), f);
-    a.confinement_a[i] += static_cast<double>(s.dt) * dot(vcon, cross(nv, wv));
-    const float nz = a.nz[i];
-    store(a.g_a, i,
-          nz == 0.0F ? D3{0.0, 0.0, 0.0}
-                     : scale(sub(n_bar, scale(nv, dot(nv, n_bar))), 1.0 / static_cast<double>(nz)));
+    a.confinement_a[w] += static_cast<double>(s.dt) * dot(vcon, cross(nv, wv));
+    const float nz = a.nz[w];
+    store_d4(a.g_a, w,
+             nz == 0.0F ? D3{0.0, 0.0, 0.0}
+                        : scale(sub(n_bar, scale(nv, dot(nv, n_bar))), 1.0 / static_cast<double>(nz)),
+             0.0);
 }
 
 struct NormalVjpArgs {
     Step s;
-    uint32_t slot;  // displacement slot of the positions read
-    CVec pos, w;
-    const float* mag;
-    DVec p_a, w_a, g_a;
+    const float4* point;  // final positions and vorticity magnitudes
+    CVec w;
+    DVec p_a;
+    double2* w_a;
+    const double2* g_a;
 };
 
 // normal_vjp_kernel (pbf.cu:635-672) and the magnitude adjoint into omega.
-__global__ void __launch_bounds__(kBlock) pbf_vjp_normal_kernel(NormalVjpArgs a) {
-    PHX_MASK_LDS(a.s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vjp_normal_kernel(NormalVjpArgs a) {
+#pragma clang fp contract(fast)
+    __shared__ GroupLds<G> lds;
     const Step& s = a.s;
-    const Float3 pi = load(a.pos, i);
-    const D3 gi = load(a.g_a, i);
-    const double mi = static_cast<double>(a.mag[i]);
+    const uint32_t base = xcd_block() * kGroupParticles<G>;
+    const uint32_t w = walked_particle<G>(base);
+    const uint32_t own = w < s.n ? w : 0u;
+    const float4 self = a.point[own];
+    const Float3 pi = xyz(self);
+    const D3 gi = load_d4(a.g_a, own).v;
+    const double mi = static_cast<double>(self.w);
+    const double h = static_cast<double>(s.h), k = static_cast<double>(s.spiky);
     D3 pcon{0.0, 0.0, 0.0};
     double mcon = 0.0;
-    int cx, cy, cz;
-    cell_of_topology(s, i, cx, cy, cz);
     struct Record {
-        Float3 x;
-        float mag;
-        D3 g;
+        float4 x;
+        D4 g;
     };
-    auto fetch = [&](uint32_t j) { return Record{load(a.pos, j), a.mag[j], load(a.g_a, j)}; };
-    visit_records<kVjpDepth>(s.grid, s.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, fetch,
-                  [&](const Record& r, uint32_t j) {
-        if (j == i) return;
-        const Float3 dd = sub(pi, r.x);
-        const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
-        const D3 both = add(gi, r.g);
-        pcon = add(pcon, spiky_hessian(dd, scale(both, static_cast<double>(r.mag) - mi), static_cast<double>(s.h),
-                                       static_cast<double>(s.spiky)));
-        mcon -= dot(gr, both);
-    });
-    store(a.p_a, i, add(load(a.p_a, i), pcon));
-    if (a.mag[i] > 0.0F) store(a.w_a, i, add(load(a.w_a, i), scale(d3(load(a.w, i)), mcon / mi)));
+    reverse_walk<G, false>(
+        s, a.point, lds, base, w, [&](uint32_t j) { return Record{a.point[j], load_d4(a.g_a, j)}; },
+        [&](const Record& r, uint32_t j) {
+            if (j == w) return;
+            const Float3 dd = sub(pi, xyz(r.x));
+            const D3 gr = d3(scale(dd, spiky_factor(dot(dd, dd), s.k)));
+            const D3 both = add(gi, r.g.v);
+            pcon = add(pcon, spiky_hessian(dd, scale(both, static_cast<double>(r.x.w) - mi), h, k));
+            mcon -= dot(gr, both);
+        },
+        [](float4) {});
+    pcon = group_sum<G>(pcon);
+    mcon = group_total<G>(mcon);
+    if (w >= s.n || threadIdx.x % G != 0u) return;
+    store(a.p_a, w, add(load(a.p_a, w), pcon));
+    if (self.w > 0.0F)
+        store_d4(a.w_a, w, add(load_d4(a.w_a, w).v, scale(d3(load(a.w, w)), mcon / mi)), 0.0);
 }
 
 struct VorticityVjpArgs {
     Step s;
-    uint32_t slot;  // displacement slot of the positions read
-    CVec pos, vrec;
-    DVec p_a, vrec_a, w_a, x_a;
+    const float4* point;  // final positions
+    const float4* vrec;
+    DVec p_a, vrec_a;
+    const double2* w_a;
+    DVec x_a;
+    IterationRecords next;
 };
 
 // vorticity_vjp_kernel (pbf.cu:529-563) and reconstruct_vjp_kernel
 // (pbf.cu:468-474).
-__global__ void __launch_bounds__(kBlock) pbf_vjp_vorticity_kernel(VorticityVjpArgs a) {
-    PHX_MASK_LDS(a.s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vjp_vorticity_kernel(VorticityVjpArgs a) {
+#pragma clang fp contract(fast)
+    __shared__ GroupLds<G> lds;
     const Step& s = a.s;
-    const Float3 pi = load(a.pos, i);
-    const D3 vi = d3(load(a.vrec, i));
-    const D3 wb = load(a.w_a, i);
+    const uint32_t base = xcd_block() * kGroupParticles<G>;
+    const uint32_t w = walked_particle<G>(base);
+    const uint32_t own = w < s.n ? w : 0u;
+    const Float3 pi = xyz(a.point[own]);
+    const D3 vi = d3(xyz(a.vrec[own]));
+    const D3 wb = load_d4(a.w_a, own).v;
+    const double h = static_cast<double>(s.h), k = static_cast<double>(s.spiky);
     D3 pcon{0.0, 0.0, 0.0};
     D3 vcon{0.0, 0.0, 0.0};
-    int cx, cy, cz;
-    cell_of_topology(s, i, cx, cy, cz);
     struct Record {
-        Float3 x, v;
-        D3 w;
+        float4 x, v;
+        D4 w;
     };
-    auto fetch = [&](uint32_t j) { return Record{load(a.pos, j), load(a.vrec, j), load(a.w_a, j)}; };
-    visit_records<kVjpDepth>(s.grid, s.mv, masked, i, cx, cy, cz, delta, smask + threadIdx.x, kBlock, fetch,
-                  [&](const Record& r, uint32_t j) {
-        if (j == i) return;
-        const Float3 dd = sub(pi, r.x);
-        const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
-        const D3 both = add(wb, r.w);
-        const D3 diff = sub(d3(r.v), vi);
-        vcon = sub(vcon, cross(gr, both));
-        pcon = add(pcon, spiky_hessian(dd, cross(both, diff), static_cast<double>(s.h), static_cast<double>(s.spiky)));
-    });
-    const D3 va = add(load(a.vrec_a, i), vcon);
+    reverse_walk<G, false>(
+        s, a.point, lds, base, w,
+        [&](uint32_t j) { return Record{a.point[j], a.vrec[j], load_d4(a.w_a, j)}; },
+        [&](const Record& r, uint32_t j) {
+            if (j == w) return;
+            const Float3 dd = sub(pi, xyz(r.x));
+            const D3 gr = d3(scale(dd, spiky_factor(dot(dd, dd), s.k)));
+            const D3 both = add(wb, r.w.v);
+            const D3 diff = sub(d3(xyz(r.v)), vi);
+            vcon = sub(vcon, cross(gr, both));
+            pcon = add(pcon, spiky_hessian(dd, cross(both, diff), h, k));
+        },
+        [](float4) {});
+    pcon = group_sum<G>(pcon);
+    vcon = group_sum<G>(vcon);
+    if (w >= s.n || threadIdx.x % G != 0u) return;
+    const D3 va = add(load(a.vrec_a, w), vcon);
     const D3 cb = scale(va, static_cast<double>(s.inv_dt));
-    store(a.x_a, i, scale(cb, -1.0));
-    store(a.p_a, i, add(add(load(a.p_a, i), pcon), cb));
+    store(a.x_a, w, scale(cb, -1.0));
+    const D3 p = add(add(load(a.p_a, w), pcon), cb);
+    if (a.next.pos.x != nullptr) {
+        write_records(a.next, w, p);
+    } else {
+        store(a.p_a, w, p);
+    }
 }
 
 struct CorrectionVjpArgs {
     Step s;
-    uint32_t slot;  // displacement slot of the positions read
     const uint8_t* vanishes;  // per particle: artificial_vanishes
     uint32_t strength_wanted;
-    CVec pos;  // positions entering the iteration
-    const float* lambda;
-    const uint8_t* mask;
-    DVec p_in;   // adjoint of the positions leaving the iteration
-    DVec p_out;  // adjoint of the positions entering it (written)
+    const float4* point;  // IterationRecords
+    const float4* artificial;  // strength, exponent, W(radius) or -1 where the pressure vanishes, mass
+    const double2* p_in;
+    DVec p_out;  // adjoint of the positions entering the iteration (written)
     double* lambda_a;
     double *m_a, *rho0_a, *strength_a, *exponent_a, *radius_a;
     // the iteration's densities and denominators, for the per-particle terms
@@ -367,6 +517,7 @@ __device__ __forceinline__ double inverse_sqrt(double x) {
 // Derivative of G(d) = f(r) d (spiky gradient) along w, with 1 / r from
 // inverse_sqrt instead of a square root and a division.
 __device__ __forceinline__ D3 spiky_hessian_one_division(Float3 d, D3 w, double h, double k) {
+#pragma clang fp contract(fast)
     const D3 dd = d3(d);
     const double r2 = dot(dd, dd);
     if (r2 == 0.0) return {0.0, 0.0, 0.0};
@@ -383,189 +534,204 @@ __device__ __forceinline__ D3 spiky_hessian_one_division(Float3 d, D3 w, double 
 // (pbf.cu:335-415). The Hessian is even in d, so the terms where i is the
 // centre and where it is the neighbour share one product; the neighbour's
 // spiky gradient is the exact negation of the centre's.
-__global__ void __launch_bounds__(kBlock) pbf_vjp_correction_kernel(CorrectionVjpArgs a) {
-    PHX_MASK_LDS(a.s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+template <int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vjp_correction_kernel(CorrectionVjpArgs a) {
+#pragma clang fp contract(fast)
+    __shared__ GroupLds<G> lds;
     const Step& s = a.s;
+    const uint32_t base = xcd_block() * kGroupParticles<G>;
+    const uint32_t w = walked_particle<G>(base);
+    const uint32_t own = w < s.n ? w : 0u;
     const double h = static_cast<double>(s.h), k = static_cast<double>(s.spiky);
-    const Float3 pi = load(a.pos, i);
-    const double inv_rho0 = s.inv_rho0[i];
-    const D3 oa = unclamped(load(a.p_in, i), a.mask[i]);
-    const float lam_i = a.lambda[i];
-    const double m_i = static_cast<double>(s.m[i]);
+    const float4 self = a.point[own];
+    const Float3 pi = xyz(self);
+    const float lam_i = self.w;
+    const D4 adjoint = load_d4(a.p_in, own);
+    const D3 oa = adjoint.v;
+    const double inv_rho0 = adjoint.w;
+    const float4 pressure = a.artificial[own];
+    const float strength_i = pressure.x, exponent_i = pressure.y, radius_i = s.radius[own];
+    const float reference_i = poly6(Float3{radius_i, 0.0F, 0.0F}, s.h);
+    const bool vanishes_i = a.vanishes[own] != 0u;
+    const double m_i = static_cast<double>(pressure.w);
     D3 pcon{0.0, 0.0, 0.0};
     double lcon = 0.0, mcon = 0.0, rcon = 0.0, scon = 0.0, econ = 0.0, qcon = 0.0;
-    int cx, cy, cz;
-    cell_of_topology(s, i, cx, cy, cz);
-    // candidate j: position, lambda, mass, artificial-pressure parameters and
-    // vanishing flag, 1 / rho0 and its unclamped position adjoint
     struct Record {
-        Float3 x;
-        float lambda, m, strength, exponent, radius;
-        uint32_t vanishes;
-        double inv_rho0;
-        D3 ob;
+        float4 x, artificial;
+        D4 ob;
     };
-    auto fetch = [&](uint32_t j) {
-        return Record{load(a.pos, j),    a.lambda[j],  s.m[j],
-                      s.strength[j],     s.exponent[j], s.radius[j],
-                      a.vanishes[j],     s.inv_rho0[j], unclamped(load(a.p_in, j), a.mask[j])};
-    };
-    const float strength_i = s.strength[i], exponent_i = s.exponent[i], radius_i = s.radius[i];
-    const bool vanishes_i = a.vanishes[i] != 0u;
-    walk_with_samples(s, masked, i, cx, cy, cz, delta, smask + threadIdx.x, fetch, [&](const Record& r, uint32_t j) {
-        if (j == i) return;
-        const Float3 dd = sub(pi, r.x);
-        const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
-        const float lam_j = r.lambda;
-        // i as the centre
-        const float kernel = poly6(dd, s.h);
-        const Artificial art =
-            artificial_at(kernel, dd, s.h, strength_i, exponent_i, radius_i, vanishes_i, a.strength_wanted != 0u);
-        const double cf = static_cast<double>(r.m) * inv_rho0;
-        const double mu = static_cast<double>(lam_i) + static_cast<double>(lam_j) + static_cast<double>(art.value);
-        const double oa_gr = dot(oa, gr);
-        const double sa = cf * oa_gr;
-        lcon += sa;
-        rcon -= cf * mu * oa_gr * inv_rho0;
-        scon += sa * static_cast<double>(art.d_strength);
-        econ += sa * static_cast<double>(art.d_exponent);
-        qcon += sa * static_cast<double>(art.d_radius);
-        // i as a neighbour of j: d_ji = -d_ij, gradient -gr
-        const Artificial rart = artificial_at(kernel, scale(dd, -1.0F), s.h, r.strength, r.exponent, r.radius,
-                                              r.vanishes != 0u, a.strength_wanted != 0u);
-        const double inv_rrho0 = r.inv_rho0;
-        const double rcf = m_i * inv_rrho0;
-        const double rmu = static_cast<double>(lam_j) + static_cast<double>(lam_i) + static_cast<double>(rart.value);
-        const D3 ob = r.ob;
-        const double ob_rgr = -dot(ob, gr);
-        const double rsa = rcf * ob_rgr;
-        lcon += rsa;
-        mcon += rmu * inv_rrho0 * ob_rgr;
-        pcon = add(pcon, spiky_hessian_one_division(dd, sub(scale(oa, cf * mu), scale(ob, rcf * rmu)), h, k));
-        pcon = add(pcon, sub(scale(d3(art.gradient), sa), scale(d3(rart.gradient), rsa)));
-    }, [&](uint32_t b) {
-        // a boundary sample: V_b (lambda_i + s_corr) grad W (pbf.cu:390-397)
-        const Float3 dd = sub(pi, sample_position(s, b));
-        const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
-        const Artificial art =
-            artificial_full(dd, s.h, strength_i, exponent_i, radius_i, vanishes_i, a.strength_wanted != 0u);
-        const double vol = static_cast<double>(s.boundary.x[b].w);
-        const double mu = static_cast<double>(lam_i) + static_cast<double>(art.value);
-        const double sa = vol * dot(oa, gr);
-        lcon += sa;
-        scon += sa * static_cast<double>(art.d_strength);
-        econ += sa * static_cast<double>(art.d_exponent);
-        qcon += sa * static_cast<double>(art.d_radius);
-        pcon = add(pcon, spiky_hessian_one_division(dd, scale(oa, vol * mu), h, k));
-        pcon = add(pcon, scale(d3(art.gradient), sa));
-    });
-    store(a.p_out, i, add(oa, pcon));
-    a.lambda_a[i] = lcon;
-    a.m_a[i] += mcon;
-    a.rho0_a[i] += rcon;
-    a.strength_a[i] += scon;
-    a.exponent_a[i] += econ;
-    a.radius_a[i] += qcon;
+    reverse_walk<G, kSamples>(
+        s, a.point, lds, base, w,
+        [&](uint32_t j) { return Record{a.point[j], a.artificial[j], load_d4(a.p_in, j)}; },
+        [&](const Record& r, uint32_t j) {
+            if (j == w) return;
+            const Float3 dd = sub(pi, xyz(r.x));
+            const float d2 = dot(dd, dd);
+            const D3 gr = d3(scale(dd, spiky_factor(d2, s.k)));
+            const float lam_j = r.x.w;
+            // i as the centre
+            const float kernel = poly6_value(d2, s.k);
+            const Artificial art = artificial_at(kernel, dd, s.h, strength_i, exponent_i, radius_i, reference_i,
+                                                 vanishes_i, a.strength_wanted != 0u);
+            const double cf = static_cast<double>(r.artificial.w) * inv_rho0;
+            const double mu = static_cast<double>(lam_i) + static_cast<double>(lam_j) + static_cast<double>(art.value);
+            const double oa_gr = dot(oa, gr);
+            const double sa = cf * oa_gr;
+            lcon += sa;
+            rcon -= cf * mu * oa_gr * inv_rho0;
+            scon += sa * static_cast<double>(art.d_strength);
+            if (!vanishes_i) {  // all exact zeros otherwise
+                econ += sa * static_cast<double>(art.d_exponent);
+                qcon += sa * static_cast<double>(art.d_radius);
+                pcon = add(pcon, scale(d3(art.gradient), sa));
+            }
+            // i as a neighbour of j: d_ji = -d_ij, gradient -gr
+            const bool vanishes_j = r.artificial.z < 0.0F;
+            const Artificial rart = artificial_at(kernel, scale(dd, -1.0F), s.h, r.artificial.x, r.artificial.y, 0.0F,
+                                                  r.artificial.z, vanishes_j, false);
+            const double inv_rrho0 = r.ob.w;
+            const double rcf = m_i * inv_rrho0;
+            const double rmu =
+                static_cast<double>(lam_j) + static_cast<double>(lam_i) + static_cast<double>(rart.value);
+            const D3 ob = r.ob.v;
+            const double ob_rgr = -dot(ob, gr);
+            const double rsa = rcf * ob_rgr;
+            lcon += rsa;
+            mcon += rmu * inv_rrho0 * ob_rgr;
+            pcon = add(pcon, spiky_hessian_one_division(dd, sub(scale(oa, cf * mu), scale(ob, rcf * rmu)), h, k));
+            if (!vanishes_j) pcon = sub(pcon, scale(d3(rart.gradient), rsa));
+        },
+        [&](float4 q) {
+            // a boundary sample: V_b (lambda_i + s_corr) grad W (pbf.cu:390-397)
+            const Float3 dd = sub(pi, xyz(q));
+            const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
+            const Artificial art = artificial_at(poly6(dd, s.h), dd, s.h, strength_i, exponent_i, radius_i, reference_i,
+                                                 vanishes_i, a.strength_wanted != 0u);
+            const double vol = static_cast<double>(q.w);
+            const double mu = static_cast<double>(lam_i) + static_cast<double>(art.value);
+            const double sa = vol * dot(oa, gr);
+            lcon += sa;
+            scon += sa * static_cast<double>(art.d_strength);
+            econ += sa * static_cast<double>(art.d_exponent);
+            qcon += sa * static_cast<double>(art.d_radius);
+            pcon = add(pcon, spiky_hessian_one_division(dd, scale(oa, vol * mu), h, k));
+            pcon = add(pcon, scale(d3(art.gradient), sa));
+        });
+    pcon = group_sum<G>(pcon);
+    for (double* sum : {&lcon, &mcon, &rcon, &scon, &econ, &qcon}) *sum = group_total<G>(*sum);
+    if (w >= s.n || threadIdx.x % G != 0u) return;
+    store(a.p_out, w, add(oa, pcon));
+    a.lambda_a[w] = lcon;
+    a.m_a[w] += mcon;
+    a.rho0_a[w] += rcon;
+    a.strength_a[w] += scon;
+    a.exponent_a[w] += econ;
+    a.radius_a[w] += qcon;
     // lambda_vjp_kernel's per-particle terms: the density adjoint
     // -lambda_bar / (D rho0) and D_bar = lambda_bar C / D^2 (pbf.cu:207-214)
-    const double rho0 = static_cast<double>(s.rho0[i]);
-    const double den = static_cast<double>(a.den[i]);
-    const double con = static_cast<double>(a.rho[i]) / rho0 - 1.0;
-    a.lambda_terms[i] = make_double2(-(lcon / (den * rho0)), lcon * con / (den * den));
+    const double rho0 = static_cast<double>(s.rho0[w]);
+    const double den = static_cast<double>(a.den[w]);
+    const double con = static_cast<double>(a.rho[w]) / rho0 - 1.0;
+    a.lambda_terms[w] = make_double2(-(lcon / (den * rho0)), lcon * con / (den * den));
 }
 
 struct LambdaVjpArgs {
     Step s;
-    uint32_t slot;  // displacement slot of the positions read
-    CVec pos;
+    const float4 *point, *gradient;  // IterationRecords
+    const double* inv_rho0;
     const float *rho, *den;
-    CVec gsum;
     const double* lambda_a;
     const double2* lambda_terms;
     DVec p_out;
     double *m_a, *rho0_a, *eps_a;
+    IterationRecords next;
 };
 
 // lambda_vjp_kernel (pbf.cu:178-252) and density_vjp_kernel (density.cu:69-98,
 // poly6) with the neighbours' density adjoints and D_bar read from the
 // per-particle terms; the centre and neighbour Hessian terms share one
 // product.
-__global__ void __launch_bounds__(kBlock) pbf_vjp_lambda_kernel(LambdaVjpArgs a) {
-    PHX_MASK_LDS(a.s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+template <int G, bool kSamples>
+__global__ void __launch_bounds__(kGroupBlock) pbf_vjp_lambda_kernel(LambdaVjpArgs a) {
+#pragma clang fp contract(fast)
+    __shared__ GroupLds<G> lds;
     const Step& s = a.s;
+    const uint32_t base = xcd_block() * kGroupParticles<G>;
+    const uint32_t w = walked_particle<G>(base);
+    const uint32_t own = w < s.n ? w : 0u;
     const double h = static_cast<double>(s.h), k = static_cast<double>(s.spiky);
-    const Float3 pi = load(a.pos, i);
-    const double rho0 = static_cast<double>(s.rho0[i]);
-    const double inv_rho0 = s.inv_rho0[i];
-    const double den = static_cast<double>(a.den[i]);
-    const double lam_a = a.lambda_a[i];
-    const double2 terms = a.lambda_terms[i];
+    const Float3 pi = xyz(a.point[own]);
+    const float4 gradient = a.gradient[own];
+    const double inv_rho0 = a.inv_rho0[own];
+    const double2 terms = a.lambda_terms[own];
     const double rho_a = terms.x;
     const double dbar = terms.y;
-    const D3 sgi = d3(load(a.gsum, i));
-    const double mi = static_cast<double>(s.m[i]);
+    const D3 sgi = d3(xyz(gradient));
+    const double mi = static_cast<double>(gradient.w);
+    const double rho0 = static_cast<double>(s.rho0[own]);
     D3 pl{0.0, 0.0, 0.0}, pd{0.0, 0.0, 0.0};
     double ml = 0.0, md = 0.0;
-    double rcon = lam_a * static_cast<double>(a.rho[i]) / (den * rho0 * rho0);
+    double rcon = 0.0;
     double rd = 0.0;  // the density's rest-density adjoint (boundary samples)
-    int cx, cy, cz;
-    cell_of_topology(s, i, cx, cy, cz);
-    // candidate j: position, mass, per-particle lambda terms, 1 / rho0 and
-    // gradient sum
     struct Record {
-        Float3 x;
-        float m;
+        float4 x, gradient;
         double2 terms;
         double inv_rho0;
-        Float3 gsum;
     };
-    auto fetch = [&](uint32_t j) {
-        return Record{load(a.pos, j), s.m[j], a.lambda_terms[j], s.inv_rho0[j], load(a.gsum, j)};
-    };
-    walk_with_samples(s, masked, i, cx, cy, cz, delta, smask + threadIdx.x, fetch, [&](const Record& r, uint32_t j) {
-        const Float3 dd = sub(pi, r.x);
-        const double2 jterms = r.terms;
-        // density term (the self term has a zero gradient)
-        const D3 gw = d3(poly6_gradient(dd, s.h));
-        pd = add(pd, scale(gw, rho_a * static_cast<double>(r.m) + jterms.x * mi));
-        md += jterms.x * static_cast<double>(poly6(dd, s.h));
-        if (j == i) return;
-        const D3 gr = d3(spiky_gradient(dd, s.h, s.spiky));
-        const double gr2 = dot(gr, gr);
-        // i as the centre: g_bar = 2 D_bar c (c g + S), c_bar = 2 D_bar (c |g|^2 + g . S)
-        const double cf = static_cast<double>(r.m) * inv_rho0;
-        const D3 gbar = scale(add(scale(gr, cf), sgi), 2.0 * dbar * cf);
-        const double cbar = 2.0 * dbar * (cf * gr2 + dot(gr, sgi));
-        rcon -= cbar * cf * inv_rho0;
-        // i as a neighbour of j: gradient -gr
-        const double inv_jrho0 = r.inv_rho0;
-        const D3 sgj = d3(r.gsum);
-        const double rcf = mi * inv_jrho0;
-        const D3 rgbar = scale(sub(sgj, scale(gr, rcf)), 2.0 * jterms.y * rcf);
-        const double rcbar = 2.0 * jterms.y * (rcf * gr2 - dot(gr, sgj));
-        ml += rcbar * inv_jrho0;
-        pl = add(pl, spiky_hessian_one_division(dd, sub(gbar, rgbar), h, k));
-    }, [&](uint32_t b) {
-        // a boundary sample: the density term rho0_i V_b W (density.cu:88-93)
-        // and V_b grad W in the gradient sum only (pbf.cu:226-229)
-        const Float3 dd = sub(pi, sample_position(s, b));
-        const double vol = static_cast<double>(s.boundary.x[b].w);
-        pd = add(pd, scale(d3(poly6_gradient(dd, s.h)), rho_a * rho0 * vol));
-        rd += rho_a * vol * static_cast<double>(poly6(dd, s.h));
-        pl = add(pl, spiky_hessian_one_division(dd, scale(sgi, 2.0 * dbar * vol), h, k));
-    });
-    store(a.p_out, i, add(add(load(a.p_out, i), pl), pd));
-    a.m_a[i] += ml;
-    a.m_a[i] += md;
-    a.rho0_a[i] += rcon;
-    a.rho0_a[i] += rd;
-    a.eps_a[i] += dbar;
+    reverse_walk<G, kSamples>(
+        s, a.point, lds, base, w,
+        [&](uint32_t j) { return Record{a.point[j], a.gradient[j], a.lambda_terms[j], a.inv_rho0[j]}; },
+        [&](const Record& r, uint32_t j) {
+            const Float3 dd = sub(pi, xyz(r.x));
+            const float d2 = dot(dd, dd);
+            const double2 jterms = r.terms;
+            const double mj = static_cast<double>(r.gradient.w);
+            // density term (the self term has a zero gradient)
+            const D3 gw = d3(poly6_gradient(dd, s.h));
+            pd = add(pd, scale(gw, rho_a * mj + jterms.x * mi));
+            md += jterms.x * static_cast<double>(poly6_value(d2, s.k));
+            if (j == w) return;
+            const D3 gr = d3(scale(dd, spiky_factor(d2, s.k)));
+            const double gr2 = dot(gr, gr);
+            // i as the centre: g_bar = 2 D_bar c (c g + S), c_bar = 2 D_bar (c |g|^2 + g . S)
+            const double cf = mj * inv_rho0;
+            const D3 gbar = scale(add(scale(gr, cf), sgi), 2.0 * dbar * cf);
+            const double cbar = 2.0 * dbar * (cf * gr2 + dot(gr, sgi));
+            rcon -= cbar * cf * inv_rho0;
+            // i as a neighbour of j: gradient -gr
+            const double inv_jrho0 = r.inv_rho0;
+            const D3 sgj = d3(xyz(r.gradient));
+            const double rcf = mi * inv_jrho0;
+            const D3 rgbar = scale(sub(sgj, scale(gr, rcf)), 2.0 * jterms.y * rcf);
+            const double rcbar = 2.0 * jterms.y * (rcf * gr2 - dot(gr, sgj));
+            ml += rcbar * inv_jrho0;
+            pl = add(pl, spiky_hessian_one_division(dd, sub(gbar, rgbar), h, k));
+        },
+        [&](float4 q) {
+            // a boundary sample: the density term rho0_i V_b W (density.cu:88-93)
+            // and V_b grad W in the gradient sum only (pbf.cu:226-229)
+            const Float3 dd = sub(pi, xyz(q));
+            const double vol = static_cast<double>(q.w);
+            pd = add(pd, scale(d3(poly6_gradient(dd, s.h)), rho_a * rho0 * vol));
+            rd += rho_a * vol * static_cast<double>(poly6(dd, s.h));
+            pl = add(pl, spiky_hessian_one_division(dd, scale(sgi, 2.0 * dbar * vol), h, k));
+        });
+    pl = group_sum<G>(pl);
+    pd = group_sum<G>(pd);
+    for (double* sum : {&ml, &md, &rcon, &rd}) *sum = group_total<G>(*sum);
+    if (w >= s.n || threadIdx.x % G != 0u) return;
+    const double den = static_cast<double>(a.den[w]);
+    const D3 p = add(add(load(a.p_out, w), pl), pd);
+    a.m_a[w] += ml;
+    a.m_a[w] += md;
+    a.rho0_a[w] += a.lambda_a[w] * static_cast<double>(a.rho[w]) / (den * rho0 * rho0) + rcon;
+    a.rho0_a[w] += rd;
+    a.eps_a[w] += dbar;
+    if (a.next.pos.x != nullptr) {
+        write_records(a.next, w, p);
+    } else {
+        store(a.p_out, w, p);
+    }
 }
 
 struct ScatterVjpArgs {
@@ -606,24 +772,47 @@ __global__ void __launch_bounds__(kBlock) pbf_vjp_scatter_kernel(ScatterVjpArgs 
         if (a.original[c] != nullptr) a.original[c][o] += a.sorted[c][i];
 }
 
-// Per-particle constants of the reverse passes: whether the artificial
-// pressure vanishes, and 1 / rho0.
-__global__ void __launch_bounds__(kBlock) pbf_vjp_setup_kernel(uint32_t n, float h, const float* strength,
-                                                               const float* exponent, const float* radius,
-                                                               const float* rho0, uint8_t* vanishes,
-                                                               double* inv_rho0) {
+// Per-particle constants of the reverse passes: the cell, whether the
+// artificial pressure vanishes, 1 / rho0 and the correction's record.
+struct SetupVjpArgs {
+    uint32_t n;
+    float h;
+    SortedGrid grid;
+    CVec xs;
+    const float *strength, *exponent, *radius, *rho0, *m;
+    uint32_t* cell;
+    uint8_t* vanishes;
+    double* inv_rho0;
+    float4* artificial;
+    double* parameter_a[8];  // sorted parameter adjoints, which start at zero
+};
+__global__ void __launch_bounds__(kBlock) pbf_vjp_setup_kernel(SetupVjpArgs a) {
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float reference = poly6(Float3{radius[i], 0.0F, 0.0F}, h);
-    vanishes[i] = artificial_vanishes(h, strength[i], exponent[i], reference) ? 1u : 0u;
-    inv_rho0[i] = 1.0 / static_cast<double>(rho0[i]);
+    if (i >= a.n) return;
+    int cx, cy, cz;
+    particle_cell(a.grid, load(a.xs, i), cx, cy, cz);
+    a.cell[i] = cell_of(a.grid, cx, cy, cz);
+    const float strength = a.strength[i], exponent = a.exponent[i];
+    const float reference = poly6(Float3{a.radius[i], 0.0F, 0.0F}, a.h);
+    const bool vanishes = artificial_vanishes(a.h, strength, exponent, reference);
+    a.vanishes[i] = vanishes ? 1u : 0u;
+    a.inv_rho0[i] = 1.0 / static_cast<double>(a.rho0[i]);
+    a.artificial[i] = make_float4(strength, exponent, vanishes ? -1.0F : reference, a.m[i]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) a.parameter_a[c][i] = 0.0;
 }
 
+// The caller's adjoints in sorted order, and the records of the first passes.
 struct GatherAdjointArgs {
     uint32_t n;
     const uint32_t* perm;
     const double *xx, *xy, *xz, *vx, *vy, *vz;
-    DVec x_a, v_a;
+    const float* xsph;
+    CVec pos, vc, vrec;
+    const float* mag;
+    DVec x_a;
+    double2* v_a;
+    float4 *point, *vc_out, *vrec_out;
 };
 
 __global__ void __launch_bounds__(kBlock) pbf_gather_adjoint_kernel(GatherAdjointArgs a) {
@@ -631,7 +820,29 @@ __global__ void __launch_bounds__(kBlock) pbf_gather_adjoint_kernel(GatherAdjoin
     if (i >= a.n) return;
     const uint32_t o = a.perm[i];
     store(a.x_a, i, D3{a.xx[o], a.xy[o], a.xz[o]});
-    store(a.v_a, i, D3{a.vx[o], a.vy[o], a.vz[o]});
+    store_d4(a.v_a, i, D3{a.vx[o], a.vy[o], a.vz[o]}, static_cast<double>(a.xsph[i]));
+    a.point[i] = record(load(a.pos, i), a.mag[i]);
+    a.vc_out[i] = record(load(a.vc, i), 0.0F);
+    a.vrec_out[i] = record(load(a.vrec, i), 0.0F);
+}
+
+// Lanes per particle of the reverse passes: 16 up to this many particles, then
+// 4 (more lanes spread a particle's chain of candidates, and idle in its last
+// trip). Sums of the five passes' times, us, with 16 / 4 lanes: 2,000 particles
+// 40 / 65, 8,000 43 / 65, 16,000 61 / 67, 32,000 96 / 77, 104,000 271 / 181.
+constexpr uint32_t kReverseGroup16Particles = 20000;
+
+// Calls launch(std::integral_constant<int, G>, blocks).
+template <class Launch>
+void with_reverse_group(uint32_t n, Launch&& launch) {
+    const uint32_t lanes = n <= kReverseGroup16Particles ? 16u : 4u;
+    const uint32_t blocks = (blocks_for(n, kGroupBlock / lanes) + 7u) / 8u * 8u;
+    if (lanes == 16u) {
+        launch(std::integral_constant<int, 16>{}, blocks);
+    } else {
+        launch(std::integral_constant<int, 4>{}, blocks);
+    }
+    PHX_LAUNCH_CHECK();
 }
 
 // ----------------------------------------------------------------------- JVP
@@ -875,8 +1086,13 @@ void PbfDerivativeWorkspace::allocate(uint32_t n) {
                                    &lambda_t, &magnitude_t})
         b->resize(n);
     for (VecBuffer* b : {&x_t, &v_t, &u_t, &p_t[0], &p_t[1], &vrec_t, &w_t, &vc_t}) b->resize(n);
-    for (DVecBuffer* b : {&p_a[0], &p_a[1], &vrec_a, &w_a, &g_a, &next_x_a, &next_v_a, &x_a, &vel_a}) b->resize(n);
-    for (DeviceBuffer<double>* b : {&lambda_a, &magnitude_a, &m_a, &rho0_a, &eps_a, &strength_a, &exponent_a, &radius_a,
+    for (DVecBuffer* b : {&p_a, &vrec_a, &next_x_a, &x_a}) b->resize(n);
+    for (DeviceBuffer<double2>* b : {&w_a, &g_a, &next_v_a, &p_in}) b->resize(2u * static_cast<size_t>(n));
+    for (DeviceBuffer<float4>* b : {&point[0], &point[1], &gradient[0], &gradient[1], &confined, &reconstructed,
+                                    &artificial})
+        b->resize(n);
+    cell.resize(n);
+    for (DeviceBuffer<double>* b : {&lambda_a, &m_a, &rho0_a, &eps_a, &strength_a, &exponent_a, &radius_a,
                                     &xsph_a, &confinement_a, &inv_rho0})
         b->resize(n);
     lambda_terms.resize(n);
@@ -974,8 +1190,10 @@ void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.xsph.data(),
            dw_.confinement.data(),
            exact_view(cache, iterations, n),
-           nullptr,
-           cache.neighborhood.boundary()};
+           cache.neighborhood.boundary(),
+           kernel_,
+           exact_mask_threshold(c.support_radius),
+           nullptr};
     const TangentParams tp{dw_.m_t.data(),        dw_.rho0_t.data(),   dw_.eps_t.data(),  dw_.strength_t.data(),
                            dw_.exponent_t.data(), dw_.radius_t.data(), dw_.xsph_t.data(), dw_.confinement_t.data()};
     PredictJvpArgs pa{n,
@@ -1072,95 +1290,158 @@ void PbfSolver::vjp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.xsph.data(),
            dw_.confinement.data(),
            exact_view(cache, iterations, n),
-           dw_.inv_rho0.data(),
-           cache.neighborhood.boundary()};
-    // sorted parameter adjoints start at zero (+0.0 is the all-zero bit pattern)
-    for (DeviceBuffer<double>* b : {&dw_.m_a, &dw_.rho0_a, &dw_.eps_a, &dw_.strength_a, &dw_.exponent_a,
-                                    &dw_.radius_a, &dw_.xsph_a, &dw_.confinement_a})
-        fill_u32(stream_, reinterpret_cast<uint32_t*>(b->data()), 2u * static_cast<size_t>(n), 0u);
-    pbf_vjp_setup_kernel<<<blocks, kBlock, 0, stream_>>>(n, c.support_radius, dw_.strength.data(),
-                                                          dw_.exponent.data(), dw_.radius.data(), dw_.rho0.data(),
-                                                          dw_.vanishes.data(), dw_.inv_rho0.data());
+           cache.neighborhood.boundary(),
+           kernel_,
+           exact_mask_threshold(c.support_radius),
+           dw_.cell.data()};
+    const SetupVjpArgs setup{n,
+                             c.support_radius,
+                             s.grid,
+                             s.xs,
+                             s.strength,
+                             s.exponent,
+                             s.radius,
+                             s.rho0,
+                             s.m,
+                             dw_.cell.data(),
+                             dw_.vanishes.data(),
+                             dw_.inv_rho0.data(),
+                             dw_.artificial.data(),
+                             {dw_.m_a.data(), dw_.rho0_a.data(), dw_.eps_a.data(), dw_.strength_a.data(),
+                              dw_.exponent_a.data(), dw_.radius_a.data(), dw_.xsph_a.data(),
+                              dw_.confinement_a.data()}};
+    pbf_vjp_setup_kernel<<<blocks, kBlock, 0, stream_>>>(setup);
     PHX_LAUNCH_CHECK();
-    GatherAdjointArgs ga{n, perm, nx.x, nx.y, nx.z, nv.x, nv.y, nv.z, dw_.next_x_a.view(), dw_.next_v_a.view()};
+    int cur = 0;  // the point and gradient records of the pass; the next iteration's are written to the others
+    const GatherAdjointArgs ga{n,
+                               perm,
+                               nx.x,
+                               nx.y,
+                               nx.z,
+                               nv.x,
+                               nv.y,
+                               nv.z,
+                               s.xsph,
+                               iterations == 0u ? cache.xs.cview() : cache.positions.cview(iterations - 1u),
+                               cache.confined.cview(),
+                               cache.velocities.cview(),
+                               cache.magnitudes.data(),
+                               dw_.next_x_a.view(),
+                               dw_.next_v_a.data(),
+                               dw_.point[cur].data(),
+                               dw_.confined.data(),
+                               dw_.reconstructed.data()};
     pbf_gather_adjoint_kernel<<<blocks, kBlock, 0, stream_>>>(ga);
     PHX_LAUNCH_CHECK();
 
-    const CVec final_pos = iterations == 0u ? cache.xs.cview() : cache.positions.cview(iterations - 1u);
-    int cur = 0;
+    // the records of iteration `it`, in the buffers `to`
+    auto records = [&](uint32_t it, int to) {
+        const size_t off = static_cast<size_t>(it) * n;
+        return IterationRecords{it == 0u ? cache.xs.cview() : cache.positions.cview(it - 1u),
+                                cache.lambda.data() + off,
+                                cache.gradient_sums.cview(it),
+                                s.m,
+                                cache.masks.data() + off,
+                                dw_.inv_rho0.data(),
+                                dw_.point[to].data(),
+                                dw_.gradient[to].data(),
+                                dw_.p_in.data()};
+    };
+    const PostVjpArgs pv{s,
+                         dw_.point[cur].data(),
+                         dw_.confined.data(),
+                         dw_.next_v_a.data(),
+                         cache.vorticities.cview(),
+                         cache.normals.cview(),
+                         cache.normalizers.data(),
+                         dw_.next_x_a.view(),
+                         dw_.p_a.view(),
+                         dw_.vrec_a.view(),
+                         dw_.w_a.data(),
+                         dw_.g_a.data(),
+                         dw_.xsph_a.data(),
+                         dw_.confinement_a.data()};
+    with_reverse_group(n, [&](auto g, uint32_t launch_blocks) {
+        pbf_vjp_post_kernel<g()><<<launch_blocks, kGroupBlock, 0, stream_>>>(pv);
+    });
+    const NormalVjpArgs nva{s,
+                            dw_.point[cur].data(),
+                            cache.vorticities.cview(),
+                            dw_.p_a.view(),
+                            dw_.w_a.data(),
+                            dw_.g_a.data()};
+    with_reverse_group(n, [&](auto g, uint32_t launch_blocks) {
+        pbf_vjp_normal_kernel<g()><<<launch_blocks, kGroupBlock, 0, stream_>>>(nva);
+    });
+    VorticityVjpArgs vva{s,
+                         dw_.point[cur].data(),
+                         dw_.reconstructed.data(),
+                         dw_.p_a.view(),
+                         dw_.vrec_a.view(),
+                         dw_.w_a.data(),
+                         dw_.x_a.view(),
+                         IterationRecords{}};
+    if (iterations > 0u) vva.next = records(iterations - 1u, cur ^ 1);
+    with_reverse_group(n, [&](auto g, uint32_t launch_blocks) {
+        pbf_vjp_vorticity_kernel<g()><<<launch_blocks, kGroupBlock, 0, stream_>>>(vva);
+    });
+    const bool samples = s.boundary.offsets != nullptr;
     Step se = s;  // the passes at one set of positions walk its exact masks
-    se.mv = exact_view(cache, iterations, n);
-    PostVjpArgs pv{se,
-                   iterations,
-                   final_pos,
-                   cache.confined.cview(),
-                   cache.vorticities.cview(),
-                   cache.normals.cview(),
-                   cache.normalizers.data(),
-                   dw_.next_x_a.view(),
-                   dw_.next_v_a.view(),
-                   dw_.p_a[cur].view(),
-                   dw_.vrec_a.view(),
-                   dw_.w_a.view(),
-                   dw_.g_a.view(),
-                   dw_.xsph_a.data(),
-                   dw_.confinement_a.data()};
-    pbf_vjp_post_kernel<<<blocks, kBlock, 0, stream_>>>(pv);
-    PHX_LAUNCH_CHECK();
-    NormalVjpArgs nva{se, iterations, final_pos, cache.vorticities.cview(), cache.magnitudes.data(), dw_.p_a[cur].view(),
-                      dw_.w_a.view(), dw_.g_a.view()};
-    pbf_vjp_normal_kernel<<<blocks, kBlock, 0, stream_>>>(nva);
-    PHX_LAUNCH_CHECK();
-    VorticityVjpArgs vva{se, iterations, final_pos, cache.velocities.cview(), dw_.p_a[cur].view(), dw_.vrec_a.view(),
-                         dw_.w_a.view(), dw_.x_a.view()};
-    pbf_vjp_vorticity_kernel<<<blocks, kBlock, 0, stream_>>>(vva);
-    PHX_LAUNCH_CHECK();
     for (uint32_t it = iterations; it-- > 0u;) {
-        const CVec pos = it == 0u ? cache.xs.cview() : cache.positions.cview(it - 1u);
+        cur ^= 1;
         const size_t off = static_cast<size_t>(it) * n;
         se.mv = exact_view(cache, it, n);
-        CorrectionVjpArgs cva{se,
-                              it,
-                              dw_.vanishes.data(),
-                              parameter_a.artificial_pressure_strength != nullptr ? 1u : 0u,
-                              pos,
-                              cache.lambda.data() + off,
-                              cache.masks.data() + off,
-                              dw_.p_a[cur].view(),
-                              dw_.p_a[cur ^ 1].view(),
-                              dw_.lambda_a.data(),
-                              dw_.m_a.data(),
-                              dw_.rho0_a.data(),
-                              dw_.strength_a.data(),
-                              dw_.exponent_a.data(),
-                              dw_.radius_a.data(),
-                              cache.rho.data() + off,
-                              cache.den.data() + off,
-                              dw_.lambda_terms.data()};
-        pbf_vjp_correction_kernel<<<blocks, kBlock, 0, stream_>>>(cva);
-        PHX_LAUNCH_CHECK();
+        const CorrectionVjpArgs cva{se,
+                                    dw_.vanishes.data(),
+                                    parameter_a.artificial_pressure_strength != nullptr ? 1u : 0u,
+                                    dw_.point[cur].data(),
+                                    dw_.artificial.data(),
+                                    dw_.p_in.data(),
+                                    dw_.p_a.view(),
+                                    dw_.lambda_a.data(),
+                                    dw_.m_a.data(),
+                                    dw_.rho0_a.data(),
+                                    dw_.strength_a.data(),
+                                    dw_.exponent_a.data(),
+                                    dw_.radius_a.data(),
+                                    cache.rho.data() + off,
+                                    cache.den.data() + off,
+                                    dw_.lambda_terms.data()};
+        with_reverse_group(n, [&](auto g, uint32_t launch_blocks) {
+            if (samples) {
+                pbf_vjp_correction_kernel<g(), true><<<launch_blocks, kGroupBlock, 0, stream_>>>(cva);
+            } else {
+                pbf_vjp_correction_kernel<g(), false><<<launch_blocks, kGroupBlock, 0, stream_>>>(cva);
+            }
+        });
         LambdaVjpArgs lva{se,
-                          it,
-                          pos,
+                          dw_.point[cur].data(),
+                          dw_.gradient[cur].data(),
+                          dw_.inv_rho0.data(),
                           cache.rho.data() + off,
                           cache.den.data() + off,
-                          cache.gradient_sums.cview(it),
                           dw_.lambda_a.data(),
                           dw_.lambda_terms.data(),
-                          dw_.p_a[cur ^ 1].view(),
+                          dw_.p_a.view(),
                           dw_.m_a.data(),
                           dw_.rho0_a.data(),
-                          dw_.eps_a.data()};
-        pbf_vjp_lambda_kernel<<<blocks, kBlock, 0, stream_>>>(lva);
-        PHX_LAUNCH_CHECK();
-        cur ^= 1;
+                          dw_.eps_a.data(),
+                          IterationRecords{}};
+        if (it > 0u) lva.next = records(it - 1u, cur ^ 1);
+        with_reverse_group(n, [&](auto g, uint32_t launch_blocks) {
+            if (samples) {
+                pbf_vjp_lambda_kernel<g(), true><<<launch_blocks, kGroupBlock, 0, stream_>>>(lva);
+            } else {
+                pbf_vjp_lambda_kernel<g(), false><<<launch_blocks, kGroupBlock, 0, stream_>>>(lva);
+            }
+        });
     }
     ScatterVjpArgs sa{};
     sa.n = n;
     sa.dt = static_cast<double>(c.time_step);
     sa.dt2 = static_cast<double>(c.time_step * c.time_step);
     sa.perm = perm;
-    sa.p_a = dw_.p_a[cur].view();
+    sa.p_a = dw_.p_a.view();
     sa.x_a = dw_.x_a.view();
     sa.prev_x = DVec{previous_a.positions.x, previous_a.positions.y, previous_a.positions.z};
     sa.prev_v = DVec{previous_a.velocities.x, previous_a.velocities.y, previous_a.velocities.z};
