@@ -53,6 +53,12 @@ class PbfRollout:
         self._recorded: Optional[Tuple[int, int]] = None
         self._scratch_states: List[PBF.State] = []
         self._scratch_cache: Optional[PBF.StepCache] = None
+        # checkpoint_every = 1: the step caches, which the next forward pass
+        # records over, and the solver they belong to. Allocated anew on every
+        # pass (some 20 device allocations a step, and their release, each of
+        # which waits for the GPU) they left it idle for a third of a pass.
+        self._kept: List[PBF.StepCache] = []
+        self._kept_of: Optional[PBF] = None
         self._partner: Optional[PBF] = None
 
     def _workspace(self, solver: PBF, count: int):
@@ -97,6 +103,8 @@ class PbfRollout:
         self._caches = []
         self._recorded = None
         keep_all = self.checkpoint_every == 1
+        if self._kept_of is not solver:
+            self._kept, self._kept_of = [], solver
         if not keep_all and not self._scratch_states:
             self._scratch_states = [solver.allocate_state(), solver.allocate_state()]
         # checkpointed: the last segment is recorded now, into the workspace of
@@ -110,9 +118,10 @@ class PbfRollout:
             checkpoint = keep_all or (k + 1) % self.checkpoint_every == 0 or k + 1 == self.steps
             if keep_all:
                 nxt = solver.allocate_state()
-                cache = solver.allocate_step_cache()
-                solver.forward_step(current, control, parameters, nxt, cache)
-                self._caches.append(cache)
+                if k == len(self._kept):
+                    self._kept.append(solver.allocate_step_cache())
+                solver.forward_step(current, control, parameters, nxt, self._kept[k])
+                self._caches.append(self._kept[k])
             elif k >= last_first:
                 nxt = solver.allocate_state() if checkpoint else seg_states[k - last_first]
                 solver.forward_step(current, control, parameters, nxt, seg_caches[k - last_first])
@@ -202,3 +211,4 @@ class PbfRollout:
         self._states, self._caches = [], []
         self._work, self._recorded = {}, None
         self._scratch_states, self._scratch_cache = [], None
+        self._kept, self._kept_of = [], None
