@@ -79,9 +79,10 @@ void DfsphCache::allocate(uint32_t n, uint32_t cells, uint32_t divergence_iterat
     if (!record) return;
     const size_t nn = n;
     const size_t updates = static_cast<size_t>(divergence_iterations) + density_iterations;
-    for (DeviceBuffer<float4>* b : {&xm, &vmu}) b->resize(nn);
+    vmu.resize(nn);
+    xm.resize(nn + kScanPadding);
     for (DeviceBuffer<float>* b : {&rho0, &relax_div, &relax_den}) b->resize(nn);
-    xs.resize(updates * nn);
+    xs.resize(updates * nn + kScanPadding);
     rs.resize(updates * nn);
     p.resize((updates + 2u) * nn);
     collisions.resize((updates + 1u) * nn);

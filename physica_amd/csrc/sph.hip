@@ -388,7 +388,8 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
         if (!cache.wcsph) cache.wcsph = std::make_unique<WcsphRecord>();
         r = cache.wcsph.get();
         r->recorded = false;
-        for (DeviceBuffer<float4>* b : {&r->xm, &r->vmu, &r->aux}) b->resize(n);
+        for (DeviceBuffer<float4>* b : {&r->vmu, &r->aux}) b->resize(n);
+        r->xm.resize(n + static_cast<size_t>(kScanPadding));
         for (DeviceBuffer<float>* b : {&r->rho0, &r->tait}) b->resize(n);
         r->collisions.resize(n);
         r->exact.resize(static_cast<size_t>(kStencil) * n);
