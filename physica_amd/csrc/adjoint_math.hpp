@@ -19,9 +19,20 @@ struct D3 {
 __device__ __forceinline__ D3 d3(Float3 a) {
     return {static_cast<double>(a.x), static_cast<double>(a.y), static_cast<double>(a.z)};
 }
-__device__ __forceinline__ D3 add(D3 a, D3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ D3 scale(D3 v, double f) { return {f * v.x, f * v.y, f * v.z}; }
-__device__ __forceinline__ double dot(D3 a, D3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// The FP64 vector arithmetic is fused where it can be (the FP32 functions of
+// the primal values, which are promoted, stay as written).
+__device__ __forceinline__ D3 add(D3 a, D3 b) {
+#pragma clang fp contract(fast)
+    return {a.x + b.x, a.y + b.y, a.z + b.z};
+}
+__device__ __forceinline__ D3 scale(D3 v, double f) {
+#pragma clang fp contract(fast)
+    return {f * v.x, f * v.y, f * v.z};
+}
+__device__ __forceinline__ double dot(D3 a, D3 b) {
+#pragma clang fp contract(fast)
+    return a.x * b.x + a.y * b.y + a.z * b.z;
+}
 __device__ __forceinline__ D3 load(DVec f, uint32_t i) { return {f.x[i], f.y[i], f.z[i]}; }
 __device__ __forceinline__ void store(DVec f, uint32_t i, D3 v) {
     f.x[i] = v.x;
@@ -60,17 +71,24 @@ __device__ __forceinline__ float viscosity_laplacian_tangent(Float3 d, Float3 dd
 
 // cubic_hessian_product (density/device.cuh:59-70): H(d) w in FP64.
 __device__ __forceinline__ D3 cubic_hessian_product(Float3 d, D3 w, float h) {
-    const double dist = sqrt(static_cast<double>(dot(d, d)));
+    // 1 / h, 1 / h^2 (of the FP32 square) and the coefficient do not change from
+    // pair to pair; 1 / |d| from inverse_sqrt in place of a square root and five
+    // divisions
+    const double inv_h = 1.0 / static_cast<double>(h);
+    const double inv_h2 = 1.0 / static_cast<double>(h * h);
     const double coef = 8.0 / (static_cast<double>(kPi) * h * h * h);
-    if (dist == 0.0) return scale(w, -12.0 * coef / (h * h));
+    const double d2 = static_cast<double>(dot(d, d));
+    if (d2 == 0.0) return scale(w, -12.0 * coef * inv_h2);
+    const double inv_dist = inverse_sqrt(d2);
+    const double dist = d2 * inv_dist;
     if (dist >= h) return {0.0, 0.0, 0.0};
-    const double q = dist / h;
+    const double q = dist * inv_h;
     const double deriv = q <= 0.5 ? 18.0 * q * q - 12.0 * q : -6.0 * (1.0 - q) * (1.0 - q);
     const double second = q <= 0.5 ? 36.0 * q - 12.0 : 12.0 * (1.0 - q);
-    const double rs = coef * deriv / (h * dist);
-    const double rsd = coef * (second / (h * h * dist) - deriv / (h * dist * dist));
+    const double rs = coef * deriv * (inv_h * inv_dist);
+    const double rsd = coef * (second * (inv_h2 * inv_dist) - deriv * (inv_h * inv_dist * inv_dist));
     const D3 dd = d3(d);
-    return add(scale(w, rs), scale(dd, rsd * dot(w, dd) / dist));
+    return add(scale(w, rs), scale(dd, rsd * dot(w, dd) * inv_dist));
 }
 
 // viscosity_laplacian_gradient (density/device.cuh:84-88) with pow(h, 6)

@@ -265,6 +265,20 @@ __device__ __forceinline__ float artificial_value(float d2, const PbfKernel& k, 
     return -strength * powf(kernel / reference, exponent);
 }
 
+// 1 / sqrt(x) for a positive normal x: the hardware estimate refined by two
+// Newton steps, y <- y + y (1 - x y^2) / 2, to within a few units of the
+// last place (the derivative passes compare with the FP64 oracle to 1e-10;
+// the square root and the division they replace cost about 30 instructions).
+__device__ __forceinline__ double inverse_sqrt(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+#pragma unroll
+    for (int step = 0; step < 2; ++step) {
+        const double e = fma(-x * y, y, 1.0);
+        y = fma(0.5 * y, e, y);
+    }
+    return y;
+}
+
 // min(C-1, max(0, floor(v))) with NaN and negatives mapped to 0, as the
 // reference's __float2int_rd + clamp (neighborhood.cu:34-36).
 __device__ __forceinline__ int cell_clamp(float v, uint32_t count) {

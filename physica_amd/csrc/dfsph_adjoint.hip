@@ -39,18 +39,15 @@
 
 #include "adjoint_math.hpp"
 #include "dfsph.hpp"
+#include "group_walk.hpp"
 #include "neighbor_mask.hpp"
+
+#include <type_traits>
 
 namespace phx {
 namespace {
 
 constexpr uint32_t kBlock = 256;
-
-#define PHX_MASK_LDS(grid)                          \
-    __shared__ uint16_t smask[kStencil * kBlock];   \
-    __shared__ int delta[kStencil];                 \
-    fill_slot_deltas(grid, delta);                  \
-    __syncthreads()
 
 // The recorded step in sorted order.
 struct Step {
@@ -85,19 +82,148 @@ __device__ __forceinline__ MaskView skin_view(const Step& s) {
     return MaskView{s.skin, s.flags, s.n, s.limit2, 0u, s.crowded};
 }
 
-// Visits the fluid candidates of particle i (through the masks where they
-// apply) or, with boundary samples, every fluid particle and every sample of
-// the 27 cells in the reference order: each cell's fluid, then its samples.
-template <class Visit, class VisitBoundary>
-__device__ __forceinline__ void walk(const Step& s, const MaskView& mv, bool masked, uint32_t i, int cx, int cy,
-                                     int cz, const int* delta, uint16_t* column, Visit&& visit,
-                                     VisitBoundary&& visit_boundary) {
-    if (s.boundary.offsets != nullptr) {
-        for_each_candidate(s.grid, s.boundary, cx, cy, cz, visit, visit_boundary);
-    } else {
-        visit_candidates(s.grid, mv, masked, i, cx, cy, cz, delta, column, kBlock, visit);
-    }
+// The derivative passes serve each particle with a group of G lanes: with one
+// lane a particle they were a chain of 40 to 60 candidates, with few waves in
+// flight. 36,000 particles, us a pass before and now: pressure VJP 53 / 20 (with
+// the non-pressure terms 75 / 42; one Hessian product a pair for two, without
+// its divisions), density VJP 43 / 24, projection JVP 51 / 23, force JVP 31 / 16.
+
+// Lists the candidates of a workgroup's particles (base ..) for its groups:
+// the fluid particles in the masks of particle w or, where they do not apply,
+// near it at the positions pos, walked with fluid(row, count); for a crowded
+// particle and in a step with boundary samples (whose masks are not used) the
+// particles and samples of the stencil near it, walked with all(row, count).
+template <int G, class Fluid, class All>
+__device__ __forceinline__ void group_candidates(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
+                                                 const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
+                                                 Fluid&& fluid, All&& all) {
+    const uint32_t i = base + threadIdx.x % kGroupParticles<G>;
+    const bool active = w < s.n;
+    // the rounding of a distance in another order than the kernels'
+    const float reach = s.kc.sqrt_support * (1.0F + 4e-6F);
+    auto near = [&](Float3 p, Float3 q) {
+        const Float3 d = sub(p, q);
+        return !(dot(d, d) >= reach);
+    };
+    const bool listed = active && exact_masked(s, w);
+    group_expand<G, false>(
+        lds,
+        [&](auto& bits, auto& first) {
+            if (i >= s.n || !exact_masked(s, i)) return;
+            int cx, cy, cz;
+            particle_cell(s.grid, xyz(s.xm[i]), cx, cy, cz);
+            if (exact || masks_apply(mv, slot, i)) {
+                stored_slots<G, false>(mv.masks, s.grid, s.grid.offsets, s.n, i, cell_of(s.grid, cx, cy, cz), bits,
+                                       first);
+            } else {
+                const Float3 p = xyz(pos[i]);
+                scanned_slots<G>(s.grid, s.grid.offsets, pos, cx, cy, cz, bits, first,
+                                 [&](Float3 q) { return near(p, q); });
+            }
+        },
+        [](auto&, auto&) {},
+        [&](const uint32_t* row, uint32_t count) {
+            if (listed) fluid(row, count);
+        });
+    if (!active || listed) return;
+    const Float3 p = xyz(pos[w]);
+    int cx, cy, cz;
+    particle_cell(s.grid, xyz(s.xm[w]), cx, cy, cz);
+    group_near_stencil<G>(
+        s.grid, s.boundary.offsets, cx, cy, cz, ~0u, group_row(lds),
+        [&](uint32_t entry) {
+            const bool is_sample = (entry & kSampleEntry) != 0u;
+            return near(p, xyz(is_sample ? s.boundary.x[entry & ~kSampleEntry] : pos[entry]));
+        },
+        all);
 }
+
+// The candidates of an adjoint: pair(load(j), j) and sample(b), each lane with
+// every G-th one; the lanes' FP64 sums are added at the end, in no order.
+template <int G, class Load, class Pair, class Sample>
+__device__ __forceinline__ void group_visit(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
+                                            const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
+                                            Load&& load_record, Pair&& pair, Sample&& sample) {
+    group_candidates<G>(
+        s, mv, exact, slot, pos, lds, base, w,
+        [&](const uint32_t* row, uint32_t count) { group_visit_list<G>(row, count, load_record, pair); },
+        [&](const uint32_t* row, uint32_t count) {
+            group_visit_list<G>(
+                row, count,
+                [&](uint32_t entry) { return load_record((entry & kSampleEntry) != 0u ? w : entry); },
+                [&](const auto& r, uint32_t entry) {
+                    if ((entry & kSampleEntry) != 0u) {
+                        sample(entry & ~kSampleEntry);
+                    } else {
+                        pair(r, entry);
+                    }
+                });
+        });
+}
+
+// The candidates of an FP32 tangent: pair(load(j), j, terms) and
+// sample(b, terms) write a candidate's F terms, which are added to sum in the
+// reference's order (group_add).
+template <int G, int F, class Load, class Pair, class Sample>
+__device__ __forceinline__ void group_tangent(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
+                                              const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
+                                              float (&sum)[F], Load&& load_record, Pair&& pair, Sample&& sample) {
+    auto fold = [&](const float (&terms)[F]) { group_add<G, F>(sum, terms); };
+    group_candidates<G>(
+        s, mv, exact, slot, pos, lds, base, w,
+        [&](const uint32_t* row, uint32_t count) { group_walk_list<G, F>(row, count, w, load_record, pair, fold); },
+        [&](const uint32_t* row, uint32_t count) {
+            group_walk_list<G, F>(
+                row, count, w,
+                [&](uint32_t entry) { return load_record((entry & kSampleEntry) != 0u ? w : entry); },
+                [&](const auto& r, uint32_t entry, float (&terms)[F]) {
+                    if ((entry & kSampleEntry) != 0u) {
+                        sample(entry & ~kSampleEntry, terms);
+                    } else {
+                        pair(r, entry, terms);
+                    }
+                },
+                fold);
+        });
+}
+
+__device__ __forceinline__ void put(float* terms, Float3 v) {
+    terms[0] = v.x;
+    terms[1] = v.y;
+    terms[2] = v.z;
+}
+
+// Lanes per particle: 16 up to this many particles, then 4. Projection JVP and
+// pressure VJP, us, with 16 / 4 lanes: 2,000 particles 9 / 17 and 9 / 14, 16,000
+// 12 / 19 and 13 / 15, 36,000 21 / 23 and 20 / 20 (with crowded cells 33 / 46
+// and 39 / 47), 100,000 53 / 59 and 71 / 65.
+constexpr uint32_t kDerivativeGroup16Particles = 40000;
+
+// Calls launch(std::integral_constant<int, G>, blocks).
+template <class Launch>
+void with_derivative_group(uint32_t n, Launch&& launch) {
+    const uint32_t lanes = n <= kDerivativeGroup16Particles ? 16u : 4u;
+    const uint32_t blocks = (blocks_for(n, kGroupBlock / lanes) + 7u) / 8u * 8u;
+    if (lanes == 16u) {
+        launch(std::integral_constant<int, 16>{}, blocks);
+    } else {
+        launch(std::integral_constant<int, 4>{}, blocks);
+    }
+    PHX_LAUNCH_CHECK();
+}
+
+template <int G>
+__device__ __forceinline__ D3 group_sum(D3 v) {
+    return D3{group_total<G>(v.x), group_total<G>(v.y), group_total<G>(v.z)};
+}
+// What a derivative kernel declares of its group: its particle w (i: w, or
+// particle 0 where there is none) and its lists.
+#define PHX_DERIVATIVE_GROUP(n)                                \
+    __shared__ GroupLds<G> lds;                                \
+    const uint32_t base = xcd_block() * kGroupParticles<G>;    \
+    const uint32_t w = base + threadIdx.x / G;                 \
+    const uint32_t i = w < (n) ? w : 0u;                       \
+    const bool writes = w < (n) && threadIdx.x % G == 0u
 
 // ----------------------------------------------------------------- JVP
 struct GatherTangentArgs {
@@ -146,35 +272,37 @@ struct DensityJvpArgs {
 
 // density_jvp_kernel (density.cu:42-67, topology = positions = x) and the
 // first terms of the two initial pressure fields.
-__global__ void __launch_bounds__(kBlock) dfsph_jvp_density_kernel(DensityJvpArgs a) {
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_density_kernel(DensityJvpArgs a) {
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const Float3 p = xyz(s.xm[i]);
     const Float3 pt = xyz(a.xt[i]);
-    int cx, cy, cz;
-    particle_cell(s.grid, p, cx, cy, cz);
-    float result = 0.0F;
+    float sum[1] = {0.0F};
     const float rest_i = s.rest[i];
     const float rest_t_i = a.rest_t[i];
-    walk(
-        s, exact_view(s), exact_masked(s, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-        [&](uint32_t j) {
-            const float4 q = s.xm[j];
-            const float4 qt = a.xt[j];
+    struct Record {
+        float4 q, qt;
+    };
+    group_tangent<G, 1>(
+        s, exact_view(s), true, 0u, s.xm, lds, base, w, sum, [&](uint32_t j) { return Record{s.xm[j], a.xt[j]}; },
+        [&](const Record& r, uint32_t, float (&terms)[1]) {
+            const float4 q = r.q;
+            const float4 qt = r.qt;
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
-            result += qt.w * cubic_value(dist, s.kc) +
-                      q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pt, xyz(qt)));
+            terms[0] = qt.w * cubic_value(dist, s.kc) +
+                       q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pt, xyz(qt)));
         },
-        [&](uint32_t b) {
+        [&](uint32_t b, float (&terms)[1]) {
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
-            result += q.w * (rest_t_i * cubic_value(dist, s.kc) +
-                             rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pt));
+            terms[0] = q.w * (rest_t_i * cubic_value(dist, s.kc) +
+                              rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pt));
         });
+    if (!writes) return;
+    const float result = sum[0];
     a.rho_t[i] = result;
     const float rho = s.rho[i];
     a.t_div[i] = first_term(a.p_div[i], a.p_t_div[i], rho, result);
@@ -212,41 +340,45 @@ struct ForceJvpArgs {
 // pressure_jvp_kernel (common.cu:196-237) for one or two pressure fields +
 // predict_jvp_kernel (dfsph.cu:46-66) of the next prediction or the next
 // state.
-template <bool kNonPressure, int kEpilogue>
-__global__ void __launch_bounds__(kBlock) dfsph_jvp_force_kernel(ForceJvpArgs a) {
+template <bool kNonPressure, int kEpilogue, int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_force_kernel(ForceJvpArgs a) {
     constexpr bool kTwo = kEpilogue == kJvpDivEnd;
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const float4 self = s.xm[i];
     const Float3 x = xyz(self);
     const float4 xt_i = a.xt[i];
     const Float3 xti = xyz(xt_i);
     const float4 vm = s.vmu[i];
     const float4 vt_i = a.vt[i];
-    Float3 acc_t{0.0F, 0.0F, 0.0F};
-    if constexpr (kNonPressure) acc_t = xyz(a.ut[i]);
     const float2 t1_i = a.t1[i];
     float2 t2_i = make_float2(0.0F, 0.0F);
     if constexpr (kTwo) t2_i = a.t2[i];
-    Float3 ap1{0.0F, 0.0F, 0.0F};
-    Float3 ap2{0.0F, 0.0F, 0.0F};
+    // the sums: the non-pressure acceleration's tangent, then the pressure
+    // accelerations'
+    constexpr int kFirst = kNonPressure ? 3 : 0;
+    constexpr int kSecond = kFirst + 3;
+    constexpr int kSums = kTwo ? kSecond + 3 : kSecond;
+    float sum[kSums] = {};
+    if constexpr (kNonPressure) put(sum, xyz(a.ut[i]));
     const float rest_i = s.rest[i];
     const float rest_t_i = a.ut[i].w;
-    int cx, cy, cz;
-    particle_cell(s.grid, x, cx, cy, cz);
     // the pressure terms of sample b (pressure_jvp_kernel's boundary half)
-    auto boundary_pressure = [&](const Float3& gradient, const Float3& gradient_t, float vol, float2 t, Float3& ap) {
+    auto boundary_pressure = [&](const Float3& gradient, const Float3& gradient_t, float vol, float2 t) {
         const float factor = -rest_i * vol * t.x;
         const float factor_t = -vol * (rest_t_i * t.x + rest_i * t.y);
-        ap = add(ap, add(scale(gradient, factor_t), scale(gradient_t, factor)));
+        return add(scale(gradient, factor_t), scale(gradient_t, factor));
     };
-    walk(s, exact_view(s), exact_masked(s, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-                     [&](uint32_t j) {
-                         if (j == i) return;
-                         const float4 q = s.xm[j];
-                         const float4 qt = a.xt[j];
+    struct Record {
+        float4 q, qt;
+        float2 t1, t2;
+    };
+    group_tangent<G, kSums>(s, exact_view(s), true, 0u, s.xm, lds, base, w, sum,
+                     [&](uint32_t j) { return Record{s.xm[j], a.xt[j], a.t1[j], kTwo ? a.t2[j] : float2{}}; },
+                     [&](const Record& r, uint32_t j, float (&terms)[kSums]) {
+                         if (j == w) return;
+                         const float4 q = r.q;
+                         const float4 qt = r.qt;
                          const float mass = q.w;
                          const Float3 d = sub(x, xyz(q));
                          const Float3 dd = sub(xti, xyz(qt));
@@ -258,44 +390,48 @@ __global__ void __launch_bounds__(kBlock) dfsph_jvp_force_kernel(ForceJvpArgs a)
                              const float nu = 0.5F * (vm.w + vq.w);
                              const float nu_t = 0.5F * (vt_i.w + vqt.w);
                              const float dens = s.rho[j];
-                             const float w = nu * mass * lap / dens;
+                             const float weight = nu * mass * lap / dens;
                              const float w_t = nu_t * mass * lap / dens + nu * qt.w * lap / dens +
                                                nu * mass * lap_t / dens - nu * mass * lap * a.rho_t[j] / (dens * dens);
                              const Float3 diff = sub(xyz(vq), xyz(vm));
                              const Float3 diff_t = sub(xyz(vqt), xyz(vt_i));
-                             acc_t = add(acc_t, add(scale(diff, w_t), scale(diff_t, w)));
+                             put(terms, add(scale(diff, w_t), scale(diff_t, weight)));
                          }
                          const Float3 gradient = scale(d, cubic_gradient_factor(length(d), s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, dd, s.kc);
-                         const float2 t1_j = a.t1[j];
+                         const float2 t1_j = r.t1;
                          const float factor = -mass * (t1_i.x + t1_j.x);
                          const float factor_t = -qt.w * (t1_i.x + t1_j.x) - mass * (t1_i.y + t1_j.y);
-                         ap1 = add(ap1, add(scale(gradient, factor_t), scale(gradient_t, factor)));
+                         put(terms + kFirst, add(scale(gradient, factor_t), scale(gradient_t, factor)));
                          if constexpr (kTwo) {
-                             const float2 t2_j = a.t2[j];
+                             const float2 t2_j = r.t2;
                              const float f2 = -mass * (t2_i.x + t2_j.x);
                              const float f2_t = -qt.w * (t2_i.x + t2_j.x) - mass * (t2_i.y + t2_j.y);
-                             ap2 = add(ap2, add(scale(gradient, f2_t), scale(gradient_t, f2)));
+                             put(terms + kSecond, add(scale(gradient, f2_t), scale(gradient_t, f2)));
                          }
                      },
-                     [&](uint32_t b) {
+                     [&](uint32_t b, float (&terms)[kSums]) {
                          const float4 q = s.boundary.x[b];
                          const float vol = q.w;
                          const Float3 d = sub(x, xyz(q));
                          if constexpr (kNonPressure) {
                              // non_pressure_jvp_kernel's boundary half: mu_i V lap (v_b - v_i)
                              const float lap = viscosity_laplacian_c(d, s.kc);
-                             const float w = vm.w * vol * lap;
+                             const float weight = vm.w * vol * lap;
                              const float w_t = vol * (vt_i.w * lap + vm.w * viscosity_laplacian_tangent(d, xti, s.kc));
                              const Float3 diff = sub(xyz(s.boundary.v[b]), xyz(vm));
-                             acc_t = add(acc_t, add(scale(diff, w_t), scale(xyz(vt_i), -w)));
+                             put(terms, add(scale(diff, w_t), scale(xyz(vt_i), -weight)));
                          }
                          const Float3 gradient = scale(d, cubic_gradient_factor(length(d), s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, xti, s.kc);
-                         boundary_pressure(gradient, gradient_t, vol, t1_i, ap1);
-                         if constexpr (kTwo) boundary_pressure(gradient, gradient_t, vol, t2_i, ap2);
+                         put(terms + kFirst, boundary_pressure(gradient, gradient_t, vol, t1_i));
+                         if constexpr (kTwo) put(terms + kSecond, boundary_pressure(gradient, gradient_t, vol, t2_i));
                      });
+    if (!writes) return;
+    const Float3 ap1{sum[kFirst], sum[kFirst + 1], sum[kFirst + 2]};
+    Float3 acc_t;
     if constexpr (kNonPressure) {
+        acc_t = Float3{sum[0], sum[1], sum[2]};
         a.anp_t[i] = make_float4(acc_t.x, acc_t.y, acc_t.z, 0.0F);
     } else {
         acc_t = xyz(a.anp_t[i]);
@@ -305,7 +441,7 @@ __global__ void __launch_bounds__(kBlock) dfsph_jvp_force_kernel(ForceJvpArgs a)
         total = ap1;
     } else if constexpr (kTwo) {
         a.adiv_t[i] = make_float4(ap1.x, ap1.y, ap1.z, 0.0F);
-        total = add(ap1, ap2);
+        total = add(ap1, Float3{sum[kSecond], sum[kSecond + 1], sum[kSecond + 2]});
     } else {
         total = add(xyz(a.adiv_t[i]), ap1);
     }
@@ -347,36 +483,40 @@ struct ProjectionJvpArgs {
 
 // density_jvp_kernel at the predicted positions (topology x) +
 // projection_update_jvp_kernel (dfsph.cu:112-121).
-__global__ void __launch_bounds__(kBlock) dfsph_jvp_projection_kernel(ProjectionJvpArgs a) {
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_projection_kernel(ProjectionJvpArgs a) {
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const float4 self = a.xs[i];
     const Float3 ps = xyz(self);
     const Float3 pst = xyz(a.xs_t[i]);
-    int cx, cy, cz;
-    particle_cell(s.grid, xyz(s.xm[i]), cx, cy, cz);
-    float rs_t = 0.0F;
+    float sum[1] = {0.0F};
     const float rest_i = s.rest[i];
     const float rest_t_i = a.rest_t[i];
     const MaskView mv = skin_view(s);
-    walk(
-        s, mv, masks_apply(mv, a.slot, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-        [&](uint32_t j) {
-            const float4 q = a.xs[j];
+    struct Record {
+        float4 q, qt;
+        float mass_t;
+    };
+    group_tangent<G, 1>(
+        s, mv, false, a.slot, a.xs, lds, base, w, sum,
+        [&](uint32_t j) { return Record{a.xs[j], a.xs_t[j], a.xt[j].w}; },
+        [&](const Record& r, uint32_t, float (&terms)[1]) {
+            const float4 q = r.q;
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
-            rs_t += a.xt[j].w * cubic_value(dist, s.kc) +
-                    q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pst, xyz(a.xs_t[j])));
+            terms[0] = r.mass_t * cubic_value(dist, s.kc) +
+                       q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pst, xyz(r.qt)));
         },
-        [&](uint32_t b) {
+        [&](uint32_t b, float (&terms)[1]) {
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
-            rs_t += q.w * (rest_t_i * cubic_value(dist, s.kc) +
-                           rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pst));
+            terms[0] = q.w * (rest_t_i * cubic_value(dist, s.kc) +
+                              rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pst));
         });
+    if (!writes) return;
+    const float rs_t = sum[0];
     const float m = self.w;
     const float m_t = a.xt[i].w;
     const float rho = s.rho[i];
@@ -470,12 +610,10 @@ struct PressureVjpArgs {
 
 // pressure_vjp_kernel (common.cu:239-294) + projection_update_vjp_kernel
 // (dfsph.cu:123-139), or + non_pressure_vjp_kernel (common.cu:98-163).
-template <bool kUpdate, bool kNonPressure>
-__global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpArgs a) {
+template <bool kUpdate, bool kNonPressure, int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_pressure_kernel(PressureVjpArgs a) {
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const float h = s.kc.h;
     const float4 self = s.xm[i];
     const Float3 x = xyz(self);
@@ -496,12 +634,16 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpA
     double visc_c = 0.0;
     double rest_c = 0.0;
     const float rest_i = s.rest[i];
-    int cx, cy, cz;
-    particle_cell(s.grid, x, cx, cy, cz);
-    walk(s, exact_view(s), exact_masked(s, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-                     [&](uint32_t j) {
-                         if (j == i) return;
-                         const float4 q = s.xm[j];
+    struct Record {
+        float4 q;
+        float p, rho;
+        D3 ap_a;
+    };
+    group_visit<G>(s, exact_view(s), true, 0u, s.xm, lds, base, w,
+                     [&](uint32_t j) { return Record{s.xm[j], a.p[j], s.rho[j], load(a.ap_a, j)}; },
+                     [&](const Record& r, uint32_t j) {
+                         if (j == w) return;
+                         const float4 q = r.q;
                          const Float3 d = sub(x, xyz(q));
                          const float mass = q.w;
                          if constexpr (kNonPressure) {
@@ -509,10 +651,10 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpA
                              const Float3 diff = sub(xyz(vq), vel);
                              const float lap = viscosity_laplacian_c(d, s.kc);
                              const float nu = 0.5F * (vm.w + vq.w);
-                             const float dens = s.rho[j];
-                             const float w = nu * mass * lap / dens;
+                             const float dens = r.rho;
+                             const float weight = nu * mass * lap / dens;
                              const double w_a = dot(lnp, d3(diff));
-                             velocity = add(velocity, scale(lnp, static_cast<double>(-w)));
+                             velocity = add(velocity, scale(lnp, static_cast<double>(-weight)));
                              const double nu_a = w_a * mass * lap / dens;
                              visc_c += 0.5 * nu_a;
                              position = add(position, viscosity_laplacian_gradient(d, h, s.pi_h6, w_a * nu * mass / dens));
@@ -527,16 +669,17 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpA
                                             viscosity_laplacian_gradient(d, h, s.pi_h6, cross_w_a * nu * m_i / rho_i));
                          }
                          const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), s.kc)));
-                         const double second = static_cast<double>(a.p[j]) / (s.rho[j] * s.rho[j]);
+                         const double second = static_cast<double>(r.p) / (r.rho * r.rho);
                          const double sum = first + second;
                          const double local_factor = -mass * sum;
                          first_a -= mass * dot(local, gradient);
-                         position = add(position, cubic_hessian_product(d, scale(local, local_factor), h));
-                         const D3 cross = load(a.ap_a, j);
+                         const D3 cross = r.ap_a;
                          const double projection = dot(cross, gradient);
                          mass_c += sum * projection;
                          first_a += m_i * projection;
-                         position = add(position, cubic_hessian_product(d, scale(cross, m_i * sum), h));
+                         // the Hessian is linear: one product for the centre's and the neighbour's terms
+                         position = add(position, cubic_hessian_product(
+                                                      d, add(scale(local, local_factor), scale(cross, m_i * sum)), h));
                      },
                      [&](uint32_t b) {
                          const float4 q = s.boundary.x[b];
@@ -546,9 +689,9 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpA
                              // non_pressure_vjp_kernel's boundary half
                              const Float3 diff = sub(xyz(s.boundary.v[b]), vel);
                              const float lap = viscosity_laplacian_c(d, s.kc);
-                             const float w = vm.w * vol * lap;
+                             const float weight = vm.w * vol * lap;
                              const double w_a = dot(lnp, d3(diff));
-                             velocity = add(velocity, scale(lnp, static_cast<double>(-w)));
+                             velocity = add(velocity, scale(lnp, static_cast<double>(-weight)));
                              visc_c += w_a * vol * lap;
                              position = add(position, viscosity_laplacian_gradient(d, h, s.pi_h6, w_a * vm.w * vol));
                          }
@@ -560,6 +703,16 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_pressure_kernel(PressureVjpA
                          first_a -= factor_a * rest_i * vol;
                          position = add(position, cubic_hessian_product(d, scale(local, factor), h));
                      });
+    position = group_sum<G>(position);
+    first_a = group_total<G>(first_a);
+    mass_c = group_total<G>(mass_c);
+    if constexpr (kNonPressure) {
+        velocity = group_sum<G>(velocity);
+        dens_c = group_total<G>(dens_c);
+        visc_c = group_total<G>(visc_c);
+    }
+    rest_c = group_total<G>(rest_c);
+    if (!writes) return;
     if (s.boundary.offsets != nullptr) a.rest_a[i] += rest_c;
     accumulate(a.pos_a, i, position);
     double m_a = a.m_a[i] + mass_c;
@@ -620,30 +773,30 @@ struct DensityVjpArgs {
 // x) + predict_vjp_kernel of the prediction that produced them; in the
 // density phase the prediction read a_div + a_p, and its adjoint goes to
 // both (add_adjoint_kernel, common.cu:376-388).
-template <bool kDensityPhase>
-__global__ void __launch_bounds__(kBlock) dfsph_vjp_density_kernel(DensityVjpArgs a) {
+template <bool kDensityPhase, int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_density_kernel(DensityVjpArgs a) {
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const float4 self = a.xs[i];
     const Float3 ps = xyz(self);
     const double out_a = a.rs_a[i];
     const float m_i = self.w;
-    int cx, cy, cz;
-    particle_cell(s.grid, xyz(s.xm[i]), cx, cy, cz);
     D3 position{0.0, 0.0, 0.0};
     double mass_c = 0.0;
     double rest_c = 0.0;
     const float rest_i = s.rest[i];
     const MaskView mv = skin_view(s);
-    walk(
-        s, mv, masks_apply(mv, a.slot, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-        [&](uint32_t j) {
-            const float4 q = a.xs[j];
+    struct Record {
+        float4 q;
+        double rs_a;
+    };
+    group_visit<G>(
+        s, mv, false, a.slot, a.xs, lds, base, w, [&](uint32_t j) { return Record{a.xs[j], a.rs_a[j]}; },
+        [&](const Record& r, uint32_t) {
+            const float4 q = r.q;
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
-            const double rs_a_j = a.rs_a[j];
+            const double rs_a_j = r.rs_a;
             position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
                                            out_a * q.w + rs_a_j * m_i));
             mass_c += rs_a_j * cubic_value(dist, s.kc);
@@ -655,6 +808,10 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_density_kernel(DensityVjpArg
             position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))), out_a * rest_i * q.w));
             rest_c += out_a * q.w * cubic_value(dist, s.kc);
         });
+    position = group_sum<G>(position);
+    mass_c = group_total<G>(mass_c);
+    rest_c = group_total<G>(rest_c);
+    if (!writes) return;
     a.m_a[i] += mass_c;
     if (s.boundary.offsets != nullptr) a.rest_a[i] += rest_c;
     D3 pos, velocity;
@@ -681,28 +838,29 @@ struct ScatterVjpArgs {
 // density_vjp_kernel of the state densities (sph.ixx:364, topology =
 // positions = x), then every sorted adjoint accumulated into the caller's
 // original-order arrays.
-__global__ void __launch_bounds__(kBlock) dfsph_vjp_scatter_kernel(ScatterVjpArgs a) {
+template <int G>
+__global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_scatter_kernel(ScatterVjpArgs a) {
     const Step& s = a.s;
-    PHX_MASK_LDS(s.grid);
-    const uint32_t i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= s.n) return;
+    PHX_DERIVATIVE_GROUP(s.n);
     const float4 self = s.xm[i];
     const Float3 x = xyz(self);
     const double out_a = a.rho_a[i];
     const float m_i = self.w;
-    int cx, cy, cz;
-    particle_cell(s.grid, x, cx, cy, cz);
     D3 position{0.0, 0.0, 0.0};
     double mass_c = 0.0;
     double rest_c = 0.0;
     const float rest_i = s.rest[i];
-    walk(
-        s, exact_view(s), exact_masked(s, i), i, cx, cy, cz, delta, smask + threadIdx.x,
-        [&](uint32_t j) {
-            const float4 q = s.xm[j];
+    struct Record {
+        float4 q;
+        double rho_a;
+    };
+    group_visit<G>(
+        s, exact_view(s), true, 0u, s.xm, lds, base, w, [&](uint32_t j) { return Record{s.xm[j], a.rho_a[j]}; },
+        [&](const Record& r, uint32_t) {
+            const float4 q = r.q;
             const Float3 d = sub(x, xyz(q));
             const float dist = length(d);
-            const double rho_a_j = a.rho_a[j];
+            const double rho_a_j = r.rho_a;
             position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
                                            out_a * q.w + rho_a_j * m_i));
             mass_c += rho_a_j * cubic_value(dist, s.kc);
@@ -714,6 +872,10 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_scatter_kernel(ScatterVjpArg
             position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))), out_a * rest_i * q.w));
             rest_c += out_a * q.w * cubic_value(dist, s.kc);
         });
+    position = group_sum<G>(position);
+    mass_c = group_total<G>(mass_c);
+    rest_c = group_total<G>(rest_c);
+    if (!writes) return;
     const uint32_t j = a.perm[i];
     const D3 pos = add(load(a.pos_a, i), position);
     if (a.out_pos.x != nullptr) accumulate(a.out_pos, j, pos);
@@ -725,8 +887,6 @@ __global__ void __launch_bounds__(kBlock) dfsph_vjp_scatter_kernel(ScatterVjpArg
     accumulate_to(a.out_relax_div, j, a.relax_div_a[i]);
     accumulate_to(a.out_relax_den, j, a.relax_den_a[i]);
 }
-
-uint32_t derivative_blocks(uint32_t n) { return (blocks_for(n, kBlock) + 7u) / 8u * 8u; }
 
 }  // namespace
 
@@ -779,9 +939,10 @@ Step make_step(const Domain& domain, const DfsphCache& cache, const KernelConsta
 }
 
 template <bool kNonPressure, int kEpilogue>
-void launch_force_jvp(hipStream_t stream, uint32_t blocks, const ForceJvpArgs& args) {
-    dfsph_jvp_force_kernel<kNonPressure, kEpilogue><<<blocks, kBlock, 0, stream>>>(args);
-    PHX_LAUNCH_CHECK();
+void launch_force_jvp(hipStream_t stream, const ForceJvpArgs& args) {
+    with_derivative_group(args.s.n, [&](auto g, uint32_t blocks) {
+        dfsph_jvp_force_kernel<kNonPressure, kEpilogue, g()><<<blocks, kGroupBlock, 0, stream>>>(args);
+    });
 }
 
 }  // namespace
@@ -803,7 +964,6 @@ void DfsphSolver::jvp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ta
     const uint32_t ne = cache.iterations[1];
     const bool warm = cache.warm_start;
     const uint32_t* perm = cache.neighborhood.perm.data();
-    const uint32_t blocks = derivative_blocks(n);
     const Step s = make_step(domain_, cache, constants_, gradient_norm_, config_.exact_no_slip_adjoint != 0u);
 
     GatherTangentArgs ga{};
@@ -842,8 +1002,9 @@ void DfsphSolver::jvp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ta
                       dw_.t_div.data(),
                       dw_.t_den.data(),
                       dw_.rest_t.data()};
-    dfsph_jvp_density_kernel<<<blocks, kBlock, 0, stream_>>>(da);
-    PHX_LAUNCH_CHECK();
+    with_derivative_group(n, [&](auto g, uint32_t blocks) {
+        dfsph_jvp_density_kernel<g()><<<blocks, kGroupBlock, 0, stream_>>>(da);
+    });
 
     ForceJvpArgs fa{};
     fa.s = s;
@@ -879,10 +1040,10 @@ void DfsphSolver::jvp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ta
     fa.collisions = collisions(slot);
     if (nd == 0u) {
         fa.final_step = ne == 0u ? 1u : 0u;
-        launch_force_jvp<true, kJvpDivEnd>(stream_, blocks, fa);
+        launch_force_jvp<true, kJvpDivEnd>(stream_, fa);
     } else {
         fa.final_step = 0u;
-        launch_force_jvp<true, kJvpDivPredict>(stream_, blocks, fa);
+        launch_force_jvp<true, kJvpDivPredict>(stream_, fa);
         pa.target = cache.densities.data();
         pa.target_t = dw_.rho_t.data();
         pa.relax = cache.relax_div.data();
@@ -895,14 +1056,15 @@ void DfsphSolver::jvp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ta
             pa.rs = cache.rs.data() + slot * nn;
             pa.p_prev = cache.pressures(0u, it - 1u);
             pa.p = cache.pressures(0u, it);
-            dfsph_jvp_projection_kernel<<<blocks, kBlock, 0, stream_>>>(pa);
-            PHX_LAUNCH_CHECK();
+            with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                dfsph_jvp_projection_kernel<g()><<<blocks, kGroupBlock, 0, stream_>>>(pa);
+            });
             fa.collisions = collisions(++slot);
             if (it < nd) {
-                launch_force_jvp<false, kJvpDivPredict>(stream_, blocks, fa);
+                launch_force_jvp<false, kJvpDivPredict>(stream_, fa);
             } else {
                 fa.final_step = ne == 0u ? 1u : 0u;
-                launch_force_jvp<false, kJvpDivEnd>(stream_, blocks, fa);
+                launch_force_jvp<false, kJvpDivEnd>(stream_, fa);
             }
         }
     }
@@ -921,11 +1083,12 @@ void DfsphSolver::jvp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ta
         pa.rs = cache.rs.data() + slot * nn;
         pa.p_prev = cache.pressures(1u, it - 1u);
         pa.p = cache.pressures(1u, it);
-        dfsph_jvp_projection_kernel<<<blocks, kBlock, 0, stream_>>>(pa);
-        PHX_LAUNCH_CHECK();
+        with_derivative_group(n, [&](auto g, uint32_t blocks) {
+            dfsph_jvp_projection_kernel<g()><<<blocks, kGroupBlock, 0, stream_>>>(pa);
+        });
         fa.collisions = collisions(++slot);
         fa.final_step = it == ne ? 1u : 0u;
-        launch_force_jvp<false, kJvpDenPredict>(stream_, blocks, fa);
+        launch_force_jvp<false, kJvpDenPredict>(stream_, fa);
     }
 }
 
@@ -951,7 +1114,6 @@ void DfsphSolver::vjp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ad
     const uint32_t ne = cache.iterations[1];
     const bool warm = cache.warm_start;
     const uint32_t* perm = cache.neighborhood.perm.data();
-    const uint32_t blocks = derivative_blocks(n);
     const Step s = make_step(domain_, cache, constants_, gradient_norm_, config_.exact_no_slip_adjoint != 0u);
     const size_t nn = n;
     auto collisions = [&](uint32_t k) { return cache.collisions.data() + k * nn; };
@@ -1034,16 +1196,21 @@ void DfsphSolver::vjp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ad
             pv.p_prev = cache.pressures(phase, it - 1u);
             pv.rs = cache.rs.data() + slot * nn;
             pv.p_prev_a = dw_.p_a[pp].data();
-            dfsph_vjp_pressure_kernel<true, false><<<blocks, kBlock, 0, stream_>>>(pv);
-            PHX_LAUNCH_CHECK();
+            with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                dfsph_vjp_pressure_kernel<true, false, g()><<<blocks, kGroupBlock, 0, stream_>>>(pv);
+            });
             dv.slot = slot;
             dv.xs = cache.xs.data() + slot * nn;
             dv.collisions = collisions(slot);
             dv.prev_ap = dw_.ap_a[pa].view();
             if (density_phase) {
-                dfsph_vjp_density_kernel<true><<<blocks, kBlock, 0, stream_>>>(dv);
+                with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                    dfsph_vjp_density_kernel<true, g()><<<blocks, kGroupBlock, 0, stream_>>>(dv);
+                });
             } else {
-                dfsph_vjp_density_kernel<false><<<blocks, kBlock, 0, stream_>>>(dv);
+                with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                    dfsph_vjp_density_kernel<false, g()><<<blocks, kGroupBlock, 0, stream_>>>(dv);
+                });
             }
             PHX_LAUNCH_CHECK();
             ca = pa;
@@ -1058,9 +1225,13 @@ void DfsphSolver::vjp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ad
                             : (density_phase ? previous_a.method.warm_density_pressure
                                              : previous_a.method.warm_divergence_pressure);
         if (density_phase) {
-            dfsph_vjp_pressure_kernel<false, false><<<blocks, kBlock, 0, stream_>>>(pv);
+            with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                dfsph_vjp_pressure_kernel<false, false, g()><<<blocks, kGroupBlock, 0, stream_>>>(pv);
+            });
         } else {
-            dfsph_vjp_pressure_kernel<false, true><<<blocks, kBlock, 0, stream_>>>(pv);
+            with_derivative_group(n, [&](auto g, uint32_t blocks) {
+                dfsph_vjp_pressure_kernel<false, true, g()><<<blocks, kGroupBlock, 0, stream_>>>(pv);
+            });
         }
         PHX_LAUNCH_CHECK();
         pv.warm_out = nullptr;
@@ -1088,8 +1259,9 @@ void DfsphSolver::vjp_step(const DfsphCache& cache, const phx_sph_dfsph_state_ad
     sa.out_visc = parameter_a.particles.viscosities;
     sa.out_relax_div = parameter_a.method.divergence_relaxation;
     sa.out_relax_den = parameter_a.method.density_relaxation;
-    dfsph_vjp_scatter_kernel<<<blocks, kBlock, 0, stream_>>>(sa);
-    PHX_LAUNCH_CHECK();
+    with_derivative_group(n, [&](auto g, uint32_t blocks) {
+        dfsph_vjp_scatter_kernel<g()><<<blocks, kGroupBlock, 0, stream_>>>(sa);
+    });
 }
 
 }  // namespace phx

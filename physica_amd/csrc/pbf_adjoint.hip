@@ -500,20 +500,6 @@ struct CorrectionVjpArgs {
     double2* lambda_terms;  // (density adjoint, D_bar) per particle (written)
 };
 
-// 1 / sqrt(x) for a positive normal x: the hardware estimate refined by two
-// Newton steps, y <- y + y (1 - x y^2) / 2, to within a few units of the
-// last place (the derivative passes compare with the FP64 oracle to 1e-10;
-// the square root and the division they replace cost about 30 instructions).
-__device__ __forceinline__ double inverse_sqrt(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int step = 0; step < 2; ++step) {
-        const double e = fma(-x * y, y, 1.0);
-        y = fma(0.5 * y, e, y);
-    }
-    return y;
-}
-
 // Derivative of G(d) = f(r) d (spiky gradient) along w, with 1 / r from
 // inverse_sqrt instead of a square root and a division.
 __device__ __forceinline__ D3 spiky_hessian_one_division(Float3 d, D3 w, double h, double k) {

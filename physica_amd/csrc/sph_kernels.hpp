@@ -198,13 +198,16 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
         if (crowded) crowd[expanded] = 1u;
     }
     // the exact mask of members from .. to - 1 at positions x[s], their skin
-    // mask in `skin`
+    // mask in `skin`; with the margin of exact_mask_threshold, as the FP64
+    // derivatives take the distance of a pair at the very edge of the support
+    // to be inside it where the FP32 passes do not
+    const float t_exact = a.kc.sqrt_support * (1.0F + 4e-6F);
     auto mark = [&](const float4* x, uint32_t from, uint32_t to, float t_skin, uint32_t& skin) {
         uint32_t bits[2];
         mark_members<2>(x, from, to, bits, [&](Float3 q, bool (&marked)[2]) {
             const Float3 d = sub(p, q);
             const float d2 = dot(d, d);
-            marked[0] = d2 < a.kc.sqrt_support;
+            marked[0] = d2 < t_exact;
             marked[1] = d2 < t_skin;
         });
         skin = bits[1];

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import oracle
+import test_gpu_dfsph_derivatives as dfsph
 from physica_amd import scenes
 from physica_amd.particle import PBF, ExecutionMode
 from physica_amd.rollout import PbfRollout
@@ -13,6 +14,7 @@ from helpers import bits_equal, pbf_setup
 
 pytestmark = pytest.mark.gpu
 
+DFSPH_LIMIT = 40000  # 16 lanes a particle up to here
 PBF_FIELDS = ("relaxation", "xsph_viscosity", "vorticity_confinement")
 
 
@@ -94,3 +96,43 @@ def test_rollout_records_over_its_caches(gpu_device):
     rollout.release()
     final, got = run(rollout, other)
     assert all(np.array_equal(got[k], fresh[1][1][k]) for k in got)
+
+
+def dfsph_case(count):
+    """A lattice of `count` particles off the cell borders, swirling, with some
+    moving further within the step than any mask skin."""
+    side = 1
+    while side ** 3 < count:
+        side += 1
+    sc = scenes.dfsph_dam_break(shape=(side, side, side), box=(0.8, 0.8, 0.8))
+    rng = np.random.default_rng(count)
+    h = sc.domain.support_radius
+    jitter = rng.uniform(-0.1, 0.1, (3, count)) * h
+    sc.positions = (0.95 * sc.positions[:, :count] + 0.1 + jitter).astype(np.float32)
+    velocities = rng.normal(0.0, 0.05, (3, count))
+    velocities[:, ::7] += 0.3 * h / sc.domain.time_step * rng.uniform(-1.0, 1.0, (3, velocities[:, ::7].shape[1]))
+    sc.velocities = velocities.astype(np.float32)
+    sc.parameters = {k: np.ascontiguousarray(v[:count]) for k, v in sc.parameters.items()}
+    sc.parameters["masses"] = (sc.parameters["masses"] * rng.uniform(0.95, 1.05, count)).astype(np.float32)
+    sc.parameters["viscosities"][:] = 0.01
+    sc.domain.particle_count = count
+    zeros = np.zeros(count, np.float32)
+    return dfsph.Case(sc, oracle.make_domain(sc.domain), (zeros, zeros))
+
+
+@pytest.mark.parametrize("count", [1, 15, 17, 63, 65, 257, 1000, DFSPH_LIMIT, DFSPH_LIMIT + 1])
+def test_dfsph_derivatives(gpu_device, count):
+    cs = dfsph_case(count)
+    run = dfsph.recorded(cs, gpu_device, 1, 2, True)
+    t, w = dfsph.directions(cs, np.random.default_rng(4))
+    x, v, u, p, wd, we = dfsph.inputs(cs, "f32")
+    got = dfsph.run_vjp(*run, w, gpu_device)
+    exp = oracle.dfsph_vjp(cs.d, 0, x, v, u, p, wd, we, w, 1, 2, True, "f32")
+    for k in dfsph.STATE + dfsph.PARAMS + dfsph.WARM:
+        # as for PBF: FP64 sums in another order
+        assert np.abs(got[k] - exp[k]).max() <= 1e-10 * max(np.abs(exp[k]).max(), 1e-300), k
+    got = dfsph.run_jvp(*run, t, gpu_device)
+    exp = oracle.dfsph_jvp(cs.d, 0, x, v, u, p, wd, we, t, 1, 2, True, "f32")
+    for k in ("positions", "velocities") + dfsph.WARM:
+        # the oracle's FP32 operations in its order; the platforms' functions differ by units of the last place
+        assert np.abs(got[k] - exp[k]).max() <= 1e-6 * max(np.abs(exp[k]).max(), 1e-30), k
