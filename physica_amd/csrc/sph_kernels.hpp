@@ -37,8 +37,9 @@ constexpr int kWalkDepth = 2;
 // candidates, idle lanes in a particle's last trip) to one that does. DFSPH
 // steps of 4 + 6 iterations, us, with 1 / 4 / 16 lanes: 2,000 particles
 // 419 / 278 / 194, 16,000 476 / 303 / 270, 32,000 432 / 297 / 346, 64,000
-// 458 / 379 / 501, 130,000 529 / 613 / 829, 1,048,576 3,071 / 3,309 / 5,780;
-// IISPH and PCISPH cross at the same counts.
+// 458 / 370 / 501, 130,000 505 / 558 / 829, 260,000 710 / 897 / -; IISPH and
+// PCISPH cross at the same counts. From 400,000 four lanes are 6 % faster on
+// cubic lattices and 6 to 20 % slower on a dam break of 128 x 64 x 128.
 constexpr uint32_t kGroup16Particles = 20000;
 constexpr uint32_t kGroup4Particles = 90000;
 
