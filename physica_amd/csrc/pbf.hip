@@ -36,10 +36,11 @@ __device__ __forceinline__ Float3 xyz(float4 q) { return Float3{q.x, q.y, q.z}; 
 constexpr uint32_t kBlock = 256;
 // Particle counts up to which 16 lanes share a particle; above, 4. One lane
 // per particle, over skin masks built once a step, is slower at every size.
-// Steps, us, with 1 / 4 / 16 lanes: 1,300 particles 532 / 169 / 106, 16,000
-// 514 / 174 / 136, 32,000 524 / 179 / 181 (30 clumps 1,799 / 613 / 524),
-// 64,000 517 / 239 / 289, 260,000 809 / 663 / 903, 1,048,576 4,080 / 2,313 /
-// 3,424.
+// Steps, us, with 1 / 4 / 16 lanes before the candidates were records: 1,300
+// particles 532 / 169 / 106, 16,000 514 / 174 / 136, 32,000 524 / 179 / 181
+// (30 clumps 1,799 / 613 / 524), 64,000 517 / 239 / 289, 1,048,576 4,080 /
+// 2,313 / 3,424; with records, 4 / 16 lanes: 32,000 165 / 168, 64,000 196 /
+// 254, 1,048,576 1,590 / 2,865.
 constexpr uint32_t kGroup16Particles = 32768;
 
 // Workgroups with crowded particles that a pass starts before all others.
@@ -821,6 +822,8 @@ PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_confi
     exact_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
     cells_.resize(n);
+    if (n >= kEarlyParticles)
+        schedule_.resize(1u + kEarlyBlocks + 2u * static_cast<size_t>(pbf_blocks(n, pbf_group(n))));
 }
 
 void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& control,
@@ -885,7 +888,6 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     const uint32_t group_blocks = pbf_blocks(n, group);
     Schedule schedule{};
     if (ordered) {
-        schedule_.resize(1u + kEarlyBlocks + 2u * static_cast<size_t>(group_blocks));
         schedule = Schedule{schedule_.data(), schedule_.data() + 1u, schedule_.data() + 1u + kEarlyBlocks,
                             schedule_.data() + 1u + kEarlyBlocks + group_blocks, kEarlyBlocks};
     }
