@@ -1254,8 +1254,8 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
         current = target;
     }
     if (iterations == 0u) {
-        pbf_reconstruct_kernel<<<blocks_for(n, kBlock), kBlock, 0, s>>>(n, current, x0_.cview(), 1.0F / dt_,
-                                                                      vel_.data(), Vec{});
+        pbf_reconstruct_kernel<<<pbf_blocks(n, 1), kBlock, 0, s>>>(n, current, x0_.cview(), 1.0F / dt_, vel_.data(),
+                                                                   Vec{});
         PHX_LAUNCH_CHECK();
         ++kernels_per_step_;
     }

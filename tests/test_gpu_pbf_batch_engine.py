@@ -28,12 +28,12 @@ def small_batch(count=5, moving=False):
     return batch
 
 
-def lone_states(batch, steps, device):
+def lone_states(batch, steps, device, iterations=ITERATIONS):
     """Each scene on its own PBF solver for `steps` steps."""
     out = []
     for sc in batch:
         solver, state, nxt, control, params, cache = pbf_setup(
-            sc, device, PBF.Configuration(pressure_iterations=ITERATIONS), ExecutionMode.forward)
+            sc, device, PBF.Configuration(pressure_iterations=iterations), ExecutionMode.forward)
         states = [state, nxt]
         for k in range(steps):
             solver.forward_step(states[k % 2], control, params, states[(k + 1) % 2], cache)
@@ -43,8 +43,8 @@ def lone_states(batch, steps, device):
     return out
 
 
-def batch_engine(batch, device, use_graph):
-    engine = PbfBatch([sc.domain for sc in batch], PBF.Configuration(pressure_iterations=ITERATIONS),
+def batch_engine(batch, device, use_graph, iterations=ITERATIONS):
+    engine = PbfBatch([sc.domain for sc in batch], PBF.Configuration(pressure_iterations=iterations),
                       use_graph=use_graph, device=device)
     state, control, params = engine.allocate_state(), engine.allocate_control(), engine.allocate_parameters()
     engine.upload(batch, state, params)
@@ -115,3 +115,22 @@ def test_batch_refuses_mixed_support_radii(gpu_device):
     batch[1].domain.support_radius = 0.05
     with pytest.raises(RuntimeError, match="support radius"):
         PbfBatch([sc.domain for sc in batch], PBF.Configuration(pressure_iterations=ITERATIONS), device=gpu_device)
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+@pytest.mark.parametrize("shapes", [((8, 8, 8), (9, 9, 9)), ((16, 16, 16), (10, 10, 10)), ((16, 16, 16),)])
+def test_batch_without_pressure_iterations(gpu_device, shapes, use_graph):
+    """0 iterations: the velocities come from the batch's reconstruction pass.
+    Its blocks of 256 particles number 5, 20 and 16: fewer than the XCDs, not a
+    multiple of them, and a multiple."""
+    batch = [scenes.pbf_dam_break(shape=shape, seed=k) for k, shape in enumerate(shapes)]
+    for k, sc in enumerate(batch):
+        sc.velocities = np.random.default_rng(k).normal(0.0, 0.5, sc.positions.shape).astype(np.float32)
+        sc.parameters["xsph_viscosity"][:] = 0.01
+        sc.parameters["vorticity_confinement"][:] = 0.5
+    engine, state, control, params = batch_engine(batch, gpu_device, use_graph, iterations=0)
+    engine.run(state, control, params, 2)
+    torch.cuda.synchronize()
+    for (x, v), (lx, lv) in zip(split(engine, state), lone_states(batch, 2, gpu_device, iterations=0)):
+        assert bits_equal(x, lx)
+        assert bits_equal(v, lv)
