@@ -79,9 +79,11 @@ __device__ __forceinline__ D3 cubic_hessian_product(Float3 d, D3 w, float h) {
     const double coef = 8.0 / (static_cast<double>(kPi) * h * h * h);
     const double d2 = static_cast<double>(dot(d, d));
     if (d2 == 0.0) return scale(w, -12.0 * coef * inv_h2);
+    // |d| >= h, from the square: inverse_sqrt takes no infinity, which a
+    // distance of 2^64 reaches (the product of two floats is exact here)
+    if (d2 >= static_cast<double>(h) * h) return {0.0, 0.0, 0.0};
     const double inv_dist = inverse_sqrt(d2);
     const double dist = d2 * inv_dist;
-    if (dist >= h) return {0.0, 0.0, 0.0};
     const double q = dist * inv_h;
     const double deriv = q <= 0.5 ? 18.0 * q * q - 12.0 * q : -6.0 * (1.0 - q) * (1.0 - q);
     const double second = q <= 0.5 ? 36.0 * q - 12.0 : 12.0 * (1.0 - q);

@@ -187,3 +187,24 @@ def test_forward_mode_refuses_derivatives():
                       solver.allocate_parameter_tangent(), solver.allocate_state_tangent())
     with pytest.raises(RuntimeError, match="differentiable mode"):
         solver.jvp_step(state, control, params, nxt, cache, st, ct, pt, nt)
+
+
+def test_vjp_with_a_particle_at_an_infinite_squared_distance():
+    """Grid cells at the box's faces hold particles at any distance beyond
+    them, and with boundary samples every candidate of the 27 cells is walked:
+    a pair whose squared distance overflows FP32 is outside the support."""
+    dev = torch.device("cuda:0")
+    cs = scene(unit_exponent=True, boundary=True)
+    sc = cs.sc
+    # the particle nearest the x = 0 face; its cell stays among its neighbours'
+    far = int(np.argmin(sc.positions[0]))
+    sc.positions[0] -= np.float32(sc.positions[0].min() - 0.1 * sc.domain.support_radius)
+    sc.positions[0, far] = np.float32(-1.0e20)
+    run = recorded(cs, dev, exact=True)
+    _, w = directions(cs, np.random.default_rng(31))
+    jw = run_vjp(*run, w)
+    x, v, u, p = inputs(cs, "f32")
+    rw = oracle.wcsph_vjp(cs.d, 0, x, v, u, p, w, "f32")
+    for k in STATE + PARAMS:
+        assert np.isfinite(rw[k]).all(), k
+        assert close(jw[k], rw[k], 1e-10), k
