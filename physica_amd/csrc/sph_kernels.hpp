@@ -201,15 +201,18 @@ __global__ void __launch_bounds__(kGroupBlock) mask_density_kernel(MaskDensityAr
     // the exact mask of members from .. to - 1 at positions x[s], their skin
     // mask in `skin`; with the margin of exact_mask_threshold, as the FP64
     // derivatives take the distance of a pair at the very edge of the support
-    // to be inside it where the FP32 passes do not
+    // to be inside it where the FP32 passes do not. With samples a distance
+    // that is NaN is kept, as its terms are (a particle at a NaN position and
+    // its neighbours have NaN sums); without, such a particle has no neighbours.
     const float t_exact = a.kc.sqrt_support * (1.0F + 4e-6F);
+    auto within = [](float d2, float bound) { return kSamples ? !(d2 >= bound) : d2 < bound; };
     auto mark = [&](const float4* x, uint32_t from, uint32_t to, float t_skin, uint32_t& skin) {
         uint32_t bits[2];
         mark_members<2>(x, from, to, bits, [&](Float3 q, bool (&marked)[2]) {
             const Float3 d = sub(p, q);
             const float d2 = dot(d, d);
-            marked[0] = d2 < t_exact;
-            marked[1] = d2 < t_skin;
+            marked[0] = within(d2, t_exact);
+            marked[1] = within(d2, t_skin);
         });
         skin = bits[1];
         return bits[0];

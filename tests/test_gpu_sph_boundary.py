@@ -10,8 +10,8 @@ import torch
 
 import oracle
 from physica_amd import scenes
-from physica_amd.particle import ExecutionMode, PCISPH, SPH, WCSPH
-from helpers import add_boundary_samples, bits_equal, sph_setup
+from physica_amd.particle import DFSPH, ExecutionMode, PCISPH, SPH, WCSPH
+from helpers import add_boundary_samples, bits_equal, dfsph_setup, sph_setup
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +73,39 @@ def test_differentiable_mode_accepts_boundary_particles(gpu_device):
     add_boundary_samples(sc)
     SPH(sc.domain, WCSPH.Configuration(), mode=ExecutionMode.differentiable, device=gpu_device)
     SPH(sc.domain, PCISPH.Configuration(), mode=ExecutionMode.differentiable, device=gpu_device)
+
+
+@pytest.mark.parametrize("method", ["dfsph", "pcisph", "iisph", "wcsph"])
+def test_a_nan_position_reaches_its_cell_with_samples(gpu_device, method):
+    """A distance that is NaN is not outside the support: the particle (its
+    cell is the grid's first) and every candidate of its 27 cells have NaN
+    densities. Later sums differ from the reference's, which adds zero times
+    the NaN of candidates that are outside the support; the masks leave those out."""
+    if method == "dfsph":
+        sc = scenes.dfsph_dam_break(shape=(16, 10, 12), seed=5)
+    else:
+        sc = scene_for(method)
+    for axis in range(3):
+        sc.positions[axis] -= np.float32(sc.positions[axis].min() - sc.domain.particle_radius)
+    samples = add_boundary_samples(sc)
+    sc.positions[1, sc.count // 4] = np.nan
+    x, v, u = sc.positions, sc.velocities, np.zeros_like(sc.positions)
+    d = oracle.make_domain(sc.domain, samples)
+    if method == "dfsph":
+        zero = np.zeros(sc.count, np.float32)
+        solver, state, nxt, control, params, cache = dfsph_setup(sc, gpu_device, DFSPH.Configuration(2, 3))
+        exp = oracle.dfsph_step(d, 0, x, v, u, sc.parameters, zero, zero, 2, 3)
+    else:
+        solver, state, nxt, control, params, cache = sph_setup(sc, gpu_device, method, 3)
+        if method == "wcsph":
+            exp = oracle.wcsph_step(d, 0, x, v, u, sc.parameters)
+        else:
+            exp = oracle.pressure_solver_step(d, 0, x, v, u, sc.parameters, method, 3)
+    solver.forward_step(state, control, params, nxt, cache)
+    torch.cuda.synchronize()
+    assert np.isnan(exp["densities"]).sum() > 1
+    assert np.array_equal(cache.densities().cpu().numpy(), exp["densities"], equal_nan=True)
+    # they reach everyone with a NaN density, and nobody whom the reference spares
+    broken = np.isnan(nxt.particles.velocities.numpy()).any(axis=0)
+    assert broken[np.isnan(exp["densities"])].all()
+    assert not (broken & ~np.isnan(exp["velocities"]).any(axis=0)).any()
