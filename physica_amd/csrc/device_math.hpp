@@ -120,6 +120,25 @@ __host__ __device__ inline float div_rn(float x, float b, float inv_b) {
     return fmaf(r1, inv_b, q1);
 }
 
+// A particle's rest density as the divisor of its candidates' masses. With
+// masses and rest densities in [2^-60, 2^60], whose quotients and remainders
+// stay normal, the reciprocal is taken once (div_rn); otherwise, zeros and
+// infinities included, each pair's quotient is the compiler's. The masses are
+// checked as a step gathers them (Channels::flag), so that the choice does not
+// change within a walk: a check of each candidate's mass made a PBF step of
+// 32,768 particles 178 us for 168.
+__device__ __forceinline__ bool outside_quick_range(float v) { return !(v >= 0x1p-60F && v <= 0x1p60F); }
+struct RestDensity {
+    float value, inverse;
+    bool plain;
+};
+__device__ __forceinline__ RestDensity rest_density_of(float rest, bool unusual_masses) {
+    return RestDensity{rest, 1.0F / rest, unusual_masses || outside_quick_range(rest)};
+}
+__device__ __forceinline__ float over_rest(float mass, const RestDensity& rest) {
+    return rest.plain ? mass / rest.value : div_rn(mass, rest.value, rest.inverse);
+}
+
 // a / b for operands whose quotient, remainders and reciprocal stay normal:
 // the compiler's own sequence of reciprocal estimate, one Newton step and two
 // quotient refinements, hence its correctly rounded result, without the

@@ -138,6 +138,8 @@ struct Channels {
     float* dst[kMaxChannels];
     uint32_t stride[kMaxChannels];
     uint32_t count;
+    const float* checked;  // optional: masses; a gather that finds one outside the quick range (device_math.hpp) ...
+    uint32_t* flag;        // ... sets this word to 1
 };
 
 class ChannelList {
@@ -166,6 +168,10 @@ class ChannelList {
     void add(const float* src, float4* dst, int component) {
         add(src, reinterpret_cast<float*>(dst) + component, 4u);
     }
+    void check_masses(const float* masses, uint32_t* flag) {
+        list_.checked = masses;
+        list_.flag = flag;
+    }
     const Channels& get() const { return list_; }
 
   private:
@@ -180,6 +186,7 @@ struct PredictInput {
     Float3 gravity{};
     float dt = 0.0F;
     Vec predicted{};
+    uint32_t* mass_flag = nullptr;  // optional: set to 0 (Channels::flag, which a later pass of the build raises)
 };
 
 // A batch of independent scenes stepped together: every scene's particles

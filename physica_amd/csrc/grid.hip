@@ -101,6 +101,7 @@ __global__ void __launch_bounds__(kBlock)
                 add(load(predict.velocities, i), scale(add(predict.gravity, load(predict.controls, i)), predict.dt));
             p = add(p, scale(pv, predict.dt));
             store(predict.predicted, i, p);
+            if (i == 0u && predict.mass_flag != nullptr) *predict.mass_flag = 0u;
         }
         key = cell_key(box, p);
         keys[i] = key;
@@ -118,6 +119,7 @@ __global__ void __launch_bounds__(kBlock)
     const BatchBlock blk = batch.blocks[blockIdx.x];
     const bool valid = threadIdx.x < blk.count;
     const uint32_t i = blk.first + threadIdx.x;
+    if (blockIdx.x == 0u && threadIdx.x == 0u && predict.mass_flag != nullptr) *predict.mass_flag = 0u;
     uint32_t key = ~0u;
     if (valid) {
         const BatchScene sc = batch.scenes[blk.scene];
@@ -253,6 +255,8 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
     for (int c = 0; c < kMaxChannels; ++c)
         if (static_cast<uint32_t>(c) < channels.count) channels.dst[c][s * channels.stride[c]] = v[c];
+    // one value for every writer
+    if (channels.checked != nullptr && outside_quick_range(channels.checked[i])) *channels.flag = 1u;
 }
 
 // ------------------------------------------------------------------- scan

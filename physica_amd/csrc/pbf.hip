@@ -192,21 +192,8 @@ struct LambdaArgs {
     uint32_t* cell;
     uint8_t* crowded;
     uint32_t first_pass;
+    const uint32_t* unusual_masses;  // rest_density_of
 };
-
-// A particle's rest density as the divisor of its candidates' masses: the
-// reciprocal is taken once (div_rn), or, outside [2^-60, 2^60], the quotient
-// of each pair by the compiler's division.
-struct RestDensity {
-    float value, inverse;
-    bool plain;
-};
-__device__ __forceinline__ RestDensity rest_density_of(float rest) {
-    return RestDensity{rest, 1.0F / rest, !(rest >= 0x1p-60F && rest <= 0x1p60F)};
-}
-__device__ __forceinline__ float over_rest(float mass, const RestDensity& rest) {
-    return rest.plain ? mass / rest.value : div_rn(mass, rest.value, rest.inverse);
-}
 
 // The terms of one candidate in the density and lambda sums: the density,
 // the gradient sum and the denominator.
@@ -401,7 +388,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_lambda_kernel(LambdaArgs a, S
     const GroupScene scene = group_scene<kBatch, G>(id, a.n, a.grid, Box{}, batch);
     const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
     const Float3 p = xyz(a.pos[own]);
-    const RestDensity rest = rest_density_of(a.rho0[own]);
+    const RestDensity rest = rest_density_of(a.rho0[own], *a.unusual_masses != 0u);
     float sum[kSums] = {0.0F, 0.0F, 0.0F, 0.0F, a.eps[own]};
     const uint32_t w = group_first_walk<G, kSamples, kSums>(
         a, scene, lds, crowd, a.boundary, ~0u,
@@ -465,6 +452,7 @@ struct CorrectionArgs {
     const uint32_t* cell;   // LambdaArgs::cell and crowded
     const uint8_t* crowded;
     float t_exact;
+    const uint32_t* unusual_masses;
 };
 
 // The artificial pressure of a particle, as its correction pass evaluates it.
@@ -515,7 +503,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_correction_kernel(CorrectionA
     const uint32_t own = threadIdx.x / G < scene.count ? scene.base + threadIdx.x / G : 0u;
     const float4 self = a.pos[own];
     const Float3 p = xyz(self);
-    const RestDensity rest = rest_density_of(a.rho0[own]);
+    const RestDensity rest = rest_density_of(a.rho0[own], *a.unusual_masses != 0u);
     const float lambda_i = a.lambda[own];
     const ArtificialPressure pressure = artificial_of(a, own);
     float sum[kSums] = {0.0F, 0.0F, 0.0F};
@@ -821,6 +809,7 @@ PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_confi
         b->resize(n);
     exact_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
+    mass_flag_.resize(1u);
     cells_.resize(n);
     if (n >= kEarlyParticles)
         schedule_.resize(1u + kEarlyBlocks + 2u * static_cast<size_t>(pbf_blocks(n, pbf_group(n))));
@@ -861,7 +850,9 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     predict.gravity = Float3{c.gravity.x, c.gravity.y, c.gravity.z};
     predict.dt = c.time_step;
     predict.predicted = cache.predicted.view();
+    predict.mass_flag = mass_flag_.data();
     ChannelList gather;
+    gather.check_masses(pp.masses, mass_flag_.data());
     gather.add(cache.predicted.cview(), xs_.data());
     gather.add(pp.masses, xs_.data(), 3);
     if (rec) gather.add(cache.predicted.cview(), cache.xs.view());
@@ -920,6 +911,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
                   xs_.data(),  rho0_.data(), eps_.data(),
                   cache.densities.data(), cache.lambdas.data()};
     la.t_exact = t_exact;
+    la.unusual_masses = mass_flag_.data();
     la.boundary = boundary;
     la.cell = cells_.data();
     la.crowded = crowded;
@@ -941,6 +933,7 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     ca.cell = cells_.data();
     ca.crowded = crowded;
     ca.t_exact = t_exact;
+    ca.unusual_masses = mass_flag_.data();
 
     // positions start at x* (pbf.cpp:171) and ping-pong between two buffers
     // (a recorded step keeps every iterate)
@@ -1140,6 +1133,7 @@ PbfBatch::PbfBatch(const phx_domain_configuration* domains, uint32_t scene_count
         b->resize(n);
     exact_.resize(static_cast<size_t>(kStencil) * n);
     crowded_.resize(n);
+    mass_flag_.resize(1u);
     cell_index_.resize(n);
     // grid build 9, schedule fills 3, cells 1, two per iteration, three post passes
     const uint32_t it = config_.pressure_iterations;
@@ -1185,7 +1179,9 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     predict.controls = cvec(control.external_accelerations);
     predict.dt = dt_;
     predict.predicted = predicted_.view();
+    predict.mass_flag = mass_flag_.data();
     ChannelList gather;
+    gather.check_masses(pp.masses, mass_flag_.data());
     gather.add(predicted_.cview(), xs_.data());
     gather.add(pp.masses, xs_.data(), 3);
     gather.add(x.cview(), x0_.view());
@@ -1218,6 +1214,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     LambdaArgs la{n,           kernel_,     grid, xs_.data(), rho0_.data(),
                   eps_.data(), rho_.data(), lambda_.data()};
     la.t_exact = t_exact;
+    la.unusual_masses = mass_flag_.data();
     la.exact_out = exact_.data();
     la.cell = cell_index_.data();
     la.crowded = crowded_.data();
@@ -1237,6 +1234,7 @@ void PbfBatch::substep(uint32_t from, uint64_t step, const phx_control& control,
     ca.cell = cell_index_.data();
     ca.crowded = crowded_.data();
     ca.t_exact = t_exact;
+    ca.unusual_masses = mass_flag_.data();
     // the exact masks of each set of positions are rebuilt by the pass that
     // first walks them, so one buffer serves every set in forward mode
     const float4* current = xs_.data();

@@ -138,6 +138,7 @@ class PbfSolver {
     DeviceBuffer<uint16_t> exact_;  // exact masks of the current set of positions (forward mode)
     DeviceBuffer<uint8_t> crowded_;  // per particle: walks the full stencil (forward mode)
     DeviceBuffer<uint32_t> cells_;   // per particle: its grid cell
+    DeviceBuffer<uint32_t> mass_flag_;  // whether the step's masses leave the quick range (rest_density_of)
     DeviceBuffer<uint32_t> schedule_;  // the order of the passes' workgroups (a large scene)
     PbfDerivativeWorkspace dw_;
 };
@@ -195,6 +196,7 @@ class PbfBatch {
     DeviceBuffer<uint8_t> crowded_;
     DeviceBuffer<uint32_t> schedule_, schedule_place_, schedule_seen_;  // the order of the passes' workgroups
     DeviceBuffer<uint32_t> cell_index_;  // per particle: its cell in its scene's grid
+    DeviceBuffer<uint32_t> mass_flag_;   // PbfSolver::mass_flag_
     // captured substeps 0 -> 1 and 1 -> 0, and the control and parameter
     // arrays they read
     hipGraphExec_t graph_[2] = {nullptr, nullptr};

@@ -50,22 +50,51 @@ __global__ void __launch_bounds__(256)
         if (bad[i] != 0u) atomicAdd(wrong + i, bad[i]);
 }
 
-}  // namespace
+// over_rest(x, rest) against x / rest, x the only mass of the step
+__global__ void __launch_bounds__(256)
+    rest_check_kernel(uint32_t first, uint32_t count, float rest, unsigned long long* wrong) {
+    const uint32_t stride = gridDim.x * blockDim.x;
+    unsigned long long bad = 0;
+    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += stride) {
+        const float x = __uint_as_float(first + t);
+        const RestDensity density = rest_density_of(rest, outside_quick_range(x));
+        bad += same(over_rest(x, density), x / rest) ? 0u : 1u;
+    }
+    if (bad != 0u) atomicAdd(wrong, bad);
+}
 
-// Mismatches of the four functions over the floats with bit patterns
-// [first, first + count); returns a hipError_t.
-extern "C" int phx_test_pair_math(float h, uint32_t first, uint32_t count, unsigned long long* mismatches) {
+// Counts mismatches on the device: launch(counter) starts the check.
+template <class Launch>
+int count_mismatches(uint32_t first, uint32_t count, unsigned long long* mismatches, int counters, Launch&& launch) {
     if (mismatches == nullptr || count == 0u || first + (count - 1u) < first) return static_cast<int>(hipErrorInvalidValue);
     unsigned long long* device = nullptr;
-    const size_t bytes = 4u * sizeof(unsigned long long);
+    const size_t bytes = static_cast<size_t>(counters) * sizeof(unsigned long long);
     hipError_t e = hipMalloc(&device, bytes);
     if (e != hipSuccess) return static_cast<int>(e);
     e = hipMemset(device, 0, bytes);
     if (e == hipSuccess) {
-        pair_check_kernel<<<4096, 256>>>(first, count, phx::pbf_kernel(h), phx::kernel_constants(h), device);
+        launch(device);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(mismatches, device, bytes, hipMemcpyDeviceToHost);
     const hipError_t f = hipFree(device);
     return static_cast<int>(e != hipSuccess ? e : f);
+}
+
+}  // namespace
+
+// Mismatches of the four functions over the floats with bit patterns
+// [first, first + count); returns a hipError_t.
+extern "C" int phx_test_pair_math(float h, uint32_t first, uint32_t count, unsigned long long* mismatches) {
+    return count_mismatches(first, count, mismatches, 4, [&](unsigned long long* wrong) {
+        pair_check_kernel<<<4096, 256>>>(first, count, phx::pbf_kernel(h), phx::kernel_constants(h), wrong);
+    });
+}
+
+// Mismatches of over_rest for the masses with bit patterns
+// [first, first + count) over the rest density `rest`; returns a hipError_t.
+extern "C" int phx_test_over_rest(float rest, uint32_t first, uint32_t count, unsigned long long* mismatches) {
+    return count_mismatches(first, count, mismatches, 1, [&](unsigned long long* wrong) {
+        rest_check_kernel<<<4096, 256>>>(first, count, rest, wrong);
+    });
 }

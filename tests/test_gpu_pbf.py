@@ -6,6 +6,7 @@ import torch
 
 import oracle
 from physica_amd import scenes
+from physica_amd.batch import PbfBatch
 from physica_amd.particle import PBF
 from helpers import bits_equal, max_rel, pbf_setup
 
@@ -71,3 +72,52 @@ def test_artificial_pressure_within_tolerance(gpu_device):
     motion = np.abs(exp["positions"] - sc.positions).max()
     assert np.abs(gx - exp["positions"]).max() <= 1e-5 * motion
     assert max_rel(gv, exp["velocities"]) <= 1e-5
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_masses_outside_the_quick_division(gpu_device, batched):
+    """Masses and rest densities whose quotients the pair terms cannot take
+    from a reciprocal (the remainders underflow), then usual ones: bit-exact
+    steps, also right after each other."""
+    sc = scenes.pbf_dam_break(shape=(12, 12, 12))
+    rng = np.random.default_rng(9)
+    usual = dict(sc.parameters)
+    tiny = dict(usual)
+    tiny["masses"] = (rng.uniform(1.0, 2.0, sc.count) * 2.0**-118).astype(np.float32)
+    tiny["rest_densities"] = np.full(sc.count, 1.37 * 2.0**-60, np.float32)
+    tiny["relaxation"] = np.full(sc.count, 2.0**-34, np.float32)  # corrections of some 1e-3
+    d = oracle.make_domain(sc.domain)
+    u = np.zeros_like(sc.positions)
+    for parameters in (tiny, usual):
+        sc.parameters = parameters
+        exp = oracle.pbf_step(d, 0, sc.positions, sc.velocities, u, parameters, 2)
+        free = oracle.pbf_step(d, 0, sc.positions, sc.velocities, u, parameters, 0)
+        assert np.abs(exp["positions"] - free["positions"]).max() > 1e-4
+        if batched:
+            engine = PbfBatch([sc.domain], PBF.Configuration(2), device=gpu_device)
+            state, control, params = engine.allocate_state(), engine.allocate_control(), engine.allocate_parameters()
+            engine.upload([sc], state, params)
+            engine.run(state, control, params, 1)
+            torch.cuda.synchronize()
+            gx, gv = state.particles.positions.numpy(), state.particles.velocities.numpy()
+        else:
+            gx, gv = gpu_step(*pbf_setup(sc, gpu_device, PBF.Configuration(2)))
+        assert bits_equal(gx, exp["positions"])
+        assert bits_equal(gv, exp["velocities"])
+
+
+def test_masses_back_in_range(gpu_device):
+    """One solver: a step with a mass outside the quick range, then one without."""
+    sc = scenes.pbf_dam_break(shape=(8, 8, 8))
+    solver, state, nxt, control, params, cache = pbf_setup(sc, gpu_device, PBF.Configuration(2))
+    d = oracle.make_domain(sc.domain)
+    for mass in (np.float32(2.0**-70), sc.parameters["masses"][7]):
+        p = dict(sc.parameters)
+        p["masses"] = p["masses"].copy()
+        p["masses"][7] = mass
+        params.particles.masses.copy_(torch.from_numpy(p["masses"]))
+        exp = oracle.pbf_step(d, 0, sc.positions, sc.velocities, np.zeros_like(sc.positions), p, 2)
+        state.particles.step_index = 0
+        gx, gv = gpu_step(solver, state, nxt, control, params, cache)
+        assert bits_equal(gx, exp["positions"])
+        assert bits_equal(gv, exp["velocities"])

@@ -27,3 +27,14 @@ def test_pair_functions_equal_their_expressions(gpu_device, h):
     for first, count in ((_bits(2.0**-90 * h * h), _bits(1.01 * h * h) - _bits(2.0**-90 * h * h)), (0, 1)):
         assert lib.phx_test_pair_math(h, first, count, wrong) == 0
         assert list(wrong) == [0, 0, 0, 0], (h, first)
+
+
+@pytest.mark.parametrize("rest", [1000.0, 1.0, 0.37, 2.0**-60, 2.0**60, 1.0e-30, 1.0e25, 0.0, float("inf")])
+def test_mass_over_rest_density_equals_the_division(gpu_device, rest):
+    """For every non-negative float mass: 0, subnormal, of any size, infinite."""
+    lib = ctypes.CDLL(str(build.PAIR_MATH_CHECK))
+    lib.phx_test_over_rest.argtypes = [ctypes.c_float, ctypes.c_uint32, ctypes.c_uint32,
+                                       ctypes.POINTER(ctypes.c_ulonglong)]
+    wrong = ctypes.c_ulonglong()
+    assert lib.phx_test_over_rest(rest, 0, _bits(np.inf) + 1, ctypes.byref(wrong)) == 0
+    assert wrong.value == 0
