@@ -99,7 +99,8 @@ struct KernelConstants {
     float sqrt_support; // smallest float t with sqrtf(t) >= h
     float inv_h;        // RN(1 / h)
     float inv_viscosity; // RN(1 / viscosity)
-    uint32_t plain;      // h lies outside [2^-20, 2^20], where div_in_range is not used
+    uint32_t plain;      // h lies outside [2^-20, 2^16], where div_in_range is not used: beyond 2^16.4 the gradient
+                         // factors next to the support's edge are subnormal
 };
 
 // Correctly rounded x / b from inv_b = RN(1 / b), for b > 0: the estimate

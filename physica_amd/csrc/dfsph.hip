@@ -100,7 +100,7 @@ KernelConstants kernel_constants(float h) {
     k.sqrt_support = sqrt_support_threshold(h);
     k.inv_h = 1.0F / h;
     k.inv_viscosity = 1.0F / k.viscosity;
-    k.plain = h >= 0x1p-20F && h <= 0x1p20F ? 0u : 1u;
+    k.plain = h >= 0x1p-20F && h <= 0x1p16F ? 0u : 1u;
     return k;
 }
 
