@@ -144,7 +144,7 @@ __device__ __forceinline__ float over_rest(float mass, const RestDensity& rest) 
 // the compiler's own sequence of reciprocal estimate, one Newton step and two
 // quotient refinements, hence its correctly rounded result, without the
 // scaling and special cases around it (8 instructions for 11). With
-// positive_sqrt it took PBF steps of 1,048,576 particles from 1,738 to
+// sqrt_rn it took PBF steps of 1,048,576 particles from 1,738 to
 // 1,625 us and WCSPH steps from 466 to 456; DFSPH's passes, held by their
 // gathers, did not move.
 __device__ __forceinline__ float div_in_range(float a, float b) {
@@ -155,24 +155,20 @@ __device__ __forceinline__ float div_in_range(float a, float b) {
     return fmaf(fmaf(-b, q, a), r, q);
 }
 
-// sqrt(x) for x > 0, correctly rounded, from the reciprocal square root s of
-// y = x 2^64 (a normal number for every such x below 2^64): g = y s is within
-// an ulp of sqrt(y), its residual y - g^2 is exact, and g + (y - g^2) s / 2
-// rounds correctly (checked on the GPU for every float below 2^64); the scale
-// is undone exactly. Two operations fewer than correcting the hardware's
-// square root by the signs of its neighbours' residuals, which also needs two
-// comparisons. x = 0 gives a root below 2^-77, which no kernel value tells
-// from 0; from 2^64 on the result is +inf; NaN stays NaN.
-__device__ __forceinline__ float positive_sqrt(float x) {
+// Correctly rounded square root of 0 <= x < 2^64 from the reciprocal square
+// root s of y = x 2^64 (a normal number for every such x but 0): g = y s is
+// within an ulp of sqrt(y), its residual y - g^2 is exact, and
+// g + (y - g^2) s / 2 rounds correctly (checked on the GPU for every float
+// below 2^64); the scale is undone exactly. x = 0 gives 0 without a branch,
+// across which the compiler does not move a pair term's later loads
+// (non-pressure pass of 4,194,304 particles 1,116 -> 1,003 us). From 2^64 on
+// the result is +inf; NaN stays NaN.
+__device__ __forceinline__ float sqrt_rn(float x) {
     const float y = x * 0x1p64F;
-    const float in_range = __builtin_amdgcn_fmed3f(y, 0x1p-90F, 0x1.fffffep127F);
-    const float s = __builtin_amdgcn_rsqf(in_range);
-    const float g = in_range * s;
+    const float s = __builtin_amdgcn_rsqf(__builtin_amdgcn_fmed3f(y, 0x1p-90F, 0x1.fffffep127F));
+    const float g = __builtin_amdgcn_fmed3f(y, 0.0F, 0x1.fffffep127F) * s;
     return fmaf(fmaf(-g, g, y), 0.5F * s, g) * 0x1p-32F;
 }
-
-// Correctly rounded square root of 0 <= x < 2^64 (positive_sqrt, and 0 at 0).
-__device__ __forceinline__ float sqrt_rn(float x) { return x == 0.0F ? 0.0F : positive_sqrt(x); }
 
 // length(d) of a neighbour pair (the same value; any |d| >= 2^32 gives +inf,
 // which lies outside every support).

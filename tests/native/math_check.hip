@@ -1,7 +1,7 @@
 // Checks of the correctly rounded helpers of device_math.hpp against the
 // compiler's IEEE operations: div_rn against x / b (on the host and on the
 // GPU) and sqrt_rn against sqrtf (on the GPU, where the hardware estimate
-// it corrects lives). Built by physica_amd.build into
+// it starts from lives). Built by physica_amd.build into
 // tests/native/libphx_math_check.so and driven from tests/test_device_math.py.
 #include <hip/hip_runtime.h>
 

@@ -10,7 +10,7 @@ compiler's division and square root (physica_amd/csrc/device_math.hpp):
   2^-105 the remainders underflow and the sequence can miss (x = 0 is exact);
   the kernels' arguments are distances, at least 2^-74.5 when nonzero.
 - sqrt_rn(x) must equal sqrtf(x) for every float in [0, 2^64) (GPU only: it
-  corrects the hardware's square-root estimate).
+  corrects a root taken from the hardware's reciprocal square root).
 """
 from __future__ import annotations
 
@@ -86,6 +86,9 @@ def test_sqrt_rn_equals_sqrtf_below_2_64():
     wrong = ctypes.c_ulonglong(0)
     last = _bits(2.0 ** 64)
     assert lib.phx_test_math_gpu(0, 0, last, 1.0, ctypes.byref(wrong)) == 0
+    assert wrong.value == 0
+    # infinity stays infinity
+    assert lib.phx_test_math_gpu(0, _bits(np.inf), 1, 1.0, ctypes.byref(wrong)) == 0
     assert wrong.value == 0
 
 
