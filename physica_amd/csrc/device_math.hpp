@@ -144,9 +144,7 @@ __device__ __forceinline__ float over_rest(float mass, const RestDensity& rest) 
 // the compiler's own sequence of reciprocal estimate, one Newton step and two
 // quotient refinements, hence its correctly rounded result, without the
 // scaling and special cases around it (8 instructions for 11). With
-// sqrt_rn it took PBF steps of 1,048,576 particles from 1,738 to
-// 1,625 us and WCSPH steps from 466 to 456; DFSPH's passes, held by their
-// gathers, did not move.
+// sqrt_rn it took PBF steps of 1,048,576 particles from 1,738 to 1,625 us.
 __device__ __forceinline__ float div_in_range(float a, float b) {
     float r = __builtin_amdgcn_rcpf(b);
     r = fmaf(fmaf(-b, r, 1.0F), r, r);
@@ -188,7 +186,14 @@ __device__ __forceinline__ float cubic_value(float dist, const KernelConstants& 
 
 // The radial factor f of cubic_gradient(d, h) = f * d (zero outside the
 // support and at d = 0), with the constants supplied; branch-free like
-// cubic_value().
+// cubic_value() but for the choice of the quotient with kQuick, which the
+// derivative passes take. The forward passes, held by their gathers, lose more
+// by the choice's branch at every pair than the shorter quotient saves (force
+// pass of 4,194,304 particles 486 us, with it 503; of 1,048,576 87.5 and 88.3;
+// WCSPH steps of 2,097,152 886 and 886); the derivatives, held by their
+// arithmetic, gain (a DFSPH step of 35,805 particles with JVP and VJP 1,717 us,
+// with it 1,691).
+template <bool kQuick = false>
 __device__ __forceinline__ float cubic_gradient_factor(float dist, const KernelConstants& k) {
     const float q = div_rn(dist, k.h, k.inv_h);
     const float near = 18.0F * q * q - 12.0F * q;
@@ -197,7 +202,7 @@ __device__ __forceinline__ float cubic_gradient_factor(float dist, const KernelC
     const float deriv = q <= 0.5F ? near : far;
     const float top = k.cubic * deriv;
     const float bottom = k.h * dist;
-    const float f = k.plain != 0u ? top / bottom : div_in_range(top, bottom);
+    const float f = !kQuick || k.plain != 0u ? top / bottom : div_in_range(top, bottom);
     return dist == 0.0F || dist >= k.h ? 0.0F : f;
 }
 

@@ -292,14 +292,14 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_density_kernel(DensityJ
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
             terms[0] = qt.w * cubic_value(dist, s.kc) +
-                       q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pt, xyz(qt)));
+                       q.w * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), sub(pt, xyz(qt)));
         },
         [&](uint32_t b, float (&terms)[1]) {
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
             terms[0] = q.w * (rest_t_i * cubic_value(dist, s.kc) +
-                              rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pt));
+                              rest_i * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), pt));
         });
     if (!writes) return;
     const float result = sum[0];
@@ -397,7 +397,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_force_kernel(ForceJvpAr
                              const Float3 diff_t = sub(xyz(vqt), xyz(vt_i));
                              put(terms, add(scale(diff, w_t), scale(diff_t, weight)));
                          }
-                         const Float3 gradient = scale(d, cubic_gradient_factor(length(d), s.kc));
+                         const Float3 gradient = scale(d, cubic_gradient_factor<true>(length(d), s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, dd, s.kc);
                          const float2 t1_j = r.t1;
                          const float factor = -mass * (t1_i.x + t1_j.x);
@@ -422,7 +422,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_force_kernel(ForceJvpAr
                              const Float3 diff = sub(xyz(s.boundary.v[b]), xyz(vm));
                              put(terms, add(scale(diff, w_t), scale(xyz(vt_i), -weight)));
                          }
-                         const Float3 gradient = scale(d, cubic_gradient_factor(length(d), s.kc));
+                         const Float3 gradient = scale(d, cubic_gradient_factor<true>(length(d), s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, xti, s.kc);
                          put(terms + kFirst, boundary_pressure(gradient, gradient_t, vol, t1_i));
                          if constexpr (kTwo) put(terms + kSecond, boundary_pressure(gradient, gradient_t, vol, t2_i));
@@ -506,14 +506,14 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_projection_kernel(Proje
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
             terms[0] = r.mass_t * cubic_value(dist, s.kc) +
-                       q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pst, xyz(r.qt)));
+                       q.w * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), sub(pst, xyz(r.qt)));
         },
         [&](uint32_t b, float (&terms)[1]) {
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
             terms[0] = q.w * (rest_t_i * cubic_value(dist, s.kc) +
-                              rest_i * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pst));
+                              rest_i * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), pst));
         });
     if (!writes) return;
     const float rs_t = sum[0];
@@ -668,7 +668,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_pressure_kernel(Pressur
                              position = add(position,
                                             viscosity_laplacian_gradient(d, h, s.pi_h6, cross_w_a * nu * m_i / rho_i));
                          }
-                         const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), s.kc)));
+                         const D3 gradient = d3(scale(d, cubic_gradient_factor<true>(length(d), s.kc)));
                          const double second = static_cast<double>(r.p) / (r.rho * r.rho);
                          const double sum = first + second;
                          const double local_factor = -mass * sum;
@@ -696,7 +696,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_pressure_kernel(Pressur
                              position = add(position, viscosity_laplacian_gradient(d, h, s.pi_h6, w_a * vm.w * vol));
                          }
                          // pressure_vjp_kernel's boundary half: -rho0_i V (p_i / rho_i^2) grad W
-                         const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), s.kc)));
+                         const D3 gradient = d3(scale(d, cubic_gradient_factor<true>(length(d), s.kc)));
                          const double factor = static_cast<double>(-rest_i * vol) * first;
                          const double factor_a = dot(local, gradient);
                          rest_c -= factor_a * vol * first;
@@ -797,7 +797,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_density_kernel(DensityV
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
             const double rs_a_j = r.rs_a;
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))),
                                            out_a * q.w + rs_a_j * m_i));
             mass_c += rs_a_j * cubic_value(dist, s.kc);
         },
@@ -805,7 +805,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_density_kernel(DensityV
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(ps, xyz(q));
             const float dist = length(d);
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))), out_a * rest_i * q.w));
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))), out_a * rest_i * q.w));
             rest_c += out_a * q.w * cubic_value(dist, s.kc);
         });
     position = group_sum<G>(position);
@@ -861,7 +861,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_scatter_kernel(ScatterV
             const Float3 d = sub(x, xyz(q));
             const float dist = length(d);
             const double rho_a_j = r.rho_a;
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))),
                                            out_a * q.w + rho_a_j * m_i));
             mass_c += rho_a_j * cubic_value(dist, s.kc);
         },
@@ -869,7 +869,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_scatter_kernel(ScatterV
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(x, xyz(q));
             const float dist = length(d);
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))), out_a * rest_i * q.w));
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))), out_a * rest_i * q.w));
             rest_c += out_a * q.w * cubic_value(dist, s.kc);
         });
     position = group_sum<G>(position);

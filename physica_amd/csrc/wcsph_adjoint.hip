@@ -132,14 +132,14 @@ __global__ void __launch_bounds__(kBlock) wcsph_jvp_density_kernel(WcsphDensityJ
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
             rho_t += qt.w * cubic_value(dist, s.kc) +
-                     q.w * dot(scale(d, cubic_gradient_factor(dist, s.kc)), sub(pti, xyz(qt)));
+                     q.w * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), sub(pti, xyz(qt)));
         },
         [&](uint32_t b) {
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(p, xyz(q));
             const float dist = length(d);
             rho_t += q.w * (rest_t * cubic_value(dist, s.kc) +
-                            rest * dot(scale(d, cubic_gradient_factor(dist, s.kc)), pti));
+                            rest * dot(scale(d, cubic_gradient_factor<true>(dist, s.kc)), pti));
         });
     a.rho_t[i] = rho_t;
     const float4 own = s.aux[i];
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_jvp_force_kernel(WcsphForceJvpAr
                          const Float3 d = sub(x, xyz(q));
                          const Float3 dd = sub(xti, xyz(qt));
                          const float dist = length(d);
-                         const Float3 gradient = scale(d, cubic_gradient_factor(dist, s.kc));
+                         const Float3 gradient = scale(d, cubic_gradient_factor<true>(dist, s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, dd, s.kc);
                          // pressure
                          const float2 tt_j = a.tt[j];
@@ -261,7 +261,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_jvp_force_kernel(WcsphForceJvpAr
                          const float vol = q.w;
                          const Float3 d = sub(x, xyz(q));
                          const float dist = length(d);
-                         const Float3 gradient = scale(d, cubic_gradient_factor(dist, s.kc));
+                         const Float3 gradient = scale(d, cubic_gradient_factor<true>(dist, s.kc));
                          const Float3 gradient_t = cubic_gradient_tangent(d, xti, s.kc);
                          // pressure: -rho0_i V (p_i / rho_i^2) grad W
                          const float factor = -rest_i * vol * tt_i.x;
@@ -352,7 +352,7 @@ __device__ __forceinline__ ViscosityAdjoint viscosity_reverse(Float3 d, Float3 d
     const double rho_sum = static_cast<double>(rho_a + rho_b);
     const double nu = 2.0 * alpha * h * speed / rho_sum;
     const double pi = -nu * compression / denominator;
-    const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), kc)));
+    const D3 gradient = d3(scale(d, cubic_gradient_factor<true>(length(d), kc)));
     r.mass_b = -pi * dot(w, gradient);
     const double pi_a = -static_cast<double>(mass_b) * dot(w, gradient);
     r.displacement = cubic_hessian_product(d, scale(w, -static_cast<double>(mass_b) * pi), h);
@@ -384,7 +384,7 @@ __device__ __forceinline__ SurfaceAdjoint surface_reverse(Float3 d, float mass_a
     const double factor_a = dot(w, d3(d));
     r.displacement = scale(w, factor);
     if (dist > s.diameter)
-        r.displacement = add(r.displacement, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
+        r.displacement = add(r.displacement, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))),
                                                    -static_cast<double>(tension) * mass_b * factor_a / mass_a));
     r.tension = -static_cast<double>(mass_b) * weight * factor_a / mass_a;
     r.mass_b = -static_cast<double>(tension) * weight * factor_a / mass_a;
@@ -432,7 +432,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_vjp_force_kernel(WcsphForceVjpAr
                          const float mass = q.w;
                          const D3 cross = load(a.total_a, j);
                          // pressure
-                         const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), s.kc)));
+                         const D3 gradient = d3(scale(d, cubic_gradient_factor<true>(length(d), s.kc)));
                          const double second = static_cast<double>(s.p[j]) / (s.aux[j].x * s.aux[j].x);
                          const double sum = first + second;
                          first_a -= mass * dot(local, gradient);
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_vjp_force_kernel(WcsphForceVjpAr
                          const float vol = q.w;
                          const Float3 d = sub(x, xyz(q));
                          // pressure: -rho0_i V (p_i / rho_i^2) grad W
-                         const D3 gradient = d3(scale(d, cubic_gradient_factor(length(d), s.kc)));
+                         const D3 gradient = d3(scale(d, cubic_gradient_factor<true>(length(d), s.kc)));
                          const double factor = static_cast<double>(-rest_i * vol) * first;
                          const double factor_a = dot(local, gradient);
                          rest_c -= factor_a * vol * first;
@@ -553,7 +553,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_vjp_density_kernel(WcsphDensityV
             const Float3 d = sub(x, xyz(q));
             const float dist = length(d);
             const double rho_a_j = a.rho_a[j];
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))),
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))),
                                            out_a * q.w + rho_a_j * self.w));
             mass_c += rho_a_j * cubic_value(dist, s.kc);
         },
@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(kBlock) wcsph_vjp_density_kernel(WcsphDensityV
             const float4 q = s.boundary.x[b];
             const Float3 d = sub(x, xyz(q));
             const float dist = length(d);
-            position = add(position, scale(d3(scale(d, cubic_gradient_factor(dist, s.kc))), out_a * rest_i * q.w));
+            position = add(position, scale(d3(scale(d, cubic_gradient_factor<true>(dist, s.kc))), out_a * rest_i * q.w));
             rest_c += out_a * q.w * cubic_value(dist, s.kc);
         });
     accumulate(a.pos_a, i, position);

@@ -22,7 +22,7 @@ __device__ bool same(float a, float b) {
     return __float_as_uint(a) == __float_as_uint(b) || (a == 0.0F && b == 0.0F);
 }
 
-// [0] poly6_value, [1] spiky_factor, [2] cubic_gradient_factor, [3] cubic_value
+// [0] poly6_value, [1] spiky_factor, [2] cubic_gradient_factor<true>, [3] cubic_value
 __global__ void __launch_bounds__(256)
     pair_check_kernel(uint32_t first, uint32_t count, PbfKernel k, KernelConstants c, unsigned long long* wrong) {
     const uint32_t stride = gridDim.x * blockDim.x;
@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256)
         const float q = dist / h;
         const float deriv = q <= 0.5F ? 18.0F * q * q - 12.0F * q : -6.0F * (1.0F - q) * (1.0F - q);
         const float f = dist == 0.0F || dist >= h ? 0.0F : c.cubic * deriv / (h * dist);
-        bad[2] += same(cubic_gradient_factor(sqrt_rn(d2), c), f) ? 0u : 1u;
+        bad[2] += same(cubic_gradient_factor<true>(sqrt_rn(d2), c), f) ? 0u : 1u;
         const float v = dist >= h ? 0.0F
                         : q <= 0.5F ? c.cubic * (6.0F * q * q * q - 6.0F * q * q + 1.0F)
                                     : c.cubic * 2.0F * (1.0F - q) * (1.0F - q) * (1.0F - q);
