@@ -280,7 +280,6 @@ void DfsphSolver::forward_step(const phx_sph_dfsph_state& state, const phx_contr
                        cache.densities.data(),
                        t_div_.data(),
                        t_den_.data(),
-                       masks_.flags(),
                        rho0};
     ma.crowded = crowded;
     ma.cell = masks_.cells();

@@ -75,11 +75,10 @@ struct Step {
 __device__ __forceinline__ bool exact_masked(const Step& s, uint32_t i) {
     return s.flags[kFlagOverflow] == 0u && s.crowded[i] == 0u;
 }
-__device__ __forceinline__ MaskView exact_view(const Step& s) {
-    return MaskView{s.exact, s.flags, s.n, s.limit2, 0u, s.crowded};
-}
-__device__ __forceinline__ MaskView skin_view(const Step& s) {
-    return MaskView{s.skin, s.flags, s.n, s.limit2, 0u, s.crowded};
+// Whether the skin masks hold at the predicted positions of displacement slot
+// `slot`: no particle moved farther than they allow.
+__device__ __forceinline__ bool skin_holds(const Step& s, uint32_t slot) {
+    return __uint_as_float(s.flags[kFlagDisplacement + slot]) <= s.limit2;
 }
 
 // The derivative passes serve each particle with a group of G lanes: with one
@@ -89,14 +88,14 @@ __device__ __forceinline__ MaskView skin_view(const Step& s) {
 // its divisions), density VJP 43 / 24, projection JVP 51 / 23, force JVP 31 / 16.
 
 // Lists the candidates of a workgroup's particles (base ..) for its groups:
-// the fluid particles in the masks of particle w or, where they do not apply,
+// the fluid particles in the masks of particle w (with exact those of the
+// state's positions, else the skin masks) or, where the skin masks do not hold,
 // near it at the positions pos, walked with fluid(row, count); for a crowded
 // particle and in a step with boundary samples (whose masks are not used) the
 // particles and samples of the stencil near it, walked with all(row, count).
 template <int G, class Fluid, class All>
-__device__ __forceinline__ void group_candidates(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
-                                                 const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
-                                                 Fluid&& fluid, All&& all) {
+__device__ __forceinline__ void group_candidates(const Step& s, bool exact, uint32_t slot, const float4* pos,
+                                                 GroupLds<G>& lds, uint32_t base, uint32_t w, Fluid&& fluid, All&& all) {
     const uint32_t i = base + threadIdx.x % kGroupParticles<G>;
     const bool active = w < s.n;
     // the rounding of a distance in another order than the kernels'
@@ -112,9 +111,9 @@ __device__ __forceinline__ void group_candidates(const Step& s, const MaskView& 
             if (i >= s.n || !exact_masked(s, i)) return;
             int cx, cy, cz;
             particle_cell(s.grid, xyz(s.xm[i]), cx, cy, cz);
-            if (exact || masks_apply(mv, slot, i)) {
-                stored_slots<G, false>(mv.masks, s.grid, s.grid.offsets, s.n, i, cell_of(s.grid, cx, cy, cz), bits,
-                                       first);
+            if (exact || skin_holds(s, slot)) {
+                stored_slots<G, false>(exact ? s.exact : s.skin, s.grid, s.grid.offsets, s.n, i,
+                                       cell_of(s.grid, cx, cy, cz), bits, first);
             } else {
                 const Float3 p = xyz(pos[i]);
                 scanned_slots<G>(s.grid, s.grid.offsets, pos, cx, cy, cz, bits, first,
@@ -141,11 +140,11 @@ __device__ __forceinline__ void group_candidates(const Step& s, const MaskView& 
 // The candidates of an adjoint: pair(load(j), j) and sample(b), each lane with
 // every G-th one; the lanes' FP64 sums are added at the end, in no order.
 template <int G, class Load, class Pair, class Sample>
-__device__ __forceinline__ void group_visit(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
-                                            const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
-                                            Load&& load_record, Pair&& pair, Sample&& sample) {
+__device__ __forceinline__ void group_visit(const Step& s, bool exact, uint32_t slot, const float4* pos,
+                                            GroupLds<G>& lds, uint32_t base, uint32_t w, Load&& load_record,
+                                            Pair&& pair, Sample&& sample) {
     group_candidates<G>(
-        s, mv, exact, slot, pos, lds, base, w,
+        s, exact, slot, pos, lds, base, w,
         [&](const uint32_t* row, uint32_t count) { group_visit_list<G>(row, count, load_record, pair); },
         [&](const uint32_t* row, uint32_t count) {
             group_visit_list<G>(
@@ -165,12 +164,12 @@ __device__ __forceinline__ void group_visit(const Step& s, const MaskView& mv, b
 // sample(b, terms) write a candidate's F terms, which are added to sum in the
 // reference's order (group_add).
 template <int G, int F, class Load, class Pair, class Sample>
-__device__ __forceinline__ void group_tangent(const Step& s, const MaskView& mv, bool exact, uint32_t slot,
-                                              const float4* pos, GroupLds<G>& lds, uint32_t base, uint32_t w,
-                                              float (&sum)[F], Load&& load_record, Pair&& pair, Sample&& sample) {
+__device__ __forceinline__ void group_tangent(const Step& s, bool exact, uint32_t slot, const float4* pos,
+                                              GroupLds<G>& lds, uint32_t base, uint32_t w, float (&sum)[F],
+                                              Load&& load_record, Pair&& pair, Sample&& sample) {
     auto fold = [&](const float (&terms)[F]) { group_add<G, F>(sum, terms); };
     group_candidates<G>(
-        s, mv, exact, slot, pos, lds, base, w,
+        s, exact, slot, pos, lds, base, w,
         [&](const uint32_t* row, uint32_t count) { group_walk_list<G, F>(row, count, w, load_record, pair, fold); },
         [&](const uint32_t* row, uint32_t count) {
             group_walk_list<G, F>(
@@ -285,7 +284,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_density_kernel(DensityJ
         float4 q, qt;
     };
     group_tangent<G, 1>(
-        s, exact_view(s), true, 0u, s.xm, lds, base, w, sum, [&](uint32_t j) { return Record{s.xm[j], a.xt[j]}; },
+        s, true, 0u, s.xm, lds, base, w, sum, [&](uint32_t j) { return Record{s.xm[j], a.xt[j]}; },
         [&](const Record& r, uint32_t, float (&terms)[1]) {
             const float4 q = r.q;
             const float4 qt = r.qt;
@@ -373,7 +372,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_force_kernel(ForceJvpAr
         float4 q, qt;
         float2 t1, t2;
     };
-    group_tangent<G, kSums>(s, exact_view(s), true, 0u, s.xm, lds, base, w, sum,
+    group_tangent<G, kSums>(s, true, 0u, s.xm, lds, base, w, sum,
                      [&](uint32_t j) { return Record{s.xm[j], a.xt[j], a.t1[j], kTwo ? a.t2[j] : float2{}}; },
                      [&](const Record& r, uint32_t j, float (&terms)[kSums]) {
                          if (j == w) return;
@@ -493,13 +492,12 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_jvp_projection_kernel(Proje
     float sum[1] = {0.0F};
     const float rest_i = s.rest[i];
     const float rest_t_i = a.rest_t[i];
-    const MaskView mv = skin_view(s);
     struct Record {
         float4 q, qt;
         float mass_t;
     };
     group_tangent<G, 1>(
-        s, mv, false, a.slot, a.xs, lds, base, w, sum,
+        s, false, a.slot, a.xs, lds, base, w, sum,
         [&](uint32_t j) { return Record{a.xs[j], a.xs_t[j], a.xt[j].w}; },
         [&](const Record& r, uint32_t, float (&terms)[1]) {
             const float4 q = r.q;
@@ -639,7 +637,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_pressure_kernel(Pressur
         float p, rho;
         D3 ap_a;
     };
-    group_visit<G>(s, exact_view(s), true, 0u, s.xm, lds, base, w,
+    group_visit<G>(s, true, 0u, s.xm, lds, base, w,
                      [&](uint32_t j) { return Record{s.xm[j], a.p[j], s.rho[j], load(a.ap_a, j)}; },
                      [&](const Record& r, uint32_t j) {
                          if (j == w) return;
@@ -785,13 +783,12 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_density_kernel(DensityV
     double mass_c = 0.0;
     double rest_c = 0.0;
     const float rest_i = s.rest[i];
-    const MaskView mv = skin_view(s);
     struct Record {
         float4 q;
         double rs_a;
     };
     group_visit<G>(
-        s, mv, false, a.slot, a.xs, lds, base, w, [&](uint32_t j) { return Record{a.xs[j], a.rs_a[j]}; },
+        s, false, a.slot, a.xs, lds, base, w, [&](uint32_t j) { return Record{a.xs[j], a.rs_a[j]}; },
         [&](const Record& r, uint32_t) {
             const float4 q = r.q;
             const Float3 d = sub(ps, xyz(q));
@@ -855,7 +852,7 @@ __global__ void __launch_bounds__(kGroupBlock) dfsph_vjp_scatter_kernel(ScatterV
         double rho_a;
     };
     group_visit<G>(
-        s, exact_view(s), true, 0u, s.xm, lds, base, w, [&](uint32_t j) { return Record{s.xm[j], a.rho_a[j]}; },
+        s, true, 0u, s.xm, lds, base, w, [&](uint32_t j) { return Record{s.xm[j], a.rho_a[j]}; },
         [&](const Record& r, uint32_t) {
             const float4 q = r.q;
             const Float3 d = sub(x, xyz(q));

@@ -20,9 +20,10 @@ namespace phx {
 constexpr int kStencil = 27;
 constexpr uint32_t kMaskBits = 16;
 
-// Device flags of a step: [0] masks unusable for every particle (boundary
-// samples); [1 + k] largest squared displacement |x* - x|^2 (float bits)
-// written by the k-th predicting pass.
+// Device flags of a step: [0] raised in the copy that a recorded step keeps
+// where its masks do not serve its derivatives (boundary samples, which have
+// masks of their own in the forward passes only); [1 + k] largest squared
+// displacement |x* - x|^2 (float bits) written by the k-th predicting pass.
 constexpr uint32_t kFlagOverflow = 0;
 constexpr uint32_t kFlagDisplacement = 1;
 
@@ -168,15 +169,6 @@ __device__ __forceinline__ uint32_t drop_self(uint32_t i, uint32_t cell_first, u
     return m == 0u ? nonzero & ~(1u << kCenter) : nonzero;
 }
 
-// ------------------------------------------------ crowded cells, wave-shared
-// A particle next to a crowded cell walks every candidate of its 27 cells.
-// Inside a crowded cell every particle has the same 27 cells, so a wave whose
-// crowded lanes all sit in one cell fetches each run of 64 candidates with
-// one coalesced load per lane and hands candidate k to every lane from scalar
-// registers (v_readlane): the walk has no memory access per candidate. Each
-// lane still adds its own terms in the reference order, so its sums are
-// unchanged bit for bit.
-
 // Workgroup index with consecutive ranges of indices on one XCD (MI355X
 // dispatches workgroup b to XCD b % 8). gridDim.x must be a multiple of 8.
 __device__ __forceinline__ uint32_t xcd_block() {
@@ -184,29 +176,11 @@ __device__ __forceinline__ uint32_t xcd_block() {
     return (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
 }
 
-// A step's skin masks and the flags that decide, pass by pass, whether they
-// apply: a pass at positions that moved at most sqrt(flags[kFlagDisplacement
-// + slot]) from the positions the masks were built at may use them while
-// that is within limit2 and no cell overflowed.
+// Masks of n particles, [kStencil][n].
 struct MaskView {
-    const uint16_t* masks;  // [kStencil][n]; null: always scan the full stencil
-    const uint32_t* flags;
+    const uint16_t* masks;
     uint32_t n;
-    float limit2;
-    // exact masks of one set of positions: they apply unless flags[kFlagOverflow]
-    // is raised; no displacement slot is read
-    uint32_t exact = 0u;
-    // per particle (sorted order): non-zero where a stencil cell holds more
-    // than kMaskBits particles; null: no particle is crowded
-    const uint8_t* crowded = nullptr;
 };
-
-// Whether particle i walks its masks in a pass reading displacement slot `slot`.
-__device__ __forceinline__ bool masks_apply(const MaskView& m, uint32_t slot, uint32_t i) {
-    if (m.masks == nullptr || m.flags[kFlagOverflow] != 0u) return false;
-    if (m.crowded != nullptr && m.crowded[i] != 0u) return false;
-    return m.exact != 0u || __uint_as_float(m.flags[kFlagDisplacement + slot]) <= m.limit2;
-}
 
 // The masks of members from .. to - 1 (the first kMaskBits of them) of the
 // records x: test(position, marked) sets the bits of a member in the M masks.

@@ -785,7 +785,6 @@ void PbfCache::allocate(uint32_t n, uint32_t cells, uint32_t pressure_iterations
     normalizers.resize(n);
     crowded.resize(n);
     exact_masks.resize(static_cast<size_t>(pressure_iterations + 1u) * kStencil * n);
-    exact_flags.resize(pressure_iterations + 1u);
 }
 
 PbfSolver::PbfSolver(const phx_domain_configuration* domain, const phx_pbf_configuration* configuration,
@@ -897,11 +896,9 @@ void PbfSolver::forward_step(const phx_pbf_state& state, const phx_control& cont
     }
     // exact masks of position set k (iterate k, the final positions last):
     // written by the pass that first walks those positions, walked by the
-    // later passes at them; a recorded step keeps every set. Each recorded set
-    // has one overflow word.
+    // later passes at them; a recorded step keeps every set
     const float t_exact = exact_mask_threshold(h);
     const uint32_t sets = config_.pressure_iterations + 1u;
-    if (rec) fill_u32(stream_, cache.exact_flags.data(), sets, 0u);
     auto exact_set = [&](uint32_t k) {
         require(k < sets, PHX_ERROR_INVALID_ARGUMENT, "exact mask set out of range");
         return rec ? cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n : exact_.data();

@@ -53,9 +53,8 @@ struct PbfCache {
     DeviceBuffer<float> normalizers;
     DeviceBuffer<uint8_t> crowded;  // per particle: walks the full stencil (a stencil cell overflows the masks)
     // exact masks of every set of positions (iterates 0 .. I - 1, then the
-    // final positions), [set][kStencil][n], and one overflow word per set
+    // final positions), [set][kStencil][n]
     DeviceBuffer<uint16_t> exact_masks;
-    DeviceBuffer<uint32_t> exact_flags;
 
     void allocate(uint32_t n, uint32_t cells, uint32_t pressure_iterations);
 };

@@ -79,10 +79,20 @@ __device__ __forceinline__ void store(DVec f, uint32_t i, D3 v) {
 // w: H(d) w = f w + (f'(r) / r) (d . w) d, f' = -k (h - r)(h + r) / r^2; zero
 // where G is zero (r = 0 or r >= h). H is symmetric and even in d
 // (spiky_hessian_product, spiky_gradient_tangent, pbf.cu:34-54).
-// The FP64 form (reverse passes) is spiky_hessian_one_division, below.
-__device__ __forceinline__ D3 spiky_hessian_one_division(Float3 d, D3 w, double h, double k);
+// The FP64 form (reverse passes) takes 1 / r from inverse_sqrt instead of a
+// square root and a division.
 __device__ __forceinline__ D3 spiky_hessian(Float3 d, D3 w, double h, double k) {
-    return spiky_hessian_one_division(d, w, h, k);
+#pragma clang fp contract(fast)
+    const D3 dd = d3(d);
+    const double r2 = dot(dd, dd);
+    if (r2 == 0.0) return {0.0, 0.0, 0.0};
+    const double inv_r = inverse_sqrt(r2);
+    const double r = r2 * inv_r;
+    if (r >= h) return {0.0, 0.0, 0.0};
+    const double hr = h - r;
+    const double f = k * hr * hr * inv_r;
+    const double fpr = -k * hr * (h + r) * inv_r * inv_r * inv_r;  // f'(r) / r
+    return add(scale(w, f), scale(dd, fpr * dot(dd, w)));
 }
 
 __device__ __forceinline__ Float3 spiky_hessian(Float3 d, Float3 w, float h, float k) {
@@ -142,7 +152,8 @@ struct Step {
     SortedGrid grid;
     CVec xs, x0;
     const float *m, *rho0, *eps, *strength, *exponent, *radius, *xsph, *confinement;
-    MaskView mv;  // the recorded step's masks and flags
+    MaskView mv;             // the exact masks of the positions read
+    const uint8_t* crowded;  // per particle: walks the full stencil
     BoundaryGrid boundary;   // the step's sorted boundary samples; offsets null: none
     // reverse passes
     PbfKernel k;
@@ -230,9 +241,9 @@ __device__ __forceinline__ void reverse_walk(const Step& s, const float4* pos, G
     uint32_t center = 0u;
     if (i < s.n) {
         center = s.cell[i];
-        masked = masks_apply(s.mv, 0u, i);
+        masked = s.crowded[i] == 0u;
     }
-    const bool listed = active && masks_apply(s.mv, 0u, w);
+    const bool listed = active && s.crowded[w] == 0u;
     auto near = [&](Float3 p, Float3 q) {
         const Float3 d = sub(p, q);
         return !(dot(d, d) >= s.t_exact);
@@ -500,22 +511,6 @@ struct CorrectionVjpArgs {
     double2* lambda_terms;  // (density adjoint, D_bar) per particle (written)
 };
 
-// Derivative of G(d) = f(r) d (spiky gradient) along w, with 1 / r from
-// inverse_sqrt instead of a square root and a division.
-__device__ __forceinline__ D3 spiky_hessian_one_division(Float3 d, D3 w, double h, double k) {
-#pragma clang fp contract(fast)
-    const D3 dd = d3(d);
-    const double r2 = dot(dd, dd);
-    if (r2 == 0.0) return {0.0, 0.0, 0.0};
-    const double inv_r = inverse_sqrt(r2);
-    const double r = r2 * inv_r;
-    if (r >= h) return {0.0, 0.0, 0.0};
-    const double hr = h - r;
-    const double f = k * hr * hr * inv_r;
-    const double fpr = -k * hr * (h + r) * inv_r * inv_r * inv_r;  // f'(r) / r
-    return add(scale(w, f), scale(dd, fpr * dot(dd, w)));
-}
-
 // project_vjp_kernel (pbf.cu:445-454) and correction_vjp_kernel
 // (pbf.cu:335-415). The Hessian is even in d, so the terms where i is the
 // centre and where it is the neighbour share one product; the neighbour's
@@ -584,7 +579,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_vjp_correction_kernel(Correct
             const double rsa = rcf * ob_rgr;
             lcon += rsa;
             mcon += rmu * inv_rrho0 * ob_rgr;
-            pcon = add(pcon, spiky_hessian_one_division(dd, sub(scale(oa, cf * mu), scale(ob, rcf * rmu)), h, k));
+            pcon = add(pcon, spiky_hessian(dd, sub(scale(oa, cf * mu), scale(ob, rcf * rmu)), h, k));
             if (!vanishes_j) pcon = sub(pcon, scale(d3(rart.gradient), rsa));
         },
         [&](float4 q) {
@@ -600,7 +595,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_vjp_correction_kernel(Correct
             scon += sa * static_cast<double>(art.d_strength);
             econ += sa * static_cast<double>(art.d_exponent);
             qcon += sa * static_cast<double>(art.d_radius);
-            pcon = add(pcon, spiky_hessian_one_division(dd, scale(oa, vol * mu), h, k));
+            pcon = add(pcon, spiky_hessian(dd, scale(oa, vol * mu), h, k));
             pcon = add(pcon, scale(d3(art.gradient), sa));
         });
     pcon = group_sum<G>(pcon);
@@ -691,7 +686,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_vjp_lambda_kernel(LambdaVjpAr
             const D3 rgbar = scale(sub(sgj, scale(gr, rcf)), 2.0 * jterms.y * rcf);
             const double rcbar = 2.0 * jterms.y * (rcf * gr2 - dot(gr, sgj));
             ml += rcbar * inv_jrho0;
-            pl = add(pl, spiky_hessian_one_division(dd, sub(gbar, rgbar), h, k));
+            pl = add(pl, spiky_hessian(dd, sub(gbar, rgbar), h, k));
         },
         [&](float4 q) {
             // a boundary sample: the density term rho0_i V_b W (density.cu:88-93)
@@ -700,7 +695,7 @@ __global__ void __launch_bounds__(kGroupBlock) pbf_vjp_lambda_kernel(LambdaVjpAr
             const double vol = static_cast<double>(q.w);
             pd = add(pd, scale(d3(poly6_gradient(dd, s.h)), rho_a * rho0 * vol));
             rd += rho_a * vol * static_cast<double>(poly6(dd, s.h));
-            pl = add(pl, spiky_hessian_one_division(dd, scale(sgi, 2.0 * dbar * vol), h, k));
+            pl = add(pl, spiky_hessian(dd, scale(sgi, 2.0 * dbar * vol), h, k));
         });
     pl = group_sum<G>(pl);
     pd = group_sum<G>(pd);
@@ -857,7 +852,6 @@ struct TangentParams {
 struct LambdaJvpArgs {
     Step s;
     TangentParams t;
-    uint32_t slot;  // displacement slot of the positions read
     CVec pos, p_t;
     const float *rho, *den;
     float* lambda_t;
@@ -869,7 +863,7 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_lambda_kernel(LambdaJvpArgs a)
     PHX_MASK_LDS(a.s.grid);
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
     if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+    const bool masked = a.s.crowded[i] == 0u;
     const Step& s = a.s;
     const Float3 pi = load(a.pos, i), ti = load(a.p_t, i);
     const float rho0 = s.rho0[i], rho0_t = a.t.rho0[i];
@@ -910,7 +904,6 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_lambda_kernel(LambdaJvpArgs a)
 struct CorrectionJvpArgs {
     Step s;
     TangentParams t;
-    uint32_t slot;  // displacement slot of the positions read
     CVec pos, p_t;
     const float *lambda, *lambda_t;
     const uint8_t* mask;
@@ -923,7 +916,7 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_correction_kernel(CorrectionJv
     PHX_MASK_LDS(a.s.grid);
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
     if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+    const bool masked = a.s.crowded[i] == 0u;
     const Step& s = a.s;
     const Float3 pi = load(a.pos, i), ti = load(a.p_t, i);
     const float rho0 = s.rho0[i], rho0_t = a.t.rho0[i];
@@ -965,7 +958,6 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_correction_kernel(CorrectionJv
 struct PostJvpArgs {
     Step s;
     TangentParams t;
-    uint32_t slot;  // displacement slot of the positions read
     CVec pos, p_t, x_t, vrec, w, nrm, vc;
     const float *mag, *nz;
     Vec w_t, vc_t;
@@ -984,7 +976,7 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_vorticity_kernel(PostJvpArgs a
     PHX_MASK_LDS(a.s.grid);
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
     if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+    const bool masked = a.s.crowded[i] == 0u;
     const Step& s = a.s;
     const Float3 pi = load(a.pos, i), ti = load(a.p_t, i);
     const Float3 vi = load(a.vrec, i), vti = vrec_tangent(a, i);
@@ -1010,7 +1002,7 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_normal_kernel(PostJvpArgs a) {
     PHX_MASK_LDS(a.s.grid);
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
     if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+    const bool masked = a.s.crowded[i] == 0u;
     const Step& s = a.s;
     const Float3 pi = load(a.pos, i), ti = load(a.p_t, i);
     Float3 gt{0.0F, 0.0F, 0.0F};
@@ -1040,7 +1032,7 @@ __global__ void __launch_bounds__(kBlock) pbf_jvp_xsph_kernel(PostJvpArgs a) {
     PHX_MASK_LDS(a.s.grid);
     const uint32_t i = xcd_block() * kBlock + threadIdx.x;
     if (i >= a.s.n) return;
-    const bool masked = masks_apply(a.s.mv, a.slot, i);
+    const bool masked = a.s.crowded[i] == 0u;
     const Step& s = a.s;
     const CVec vct{a.vc_t.x, a.vc_t.y, a.vc_t.z};
     const Float3 pi = load(a.pos, i), ti = load(a.p_t, i);
@@ -1120,8 +1112,7 @@ namespace {
 // set's overflow word is raised.
 MaskView exact_view(const PbfCache& cache, uint32_t k, uint32_t n) {
     require(k <= cache.iterations, PHX_ERROR_INVALID_ARGUMENT, "exact mask set out of range");
-    return MaskView{cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n, cache.exact_flags.data() + k, n,
-                    0.0F, 1u, cache.crowded.data()};
+    return MaskView{cache.exact_masks.data() + static_cast<size_t>(k) * kStencil * n, n};
 }
 }  // namespace
 
@@ -1176,6 +1167,7 @@ void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.xsph.data(),
            dw_.confinement.data(),
            exact_view(cache, iterations, n),
+           cache.crowded.data(),
            cache.neighborhood.boundary(),
            kernel_,
            exact_mask_threshold(c.support_radius),
@@ -1198,13 +1190,12 @@ void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& c
         const CVec pos = it == 0u ? cache.xs.cview() : cache.positions.cview(it - 1u);
         const size_t off = static_cast<size_t>(it) * n;
         se.mv = exact_view(cache, it, n);
-        LambdaJvpArgs la{se, tp, it, pos, dw_.p_t[cur].cview(), cache.rho.data() + off, cache.den.data() + off,
+        LambdaJvpArgs la{se, tp, pos, dw_.p_t[cur].cview(), cache.rho.data() + off, cache.den.data() + off,
                          dw_.lambda_t.data()};
         pbf_jvp_lambda_kernel<<<blocks, kBlock, 0, stream_>>>(la);
         PHX_LAUNCH_CHECK();
         CorrectionJvpArgs ca{se,
                              tp,
-                             it,
                              pos,
                              dw_.p_t[cur].cview(),
                              cache.lambda.data() + off,
@@ -1217,7 +1208,6 @@ void PbfSolver::jvp_step(const phx_pbf_parameters& parameters, const PbfCache& c
     }
     PostJvpArgs post{};
     post.t = tp;
-    post.slot = iterations;
     post.pos = iterations == 0u ? cache.xs.cview() : cache.positions.cview(iterations - 1u);
     se.mv = exact_view(cache, iterations, n);
     post.s = se;
@@ -1276,6 +1266,7 @@ void PbfSolver::vjp_step(const phx_pbf_parameters& parameters, const PbfCache& c
            dw_.xsph.data(),
            dw_.confinement.data(),
            exact_view(cache, iterations, n),
+           cache.crowded.data(),
            cache.neighborhood.boundary(),
            kernel_,
            exact_mask_threshold(c.support_radius),

@@ -40,7 +40,6 @@ struct WcsphForceArgs {
     const float4* aux;  // density, p / rho^2, speed of sound, surface tension
     CVec u;
     const uint16_t* exact;
-    const uint32_t* flags;
     const uint32_t* perm;
     Vec next_x, next_v;
     uint8_t* collisions;  // optional (recorded step): box-collision bits of the integration
@@ -85,12 +84,11 @@ __global__ void __launch_bounds__(kGroupBlock) wcsph_force_kernel(WcsphForceArgs
     __shared__ GroupLds<G> lds;
     const uint32_t base = xcd_block() * kParticles;
     const uint32_t i = base + threadIdx.x % kParticles;
-    const bool usable = a.flags[kFlagOverflow] == 0u;
     uint32_t center = 0u;
     bool listed = false;
     if (i < a.n) {
         center = a.cell[i];
-        listed = usable && a.crowded[i] == 0u;
+        listed = a.crowded[i] == 0u;
     }
     const uint32_t w = base + threadIdx.x / G;
     const bool active = w < a.n;
@@ -156,7 +154,7 @@ __global__ void __launch_bounds__(kGroupBlock) wcsph_force_kernel(WcsphForceArgs
             if (active) group_walk_list<G, kSums>(row, count, w, fetch, pair, fold);
         });
     if (!active) return;
-    if (!usable || a.crowded[w] != 0u) {
+    if (a.crowded[w] != 0u) {
         int cx, cy, cz;
         cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
         group_walk_stencil<G, kSums>(
@@ -436,7 +434,6 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
     ma.exact = exact;
     ma.skin = masks_.skin_mask();
     ma.rho = cache.densities.data();
-    ma.flags = masks_.flags();
     ma.rest_density = rho0;
     ma.tait_exponent = tait;
     ma.pressures = cache.pressures.data();
@@ -460,7 +457,6 @@ void SphSolver::forward_wcsph(const phx_sph_state& state, const phx_control& con
     wa.aux = aux;
     wa.u = u_.cview();
     wa.exact = exact;
-    wa.flags = masks_.flags();
     wa.perm = cache.neighborhood.perm.data();
     wa.next_x = vec(next.particles.positions);
     wa.next_v = vec(next.particles.velocities);
@@ -553,7 +549,6 @@ void SphSolver::forward_pressure(const phx_sph_state& state, const phx_control& 
     ma.exact = masks_.exact();
     ma.skin = masks_.skin_mask();
     ma.rho = cache.densities.data();
-    ma.flags = masks_.flags();
     ma.crowded = masks_.crowded();
     ma.cell = masks_.cells();
     ma.exact_samples = exact_samples_.data();

@@ -82,7 +82,6 @@ struct MaskDensityArgs {
     float* rho;
     float* t_div;
     float* t_den;
-    uint32_t* flags;
     // rho0 (boundary terms), and the equation of state (WCSPH): p = EOS(rho),
     // aux = (rho, p / rho^2, c, sigma)
     const float* rest_density;
@@ -391,7 +390,7 @@ __device__ __forceinline__ bool projection_masked(const ProjectionArgs& a, uint3
     const bool moved_within = a.taint != nullptr
                                   ? a.taint[cell] != a.stamp
                                   : __uint_as_float(a.flags[kFlagDisplacement + a.slot]) <= a.limit2;
-    return a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u && moved_within;
+    return a.crowded[i] == 0u && moved_within;
 }
 
 // The pressure update of particle i from its predicted density rs; returns
@@ -442,7 +441,7 @@ __global__ void __launch_bounds__(kBlock) projection_kernel(ProjectionArgs a) {
     if (i < a.n) {
         const float4 topology = a.xm[i];
         const uint32_t center = a.cell[i];
-        const bool crowded = a.flags[kFlagOverflow] != 0u || a.crowded[i] != 0u;
+        const bool crowded = a.crowded[i] != 0u;
         const bool masked = projection_masked(a, i, center);
         const float4 self = a.xs[i];
         const Float3 ps = xyz(self);
@@ -491,14 +490,13 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
     if (tolerance && *a.cv.done != 0u) return;  // the phase ended at an earlier iteration
     const uint32_t base = xcd_block() * kParticles;
     const uint32_t i = base + threadIdx.x % kParticles;
-    const bool usable = a.flags[kFlagOverflow] == 0u;
     uint32_t center = 0u;
     bool listed = false, masked = false;
     Float3 expanded{0.0F, 0.0F, 0.0F};
     int cx = 0, cy = 0, cz = 0;
     if (i < a.n) {
         center = a.cell[i];
-        listed = usable && a.crowded[i] == 0u;
+        listed = a.crowded[i] == 0u;
         masked = projection_masked(a, i, center);
         if (listed && !masked) {  // moved past the skin: marked at the predicted positions below
             expanded = xyz(a.xs[i]);
@@ -544,7 +542,7 @@ __global__ void __launch_bounds__(kGroupBlock) projection_group_kernel(Projectio
         });
     double error = 0.0;
     if (active) {
-        if (!usable || a.crowded[w] != 0u) {
+        if (a.crowded[w] != 0u) {
             cell_coordinates(a.grid, a.cell[w], cx, cy, cz);
             group_walk_stencil<G, 1>(
                 a.grid, kSamples ? a.boundary.offsets : nullptr, cx, cy, cz, ~0u, w, group_row(lds),
@@ -694,7 +692,7 @@ __global__ void __launch_bounds__(kBlock) force_kernel(ForceArgs a) {
     const bool active = i < a.n;
     float moved2 = 0.0F;
     if (active) {
-        const bool masked = a.flags[kFlagOverflow] == 0u && a.crowded[i] == 0u;
+        const bool masked = a.crowded[i] == 0u;
         const float4 self = a.xm[i];
         const Float3 p = xyz(self);
         const float4 vm = a.vmu[i];
@@ -816,11 +814,10 @@ __global__ void __launch_bounds__(kGroupBlock) force_group_kernel(ForceArgs a) {
     const uint32_t base = xcd_block() * kParticles;
     const uint32_t i = base + threadIdx.x % kParticles;
     uint32_t center = 0u;
-    const bool usable = a.flags[kFlagOverflow] == 0u;
     bool listed = false;
     if (i < a.n) {
         center = a.cell[i];
-        listed = usable && a.crowded[i] == 0u;
+        listed = a.crowded[i] == 0u;
     }
     const uint32_t w = base + threadIdx.x / G;
     const bool active = w < a.n;
@@ -916,7 +913,7 @@ __global__ void __launch_bounds__(kGroupBlock) force_group_kernel(ForceArgs a) {
     float moved2 = 0.0F;
     if (active) {
         const uint32_t cell = a.cell[w];
-        if (!usable || a.crowded[w] != 0u) {
+        if (a.crowded[w] != 0u) {
             int cx, cy, cz;
             cell_coordinates(a.grid, cell, cx, cy, cz);
             group_walk_stencil<G, kSums>(

@@ -52,7 +52,7 @@ struct WcsphStep {
 };
 
 __device__ __forceinline__ MaskView exact_view(const WcsphStep& s) {
-    return MaskView{s.exact, s.flags, s.n, 0.0F, 0u, s.crowded};
+    return MaskView{s.exact, s.n};
 }
 // Whether particle i walks the step's exact masks (not crowded, no boundary samples).
 __device__ __forceinline__ bool exact_masked(const WcsphStep& s, uint32_t i) {

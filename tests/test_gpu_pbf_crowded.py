@@ -1,12 +1,11 @@
 """PBF with crowded cells on the GPU against the oracle.
 
-A particle whose 27 stencil cells include one of more than 16 particles walks
-the full stencil in every pass. A wave whose crowded particles all sit in one
-cell walks that stencil together: each lane loads one candidate of a run of 64
-and the candidates reach every lane from scalar registers, while each lane
-still adds its own terms in the reference order. The scene clumps a few
-hundred particles into single cells, so whole waves, waves that mix crowded
-and uncrowded lanes, and waves whose crowded lanes span two cells all occur.
+A particle whose 27 stencil cells include one of more than 16 particles has no
+masks: its group of lanes tests the stencil's candidates by distance, lists
+those near enough and walks the list, emptying it whenever it is full. The
+scene clumps a few hundred particles into single cells, so lists that fill
+several times, workgroups of crowded particles only, and workgroups that mix
+crowded and uncrowded ones all occur.
 Forward steps are bit-exact against the FP32 oracle (forward and
 differentiable mode, and in the batched engine), the VJP is within 1e-10 of
 the oracle's."""
@@ -55,7 +54,7 @@ def clumped_scene(seed=5):
 
 
 def test_clumps_fill_whole_waves():
-    """The scene has the cases the wave-shared walk distinguishes."""
+    """The scene has cells above 256 particles, above two waves and above the mask limit."""
     sc = clumped_scene()
     h = sc.domain.support_radius
     cells = np.floor(sc.positions / h).astype(np.int64)
