@@ -1,12 +1,12 @@
 """Autotuner of the batched PBF engine.
 
-Times a batch of scenes for each candidate setting the engine exposes (the
-neighbour-mask skin, which trades candidates per walk against passes that
-fall back to the full stencil, and replay of a captured substep against
-eager launches) and writes every timing and the fastest setting to a JSON
-file, which PbfBatch reads for its defaults (physica_amd/tuning/
-pbf_batch.json). The engine's results do not depend on these settings, so
-the tuner checks that every candidate ends in the same state bit for bit.
+Times a batch of scenes with replay of a captured substep and with eager
+launches and writes both timings and the faster setting to a JSON file, which
+PbfBatch reads for its defaults (physica_amd/tuning/pbf_batch.json). The
+engine's results do not depend on the settings, so the tuner checks that every
+candidate ends in the same state bit for bit. The mask skin is accepted by the
+engine but sizes nothing (its passes keep no skin masks), so one value is
+tried unless the caller names others.
 
     python -m physica_amd.autotune --out gpurun_out/pbf_batch.json
 """
@@ -25,7 +25,7 @@ from . import scenes
 from .batch import TUNING, PbfBatch
 from .particle import PBF
 
-SKINS = (0.1, 0.2, 0.3, 0.45, 0.6)
+SKINS = (0.3,)
 
 
 def tune(batch_scenes, steps=100, skins=SKINS, graphs=(True, False), device="cuda"):
