@@ -83,9 +83,9 @@ __device__ __forceinline__ bool skin_holds(const Step& s, uint32_t slot) {
 
 // The derivative passes serve each particle with a group of G lanes: with one
 // lane a particle they were a chain of 40 to 60 candidates, with few waves in
-// flight. 36,000 particles, us a pass before and now: pressure VJP 53 / 20 (with
-// the non-pressure terms 75 / 42; one Hessian product a pair for two, without
-// its divisions), density VJP 43 / 24, projection JVP 51 / 23, force JVP 31 / 16.
+// flight. 35,805 particles, us a pass before and now: pressure VJP 53 / 25 (with
+// the non-pressure terms 75 / 47; one Hessian product a pair for two, without
+// its divisions), density VJP 43 / 24, projection JVP 51 / 21, force JVP 31 / 16.
 
 // Lists the candidates of a workgroup's particles (base ..) for its groups:
 // the fluid particles in the masks of particle w (with exact those of the

@@ -39,7 +39,13 @@ constexpr int kWalkDepth = 2;
 // 419 / 278 / 194, 16,000 476 / 303 / 270, 32,000 432 / 297 / 346, 64,000
 // 458 / 370 / 501, 130,000 505 / 558 / 829, 260,000 710 / 897 / -; IISPH and
 // PCISPH cross at the same counts. From 400,000 four lanes are 6 % faster on
-// cubic lattices and 6 to 20 % slower on a dam break of 128 x 64 x 128.
+// cubic lattices and 6 to 20 % slower on a dam break of 128 x 64 x 128. These
+// scenes have no crowded cells, for which the rule has no term: a crowded lane
+// of the one-lane passes evaluates every candidate of its stencil while its
+// wave waits. On a lattice whose planes lie on cell borders, so that a few
+// cells hold 17 or 18 particles, one lane takes 1,900 us and four take 924 at
+// 103,823 particles (2,160 and 1,295 at 262,144; with the planes inside the
+// cells 437 and 440, 635 and 770).
 constexpr uint32_t kGroup16Particles = 20000;
 constexpr uint32_t kGroup4Particles = 90000;
 
