@@ -14,10 +14,11 @@
 // first pass at a set of positions (lambda, vorticity) scans the 27 cells and
 // writes the exact neighbour masks that the others at those positions walk.
 // Candidates are fetched as 16-byte records (position and mass, or velocity):
-// the passes keep the CU's address unit busy 80 % of the time, and a record
+// single floats kept the CU's address unit busy 80 % of the time, and a record
 // costs it about as much as one of the three to five single floats it
 // replaces (814,213 particles in 12 scenes: lambda 270 -> 176 us, correction
-// 147 -> 122, vorticity 306 -> 170, normal 118 -> 92, XSPH 151 -> 89).
+// 147 -> 122, vorticity 306 -> 170, normal 118 -> 92, XSPH 151 -> 89; with the
+// pair arithmetic of device_math.hpp 172, 102, 174, 78 and 78).
 // Per-particle sums run in the reference order, so each value is the IEEE
 // result of the reference expression.
 #include "pbf.hpp"
