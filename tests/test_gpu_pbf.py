@@ -77,8 +77,8 @@ def test_artificial_pressure_within_tolerance(gpu_device):
 @pytest.mark.parametrize("batched", [False, True])
 def test_masses_outside_the_quick_division(gpu_device, batched):
     """Masses and rest densities whose quotients the pair terms cannot take
-    from a reciprocal (the remainders underflow), then usual ones: bit-exact
-    steps, also right after each other."""
+    from a reciprocal (the remainders underflow), then usual ones, then the
+    first again: bit-exact steps, of a solver and of one batch's replays."""
     sc = scenes.pbf_dam_break(shape=(12, 12, 12))
     rng = np.random.default_rng(9)
     usual = dict(sc.parameters)
@@ -88,15 +88,16 @@ def test_masses_outside_the_quick_division(gpu_device, batched):
     tiny["relaxation"] = np.full(sc.count, 2.0**-34, np.float32)  # corrections of some 1e-3
     d = oracle.make_domain(sc.domain)
     u = np.zeros_like(sc.positions)
-    for parameters in (tiny, usual):
+    engine = PbfBatch([sc.domain], PBF.Configuration(2), use_graph=True, device=gpu_device)
+    state, control, params = engine.allocate_state(), engine.allocate_control(), engine.allocate_parameters()
+    for parameters in (tiny, usual, tiny):
         sc.parameters = parameters
         exp = oracle.pbf_step(d, 0, sc.positions, sc.velocities, u, parameters, 2)
         free = oracle.pbf_step(d, 0, sc.positions, sc.velocities, u, parameters, 0)
         assert np.abs(exp["positions"] - free["positions"]).max() > 1e-4
         if batched:
-            engine = PbfBatch([sc.domain], PBF.Configuration(2), device=gpu_device)
-            state, control, params = engine.allocate_state(), engine.allocate_control(), engine.allocate_parameters()
-            engine.upload([sc], state, params)
+            engine.upload([sc], state, params)  # into the arrays that the captured substep reads
+            state.particles.step_index = 0
             engine.run(state, control, params, 1)
             torch.cuda.synchronize()
             gx, gv = state.particles.positions.numpy(), state.particles.velocities.numpy()

@@ -82,3 +82,27 @@ def test_autograd_function_returns_chained_vjp(gpu_device):
         expected = ref_field.numpy()
         assert np.abs(got.cpu().numpy() - expected).max() <= 1e-5 * np.abs(expected).max()
     assert rollout.last_parameter_adjoint is not None
+
+
+def test_a_rollout_used_again_records_anew(gpu_device):
+    """The step caches of a store-all rollout are recorded over by its next
+    forward pass, or dropped for another solver's: each pass's gradient is that
+    of a rollout used once."""
+    sc, solver, state, control, params = setup(gpu_device)
+    other = setup(gpu_device)[1]
+    w = np.random.default_rng(2).normal(0, 1, size=(3, sc.count))
+    rollout = PbfRollout(solver, 5)
+    for used, kick in ((solver, 0.0), (solver, 0.3), (other, -0.2), (solver, 0.1)):
+        state.particles.velocities.upload(sc.velocities + np.float32(kick))
+        rollout.solver = used
+        grads = []
+        for r in (rollout, PbfRollout(used, 5)):
+            final = r.forward(state, control, params)
+            seed = used.allocate_state_adjoint()
+            seed.particles.positions.upload(w)
+            initial, control_adjoint, parameter_adjoint = r.backward(seed)
+            torch.cuda.synchronize()
+            grads.append((final.particles.positions.numpy(), initial.particles.velocities.numpy(),
+                          parameter_adjoint.relaxation.cpu().numpy(), control_adjoint.external_accelerations.numpy()))
+        for a, b in zip(*grads):
+            np.testing.assert_array_equal(a, b)
